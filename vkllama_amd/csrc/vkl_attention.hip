@@ -251,11 +251,16 @@ attn_prefill_kernel (const AttnArgs a)
     {
       // j: position in the XCD's queue.  Its 32 compute units take the first
       // 32 workgroups, then the next 32 beside them, and so on: every other
-      // such layer runs the tiles in the opposite order, so that a heavy tile
-      // and a light one share a compute unit.
-      const int j = b >> 3;
+      // such layer runs in the opposite order, so that a heavy tile and a
+      // light one share a compute unit.  (The order of the queue is reversed
+      // within the layer, the last of which may be shorter: whatever the
+      // number of tiles, every tile of every head has one place.)
+      int j = b >> 3;
+      const int queue = (a.H >> 3) * a.ntq, j0 = j & ~31;
+      if ((j >> 5) & 1)
+        j = j0 + min (queue, j0 + 32) - 1 - j;
       head = (b & 7) + 8 * (j / a.ntq);
-      qt = ((j >> 5) & 1) ? j % a.ntq : a.ntq - 1 - (j % a.ntq);
+      qt = a.ntq - 1 - (j % a.ntq);
     }
   else
     {

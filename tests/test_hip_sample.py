@@ -118,3 +118,29 @@ def test_arguments_are_checked(dev, logits):
     assert L.vkl_sample_f32(dl.ptr, 32000, 0, C.c_float(-1.0), 1, 0, None, tok.ptr, None, None, None, dev.stream) != 0
     assert L.vkl_sample_f32(dl.ptr, 32000, 0, C.c_float(1.5), 1, 0, None, tok.ptr, None, None, None, dev.stream) != 0
     assert L.vkl_sample_f32(None, 32000, 4, C.c_float(-1.0), 1, 0, None, tok.ptr, None, None, None, dev.stream) != 0
+
+
+@pytest.mark.parametrize("V", [1, 63, 32768, 32769, 70001])
+@pytest.mark.parametrize("k,p,spread", [(1, -1.0, 3.0), (256, -1.0, 3.0), (257, -1.0, 3.0), (40, -1.0, 0.0), (300, -1.0, 0.0),
+                                        (0, 0.95, 8.0), (0, 0.95, 0.5), (0, 0.6, 0.0)])
+def test_every_way_of_selection(dev, V, k, p, spread):
+    """Ranking by counting and radix selection, rows in registers and re-read, logits that are all equal (spread 0, but for
+    a few), top-p within the first 64 candidates and beyond them."""
+    rng = np.random.default_rng(V + k)
+    x = (rng.standard_normal(V) * spread).astype(np.float32)
+    x += np.float32(0)                             # no negative zeros, which rank below zero
+    x[::max(V // 7, 1)] += np.float32(0.5)
+    tok, ids, probs = run(dev, x, k, p, 11, 5)
+    order = ranked(x)
+    if p >= 0:
+        # prefix of the ranking whose mass reaches p; sums of 32-bit shares, each off by about 1e-7 of itself
+        e = np.exp((x[order] - x[order[0]]).astype(np.float64))
+        before = np.concatenate(([0.0], np.cumsum(e)[:-1])) / e.sum()
+        lo, hi = (min(max(int(np.sum(before < p + d)), 1), 1024) for d in (-1e-4, 1e-4))
+        assert lo <= ids.size <= min(hi, V)
+    else:
+        assert ids.size == min(k, V)
+    assert np.array_equal(ids, order[:ids.size])
+    assert np.allclose(probs, softmax_seq(x[ids]), rtol=1e-4, atol=1e-12)
+    hit = np.nonzero(np.cumsum(probs, dtype=np.float32) > uniform01(11, 5))[0]
+    assert tok == ids[hit[0] if hit.size else ids.size - 1]

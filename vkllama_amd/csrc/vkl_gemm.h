@@ -65,6 +65,9 @@ struct GemmSegArgs : GemmArgs
 // the fp32 product (vkl_gemm_f32.hip) and the bf16 one (vkl_gemm_wide.hip)
 int gemm_f32_launch (const GemmSegArgs &a, hipStream_t s);
 int gemm_wide_bf16_launch (const GemmSegArgs &a, hipStream_t s);
+// the fp32 product on the bf16 matrix cores; false (nothing launched) if there is no
+// scratch for it
+bool gemm_wide_f32_launch (const GemmSegArgs &a, hipStream_t s, int &err);
 
 // smallest M for which the matrix-core kernels beat one weight-streaming pass
 // per token row (measured on the 7B shapes): Q8_0 weights, fp16 weights, and

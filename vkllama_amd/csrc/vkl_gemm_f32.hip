@@ -1,6 +1,8 @@
 // y[M,N] = x[M,K] W[N,K]^T in 32-bit: fp32 activations, bf16 weights (exact as
 // fp32), products and sums on v_mfma_f32_32x32x2_f32, which multiplies and adds
-// in full fp32.  The output columns fall into segments (GemmSegArgs).
+// in full fp32: the short products, for which the planes of vkl_gemm_wide.hip do
+// not pay, and those without scratch.  The output columns fall into segments
+// (GemmSegArgs).
 //
 // Workgroup = 4 waves on a 64 x 64 output tile, each wave one 32 x 32 block;
 // k-steps of 32 through LDS, the next step's loads in flight in registers.
@@ -73,6 +75,9 @@ gemm_f32_kernel (const GemmSegArgs a)
 int
 gemm_f32_launch (const GemmSegArgs &a, hipStream_t s)
 {
+  int err = 0;
+  if (gemm_wide_f32_launch (a, s, err))
+    return err;
   const int tn = (a.N + FT - 1) / FT, tm = (a.M + FT - 1) / FT;
   if (tm > 65535)
     return (int)hipErrorInvalidValue;

@@ -192,7 +192,9 @@ wide_lds_f16 ()
 
 // BM: token rows of a tile, 256 or (where 256-row tiles would be too few to
 // occupy the compute units) 128, i.e. 64 x 64 per wave.
-template <int BM, bool UPGATE, class Args = GemmArgs>
+// PLANES > 1: x holds PLANES values for every weight, in blocks of 64 (one k-step of
+// each plane in turn): see the 32-bit product below.
+template <int BM, bool UPGATE, class Args = GemmArgs, int PLANES = 1>
 __global__ __launch_bounds__ (WWAVES * 64) void
 gemm_wide_f16_kernel (const Args a, int tiles_m, int tiles_n, int per_xcd, int vec, int ksplit, float *ws)
 {
@@ -245,7 +247,7 @@ gemm_wide_f16_kernel (const Args a, int tiles_m, int tiles_n, int per_xcd, int v
       const int mat = UPGATE ? v >> 6 : zmat;
       const int n = min (UPGATE ? n0 + (v & 63) : n0 + v, a.N - 1);
       const uint16_t *w = mat == 0 ? a.wh[0] : (mat == 1 ? a.wh[1] : a.wh[2]);
-      src[i] = w + (size_t)n * a.ws + chunk * 8 + (size_t)kbase * WBK;
+      src[i] = w + (size_t)n * a.ws + chunk * 8 + (PLANES > 1 ? 0 : (size_t)kbase * WBK);
     }
 
   // fragment reads: lane l holds row l%32 of a 32-row block, k = 16 ks + 8 (l/32) .. +7
@@ -270,11 +272,12 @@ gemm_wide_f16_kernel (const Args a, int tiles_m, int tiles_n, int per_xcd, int v
         acc[i][jn][q] = 0.f;
 
   auto issue_part = [&] (int kt, int st, int i0, int i1) {
+    const int kw = PLANES > 1 ? (kbase + kt) / PLANES : kt; // k-step of the weights
 #pragma unroll
     for (int i = i0; i < i1; ++i)
       {
         const int g = i < AG ? wave + WWAVES * i : BM / 8 + wave + WWAVES * (i - AG);
-        __builtin_amdgcn_global_load_lds ((const VKL_GLOBAL void *)(src[i] + (size_t)kt * WBK),
+        __builtin_amdgcn_global_load_lds ((const VKL_GLOBAL void *)(src[i] + (size_t)(i < AG ? kt : kw) * WBK),
                                           (VKL_LDS void *)(wide_lds + st * STAGE_BYTES + g * 1024), 16, 0, 0);
       }
   };
@@ -841,7 +844,7 @@ wide_reduce_seg_kernel (const GemmSegArgs a, const float *ws, int parts)
 // allowed and, where the tiles are few, up to 16 parts of at least 4 k-steps:
 // with few token rows the workgroups exist to stream the weights.
 WidePlan
-wide_plan_bf16 (const GemmSegArgs &a)
+wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
 {
   WidePlan best = { 0, 1 };
   double best_cost = 0;
@@ -852,7 +855,7 @@ wide_plan_bf16 (const GemmSegArgs &a)
         if (a.M < bm && bm > 128)
           continue;
         if (ks > 1
-            && (nk / ks < 4 || (size_t)ks * a.M * a.N * sizeof (float) > gemm_stream_workspace_bytes ()))
+            && (nk / ks < 4 || (size_t)ks * a.M * a.N * sizeof (float) > scratch))
           continue;
         const long groups = (long)((a.M + bm - 1) / bm) * ((a.N + WBN - 1) / WBN) * ks;
         const double round = (bm == WBM ? 0.95 : 0.55) * nk / ks + (bm == WBM ? 8 : 6);
@@ -864,17 +867,17 @@ wide_plan_bf16 (const GemmSegArgs &a)
   return best;
 }
 
-template <int BM>
+// ws: scratch for the parts of a split k range (null: the stream's)
+template <int BM, int PLANES = 1>
 int
-launch_wide_bf16 (const GemmSegArgs &a, int ksplit, hipStream_t s)
+launch_wide_bf16 (const GemmSegArgs &a, int ksplit, float *ws, hipStream_t s)
 {
   static LdsLimit limit;
   constexpr size_t lds = wide_lds_f16<BM> ();
-  const auto kernel = gemm_wide_f16_kernel<BM, false, GemmSegArgs>;
+  const auto kernel = gemm_wide_f16_kernel<BM, false, GemmSegArgs, PLANES>;
   if (int e = limit.raise ((const void *)kernel, lds))
     return e;
-  float *ws = nullptr;
-  if (ksplit > 1 && !(ws = gemm_stream_workspace (s)))
+  if (ksplit > 1 && !ws && !(ws = gemm_stream_workspace (s)))
     ksplit = 1;
   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + WBN - 1) / WBN;
   const int per_xcd = (tiles_m * tiles_n * ksplit + 7) / 8;
@@ -886,13 +889,120 @@ launch_wide_bf16 (const GemmSegArgs &a, int ksplit, hipStream_t s)
     }
   return (int)hipGetLastError ();
 }
+
+// ---------------------------------------------------------------------------
+// 32-bit activations on the bf16 matrix cores
+// ---------------------------------------------------------------------------
+// An fp32 value is the sum of three bf16 values (its 24 significant bits, eight at
+// a time), and a product of two bf16 values is exact in fp32: x W^T is the product
+// of three planes of x with the same weights, summed in the same fp32 accumulator,
+// without any rounding that the 32-bit matrix instructions would not do (they add
+// one product at a time, these sixteen before they round).  The matrix cores do
+// three such products in a fifth of the time of one in fp32.  Against 64 bits the
+// result is closer than that of the 32-bit instructions: relative error 2e-7 to 7e-7
+// instead of 8e-7 to 1.4e-6 over K = 2048 to 5504 (1.4e-7 / 4e-7 at K = 512).  Two
+// limits: values below 1e-33 lose their last bits (planes below the smallest normal
+// bf16 are taken as zero), and an infinite weight meets zeros in the lower planes.
+//
+// Planes lie in blocks of 64 columns, [plane 0 | plane 1 | plane 2] of a block next
+// to each other, so that the wide kernel walks them as one row of 3 K values and
+// takes every k-step of the weights three times (the second and third time from
+// the L2).
+constexpr int kPlanes = 3;
+
+__global__ __launch_bounds__ (256) void
+split_planes_kernel (const float *x, size_t xs, int M, int K, uint16_t *out)
+{
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const int k8 = K / 8;
+  if (i >= (size_t)M * k8)
+    return;
+  const int m = (int)(i / k8), c = (int)(i % k8) * 8;
+  const float *src = x + (size_t)m * xs + c;
+  const uint4 w0 = ldg4 (src), w1 = ldg4 (src + 4);
+  const uint32_t in[8] = { w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w };
+  uint32_t p[kPlanes][8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    {
+      // truncation: no plane overflows, and each remainder is exact.  Infinities and
+      // NaN go into the first plane alone.
+      const bool finite = (in[e] & 0x7f800000u) != 0x7f800000u;
+      const float v = __uint_as_float (in[e]);
+      p[0][e] = finite ? in[e] >> 16 : (uint32_t)f2bf (v);
+      const float r = finite ? v - __uint_as_float (in[e] & 0xffff0000u) : 0.f;
+      p[1][e] = __float_as_uint (r) >> 16;
+      p[2][e] = __float_as_uint (r - __uint_as_float (__float_as_uint (r) & 0xffff0000u)) >> 16;
+    }
+  uint16_t *dst = out + (size_t)m * kPlanes * K + (size_t)(c / WBK) * kPlanes * WBK + c % WBK;
+#pragma unroll
+  for (int q = 0; q < kPlanes; ++q)
+    {
+      vkl_u32x4 pk;
+      pk.x = p[q][0] | (p[q][1] << 16), pk.y = p[q][2] | (p[q][3] << 16);
+      pk.z = p[q][4] | (p[q][5] << 16), pk.w = p[q][6] | (p[q][7] << 16);
+      *(VKL_GLOBAL vkl_u32x4 *)(dst + q * WBK) = pk;
+    }
+}
 } // namespace
 
 int
 gemm_wide_bf16_launch (const GemmSegArgs &a, hipStream_t s)
 {
-  const WidePlan p = wide_plan_bf16 (a);
-  return p.bm == WBM ? launch_wide_bf16<WBM> (a, p.ksplit, s) : launch_wide_bf16<128> (a, p.ksplit, s);
+  const WidePlan p = wide_plan_bf16 (a, gemm_stream_workspace_bytes ());
+  return p.bm == WBM ? launch_wide_bf16<WBM> (a, p.ksplit, nullptr, s) : launch_wide_bf16<128> (a, p.ksplit, nullptr, s);
+}
+
+bool
+gemm_wide_f32_launch (const GemmSegArgs &a, hipStream_t s, int &err)
+{
+  // Short rows of few values are over in the time of two more launches.  Measured, us,
+  // 32-bit instructions / planes: K = 256, N = 2048, 300 rows 10 / 16, 4000 rows 48 / 36;
+  // K = 512, N = 512, 1000 rows 15.5 / 20; K = 768, N = 128, 1 row 20 / 13; K = 2048,
+  // N = 2048, 1 row 47 / 14, 2000 rows 162 / 65; K = 2048, N = 8064, 300 rows 121 / 51;
+  // K = 5504, N = 2048, 300 rows 161 / 43; K = 4096, N = 11008, 2000 rows 1530 / 628.
+  if (a.K <= 512 && (size_t)a.M * a.N * a.K <= (size_t)1 << 30)
+    return false;
+  // nothing is allocated while the stream is captured
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing (s, &capture) != hipSuccess)
+    {
+      (void)hipGetLastError (); // (the default stream while another one is captured)
+      return false;
+    }
+  if (capture != hipStreamCaptureStatusNone)
+    return false;
+  // the planes of as many rows as half of the scratch holds at a time, the parts of
+  // a split k range behind them
+  const size_t row = (size_t)kPlanes * a.K * sizeof (uint16_t), half = gemm_stream_workspace_bytes () / 2;
+  const size_t most = half / row;
+  const int rows = most >= (size_t)a.M ? a.M : (int)(most / WBM * WBM);
+  float *ws = rows > 0 ? gemm_stream_workspace (s) : nullptr;
+  if (!ws)
+    return false;
+  for (int m0 = 0; m0 < a.M; m0 += rows)
+    {
+      GemmSegArgs b = a;
+      b.M = a.M - m0 < rows ? a.M - m0 : rows;
+      const size_t total = (size_t)b.M * (a.K / 8);
+      split_planes_kernel<<<dim3 ((unsigned)((total + 255) / 256)), dim3 (256), 0, s>>> (a.xf + (size_t)m0 * a.xs, a.xs, b.M, a.K,
+                                                                                         (uint16_t *)ws);
+      b.x = (const uint16_t *)ws, b.xf = nullptr;
+      b.K = kPlanes * a.K, b.xs = (size_t)b.K;
+      for (int i = 0; i < a.nseg; ++i)
+        {
+          b.seg[i].y = (char *)a.seg[i].y + (size_t)m0 * a.seg[i].ys * (a.seg[i].f32 ? 4 : 2);
+          if (a.seg[i].residual)
+            b.seg[i].residual = a.seg[i].residual + (size_t)m0 * a.seg[i].ys;
+        }
+      const WidePlan p = wide_plan_bf16 (b, half);
+      float *parts = ws + half / sizeof (float);
+      err = p.bm == WBM ? launch_wide_bf16<WBM, kPlanes> (b, p.ksplit, parts, s)
+                        : launch_wide_bf16<128, kPlanes> (b, p.ksplit, parts, s);
+      if (err)
+        return true;
+    }
+  return true;
 }
 } // namespace vkl
 

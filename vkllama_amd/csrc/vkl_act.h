@@ -21,5 +21,29 @@ activate (int act, float v)
     return 0.5f * v * (1.0f + erff (v * 0.70710678118654752440f));
   return v;
 }
+
+// the same for eight, with one look at `act`
+__device__ __forceinline__ void
+activate8 (int act, float (&v)[8])
+{
+  if (act == VKL_ACT_SILU)
+    {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        v[e] = activate (VKL_ACT_SILU, v[e]);
+    }
+  else if (act == VKL_ACT_RELU2)
+    {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        v[e] = activate (VKL_ACT_RELU2, v[e]);
+    }
+  else if (act == VKL_ACT_GELU)
+    {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        v[e] = activate (VKL_ACT_GELU, v[e]);
+    }
+}
 } // namespace vkl
 #endif

@@ -65,6 +65,81 @@ template <> struct WideElem<GemmSegArgs>
   }
 };
 
+// Where a workgroup's output tile lies
+struct WidePlace
+{
+  int m0, tn, zmat, ks; // first token row, tile of weight rows, matrix, part of the k range
+};
+enum WideKind
+{
+  WIDE_NONE,
+  WIDE_TILE,
+  WIDE_HALF // of half the token rows
+};
+
+// The tiles of a launch, token-row tile fastest, then weight tile, matrix, part of the k
+// range.  Workgroups go to the XCDs in turn: each XCD gets a contiguous range of tiles,
+// so the weight tiles that they share stay in its L2.
+//
+// Tiles beyond the last whole round over the 256 compute units are cut in two where they
+// fill at most half of a round: a round of 128-row tiles takes 0.6 of one of 256-row
+// tiles.  Measured, us whole / cut: Q8_0 at 2048 rows 5120 x 5120 (1.25 rounds) 199 / 173,
+// 5120 x 13824 506 / 429, at 3967 rows (2.5 rounds) 847 / 803, up/gate 13824 x 5120 (13.5)
+// 1597 / 1556, at 512 rows up/gate 11008 x 4096 (1.34) 160 / 136; bf16 at 2048 rows 12544 x
+// 4096 (3.06) 223 / 215.
+struct WideGrid
+{
+  int tiles_m, tiles_n, nmat, ksplit;
+  int whole; // tiles that are not cut
+
+  static constexpr int kUnits = 256;
+  __host__ __device__ int
+  tiles () const
+  {
+    return tiles_m * tiles_n * nmat * ksplit;
+  }
+  __host__ WideGrid (int tm, int tn, int mats, int parts, bool cut)
+      : tiles_m (tm), tiles_n (tn), nmat (mats), ksplit (parts)
+  {
+    const int rest = tiles () % kUnits;
+    whole = cut && rest > 0 && rest <= kUnits / 2 ? tiles () - rest : tiles ();
+  }
+  // workgroups to launch: multiples of 8 of either kind
+  __host__ __device__ int
+  whole_groups () const
+  {
+    return (whole + 7) / 8 * 8;
+  }
+  __host__ int
+  groups () const
+  {
+    return whole_groups () + (2 * (tiles () - whole) + 7) / 8 * 8;
+  }
+  template <int BM>
+  __device__ __forceinline__ WideKind
+  place (int M, WidePlace &at) const
+  {
+    const int first = whole_groups (), id = (int)blockIdx.x;
+    const bool cut = id >= first;
+    const int g = cut ? id - first : id, count = cut ? 2 * (tiles () - whole) : whole;
+    const int per_xcd = (count + 7) / 8, j = g >> 3;
+    const int i = (g & 7) * per_xcd + j;
+    if (j >= per_xcd || i >= count)
+      return WIDE_NONE;
+    int t = cut ? whole + (i >> 1) : i;
+    const int tm = t % tiles_m;
+    t /= tiles_m;
+    at.tn = t % tiles_n;
+    t /= tiles_n;
+    at.zmat = t % nmat;
+    at.ks = t / nmat;
+    at.m0 = tm * BM + (cut ? (i & 1) * (BM / 2) : 0);
+    if (at.m0 >= M)
+      return WIDE_NONE; // the empty half of the last tile
+    return cut ? WIDE_HALF : WIDE_TILE;
+  }
+};
+
 // Issue order of one quarter of a k-step: after product Q one fragment read
 // (the first NR products) and an even share of the quarter's LQ loads.
 template <int Q, int NP, int NR, int LQ> struct WideOrder
@@ -88,60 +163,224 @@ template <int V> struct WideInt
   static constexpr int value = V;
 };
 
-// Epilogue through LDS (the k loop's stages are free by then): every wave parks
-// its 128 x 64 fp32 block in a region of its own, then walks it row-wise so
-// that a lane handles 8 neighbouring columns: 16-byte loads and stores, whole
-// cache lines per row, and a short loop instead of 128 unrolled elements.
-// Accumulator register q of lane l is row 8 (q/4) + 4 (l/32) + q%4, column
-// l%32 of its 32 x 32 block.
+// The products are formed transposed (the weights are the first operand): of a 32 x 32
+// block lane l holds token row l%32, and register q output column 8 (q/4) + 4 (l/32) +
+// q%4.  After exchanging half waves between the registers of two groups of four
+// (v_permlane32_swap) a lane has eight neighbouring columns of its row.
+//
+// The epilogue takes that straight from the registers where it is simple: a wave's
+// columns all there, in one segment, vector stores, nothing but an optional residual (or
+// SiLU of the fused pair) on the way.  Everything else is parked in LDS (the k loop's
+// stages are free by then) and walked row-wise in a short loop, eight neighbouring
+// columns per lane.  Both are about latency and instruction fetch, with one wave per SIMD
+// and code that runs once: the loop took 15 thousand cycles for a 256 x 128 tile (26 with
+// segments) where the k loop takes 84 at K = 4096, and all cases unrolled as much.
+// Straight, us per product at 2048 rows before / after: 4096 x 4096 fp16 71 / 66, bf16
+// 69 / 60; bf16 8064 x 2048 82 / 63, 11008 x 4096 193 / 165; at 300 rows 8064 x 2048 21 / 16.
 constexpr int kWideParkLd = 68; // floats per parked row: 16-byte aligned, rows 4 banks apart
 
-template <bool UPGATE, int TM, class Args>
+// x, y -> the lower halves of both, the upper halves of both
 __device__ __forceinline__ void
-wide_epilogue (const Args &a, const float16v (&acc)[TM][WTN], uint8_t *wide_lds, int wave, int lane,
-               int m0, int n0, int zmat, int vec, float *part)
+half_swap (float x, float y, float &lo, float &hi)
 {
-  // waves are numbered row block first: wave = 2 wm + wn, TM x 32 rows by 64 columns each
-  constexpr int ROWS = TM * 32;
-  const int wm = wave >> 1, wn = wave & 1;
-  __builtin_amdgcn_s_barrier (); // every wave has read its last fragments
-  constexpr int LD = kWideParkLd;
-  float *park = (float *)(wide_lds + wave * (ROWS * LD * 4));
+  const auto r = __builtin_amdgcn_permlane32_swap (__float_as_uint (x), __float_as_uint (y), false, false);
+  lo = __uint_as_float (r[0]), hi = __uint_as_float (r[1]);
+}
+
+// Eight values of a simple epilogue
+template <bool UPGATE, class Args> struct WideSimple;
+
+template <bool UPGATE> struct WideSimple<UPGATE, GemmArgs>
+{
+  static constexpr int NR = 1; // 16-byte words of a residual
+  const uint16_t *r;
+  uint16_t *y;
+  size_t ys;
+  bool ok;
+
+  // ncol: first of the wave's `n` columns
+  __device__ __forceinline__
+  WideSimple (const GemmArgs &a, int ncol, int n, int zmat, int vec, const float *part)
   {
-    float *pl = park + (lane >> 5) * 4 * LD + (lane & 31);
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int jn = 0; jn < WTN; ++jn)
-#pragma unroll
-        for (int q = 0; q < 16; ++q)
-          pl[(i * 32 + (q >> 2) * 8 + (q & 3)) * LD + jn * 32] = acc[i][jn][q];
+    ok = vec && !part && ncol + n <= a.N
+         && (UPGATE || a.nmat != 1 || (a.scale == 1.f && a.bias == 0.f && a.act == 0 && !a.y32));
+    y = (UPGATE ? a.y[0] : pick3 (a.y[0], a.y[1], a.y[2], zmat)) + ncol, ys = a.ys;
+    r = !UPGATE && a.nmat == 1 && a.residual ? a.residual + ncol : nullptr;
   }
-  // (a wave reads back only what it wrote itself: no barrier)
-  constexpr int CPR = UPGATE ? 4 : 8;   // lanes per row
-  constexpr int RPI = 64 / CPR;         // rows per iteration
-  const int er = lane / CPR, ec = (lane % CPR) * 8;
-  const int ncol0 = n0 + (UPGATE ? wn * 32 : wn * 64) + ec;
-  for (int it = 0; it < ROWS / RPI; ++it)
+  __device__ __forceinline__ void
+  request (size_t m, int col, uint4 (&w)[NR]) const
+  {
+    w[0] = ldg4 (r + m * ys + col);
+  }
+  __device__ __forceinline__ void
+  store (size_t m, int col, const float (&v)[8], const float (&g)[8], const uint4 *w) const
+  {
+    uint16_t h[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      h[e] = f2h (UPGATE ? silu (g[e]) * v[e] : v[e]);
+    if (w)
+      {
+        const uint32_t rw[4] = { w->x, w->y, w->z, w->w };
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          h[e] = f2h (h2f (h[e]) + h2f ((uint16_t)(rw[e >> 1] >> ((e & 1) * 16))));
+      }
+    vkl_u32x4 pk;
+    pk.x = h[0] | ((uint32_t)h[1] << 16), pk.y = h[2] | ((uint32_t)h[3] << 16);
+    pk.z = h[4] | ((uint32_t)h[5] << 16), pk.w = h[6] | ((uint32_t)h[7] << 16);
+    *(VKL_GLOBAL vkl_u32x4 *)(y + m * ys + col) = pk;
+  }
+};
+
+template <bool UPGATE> struct WideSimple<UPGATE, GemmSegArgs>
+{
+  static constexpr int NR = 2;
+  const float *r;
+  char *y;
+  size_t ys;
+  int f32, relu2;
+  bool ok;
+
+  __device__ __forceinline__
+  WideSimple (const GemmSegArgs &a, int ncol, int n, int, int, const float *part)
+  {
+    const SegCol c = seg_col (a, ncol); // (ncol is the same in all lanes)
+    ok = !part && ncol + n <= a.N && c.whole && n <= c.n && c.cap <= 0.f
+         && (c.act == VKL_ACT_NONE || c.act == VKL_ACT_RELU2);
+    y = c.y, ys = c.ys, r = c.r, f32 = c.f32, relu2 = c.act == VKL_ACT_RELU2;
+  }
+  __device__ __forceinline__ void
+  request (size_t m, int col, uint4 (&w)[NR]) const
+  {
+    w[0] = ldg4 (r + m * ys + col), w[1] = ldg4 (r + m * ys + col + 4);
+  }
+  __device__ __forceinline__ void
+  store (size_t m, int col, float (&v)[8], const float (&)[8], const uint4 *w) const
+  {
+    typedef float f32x4 __attribute__ ((ext_vector_type (4)));
+    if (relu2)
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        v[e] = activate (VKL_ACT_RELU2, v[e]);
+    if (f32)
+      {
+        f32x4 w0 = { v[0], v[1], v[2], v[3] }, w1 = { v[4], v[5], v[6], v[7] };
+        if (w)
+          w0 += __builtin_bit_cast (f32x4, w[0]), w1 += __builtin_bit_cast (f32x4, w[1]);
+        float *o = (float *)y + m * ys + col;
+        *(VKL_GLOBAL f32x4 *)o = w0;
+        *(VKL_GLOBAL f32x4 *)(o + 4) = w1;
+      }
+    else
+      {
+        vkl_u32x4 pk;
+        pk.x = f2bf (v[0]) | ((uint32_t)f2bf (v[1]) << 16), pk.y = f2bf (v[2]) | ((uint32_t)f2bf (v[3]) << 16);
+        pk.z = f2bf (v[4]) | ((uint32_t)f2bf (v[5]) << 16), pk.w = f2bf (v[6]) | ((uint32_t)f2bf (v[7]) << 16);
+        *(VKL_GLOBAL vkl_u32x4 *)((uint16_t *)y + m * ys + col) = pk;
+      }
+  }
+};
+
+// TN: 32-column accumulators of a wave, of the fused pair the first half up, the second
+// gate; mrow, ncol: the first row and output column of the wave's block
+template <bool UPGATE, int TM, int TN, class Args>
+__device__ __forceinline__ void
+wide_epilogue (const Args &a, const float16v (&acc)[TM][TN], uint8_t *wide_lds, int wave, int lane, int mrow, int ncol,
+               int zmat, int vec, float *part)
+{
+  constexpr int NB = UPGATE ? TN / 2 : TN; // blocks of 32 output columns
+  const WideSimple<UPGATE, Args> simple (a, ncol, NB * 32, zmat, vec, part);
+  if (simple.ok)
     {
-      const int row = it * RPI + er;
-      const float4 p0 = *(const float4 *)(park + row * LD + ec);
-      const float4 p1 = *(const float4 *)(park + row * LD + ec + 4);
-      float v[8] = { p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w };
-      float g[8] = { 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f };
-      if (UPGATE)
+      const int m0 = mrow + (lane & 31);
+      auto walk = [&] (auto with) {
+        constexpr bool RES = decltype (with)::value != 0;
+        constexpr int NR = WideSimple<UPGATE, Args>::NR;
+#pragma unroll
+        for (int jn = 0; jn < NB; ++jn)
+          {
+            uint4 res[TM][2][NR];
+            if (RES)
+#pragma unroll
+              for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int p = 0; p < 2; ++p)
+                  simple.request ((size_t)min (m0 + i * 32, a.M - 1), jn * 32 + p * 16 + (lane >> 5) * 8, res[i][p]);
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+              for (int p = 0; p < 2; ++p)
+                {
+                  float v[8], g[8];
+#pragma unroll
+                  for (int e = 0; e < 4; ++e)
+                    {
+                      half_swap (acc[i][jn][8 * p + e], acc[i][jn][8 * p + 4 + e], v[e], v[4 + e]);
+                      g[e] = g[4 + e] = 0.f;
+                      if (UPGATE)
+                        half_swap (acc[i][NB + jn][8 * p + e], acc[i][NB + jn][8 * p + 4 + e], g[e], g[4 + e]);
+                    }
+                  if (m0 + i * 32 < a.M)
+                    simple.store ((size_t)(m0 + i * 32), jn * 32 + p * 16 + (lane >> 5) * 8, v, g, RES ? res[i][p] : nullptr);
+                }
+          }
+      };
+      if (simple.r)
+        walk (WideInt<1> ());
+      else
+        walk (WideInt<0> ());
+      return;
+    }
+  // through LDS, 64 accumulator columns at a time
+  constexpr int ROWS = TM * 32, LD = kWideParkLd;
+  float *park = (float *)(wide_lds + wave * (ROWS * LD * 4));
+  __builtin_amdgcn_s_barrier (); // every wave has read its last fragments
+#pragma unroll
+  for (int half = 0; half < TN / 2; ++half)
+    {
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
         {
-          const float4 g0 = *(const float4 *)(park + row * LD + 32 + ec);
-          const float4 g1 = *(const float4 *)(park + row * LD + 32 + ec + 4);
-          g[0] = g0.x, g[1] = g0.y, g[2] = g0.z, g[3] = g0.w, g[4] = g1.x, g[5] = g1.y, g[6] = g1.z, g[7] = g1.w;
+          // of the fused pair a block of up, then its gate
+          const int jn = UPGATE ? c * NB + half : 2 * half + c;
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int q = 0; q < 16; q += 4)
+              *(float4 *)(park + (i * 32 + (lane & 31)) * LD + c * 32 + 2 * q + 4 * (lane >> 5))
+                  = make_float4 (acc[i][jn][q], acc[i][jn][q + 1], acc[i][jn][q + 2], acc[i][jn][q + 3]);
         }
-      gemm_finish8<UPGATE> (a, v, g, m0 + wm * ROWS + row, ncol0, zmat, vec, part);
+      // (a wave reads back only what it wrote itself: no barrier)
+      constexpr int CPR = UPGATE ? 4 : 8;   // lanes per row
+      constexpr int RPI = 64 / CPR;         // rows per iteration
+      const int er = lane / CPR, ec = (lane % CPR) * 8;
+      const FinishRows<UPGATE, Args> fin (a, ncol + half * (UPGATE ? 32 : 64) + ec, zmat, vec, part);
+      for (int it = 0; it < ROWS / RPI; ++it)
+        {
+          const int row = it * RPI + er;
+          uint4 res[2];
+          fin.request (mrow + row, res);
+          const float *pr = park + row * LD + ec;
+          const float4 p0 = *(const float4 *)pr, p1 = *(const float4 *)(pr + 4);
+          float v[8] = { p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w };
+          float g[8] = { 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f };
+          if (UPGATE)
+            {
+              const float4 g0 = *(const float4 *)(pr + 32), g1 = *(const float4 *)(pr + 36);
+              g[0] = g0.x, g[1] = g0.y, g[2] = g0.z, g[3] = g0.w, g[4] = g1.x, g[5] = g1.y, g[6] = g1.z, g[7] = g1.w;
+            }
+          fin.store (mrow + row, v, g, res);
+        }
     }
 }
 
-// The same for waves in a 2 x 4 grid (TM x 32 rows by 32 columns each; of the
-// fused pair the waves 0, 1 of a row block hold up, 2, 3 gate): the whole
-// BM x 128 tile is parked, and after a barrier all threads walk it row-wise.
+// Epilogue through LDS (the k loop's stages are free by then) of the kernel for Q8_0
+// weights, eight waves in a 2 x 4 grid (TM x 32 rows by 32 columns each; of the fused
+// pair the waves 0, 1 of a row block hold up, 2, 3 gate): the BM x 128 tile is parked, and
+// after a barrier all threads walk it row-wise, eight neighbouring columns per lane.
+// Accumulator register q of lane l is row 8 (q/4) + 4 (l/32) + q%4, column l%32 of its
+// 32 x 32 block.
 constexpr int kWideTileLd = 132;
 
 template <int BM, bool UPGATE, int TM>
@@ -194,9 +433,9 @@ wide_lds_f16 ()
 // occupy the compute units) 128, i.e. 64 x 64 per wave.
 // PLANES > 1: x holds PLANES values for every weight, in blocks of 64 (one k-step of
 // each plane in turn): see the 32-bit product below.
-template <int BM, bool UPGATE, class Args = GemmArgs, int PLANES = 1>
-__global__ __launch_bounds__ (WWAVES * 64) void
-gemm_wide_f16_kernel (const Args a, int tiles_m, int tiles_n, int per_xcd, int vec, int ksplit, float *ws)
+template <int BM, bool UPGATE, class Args, int PLANES>
+__device__ __forceinline__ void
+wide_f16_tile (const Args &a, const WidePlace &at, int vec, int ksplit, float *ws)
 {
   typedef typename WideElem<Args>::v8 v8;
   constexpr int TM = BM / 2 / 32;                    // 32-row accumulators per wave
@@ -204,24 +443,12 @@ gemm_wide_f16_kernel (const Args a, int tiles_m, int tiles_n, int per_xcd, int v
   constexpr int GPW = (BM + WBN) / 8 / WWAVES;       // 1 KiB load instructions per wave and k-step
   constexpr int AG = BM / 8 / WWAVES;                // of which rows of x
   extern __shared__ __align__ (16) uint8_t wide_lds[];
-  // workgroups go to the XCDs in turn: each XCD gets a contiguous range of
-  // tiles, token-row tile fastest, so the weight tiles it shares stay in its L2
-  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
-  const int tile = xcd * per_xcd + j;
-  // ksplit > 1: the k range is divided among ksplit workgroups per output
-  // tile; each writes its fp32 sums to the workspace, a second kernel adds them
-  const int plane = tiles_m * tiles_n;
-  if (j >= per_xcd || tile >= plane * ksplit)
-    return;
-  const int ks = tile / plane, t2 = tile - ks * plane;
-  const int tn = t2 / tiles_m, tm = t2 - tn * tiles_m;
+  const int ks = at.ks, zmat = at.zmat;
   const int nk_all = a.K / WBK;
   const int kbase = (int)((long)nk_all * ks / ksplit);
   const int nk = (int)((long)nk_all * (ks + 1) / ksplit) - kbase; // k-steps of this workgroup
   float *part = ksplit > 1 ? ws + (size_t)ks * a.M * a.N : nullptr;
-  const int bn_rows = UPGATE ? WBN / 2 : WBN; // weight rows per matrix and tile
-  const int m0 = tm * BM, n0 = tn * bn_rows;
-  const int zmat = blockIdx.z;
+  const int m0 = at.m0, n0 = at.tn * (UPGATE ? WBN / 2 : WBN); // weight rows per matrix and tile
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane (threadIdx.x >> 6);
   const int wm = wave >> 1, wn = wave & 1;
@@ -246,7 +473,7 @@ gemm_wide_f16_kernel (const Args a, int tiles_m, int tiles_n, int per_xcd, int v
       const int v = (wave + WWAVES * (i - AG)) * 8 + lr; // row of the weight tile
       const int mat = UPGATE ? v >> 6 : zmat;
       const int n = min (UPGATE ? n0 + (v & 63) : n0 + v, a.N - 1);
-      const uint16_t *w = mat == 0 ? a.wh[0] : (mat == 1 ? a.wh[1] : a.wh[2]);
+      const uint16_t *w = pick3 (a.wh[0], a.wh[1], a.wh[2], mat);
       src[i] = w + (size_t)n * a.ws + chunk * 8 + (PLANES > 1 ? 0 : (size_t)kbase * WBK);
     }
 
@@ -333,7 +560,7 @@ gemm_wide_f16_kernel (const Args a, int tiles_m, int tiles_n, int per_xcd, int v
         for (int i = 0; i < TM; ++i)
 #pragma unroll
           for (int jn = 0; jn < WTN; ++jn)
-            acc[i][jn] = WideElem<Args>::mfma (af[ks & 1][i], bf[ks & 1][jn], acc[i][jn]);
+            acc[i][jn] = WideElem<Args>::mfma (bf[ks & 1][jn], af[ks & 1][i], acc[i][jn]);
         if (ks == 0)
           WideOrder<0, NP, NR, LB1>::run ();
         else if (ks == 1)
@@ -362,7 +589,22 @@ gemm_wide_f16_kernel (const Args a, int tiles_m, int tiles_n, int per_xcd, int v
     step (kt + 1, WideInt<1> ());
   __builtin_amdgcn_s_waitcnt (0x0f70); // no load may outlive the workgroup's LDS
 
-  wide_epilogue<UPGATE, TM> (a, acc, wide_lds, wave, lane, m0, n0, zmat, vec, part);
+  wide_epilogue<UPGATE, TM, WTN> (a, acc, wide_lds, wave, lane, m0 + wm * TM * 32, n0 + (UPGATE ? wn * 32 : wn * 64), zmat, vec, part);
+}
+
+template <int BM, bool UPGATE, class Args = GemmArgs, int PLANES = 1>
+__global__ __launch_bounds__ (WWAVES * 64) void
+gemm_wide_f16_kernel (const Args a, WideGrid grid, int vec, int ksplit, float *ws)
+{
+  WidePlace at;
+  switch (grid.place<BM> (a.M, at))
+    {
+    case WIDE_TILE:
+      return wide_f16_tile<BM, UPGATE, Args, PLANES> (a, at, vec, ksplit, ws);
+    case WIDE_HALF:
+      if constexpr (BM == WBM)
+        return wide_f16_tile<BM / 2, UPGATE, Args, PLANES> (a, at, vec, ksplit, ws);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -384,9 +626,9 @@ gemm_wide_f16_kernel (const Args a, int tiles_m, int tiles_n, int per_xcd, int v
 // the compiler takes reads of a struct type to alias the tiles that the
 // direct-to-LDS loads still have in flight and waits for all of them.)
 constexpr int QWAVES = 8;
-// waves along N: 4 (2 x 4 waves, 128 x 32 each) measured 5-12 % faster than 2
-// (4 x 2 waves, 64 x 64 each) on the 7B and 13B shapes
-constexpr int QGRID = 4;
+// waves along N: 2 x 4 waves, 128 x 32 each (every weight fragment is converted by two
+// waves), measured 5-12 % faster than 4 x 2, 64 x 64 each, on the 7B and 13B shapes
+constexpr int WGN = 4;
 // Three stages, laid out by kind (x tiles, then quants, then scales).
 constexpr int QSTAGES = 3;
 constexpr int QB_BYTES = WBN * WBK;
@@ -396,7 +638,7 @@ template <int BM>
 constexpr size_t
 wide_lds_q8 ()
 {
-  const size_t stages = (size_t)QSTAGES * (BM * WROWB + QB_BYTES + QS_BYTES), park = (size_t)BM * 2 * kWideParkLd * 4; // (>= BM * kWideTileLd * 4)
+  const size_t stages = (size_t)QSTAGES * (BM * WROWB + QB_BYTES + QS_BYTES), park = (size_t)BM * kWideTileLd * 4;
   return stages > park ? stages : park;
 }
 
@@ -416,37 +658,24 @@ q8_frag (u32x2 r)
   return o;
 }
 
-// WGN: waves along N, 2 (4 x 2 waves of 64 columns) or 4 (2 x 4 waves of 32
-// columns and twice the rows: every weight fragment is converted by two waves
-// instead of four).
-template <int BM, int WGN, bool UPGATE>
-__global__ __launch_bounds__ (QWAVES * 64) void
-gemm_wide_q8_kernel (const GemmArgs a, int tiles_m, int tiles_n, int per_xcd, int vec, int ksplit, float *ws)
+template <int BM, bool UPGATE>
+__device__ __forceinline__ void
+wide_q8_tile (const GemmArgs &a, const WidePlace &at, int vec, int ksplit, float *ws)
 {
   constexpr int QTM = BM / (QWAVES / WGN) / 32; // 32-row accumulators per wave
-  constexpr int QTN = 4 / WGN;                  // 32-column accumulators per wave
+  constexpr int QTN = 1;                        // 32-column accumulators per wave
   constexpr int QAG = BM / 8 / QWAVES;       // x load instructions per wave and k-step
   constexpr int QA_BYTES = BM * WROWB;
   constexpr int QB_BASE = QSTAGES * QA_BYTES;
   constexpr int QS_BASE = QB_BASE + QSTAGES * QB_BYTES;
   constexpr int QLOADS = QAG + 1 + 1;        // per wave and k-step: x, quants, scales
   extern __shared__ __align__ (16) uint8_t wide_lds[];
-  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
-  const int tile = xcd * per_xcd + j;
-  // ksplit > 1: the k range is divided among ksplit workgroups per output
-  // tile; each writes its fp32 sums to the workspace, a second kernel adds them
-  const int plane = tiles_m * tiles_n;
-  if (j >= per_xcd || tile >= plane * ksplit)
-    return;
-  const int ks = tile / plane, t2 = tile - ks * plane;
-  const int tn = t2 / tiles_m, tm = t2 - tn * tiles_m;
+  const int ks = at.ks, zmat = at.zmat;
   const int nk_all = a.K / WBK;
   const int kbase = (int)((long)nk_all * ks / ksplit);
   const int nk = (int)((long)nk_all * (ks + 1) / ksplit) - kbase; // k-steps of this workgroup
   float *part = ksplit > 1 ? ws + (size_t)ks * a.M * a.N : nullptr;
-  const int bn_rows = UPGATE ? WBN / 2 : WBN;
-  const int m0 = tm * BM, n0 = tn * bn_rows;
-  const int zmat = blockIdx.z;
+  const int m0 = at.m0, n0 = at.tn * (UPGATE ? WBN / 2 : WBN);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane (threadIdx.x >> 6);
   const int wm = wave / WGN, wn = wave % WGN;
@@ -486,7 +715,7 @@ gemm_wide_q8_kernel (const GemmArgs a, int tiles_m, int tiles_n, int per_xcd, in
   // fragment reads
   const int fsw = (lane & 7) ^ ((lane >> 3) & 1);
   // (rows of the weight tile: for the fused pair 0 .. 63 are up, 64 .. 127 gate)
-  const int brow = (WGN == 4 ? wn * 32 : UPGATE ? wn * 32 : wn * 64) + (lane & 31);
+  const int brow = wn * 32 + (lane & 31);
   const int qsw = (lane >> 1) & 3;
   uint32_t aoff[4], qoff[4];
 #pragma unroll
@@ -624,10 +853,22 @@ gemm_wide_q8_kernel (const GemmArgs a, int tiles_m, int tiles_n, int per_xcd, in
       st = s1;
     }
   __builtin_amdgcn_s_waitcnt (0x0f70); // no load may outlive the workgroup's LDS
-  if constexpr (WGN == 4)
-    wide_epilogue_tile<BM, UPGATE, QTM> (a, acc, wide_lds, wave, lane, m0, n0, zmat, vec, part);
-  else
-    wide_epilogue<UPGATE, QTM> (a, acc, wide_lds, wave, lane, m0, n0, zmat, vec, part);
+  wide_epilogue_tile<BM, UPGATE, QTM> (a, acc, wide_lds, wave, lane, m0, n0, zmat, vec, part);
+}
+
+template <int BM, bool UPGATE>
+__global__ __launch_bounds__ (QWAVES * 64) void
+gemm_wide_q8_kernel (const GemmArgs a, WideGrid grid, int vec, int ksplit, float *ws)
+{
+  WidePlace at;
+  switch (grid.place<BM> (a.M, at))
+    {
+    case WIDE_TILE:
+      return wide_q8_tile<BM, UPGATE> (a, at, vec, ksplit, ws);
+    case WIDE_HALF:
+      if constexpr (BM == WBM)
+        return wide_q8_tile<BM / 2, UPGATE> (a, at, vec, ksplit, ws);
+    }
 }
 
 // Which tile height and how many parts of the k range: the pair with the
@@ -736,8 +977,8 @@ gemm_wide_launch (const GemmArgs &a, hipStream_t s)
   const void *const kernels[8]
       = { (const void *)gemm_wide_f16_kernel<256, false>,       (const void *)gemm_wide_f16_kernel<256, true>,
           (const void *)gemm_wide_f16_kernel<128, false>,       (const void *)gemm_wide_f16_kernel<128, true>,
-          (const void *)gemm_wide_q8_kernel<256, QGRID, false>, (const void *)gemm_wide_q8_kernel<256, QGRID, true>,
-          (const void *)gemm_wide_q8_kernel<128, QGRID, false>, (const void *)gemm_wide_q8_kernel<128, QGRID, true> };
+          (const void *)gemm_wide_q8_kernel<256, false>, (const void *)gemm_wide_q8_kernel<256, true>,
+          (const void *)gemm_wide_q8_kernel<128, false>, (const void *)gemm_wide_q8_kernel<128, true> };
   const size_t need[8] = { lds256, lds256, lds128, lds128, q256, q256, q128, q128 };
   for (int i = 0; i < 8; ++i)
     if (int e = limits[i].raise (kernels[i], need[i]))
@@ -752,8 +993,8 @@ gemm_wide_launch (const GemmArgs &a, hipStream_t s)
     ksplit = 1;
   const int tiles_m = (a.M + bm - 1) / bm;
   const int tiles_n = (a.N + (a.upgate ? 63 : 127)) / (a.upgate ? 64 : 128);
-  const int per_xcd = (tiles_m * tiles_n * ksplit + 7) / 8;
-  const dim3 grid ((unsigned)(per_xcd * 8), 1, (unsigned)(a.upgate ? 1 : a.nmat));
+  const WideGrid tiles (tiles_m, tiles_n, a.upgate ? 1 : a.nmat, ksplit, bm == WBM);
+  const dim3 grid ((unsigned)tiles.groups ());
   const dim3 block ((a.wtype == 8 ? QWAVES : WWAVES) * 64);
   // 16-byte accesses to the outputs (and the residual) where their rows allow it
   int vec = (a.ys % 8) == 0 && (!a.residual || ((uintptr_t)a.residual % 16) == 0)
@@ -763,28 +1004,28 @@ gemm_wide_launch (const GemmArgs &a, hipStream_t s)
   if (a.wtype == 8 && bm == 256)
     {
       if (a.upgate)
-        gemm_wide_q8_kernel<256, QGRID, true><<<grid, block, q256, s>>> (a, tiles_m, tiles_n, per_xcd, vec, ksplit, ws);
+        gemm_wide_q8_kernel<256, true><<<grid, block, q256, s>>> (a, tiles, vec, ksplit, ws);
       else
-        gemm_wide_q8_kernel<256, QGRID, false><<<grid, block, q256, s>>> (a, tiles_m, tiles_n, per_xcd, vec, ksplit, ws);
+        gemm_wide_q8_kernel<256, false><<<grid, block, q256, s>>> (a, tiles, vec, ksplit, ws);
     }
   else if (a.wtype == 8)
     {
       if (a.upgate)
-        gemm_wide_q8_kernel<128, QGRID, true><<<grid, block, q128, s>>> (a, tiles_m, tiles_n, per_xcd, vec, ksplit, ws);
+        gemm_wide_q8_kernel<128, true><<<grid, block, q128, s>>> (a, tiles, vec, ksplit, ws);
       else
-        gemm_wide_q8_kernel<128, QGRID, false><<<grid, block, q128, s>>> (a, tiles_m, tiles_n, per_xcd, vec, ksplit, ws);
+        gemm_wide_q8_kernel<128, false><<<grid, block, q128, s>>> (a, tiles, vec, ksplit, ws);
     }
   else if (bm == 256)
     {
       if (a.upgate)
-        gemm_wide_f16_kernel<256, true><<<grid, block, lds256, s>>> (a, tiles_m, tiles_n, per_xcd, vec, ksplit, ws);
+        gemm_wide_f16_kernel<256, true><<<grid, block, lds256, s>>> (a, tiles, vec, ksplit, ws);
       else
-        gemm_wide_f16_kernel<256, false><<<grid, block, lds256, s>>> (a, tiles_m, tiles_n, per_xcd, vec, ksplit, ws);
+        gemm_wide_f16_kernel<256, false><<<grid, block, lds256, s>>> (a, tiles, vec, ksplit, ws);
     }
   else if (a.upgate)
-    gemm_wide_f16_kernel<128, true><<<grid, block, lds128, s>>> (a, tiles_m, tiles_n, per_xcd, vec, ksplit, ws);
+    gemm_wide_f16_kernel<128, true><<<grid, block, lds128, s>>> (a, tiles, vec, ksplit, ws);
   else
-    gemm_wide_f16_kernel<128, false><<<grid, block, lds128, s>>> (a, tiles_m, tiles_n, per_xcd, vec, ksplit, ws);
+    gemm_wide_f16_kernel<128, false><<<grid, block, lds128, s>>> (a, tiles, vec, ksplit, ws);
   if (ksplit > 1)
     return gemm_reduce_parts (a, ws, ksplit, a.M, s);
   return (int)hipGetLastError ();
@@ -880,8 +1121,8 @@ launch_wide_bf16 (const GemmSegArgs &a, int ksplit, float *ws, hipStream_t s)
   if (ksplit > 1 && !ws && !(ws = gemm_stream_workspace (s)))
     ksplit = 1;
   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + WBN - 1) / WBN;
-  const int per_xcd = (tiles_m * tiles_n * ksplit + 7) / 8;
-  kernel<<<dim3 ((unsigned)(per_xcd * 8)), dim3 (WWAVES * 64), lds, s>>> (a, tiles_m, tiles_n, per_xcd, 1, ksplit, ws);
+  const WideGrid tiles (tiles_m, tiles_n, 1, ksplit, BM == WBM);
+  kernel<<<dim3 ((unsigned)tiles.groups ()), dim3 (WWAVES * 64), lds, s>>> (a, tiles, 1, ksplit, ws);
   if (ksplit > 1)
     {
       const size_t total = (size_t)a.M * ((a.N + 7) / 8);

@@ -3,23 +3,18 @@
 // score and probability tensors ever reaching memory.
 //
 // One pass over the keys with a running maximum (online softmax): per tile of
-// 64 keys the scores are formed (rounded to fp16 like the stand-alone product:
-// score = fp16(scale * q.k)), the maximum m is raised if needed - the products
-// accumulated so far and the sum of exponentials are then multiplied by
-// exp(m_old - m_new) -, the weights fp16(exp(score - m)) go into the second
-// product as they are, and the division by the sum of exponentials comes last,
-// in fp32, before the one rounding of the output.  The separate operators round
-// the NORMALISED probability to fp16 instead (p = fp16(exp(score - max) / sum));
-// the two differ by at most two half-ulp roundings of a weight, i.e. by
-// 2 * 2^-12 * sum_l p[l] |v[l]|, inside the 1e-2 the outputs are held to.  (A first
-// version walked the keys twice - maximum and sum first, then the very
-// probabilities of the operators - and took twice as long: two exponentials
-// per score and the scores computed twice.)
+// 64 keys the scores are formed (fp16: rounded like the stand-alone product: score =
+// fp16(scale * q.k)), the maximum m is raised if needed - the products accumulated
+// so far and the sum of exponentials are then multiplied by exp(m_old - m_new) -, the
+// weights, rounded once as the operand of the second product, go into it as they
+// are, and the division by their sum comes last, in fp32, before the one rounding
+// of the output.  The separate operators round the NORMALISED probability to fp16
+// instead; the two differ by two half-ulp roundings of a weight, i.e. by
+// 2 * 2^-12 * sum_l p[l] |v[l]|, inside the 1e-2 the outputs are held to.
 //
 // Workgroup = 4 waves = 128 query rows of one head, 32 per wave; the keys come
-// through LDS in tiles of 64.  Both products run on v_mfma_f32_32x32x16_f16 in
-// the transposed form, so that a lane's accumulator registers belong to ONE
-// query:
+// through LDS in tiles of 64.  Both products run on v_mfma_f32_32x32x16 in the
+// transposed form, so that a lane's accumulator registers belong to ONE query:
 //   S^T[key, q] = sum_d K[key, d] Q[q, d]      A = K tile (LDS), B = Q (regs)
 //   O^T[d, q]   = sum_key V^T[d, key] P^T[key, q]   A = V^T tile (LDS), B = P^T
 // Lane l of a wave owns query l % 32.  Of a 32-key block its 16 accumulator
@@ -27,22 +22,40 @@
 // keys are sums over a lane's own registers (the two lane halves are merged
 // after every tile), and the weights it forms are, as they lie, the B
 // operand of the second product: registers 8t .. 8t+7 are the eight k values
-// of lane half l/32 in k-step t.  The V tile is written to LDS transposed and
-// with its keys permuted to that same order (slot 16t + 8h + j holds key
-// 16t + 8*(j/4) + 4h + j%4 of the block), so the A operand of the second
-// product is one 16-byte LDS read.
+// of lane half l/32 in k-step t.
 //
-// The element type is a template parameter: fp16 (Llama-2, the score rounded
-// to fp16 as above) or bf16 (scores stay in fp32; weights are rounded once, as
-// the operand of the second product).  Query heads may share key/value heads,
-// the score factor may grow with the query's position, and a head's output may
-// be scaled by the sigmoid of a per-token gate.
+// Heads of 64 and 128 values (attn_tiles_kernel): K and V tiles go straight into LDS
+// as they lie in memory (global_load_lds), the next tile while this one is multiplied,
+// one barrier per tile; the V^T operand is read transposed (ds_read_b64_tr_b16: four
+// keys of a column per lane, two reads make the eight k values above).  Other head sizes
+// (attn_prefill_kernel): tiles travel through registers and V is written to LDS
+// transposed, its keys permuted to the operand's order (slot 16t + 8h + j holds key
+// 16t + 8*(j/4) + 4h + j%4 of the block).
+//
+// What bounds it: matrix cores 1024 cycles per wave and tile, vector ALU 13 instructions
+// per two scores (two FMAs, two exponentials at a quarter of the rate, a maximum, one
+// conversion, one dot product with ones for the sum) = 830, with rounded scores two more
+// (mixed-precision FMAs round and widen on the way), LDS reads 32 KB; two workgroups on a
+// compute unit overlap them.  The maximum is only raised by more than a
+// factor of 2^6 in the weights at a time, which keeps nearly all tiles free of rescaling.
+// Measured, us per call before (registers and two barriers per tile for all head sizes) and
+// now: fp16, 32 heads of 128, 2048 rows 85 / 60, 40 heads, 3967 rows 308 / 224; bf16 in chunks
+// with a sink, 2048 rows 100 / 51; 16 heads, 1500 rows behind 600 keys 67 / 46.
+// Few query tiles (a turn of some dozen tokens behind a long context) would leave most
+// compute units idle: then the keys of a query tile are divided among workgroups, whose
+// unnormalised outputs a second launch adds up.
+//
+// The element type is a template parameter: fp16 (Llama-2) or bf16.  Query heads may share
+// key/value heads, the score factor may grow with the query's position, and a head's output
+// may be scaled by the sigmoid of a per-token gate.
 //
 // A second, small kernel in this file prepares the inputs of the first from
 // the projection outputs: RoPE of Q (in place) and K, and the K/V cache write.
 #include "../../include/vkl_hip.h"
 #include "../../include/vkl_stack.h"
 #include "vkl_common.h"
+#include "vkl_gemm.h"
+#include <algorithm>
 
 namespace
 {
@@ -69,13 +82,15 @@ struct AttnArgs
   const float *gate;  // optional [S, gs]: head h's output times sigmoid (gate[s, h])
   size_t gs;
   int chunk, sink;    // CHUNKED kernels: see vkl_attn_prefill_chunked_bf16
+  int parts;          // workgroups that share the keys of a query tile
+  float *ws;          // parts > 1: their results, see part_row
 };
 
 // the two element types of the operands
 struct F16Elem
 {
   typedef half8 v8;
-  static constexpr bool round_scores = true;
+  static constexpr bool round_scores = true; // to fp16, as the stand-alone product stores them
   static __device__ __forceinline__ float16v
   mfma (v8 a, v8 b, float16v c)
   {
@@ -87,6 +102,13 @@ struct F16Elem
     return vkl::f2h (f);
   }
   typedef _Float16 t;
+  typedef _Float16 t2 __attribute__ ((ext_vector_type (2)));
+  // sum + a[0] + a[1]
+  static __device__ __forceinline__ float
+  add2 (t2 a, float sum)
+  {
+    return __builtin_amdgcn_fdot2 (a, t2{ (_Float16)1.f, (_Float16)1.f }, sum, false);
+  }
 };
 
 struct Bf16Elem
@@ -104,6 +126,12 @@ struct Bf16Elem
     return vkl::f2bf (f);
   }
   typedef __bf16 t;
+  typedef __bf16 t2 __attribute__ ((ext_vector_type (2)));
+  static __device__ __forceinline__ float
+  add2 (t2 a, float sum)
+  {
+    return __builtin_amdgcn_fdot2_f32_bf16 (a, t2{ (__bf16)1.f, (__bf16)1.f }, sum, false);
+  }
 };
 
 __device__ __align__ (16) const uint32_t g_zero16[4] = { 0, 0, 0, 0 };
@@ -114,6 +142,35 @@ fast_exp (float x)
   return __builtin_amdgcn_exp2f (x * 1.44269504088896340736f);
 }
 
+
+// Which query tile of which head a workgroup has.
+// Heavy query tiles (the last ones: most keys) first.  With a head count
+// that is a multiple of 8 the workgroups of one head share id % 8, which
+// keeps the head's K and V in the L2 of one XCD.
+__device__ __forceinline__ void
+tile_of (const AttnArgs &a, int b, int &head, int &qt)
+{
+  if ((a.H & 7) == 0)
+    {
+      // j: position in the XCD's queue.  Its 32 compute units take the first
+      // 32 workgroups, then the next 32 beside them, and so on: every other
+      // such layer runs in the opposite order, so that a heavy tile and a
+      // light one share a compute unit.  (The order of the queue is reversed
+      // within the layer, the last of which may be shorter: whatever the
+      // number of tiles, every tile of every head has one place.)
+      int j = b >> 3;
+      const int queue = (a.H >> 3) * a.ntq, j0 = j & ~31;
+      if ((j >> 5) & 1)
+        j = j0 + min (queue, j0 + 32) - 1 - j;
+      head = (b & 7) + 8 * (j / a.ntq);
+      qt = a.ntq - 1 - (j % a.ntq);
+    }
+  else
+    {
+      head = b / a.ntq;
+      qt = a.ntq - 1 - (b % a.ntq);
+    }
+}
 
 template <int HD> struct Tile
 {
@@ -242,31 +299,8 @@ attn_prefill_kernel (const AttnArgs a)
   __shared__ __align__ (16) uint16_t Ks[kBKey * LDK];
   __shared__ __align__ (16) uint16_t Vt[HD * LDV];
 
-  // Heavy query tiles (the last ones: most keys) first.  With a head count
-  // that is a multiple of 8 the workgroups of one head share id % 8, which
-  // keeps the head's K and V in the L2 of one XCD.
-  const int b = blockIdx.x;
   int head, qt;
-  if ((a.H & 7) == 0)
-    {
-      // j: position in the XCD's queue.  Its 32 compute units take the first
-      // 32 workgroups, then the next 32 beside them, and so on: every other
-      // such layer runs in the opposite order, so that a heavy tile and a
-      // light one share a compute unit.  (The order of the queue is reversed
-      // within the layer, the last of which may be shorter: whatever the
-      // number of tiles, every tile of every head has one place.)
-      int j = b >> 3;
-      const int queue = (a.H >> 3) * a.ntq, j0 = j & ~31;
-      if ((j >> 5) & 1)
-        j = j0 + min (queue, j0 + 32) - 1 - j;
-      head = (b & 7) + 8 * (j / a.ntq);
-      qt = a.ntq - 1 - (j % a.ntq);
-    }
-  else
-    {
-      head = b / a.ntq;
-      qt = a.ntq - 1 - (b % a.ntq);
-    }
+  tile_of (a, (int)blockIdx.x, head, qt);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lq = lane & 31, hh = lane >> 5;
   const int q0 = qt * kBQ;
@@ -280,12 +314,12 @@ attn_prefill_kernel (const AttnArgs a)
   const int klow = chunk_start (qrow), wave_low = chunk_start (q0 + wave * 32);
   const int wave_high = chunk_start (q0 + wave * 32 + 31);
   const int t0 = CHUNKED ? chunk_start (q0) / kBKey : 0;
-  const int kvh = E::round_scores ? head : head / a.rep;
+  const int kvh = head / a.rep;
   const uint16_t *kb = a.k + (size_t)kvh * a.kcs;
   const uint16_t *vb = a.v + (size_t)kvh * a.vcs;
   // this query's score factor
   float scale = a.scale;
-  if (!E::round_scores && a.temp_coef != 0.f)
+  if (a.temp_coef != 0.f)
     scale *= 1.0f + a.temp_coef * logf ((float)((qrow + shift + 1) / a.temp_every + 1));
 
   v8 qf[KT];
@@ -326,8 +360,8 @@ attn_prefill_kernel (const AttnArgs a)
         }
       if (t * kBKey > wave_last || (CHUNKED && t * kBKey + kBKey <= wave_low))
         continue;
-      // scores of the tile's 64 keys, rounded to fp16 like the stand-alone
-      // product; a key the query must not see counts as "never seen"
+      // scores of the tile's 64 keys; a key the query must not see counts as "never
+      // seen"
       float sv[2][16];
       float bm = kNeg;
       const bool inner = t * kBKey + kBKey - 1 <= q0 + wave * 32 + shift // every key visible to every query of the wave
@@ -341,7 +375,7 @@ attn_prefill_kernel (const AttnArgs a)
           for (int r = 0; r < 16; ++r)
             {
               const int key = key0 + 8 * (r >> 2) + (r & 3);
-              const float sc = E::round_scores ? vkl::h2f (vkl::f2h (acc[r] * scale)) : acc[r] * scale;
+              const float sc = acc[r] * scale;
               sv[blk][r] = inner || (key <= qrow + shift && (!CHUNKED || key >= klow)) ? sc : kNeg;
               bm = fmaxf (bm, sv[blk][r]);
             }
@@ -368,8 +402,7 @@ attn_prefill_kernel (const AttnArgs a)
         for (int r = 0; r < 16; ++r)
           {
             // exp (kNeg - m) = 0.  The sum takes the weight as the product
-            // below consumes it, rounded to fp16: the weights then add up to
-            // one exactly.
+            // below consumes it, rounded: the weights then add up to one exactly.
             const typename E::t e = (typename E::t)fast_exp (sv[blk][r] - m);
             sum += (float)e;
             pf[blk][r >> 3][r & 7] = e;
@@ -388,7 +421,7 @@ attn_prefill_kernel (const AttnArgs a)
   // the other half of the lanes has summed the other keys of the same query
   sum += __shfl_xor (sum, 32, 64);
   float inv = 1.0f / sum;
-  if (!E::round_scores && a.gate)
+  if (a.gate)
     inv = inv / (1.0f + expf (-vkl::ldg (a.gate + (size_t)min (qrow, a.S - 1) * a.gs + head)));
 #pragma unroll
   for (int db = 0; db < DB; ++db)
@@ -412,6 +445,460 @@ attn_prefill_kernel (const AttnArgs a)
         *(VKL_GLOBAL u32x2 *)(op + d) = w;
       }
 }
+// ---------------------------------------------------------------------------
+// heads of 64 and 128 values
+// ---------------------------------------------------------------------------
+#define VKL_LDS __attribute__ ((address_space (3)))
+
+// Weights grow by at most this power of two before the maximum is raised
+constexpr float kRaise = 6.0f;
+
+__device__ __forceinline__ float
+max3 (float a, float b, float c)
+{
+  // (fmaxf would quiet its operands first)
+  float r;
+  asm ("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
+template <class T>
+__device__ __forceinline__ T
+pk_max (T a, T b)
+{
+  T r;
+  asm ("v_pk_max_f16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
+// the larger of a lane's value and of that of the lane 32 away
+__device__ __forceinline__ float
+max_halves (float x)
+{
+  const auto r = __builtin_amdgcn_permlane32_swap (__float_as_uint (x), __float_as_uint (x), false, false);
+  return fmaxf (__uint_as_float (r[0]), __uint_as_float (r[1]));
+}
+
+// Results of a part of the keys: per part, head and query row the maximum (in powers of
+// two), the sum of weights and HD unnormalised outputs
+template <int HD>
+__device__ __forceinline__ float *
+part_row (const AttnArgs &a, int part, int head, int row)
+{
+  return a.ws + ((size_t)(part * a.H + head) * a.S + row) * (HD + 4);
+}
+
+// Tiles in LDS hold their rows as they lie, except that the 16-byte chunks of a row are
+// exchanged: chunk c of key k is at slot c ^ swizzle (k).  Both kinds of reads, sixteen
+// keys at one chunk (K) and four keys of 32 columns (V, transposed), then meet every bank
+// once.
+template <int HD>
+__device__ __forceinline__ int
+swizzle (int key)
+{
+  return HD == 128 ? ((key & 3) << 2) | ((key >> 2) & 3) : (((key >> 1) & 1) << 2) | ((key >> 2) & 3);
+}
+
+// Issue order of N products, each with PER reads, the reads of AHEAD products in front
+template <int KIND, int PER, int N, int AHEAD> struct Alternate
+{
+  template <int I>
+  static __device__ __forceinline__ void
+  from ()
+  {
+    __builtin_amdgcn_sched_group_barrier (0x008, 1, 0);
+    if constexpr (I + AHEAD < N)
+      __builtin_amdgcn_sched_group_barrier (KIND, PER, 0);
+    if constexpr (I + 1 < N)
+      from<I + 1> ();
+  }
+  static __device__ __forceinline__ void
+  run ()
+  {
+    __builtin_amdgcn_sched_group_barrier (KIND, PER * AHEAD, 0);
+    from<0> ();
+  }
+};
+
+template <int HD, class E, bool CHUNKED, bool PARTS>
+__global__ __launch_bounds__ (kThreads, 2) void
+attn_tiles_kernel (const AttnArgs a)
+{
+  typedef typename E::v8 v8;
+  typedef typename E::t2 t2;
+  constexpr int KT = HD / 16, DB = HD / 32, CPR = HD / 8, ROWB = HD * 2;
+  constexpr int TILE = kBKey * ROWB;     // bytes of a K or V tile
+  constexpr int RPI = 1024 / ROWB;       // keys per 1 KiB load
+  constexpr int LPW = TILE / 1024 / 4;   // loads per wave and tile
+  // four objects: a read of one is then not made to wait for the loads on their way into
+  // another
+  __shared__ __align__ (16) uint8_t lk0[TILE], lv0[TILE], lk1[TILE], lv1[TILE];
+
+  int head, qt, part = 0;
+  {
+    int b = (int)blockIdx.x;
+    if (PARTS)
+      part = b / (a.ntq * a.H), b -= part * (a.ntq * a.H);
+    tile_of (a, b, head, qt);
+  }
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane (threadIdx.x >> 6);
+  const int lq = lane & 31, hh = lane >> 5;
+  const int q0 = qt * kBQ;
+  const int qrow = q0 + wave * 32 + lq; // this lane's query
+  const int shift = a.L - a.S;          // key l is visible iff l <= qrow + shift
+  const int kmax = min (a.L, q0 + kBQ + shift);
+  const int wave_last = q0 + wave * 32 + 31 + shift; // last key any query of the wave sees
+  // first key of the chunk of this lane's query, of the wave's first and last
+  auto chunk_start = [&] (int row) { return CHUNKED && a.chunk ? (row + shift) / a.chunk * a.chunk : 0; };
+  const int klow = chunk_start (qrow), wave_low = chunk_start (q0 + wave * 32);
+  const int wave_high = chunk_start (q0 + wave * 32 + 31);
+  int t0 = CHUNKED ? chunk_start (q0) / kBKey : 0, t1 = (kmax + kBKey - 1) / kBKey;
+  if (PARTS)
+    {
+      const int n = t1 - t0, first = t0;
+      t0 = first + n * part / a.parts, t1 = first + n * (part + 1) / a.parts;
+    }
+  const int kvh = head / a.rep;
+  const uint16_t *kb = a.k + (size_t)kvh * a.kcs;
+  const uint16_t *vb = a.v + (size_t)kvh * a.vcs;
+  // from what the maximum is taken over to powers of two: rounded scores, or the products,
+  // with this query's score factor
+  float c = (E::round_scores ? 1.f : a.scale) * 1.44269504088896340736f;
+  if (!E::round_scores && a.temp_coef != 0.f)
+    c *= 1.0f + a.temp_coef * logf ((float)((qrow + shift + 1) / a.temp_every + 1));
+
+  v8 qf[KT];
+  {
+    // the maximum is taken over the products: a negative factor goes into the query (of
+    // the factor 0 all scores are 0)
+    const uint32_t flip = c < 0.f ? 0x80008000u : 0u, keep = c == 0.f ? 0u : ~0u;
+    c = c == 0.f ? 1.f : fabsf (c);
+    const uint16_t *qp = a.q + (size_t)head * a.qcs + (size_t)min (qrow, a.S - 1) * a.qhs + hh * 8;
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+      {
+        uint4 w = vkl::ldg4 (qp + kt * 16);
+        w.x = (w.x ^ flip) & keep, w.y = (w.y ^ flip) & keep, w.z = (w.z ^ flip) & keep, w.w = (w.w ^ flip) & keep;
+        qf[kt] = __builtin_bit_cast (v8, w);
+      }
+  }
+
+  // loads: instruction i of a wave covers RPI keys from (wave + 4 i) RPI on; lane l fetches
+  // the chunk that belongs into slot l % CPR of its key (keys beyond the last repeat it:
+  // no query sees them)
+  const int lr = lane / CPR;
+  auto issue = [&] (int t, uint8_t *lk, uint8_t *lv) {
+#pragma unroll
+    for (int i = 0; i < LPW; ++i)
+      {
+        const int r = (wave + 4 * i) * RPI + lr;
+        const size_t key = (size_t)min (t * kBKey + r, a.L - 1);
+        const int col = ((lane % CPR) ^ swizzle<HD> (r)) * 8;
+        __builtin_amdgcn_global_load_lds ((const VKL_GLOBAL void *)(kb + key * a.khs + col),
+                                          (VKL_LDS void *)(lk + (wave + 4 * i) * 1024), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds ((const VKL_GLOBAL void *)(vb + key * a.vhs + col),
+                                          (VKL_LDS void *)(lv + (wave + 4 * i) * 1024), 16, 0, 0);
+      }
+  };
+  // reads of K: key l % 32 of a block, values 16 kt + 8 (l / 32) .. + 7
+  uint32_t koff[KT];
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt)
+    koff[kt] = lq * ROWB + (((2 * kt + hh) ^ swizzle<HD> (lq)) << 4);
+  // reads of V: of sixteen lanes four each give the columns 16 ((l / 16) % 2) .. + 15 of four
+  // neighbouring keys from 8 g + 4 (l / 32) on, of which each receives one column
+  uint32_t voff[DB][2];
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+      {
+        const int key = 8 * g + 4 * hh + ((lane & 15) >> 2);
+        const int chunk = 4 * db + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
+        voff[db][g] = key * ROWB + ((chunk ^ swizzle<HD> (key)) << 4) + (lane & 1) * 8;
+      }
+
+  // (the sink is a key that every query has seen before the first tile; the sums of the
+  // two lane halves are added at the end, one of them has it)
+  // (a tile may hold no key that a query sees: its first maximum lies far above the score
+  // of a hidden key, whose weight is then zero)
+  const bool sink = CHUNKED && a.sink && part == 0;
+  float m = sink ? 0.f : 0.1f * kNeg, sum = sink && hh == 0 ? 1.f : 0.f;
+  float16v oacc[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      oacc[db][r] = 0.f;
+  // one tile, in (ks, vs); the next one goes to (kn, vn)
+  auto step = [&] (int t, const uint8_t *ks, const uint8_t *vs, uint8_t *kn, uint8_t *vn) {
+    // this tile has landed (the wave's part; the barrier covers the others'), and every
+    // wave is done with the tile before, whose place the next one takes
+    __builtin_amdgcn_s_waitcnt (0x0f70);
+    __builtin_amdgcn_s_barrier ();
+    __builtin_amdgcn_sched_barrier (0);
+    if (t + 1 < t1)
+      issue (t + 1, kn, vn);
+    if (t * kBKey > wave_last || (CHUNKED && t * kBKey + kBKey <= wave_low))
+      return;
+    const bool inner = t * kBKey + kBKey - 1 <= q0 + wave * 32 + shift // every key visible to every query of the wave
+                       && (!CHUNKED || t * kBKey >= wave_high);
+    float16v s[2];
+#pragma unroll
+    for (int blk = 0; blk < 2; ++blk)
+      {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          s[blk][r] = 0.f;
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt)
+          s[blk] = E::mfma (*(const v8 *)(ks + koff[kt] + blk * 32 * ROWB), qf[kt], s[blk]);
+      }
+    Alternate<0x100, 1, 2 * KT, 6>::run (); // reads stay six ahead of the products
+    __builtin_amdgcn_sched_barrier (0);
+    auto hidden = [&] (int blk, int r) {
+      const int key = t * kBKey + 4 * hh + 32 * blk + 8 * (r >> 2) + (r & 3);
+      return key > qrow + shift || (CHUNKED && key < klow);
+    };
+    float bm;
+    t2 sh[2][8]; // the scores as fp16 pairs
+    if constexpr (E::round_scores)
+      {
+#pragma unroll
+        for (int blk = 0; blk < 2; ++blk)
+#pragma unroll
+          for (int r = 0; r < 16; r += 2)
+            sh[blk][r / 2] = t2{ (typename E::t)__builtin_fmaf (s[blk][r], a.scale, 0.f),
+                                 (typename E::t)__builtin_fmaf (s[blk][r + 1], a.scale, 0.f) };
+        if (!inner)
+          {
+            const typename E::t never = -__builtin_inff ();
+#pragma unroll
+            for (int blk = 0; blk < 2; ++blk)
+#pragma unroll
+              for (int r = 0; r < 16; ++r)
+                if (hidden (blk, r))
+                  sh[blk][r / 2][r & 1] = never;
+          }
+        t2 top = sh[0][0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i)
+          top = pk_max (top, sh[i >> 3][i & 7]);
+        bm = fmaxf ((float)top[0], (float)top[1]);
+      }
+    else
+      {
+        if (!inner)
+          {
+#pragma unroll
+            for (int blk = 0; blk < 2; ++blk)
+#pragma unroll
+              for (int r = 0; r < 16; ++r)
+                if (hidden (blk, r))
+                  s[blk][r] = kNeg;
+          }
+        bm = kNeg;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          bm = max3 (s[0][r], s[1][r], bm);
+      }
+    // the two halves of the lanes hold different keys of the same query and feed one
+    // product: they need the same maximum
+    bm = max_halves (bm);
+    const bool raise = (bm - m) * c > kRaise;
+    if (__builtin_amdgcn_ballot_w64 (raise) != 0)
+      {
+        const float mn = raise ? bm : m;
+        const float alpha = __builtin_amdgcn_exp2f ((m - mn) * c); // 0 before the first key, 1 where the maximum stays
+        sum *= alpha;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            oacc[db][r] *= alpha;
+        m = mn;
+      }
+    const float mc = m * c;
+    v8 pf[2][2];
+#pragma unroll
+    for (int blk = 0; blk < 2; ++blk)
+#pragma unroll
+      for (int r = 0; r < 16; r += 2)
+        {
+          typedef float f32x2 __attribute__ ((ext_vector_type (2)));
+          const float s0 = E::round_scores ? (float)sh[blk][r / 2][0] : s[blk][r];
+          const float s1 = E::round_scores ? (float)sh[blk][r / 2][1] : s[blk][r + 1];
+          const f32x2 e = { __builtin_amdgcn_exp2f (__builtin_fmaf (s0, c, -mc)),
+                            __builtin_amdgcn_exp2f (__builtin_fmaf (s1, c, -mc)) };
+          // the sum takes the weights as the product below consumes them, rounded: they
+          // then add up to one exactly
+          const t2 w = __builtin_convertvector (e, t2);
+          sum = E::add2 (w, sum);
+          pf[blk][r >> 3][r & 7] = w[0], pf[blk][r >> 3][(r & 7) + 1] = w[1];
+        }
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int blk = 0; blk < 2; ++blk)
+#pragma unroll
+        for (int t2i = 0; t2i < 2; ++t2i)
+          {
+            typedef short i16x4 __attribute__ ((ext_vector_type (4)));
+            typedef short i16x8 __attribute__ ((ext_vector_type (8)));
+            const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16 (
+                (VKL_LDS i16x4 *)(vs + voff[db][0] + (32 * blk + 16 * t2i) * ROWB));
+            const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16 (
+                (VKL_LDS i16x4 *)(vs + voff[db][1] + (32 * blk + 16 * t2i) * ROWB));
+            const i16x8 v = __builtin_shufflevector (lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+            oacc[db] = E::mfma (__builtin_bit_cast (v8, v), pf[blk][t2i], oacc[db]);
+          }
+    Alternate<0x100, 2, 4 * DB, 4>::run ();
+    __builtin_amdgcn_sched_barrier (0);
+  };
+  if (t0 < t1)
+    issue (t0, lk0, lv0);
+  for (int t = t0; t < t1; t += 2)
+    {
+      step (t, lk0, lv0, lk1, lv1);
+      if (t + 1 < t1)
+        step (t + 1, lk1, lv1, lk0, lv0);
+    }
+  // the other half of the lanes has summed the other keys of the same query
+  sum += __shfl_xor (sum, 32, 64);
+  if (PARTS)
+    {
+      if (qrow >= a.S)
+        return;
+      typedef float f32x4 __attribute__ ((ext_vector_type (4)));
+      float *pr = part_row<HD> (a, part, head, qrow);
+      if (hh == 0)
+        *(VKL_GLOBAL f32x4 *)(pr + HD) = f32x4{ m * c, sum, 0.f, 0.f };
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *(VKL_GLOBAL f32x4 *)(pr + 32 * db + 8 * g + 4 * hh)
+              = f32x4{ oacc[db][4 * g], oacc[db][4 * g + 1], oacc[db][4 * g + 2], oacc[db][4 * g + 3] };
+      return;
+    }
+  float inv = 1.0f / sum;
+  if (a.gate)
+    inv = inv / (1.0f + expf (-vkl::ldg (a.gate + (size_t)min (qrow, a.S - 1) * a.gs + head)));
+  if (qrow >= a.S)
+    return;
+  uint16_t *op = a.out + (size_t)qrow * a.ors + (size_t)head * a.ohs;
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      {
+        const int d = 32 * db + 8 * g + 4 * hh;
+        u32x2 w;
+        w.x = (uint32_t)E::bits (oacc[db][4 * g] * inv) | ((uint32_t)E::bits (oacc[db][4 * g + 1] * inv) << 16);
+        w.y = (uint32_t)E::bits (oacc[db][4 * g + 2] * inv) | ((uint32_t)E::bits (oacc[db][4 * g + 3] * inv) << 16);
+        *(VKL_GLOBAL u32x2 *)(op + d) = w;
+      }
+}
+
+// adds the parts of the keys up: one wave per query row and head
+template <int HD, class E>
+__global__ __launch_bounds__ (256) void
+attn_parts_kernel (const AttnArgs a)
+{
+  constexpr int VPL = HD / 64; // values per lane
+  const int i = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const int row = i / a.H, head = i - row * a.H;
+  if (row >= a.S)
+    return;
+  // lane p looks at part p
+  float pm = -3.0e38f, ps = 0.f;
+  if (lane < a.parts)
+    {
+      const float *pr = part_row<HD> (a, lane, head, row);
+      pm = vkl::ldg (pr + HD), ps = vkl::ldg (pr + HD + 1);
+    }
+  float top = pm;
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1)
+    top = fmaxf (top, __shfl_xor (top, d, 64));
+  const float w = lane < a.parts ? __builtin_amdgcn_exp2f (pm - top) : 0.f;
+  float total = w * ps;
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1)
+    total += __shfl_xor (total, d, 64);
+  float o[VPL];
+#pragma unroll
+  for (int e = 0; e < VPL; ++e)
+    o[e] = 0.f;
+  for (int p = 0; p < a.parts; ++p)
+    {
+      const float wp = __shfl (w, p, 64);
+      const float *pr = part_row<HD> (a, p, head, row) + lane * VPL;
+#pragma unroll
+      for (int e = 0; e < VPL; ++e)
+        o[e] = __builtin_fmaf (wp, vkl::ldg (pr + e), o[e]);
+    }
+  float inv = 1.0f / total;
+  if (a.gate)
+    inv = inv / (1.0f + expf (-vkl::ldg (a.gate + (size_t)row * a.gs + head)));
+  uint16_t *op = a.out + (size_t)row * a.ors + (size_t)head * a.ohs + lane * VPL;
+  if constexpr (VPL == 2)
+    *(VKL_GLOBAL uint32_t *)op = (uint32_t)E::bits (o[0] * inv) | ((uint32_t)E::bits (o[1] * inv) << 16);
+  else
+    *op = E::bits (o[0] * inv);
+}
+
+// Into how many parts the keys go, where two workgroups fit a compute unit and fewer than
+// half of those would exist: the number with the lowest estimated time, from a model fitted
+// to measurements at 8 to 40 heads, 1 to 900 query rows and 32 to 4000 keys (microseconds:
+// a tile of the longest row takes 1.15; parts cost a second launch and 0.45 per MB that they
+// write and it reads).  Measured, one part / as chosen: 32 heads of 128, 77 rows behind 1500
+// keys 34 / 18, 10 rows behind 4000 83 / 22, 200 behind 1800 40 / 27; 384 rows of their own
+// stay in one part (12; in two 20).
+int
+key_parts (const AttnArgs &a, int hd)
+{
+  const int groups = a.ntq * a.H, tiles = (a.L + kBKey - 1) / kBKey;
+  const double mb = (double)a.H * a.S * (hd + 4) * sizeof (float) * 1e-6;
+  int best = 1;
+  double least = 1.15 * tiles;
+  for (int p = 2; p <= 16 && p * groups <= 512 && p <= tiles; ++p)
+    {
+      const double cost = 5 + 1.15 * tiles / p + 0.45 * mb * p;
+      if (cost < least)
+        best = p, least = cost;
+    }
+  return best;
+}
+
+template <int HD, class E, bool CHUNKED>
+int
+launch_tiles (AttnArgs a, hipStream_t s)
+{
+  a.parts = key_parts (a, HD);
+  if (a.parts > 1)
+    {
+      // scratch of the stream, not allocated while the stream is captured
+      hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+      if (hipStreamIsCapturing (s, &capture) != hipSuccess)
+        (void)hipGetLastError (); // (the default stream while another one is captured)
+      else if (capture == hipStreamCaptureStatusNone
+               && (size_t)a.parts * a.H * a.S * (HD + 4) * sizeof (float) <= vkl::gemm_stream_workspace_bytes ())
+        a.ws = vkl::gemm_stream_workspace (s);
+    }
+  const int groups = a.ntq * a.H;
+  if (!a.ws)
+    {
+      a.parts = 1;
+      attn_tiles_kernel<HD, E, CHUNKED, false><<<dim3 ((unsigned)groups), dim3 (kThreads), 0, s>>> (a);
+      return vkl_launch_status ();
+    }
+  attn_tiles_kernel<HD, E, CHUNKED, true><<<dim3 ((unsigned)(groups * a.parts)), dim3 (kThreads), 0, s>>> (a);
+  attn_parts_kernel<HD, E><<<dim3 ((unsigned)((a.S * a.H + 3) / 4)), dim3 (256), 0, s>>> (a);
+  return vkl_launch_status ();
+}
+
 // ---------------------------------------------------------------------------
 // RoPE of Q and K and the K/V cache write, straight from the [S, H*hd]
 // outputs of the projections: one thread per 8 consecutive elements of a
@@ -532,12 +1019,8 @@ vkl_attn_prefill_causal_f16 (const void *q, const void *k, const void *v,
   a.H = H, a.S = S, a.L = L, a.ntq = (S + kBQ - 1) / kBQ;
   a.qcs = qcs, a.qhs = qhs, a.kcs = kcs, a.khs = khs, a.vcs = vcs, a.vhs = vhs;
   a.ors = ors, a.ohs = ohs, a.scale = scale;
-  const dim3 grid ((unsigned)(a.ntq * H));
-  if (hd == 128)
-    attn_prefill_kernel<128, F16Elem><<<grid, dim3 (kThreads), 0, (hipStream_t)stream>>> (a);
-  else
-    attn_prefill_kernel<64, F16Elem><<<grid, dim3 (kThreads), 0, (hipStream_t)stream>>> (a);
-  return vkl_launch_status ();
+  return hd == 128 ? launch_tiles<128, F16Elem, false> (a, (hipStream_t)stream)
+                   : launch_tiles<64, F16Elem, false> (a, (hipStream_t)stream);
 }
 
 namespace
@@ -550,9 +1033,9 @@ launch_prefill_bf16 (const AttnArgs &a, int hd, hipStream_t s)
   switch (hd)
     {
     case 32: attn_prefill_kernel<32, Bf16Elem, CHUNKED><<<grid, block, 0, s>>> (a); break;
-    case 64: attn_prefill_kernel<64, Bf16Elem, CHUNKED><<<grid, block, 0, s>>> (a); break;
+    case 64: return launch_tiles<64, Bf16Elem, CHUNKED> (a, s);
     case 96: attn_prefill_kernel<96, Bf16Elem, CHUNKED><<<grid, block, 0, s>>> (a); break;
-    case 128: attn_prefill_kernel<128, Bf16Elem, CHUNKED><<<grid, block, 0, s>>> (a); break;
+    case 128: return launch_tiles<128, Bf16Elem, CHUNKED> (a, s);
     case 160: attn_prefill_kernel<160, Bf16Elem, CHUNKED><<<grid, block, 0, s>>> (a); break;
     case 192: attn_prefill_kernel<192, Bf16Elem, CHUNKED><<<grid, block, 0, s>>> (a); break;
     case 224: attn_prefill_kernel<224, Bf16Elem, CHUNKED><<<grid, block, 0, s>>> (a); break;

@@ -166,6 +166,11 @@ int vkl_matmul_f16_nn (const void *a, const void *b, int C, int M, int N,
                        int K, size_t acs, size_t ahs, size_t bcs, size_t bhs,
                        size_t ycs, size_t yhs, float scale, float bias,
                        int act, void *y, void *stream);
+/* The three projections of src/ops/multiheadattention_v2.cpp:190-202 with fp16
+ * matrices, as vkl_kqv_q8_0: k = x Wk^T, q = x Wq^T, v = x Wv^T, all dense. */
+int vkl_kqv_f16 (const void *x, const void *wk, const void *wq,
+                 const void *wv, int M, int N, int K, void *k, void *q,
+                 void *v, void *stream);
 /* src/shaders/ffn_up_and_gate_fp16.comp */
 int vkl_ffn_upgate_f16 (const void *x, const void *wup, const void *wgate,
                         int M, int N, int K, void *out, void *stream);

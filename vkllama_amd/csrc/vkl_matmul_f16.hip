@@ -231,6 +231,34 @@ vkl_ffn_upgate_f16 (const void *x, const void *wup, const void *wgate, int M,
 }
 
 extern "C" int
+vkl_kqv_f16 (const void *x, const void *wk, const void *wq, const void *wv, int M, int N, int K, void *k, void *q,
+             void *v, void *stream)
+{
+  VKL_CHECK_ARG (x && wk && wq && wv && k && q && v && M > 0 && N > 0 && K > 0);
+  if (M >= vkl::kGemmMinRowsF16)
+    {
+      vkl::GemmArgs g = {};
+      g.x = (const uint16_t *)x, g.xs = (size_t)K;
+      g.M = M, g.N = N, g.K = K, g.Kp = (K + 31) / 32 * 32;
+      g.wtype = 1, g.nmat = 3;
+      g.wh[0] = (const uint16_t *)wk, g.wh[1] = (const uint16_t *)wq, g.wh[2] = (const uint16_t *)wv;
+      g.ws = (size_t)K;
+      g.y[0] = (uint16_t *)k, g.y[1] = (uint16_t *)q, g.y[2] = (uint16_t *)v;
+      g.ys = (size_t)N;
+      g.scale = 1.f;
+      if (vkl::gemm_mfma_supported (g))
+        return vkl::gemm_mfma_launch (g, (hipStream_t)stream);
+    }
+  const void *w[3] = { wk, wq, wv };
+  void *y[3] = { k, q, v };
+  for (int i = 0; i < 3; ++i)
+    if (int e = vkl_matmul_f16_tb (x, w[i], 1, M, N, K, 0, (size_t)K, 0, (size_t)K, 0, (size_t)N, 1.f, 0.f, 0, nullptr, y[i],
+                                   nullptr, stream))
+      return e;
+  return 0;
+}
+
+extern "C" int
 vkl_matmul_f16_nn (const void *a, const void *b, int C, int M, int N, int K,
                    size_t acs, size_t ahs, size_t bcs, size_t bhs, size_t ycs,
                    size_t yhs, float scale, float bias, int act, void *y,

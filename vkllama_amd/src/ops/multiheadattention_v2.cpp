@@ -146,7 +146,12 @@ MultiHeadAttentionV2::operator() (Tensor X, const size_t offset) noexcept
         offset, offset + S, maxlen_));
 
   Tensor k, q, v;
-  if (wk_.dtype () == Q8_0)
+  // one launch for the three projections (fp16 matrices: of one token row they
+  // run one by one on the weight-streaming kernel)
+  auto same = [this] (const Tensor &w) {
+    return w.dtype () == wk_.dtype () && w.height () == wk_.height () && w.width () == wk_.width ();
+  };
+  if (wk_.dtype () == Q8_0 || (S > 2 && same (wq_) && same (wv_) && X.hs () == X.width () * 2))
     {
       if (!(k_.channels () == 1 && k_.height () == S && k_.width () == N))
         {
@@ -161,10 +166,10 @@ MultiHeadAttentionV2::operator() (Tensor X, const size_t offset) noexcept
       VKLLAMA_STATUS_OK (q_.reshape (1, S, N));
       VKLLAMA_STATUS_OK (v_.reshape (1, S, N));
       timer_.start (dev_);
-      const int err = vkl_kqv_q8_0 (X.data (), wk_.data (), wq_.data (),
-                                    wv_.data (), (int)S, (int)N,
-                                    (int)X.width (), k_.data (), q_.data (),
-                                    v_.data (), dev_->stream ());
+      const auto project = wk_.dtype () == Q8_0 ? vkl_kqv_q8_0 : vkl_kqv_f16;
+      const int err = project (X.data (), wk_.data (), wq_.data (), wv_.data (),
+                               (int)S, (int)N, (int)X.width (), k_.data (),
+                               q_.data (), v_.data (), dev_->stream ());
       timer_.stop (dev_);
       VKLLAMA_STATUS_OK (launch_status ("kqv", err));
       k = k_, q = q_, v = v_;

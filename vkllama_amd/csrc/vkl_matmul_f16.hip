@@ -230,6 +230,10 @@ vkl_ffn_upgate_f16 (const void *x, const void *wup, const void *wgate, int M,
   return launch_tb (p, true, (hipStream_t)stream);
 }
 
+// The three projections as one product over three matrices (what vkl_kqv_q8_0 does for
+// Q8_0): apart, each fills a part of the chip only and has a reduction of its own where its
+// k range is split.  Three 7B layers, one launch each against three: 77 rows 642 -> 592 us,
+// 2048 rows 2345 -> 2309.
 extern "C" int
 vkl_kqv_f16 (const void *x, const void *wk, const void *wq, const void *wv, int M, int N, int K, void *k, void *q,
              void *v, void *stream)

@@ -1081,9 +1081,14 @@ wide_reduce_seg_kernel (const GemmSegArgs a, const float *ws, int parts)
   gemm_finish8<false> (a, v, g, m, n, 0, 0, nullptr);
 }
 
-// As wide_plan (the same cost model; it holds for bf16), with every row count
-// allowed and, where the tiles are few, up to 16 parts of at least 4 k-steps:
-// with few token rows the workgroups exist to stream the weights.
+// As wide_plan, with every row count allowed and, where the tiles are few, up to 16 parts
+// of at least 4 k-steps: with few token rows the workgroups exist to stream the weights.
+// The model is fitted to the products of this form (microseconds: a round of 256-row tiles
+// 0.79 per k-step + 5, of 128-row tiles 0.47 + 4, cut tiles likewise; a reduction launch 5
+// + its bytes at 2.5 TB/s).  wide_plan's own fit, of the slower Q8_0 rounds, kept 128-row
+// tiles too long and split too much; with it / with this one (rows x N x K): 1500 x 12544 x
+// 4096 161 / 145 us, 1000 x 11008 x 4096 94 / 86, 1500 x 5504 x 2048 51 / 46, 500 x 2048 x
+// 2048 21 / 14, 150 x 2048 x 2048 15 / 13; of 88 products no other plan was slower.
 WidePlan
 wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
 {
@@ -1098,10 +1103,13 @@ wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
         if (ks > 1
             && (nk / ks < 4 || (size_t)ks * a.M * a.N * sizeof (float) > scratch))
           continue;
-        const long groups = (long)((a.M + bm - 1) / bm) * ((a.N + WBN - 1) / WBN) * ks;
-        const double round = (bm == WBM ? 0.95 : 0.55) * nk / ks + (bm == WBM ? 8 : 6);
+        const WideGrid tiles ((a.M + bm - 1) / bm, (a.N + WBN - 1) / WBN, 1, ks, bm == WBM);
+        const int whole = (tiles.whole + WideGrid::kUnits - 1) / WideGrid::kUnits;
+        const double steps = (double)nk / ks;
+        const double round = bm == WBM ? 0.79 * steps + 5 : 0.47 * steps + 4;
+        const double cut = tiles.whole < tiles.tiles () ? 0.47 * steps + 4 : 0;
         const double reduce = ks > 1 ? 5 + (double)ks * a.M * a.N * sizeof (float) / 2.5e6 : 0;
-        const double cost = (double)((groups + 255) / 256) * round + reduce;
+        const double cost = whole * round + cut + reduce;
         if (!best.bm || cost < best_cost)
           best = { bm, ks }, best_cost = cost;
       }

@@ -574,10 +574,26 @@ layer_launch_supported (const vkl_decode_model &m, int G)
          && 2 * (lds_bytes_needed (m.dim, m.ffn, m.maxlen, m.head_dim) + 32) <= 160 * 1024;
 }
 
+// Workgroups of a layer launch out of the G that fit (two per compute unit).  A layer of
+// little weight is bound by its hand-overs, not by the bytes in flight: half the workgroups
+// are half the arrivals to count and half the copies of the row to stage.  us per token, G /
+// G / 2, 8 layers, by MB of weights per layer: 3 (512 wide) 185 / 169, 14 197 / 182, 54 (2048
+// Q8_0) 261 / 236, 84 290 / 277, 101 (2048 fp16) 277 / 263, 120 321 / 317, 158 346 / 371, 215
+// (4096 Q8_0, 4 layers) 222 / 235.  Heads that take more than an eighth of the half leave the
+// phases beside them too few.
+static int
+layer_groups (const vkl_decode_model &m, int G)
+{
+  const double per = m.wtype == 8 ? 34.0 / 32.0 : 2.0;
+  const double bytes = (4.0 * m.dim * m.dim + 3.0 * (double)m.dim * m.ffn) * per;
+  return bytes <= 110e6 && m.n_heads * 8 <= G / 2 && (G / 2) % 8 == 0 ? G / 2 : G;
+}
+
 int
 launch_layer (const Params &p, const vkl_layer_weights &lw, int layer, int G,
               hipStream_t s)
 {
+  G = layer_groups (p.m, G);
   return p.m.wtype == 8 ? launch_layer_wt<8> (p, lw, layer, G, s)
                         : launch_layer_wt<1> (p, lw, layer, G, s);
 }

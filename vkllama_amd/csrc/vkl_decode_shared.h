@@ -567,8 +567,8 @@ flags_equal_scalar (const uint32_t *flag, int nflags, uint32_t want)
 }
 
 // One layer of the step as a single launch (vkl_decode_layer.hip): K/Q/V,
-// attention with one workgroup per head, Wo, up/gate, down.  G workgroups that
-// must all be resident at once.
+// attention with one workgroup per head, Wo, up/gate, down.  G workgroups (or half, where
+// a layer has little weight) that must all be resident at once.
 bool layer_launch_supported (const vkl_decode_model &m, int G);
 int launch_layer (const Params &p, const vkl_layer_weights &lw, int layer, int G, hipStream_t s);
 // the token's embedding row -> residual stream (one small launch in front of layer 0)

@@ -126,6 +126,9 @@ int vkl_decode_step (const vkl_decode_model *m, const uint32_t *tok,
  * repeats the step with mode 0 and separate_attn_wo = 1, which wait for
  * nothing.  No counterpart in the reference, which has no such kernels. */
 int vkl_decode_status (const vkl_decode_model *m, void *stream);
+/* the device word that vkl_decode_status looks at: zero if nothing of the kind
+ * happened (null for a model without scratch) */
+const uint32_t *vkl_decode_status_word (const vkl_decode_model *m);
 
 /* n_steps greedy tokens without a host round trip per token: step i reads
  * ids[i] (device memory) at position pos0 + i and writes its arg-max id to

@@ -57,6 +57,9 @@ int vkl_host_free_h (void *p);
 int vkl_memcpy_h2d (void *dst, const void *src_h, size_t bytes, void *stream);
 int vkl_memcpy_d2h (void *dst_h, const void *src, size_t bytes, void *stream);
 int vkl_memcpy_d2d (void *dst, const void *src, size_t bytes, void *stream);
+/* n 32-bit words and, if `word` is given, *word behind them (dst[n]) to pinned
+ * host memory by one launch: there once the stream has been synchronised */
+int vkl_send_words (const void *src, size_t n, const void *word, void *dst_pinned, void *stream);
 int vkl_memset (void *dst, int value, size_t bytes, void *stream);
 /* free and total device memory in bytes (the budget query of the reference's
  * allocator, src/core/allocator.cpp, as far as callers need it) */

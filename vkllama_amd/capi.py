@@ -47,6 +47,7 @@ SIGNATURES = {
     "vkl_host_free_h": (i32, [vp]),
     "vkl_memcpy_h2d": (i32, [vp, vp, sz, vp]),
     "vkl_memcpy_d2h": (i32, [vp, vp, sz, vp]),
+    "vkl_send_words": (i32, [vp, sz, vp, vp, vp]),
     "vkl_memcpy_d2d": (i32, [vp, vp, sz, vp]),
     "vkl_memset": (i32, [vp, i32, sz, vp]),
     "vkl_copy_kernel": (i32, [vp, vp, sz, vp]),

@@ -1215,6 +1215,14 @@ vkl_decode_flags_release (void *flags)
       }
 }
 
+extern "C" const uint32_t *
+vkl_decode_status_word (const vkl_decode_model *m)
+{
+  if (!m || !m->scratch)
+    return nullptr;
+  return carve (m->scratch, m->dim, m->ffn, m->vocab, m->n_heads, m->maxlen, m->head_dim, m->n_layers).sync + 1;
+}
+
 extern "C" int
 vkl_decode_status (const vkl_decode_model *m, void *stream)
 {

@@ -202,11 +202,9 @@ vkl_model_forward (vkl_model *m, const uint32_t *toks, size_t n_toks,
   try
     {
       std::vector<uint32_t> v (toks, toks + n_toks);
-      auto r = (*m->model) (v, offset);
-      if (!r.ok ())
-        return fail (m, r.status ());
-      const size_t V = m->model->vocab_size ();
-      std::copy (r->end () - V, r->end (), logits);
+      const auto st = m->model->forward_rows_into (v, offset, { (uint32_t)(n_toks ? n_toks - 1 : 0) }, logits);
+      if (!st.ok ())
+        return fail (m, st);
     }
   catch (const std::exception &e)
     {
@@ -223,11 +221,10 @@ vkl_model_forward_rows (vkl_model *m, const uint32_t *toks, size_t n_toks, size_
     return (int)absl::StatusCode::kInvalidArgument;
   try
     {
-      auto r = m->model->forward_rows (std::vector<uint32_t> (toks, toks + n_toks), offset,
-                                       std::vector<uint32_t> (rows, rows + n_rows));
-      if (!r.ok ())
-        return fail (m, r.status ());
-      std::copy (r->begin (), r->end (), logits);
+      const auto st = m->model->forward_rows_into (std::vector<uint32_t> (toks, toks + n_toks), offset,
+                                                   std::vector<uint32_t> (rows, rows + n_rows), logits);
+      if (!st.ok ())
+        return fail (m, st);
     }
   catch (const std::exception &e)
     {

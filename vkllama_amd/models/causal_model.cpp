@@ -50,6 +50,15 @@ CausalModel::operator() (std::vector<uint32_t> const &toks, const size_t offset)
 absl::StatusOr<std::vector<float> >
 CausalModel::forward_rows (std::vector<uint32_t> const &toks, const size_t offset, std::vector<uint32_t> const &rows)
 {
+  std::vector<float> out (rows.size () * vocab_);
+  VKLLAMA_STATUS_OK (forward_rows_into (toks, offset, rows, out.data ()));
+  return out;
+}
+
+absl::Status
+CausalModel::forward_rows_into (std::vector<uint32_t> const &toks, const size_t offset, std::vector<uint32_t> const &rows,
+                                float *out)
+{
   StepPlan *plan = plan_ptr_ ();
   if (!plan)
     return absl::InternalError ("model used before init()");
@@ -58,35 +67,41 @@ CausalModel::forward_rows (std::vector<uint32_t> const &toks, const size_t offse
     if (r >= toks.size ())
       return absl::OutOfRangeError (absl::StrFormat ("row %u of a pass over %zu tokens", r, toks.size ()));
   VKLLAMA_STATUS_OK (begin_pass_ (offset));
-  std::vector<float> out (rows.size () * vocab_);
   if (fused_decode_ && toks.size () == 1 && plan->usable ())
     {
+      float *first = rows.empty () ? nullptr : out;
       VKLLAMA_STATUS_OK (wait_all_ ());
       VKLLAMA_STATUS_OK (plan->step_host_token (toks[0], offset));
-      std::vector<float> one (vocab_);
-      auto rs = plan->read_logits (one.data ());
+      auto rs = plan->read_logits (first);
       if (absl::IsUnavailable (rs))
         {
           // a wait between workgroups gave up; the plan has switched to the
           // launches that wait for nothing: the same step once more
           ++decode_recoveries_;
           VKLLAMA_STATUS_OK (plan->step_host_token (toks[0], offset));
-          rs = plan->read_logits (one.data ());
+          rs = plan->read_logits (first);
         }
       VKLLAMA_STATUS_OK (rs);
-      for (size_t i = 0; i < rows.size (); ++i)
-        std::copy (one.begin (), one.end (), out.begin () + i * vocab_);
+      for (size_t i = 1; i < rows.size (); ++i)
+        std::copy (out, out + vocab_, out + i * vocab_);
       end_pass_ (offset + 1);
-      return out;
+      return absl::OkStatus ();
     }
   auto logits = forward_ (toks, offset, rows);
   VKLLAMA_STATUS_OK (logits);
-  if (!rows.empty ())
-    if (int e = vkl_memcpy_d2h (out.data (), logits->data (), out.size () * sizeof (float), gpu_->stream ()))
+  // (one row by way of the plan's pinned row; more are copied where they go)
+  if (rows.size () == 1)
+    {
+      VKLLAMA_STATUS_OK (plan->send_row ((const float *)logits->data ()));
+    }
+  else if (!rows.empty ())
+    if (int e = vkl_memcpy_d2h (out, logits->data (), rows.size () * vocab_ * sizeof (float), gpu_->stream ()))
       return absl::InternalError (vkl_error_string (e));
   VKLLAMA_STATUS_OK (wait_all_ ());
+  if (rows.size () == 1)
+    std::copy (plan->received (), plan->received () + vocab_, out);
   end_pass_ (offset + toks.size ());
-  return out;
+  return absl::OkStatus ();
 }
 
 // the next token from the logits of the last pass: arg-max, or a draw from

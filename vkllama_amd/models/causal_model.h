@@ -28,6 +28,10 @@ public:
   // none): [rows, vocab]
   absl::StatusOr<std::vector<float> > forward_rows (std::vector<uint32_t> const &toks, const size_t offset,
                                                     std::vector<uint32_t> const &rows);
+  // the same into memory of the caller, which a pass that fails may have
+  // written in part
+  absl::Status forward_rows_into (std::vector<uint32_t> const &toks, const size_t offset,
+                                  std::vector<uint32_t> const &rows, float *out);
 
   // single tokens on the fused step (default) or on the operator chain
   void set_fused_decode (bool on) { fused_decode_ = on; }

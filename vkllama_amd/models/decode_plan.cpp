@@ -196,6 +196,12 @@ DecodePlan::set_option (const char *name, int value)
   return true;
 }
 
+const uint32_t *
+DecodePlan::error_word () const
+{
+  return usable_ ? vkl_decode_status_word (&desc_) : nullptr;
+}
+
 absl::Status
 DecodePlan::check ()
 {

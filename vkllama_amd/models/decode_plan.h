@@ -38,6 +38,7 @@ struct DecodePlan : public StepPlan
   // (vkl_decode_status)?  If so the plan switches to the launches that wait for
   // nothing (mode 0, attention and Wo apart) and the status is Unavailable.
   absl::Status check () override;
+  const uint32_t *error_word () const override;
 
 private:
   bool usable_;

@@ -3,6 +3,7 @@
 #include "src/core/gpu_device.h"
 #include "vkl_decode.h"
 #include "vkl_hip.h"
+#include <string.h>
 
 namespace vkllama
 {
@@ -23,6 +24,8 @@ StepPlan::create_buffers (GPUDevice *gpu, size_t vocab)
   vocab_ = vocab;
   tok_slot_ = Tensor (1, 1, 1, gpu, UINT32, true);
   VKLLAMA_STATUS_OK (tok_slot_.create ());
+  row_h_ = Tensor (1, 1, (int)vocab_ + 1, gpu, FP32, true);
+  VKLLAMA_STATUS_OK (row_h_.create ());
   logits32_ = Tensor (1, 1, (int)vocab_, gpu, FP32, false);
   return logits32_.create ();
 }
@@ -54,12 +57,25 @@ StepPlan::current_logits () const
 }
 
 absl::Status
+StepPlan::send_row (const float *row, const uint32_t *word)
+{
+  return hip_status ("downloading logits", vkl_send_words (row, vocab_, word, row_h_.host (), gpu_->stream ()));
+}
+
+absl::Status
 StepPlan::read_logits (float *dst)
 {
-  VKLLAMA_STATUS_OK (hip_status ("downloading logits", vkl_memcpy_d2h (dst, current_logits (), vocab_ * sizeof (float),
-                                                                       gpu_->stream ())));
+  const uint32_t *word = error_word ();
+  VKLLAMA_STATUS_OK (send_row (current_logits (), word));
   VKLLAMA_STATUS_OK (hip_status ("downloading logits", vkl_stream_sync (gpu_->stream ())));
-  return check ();
+  uint32_t failed = 0;
+  if (word)
+    memcpy (&failed, received () + vocab_, sizeof (failed));
+  if (failed)
+    VKLLAMA_STATUS_OK (check ());
+  if (dst)
+    memcpy (dst, received (), vocab_ * sizeof (float));
+  return absl::OkStatus ();
 }
 
 absl::Status

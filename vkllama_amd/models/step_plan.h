@@ -37,8 +37,13 @@ public:
 
   // token id given by the host
   absl::Status step_host_token (uint32_t tok, size_t offset);
-  // copies the fp32 logits of the last step (fused or adopted) to the host
+  // copies the fp32 logits of the last step (fused or adopted) to the host once
+  // check () has passed
   absl::Status read_logits (float *dst);
+  // queues one row of logits for received (), which holds it after the stream
+  // has been synchronised
+  absl::Status send_row (const float *row, const uint32_t *word = nullptr);
+  const float *received () { return (const float *)row_h_.host (); }
   // remember the fp32 logits tensor of an operator-chain pass
   absl::Status adopt_logits (Tensor logits32);
   // arg-max of the current logits into device-visible memory
@@ -49,11 +54,14 @@ public:
 
 protected:
   absl::Status create_buffers (GPUDevice *gpu, size_t vocab);
+  // device word that is zero if check () would pass; null: it always does
+  virtual const uint32_t *error_word () const { return nullptr; }
   static absl::Status hip_status (const char *what, int e);
   const float *current_logits () const;
   GPUDevice *gpu_ = nullptr;
   Tensor logits32_; // fp32 [vocab] written by the fused step
   Tensor tok_slot_; // pinned uint32
+  Tensor row_h_;    // pinned: a row of logits and a status word
   Tensor adopted_;  // logits of the operator chain, if newer
   bool adopted_valid_ = false;
   size_t vocab_ = 0;

@@ -96,7 +96,8 @@ size_t vkl_decode_scratch_bytes (const vkl_decode_model *m);
 /* One token at KV position `pos` (context length becomes pos + 1).
  *  tok      device-visible uint32: the input token id (ids >= vocab -> 0)
  *  mode     0 = one launch per phase (attention and Wo share one below the
- *           split length); 1 = one launch per layer: all workgroups stay
+ *           split length); 1 = one launch per layer, or for all layers where
+ *           rows are narrow (up to about 1792 values): all workgroups stay
  *           resident through the five phases, hand activations over through
  *           memory with bounded waits for one another, and have the next
  *           phase's weights on the way meanwhile.  Results are bit for bit

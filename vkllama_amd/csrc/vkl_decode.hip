@@ -1027,14 +1027,18 @@ launch_step (const Params &p, const vkl_decode_model *m, int mode, int n_cu, int
   if (per_layer && !(p.loop && !p.sample))
     if (int e = launch_embed_row (p, s))
       return e;
-  for (int l = 0; l < m->n_layers; ++l)
+  const bool many = per_layer && layers_launch_supported (*m, n_cu);
+  if (many && !g_timer.on)
+    if (int e = launch_layers (p, 0, m->n_layers, s))
+      return e;
+  for (int l = 0; l < m->n_layers && !(many && !g_timer.on); ++l)
     {
       const vkl_layer_weights &lw = m->layers_h[l];
       if (per_layer)
         {
           if (int e = timer_mark (PH_LAYER, false, s))
             return e;
-          if (int e = launch_layer (p, lw, l, G, s))
+          if (int e = many ? launch_layers (p, l, 1, s) : launch_layer (p, lw, l, G, s))
             return e;
           if (int e = timer_mark (PH_LAYER, true, s))
             return e;
@@ -1515,7 +1519,7 @@ vkl_decode_phase_replay (const vkl_decode_model *m, int kind, uint32_t pos,
               err = launch_phase<PH_UPGATE> (p, lw, l, G, G, lds, s);
               break;
             case PH_LAYER:
-              err = launch_layer (p, lw, l, G, s);
+              err = layers_launch_supported (*m, n_cu) ? launch_layers (p, l, 1, s) : launch_layer (p, lw, l, G, s);
               break;
             default:
               err = launch_phase<PH_DOWN> (p, lw, l, G, G, lds, s);

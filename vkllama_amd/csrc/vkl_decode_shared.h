@@ -30,8 +30,34 @@ struct Scratch
   float *part_sum;    // [heads][kAttnChunks]
   float *part_out;    // [heads][kAttnChunks][head_dim]
   uint32_t *attn_cnt; // [heads] chunks of the head that have published their part (zero between launches)
+  // several layers in one launch (vkl_decode_layers.hip); null for wider rows
+  uint32_t *tagged;   // rows of words that carry a value and a tag, TaggedRows
   size_t bytes;
 };
+
+// The rows that workgroups of one launch hand to one another as words {tag, fp16 value}: a
+// reader knows by the tag that a word has arrived.  k | q | v are read by one workgroup per
+// head; the others by all, from one copy per XCD.
+constexpr int kTagCopies = 8;
+constexpr int kTaggedMaxDim = 2048; // rows of up to so many (and three times as many) values
+struct TaggedRows
+{
+  // words from Scratch::tagged: rows, and from copy to copy
+  int kqv, att, xm, x, t, copy_d, copy_f, words;
+};
+
+__host__ __device__ inline TaggedRows
+tagged_rows (int dim, int ffn)
+{
+  TaggedRows r;
+  r.copy_d = (dim + 63) & ~63, r.copy_f = (ffn + 63) & ~63;
+  r.kqv = 0, r.att = 3 * r.copy_d;
+  r.xm = r.att + kTagCopies * r.copy_d;
+  r.x = r.xm + kTagCopies * r.copy_d;
+  r.t = r.x + kTagCopies * r.copy_d;
+  r.words = r.t + kTagCopies * r.copy_f;
+  return r;
+}
 
 constexpr int kLayerSyncBytes = 12288; // see vkl_decode_layer.hip
 constexpr int kAttnChunks = 32;      // upper bound on chunks per head
@@ -69,6 +95,9 @@ carve (void *base, int dim, int ffn, int vocab, int heads, int maxlen, int hd,
   s.part_sum = (float *)(p + o), o += align256 ((size_t)heads * kAttnChunks * 4);
   s.part_out = (float *)(p + o), o += align256 ((size_t)heads * kAttnChunks * hd * 4);
   s.attn_cnt = (uint32_t *)(p + o), o += align256 ((size_t)heads * 4);
+  const bool tagged = dim <= kTaggedMaxDim && ffn <= 3 * dim;
+  s.tagged = tagged ? (uint32_t *)(p + o) : nullptr;
+  o += tagged ? align256 ((size_t)tagged_rows (dim, ffn).words * 4) : 0;
   s.bytes = o;
   return s;
 }
@@ -185,13 +214,45 @@ struct NoWait
   __device__ __forceinline__ bool operator() () const { return true; }
 };
 
+// Where a head finds this token's k, q and v (three rows behind one another; the head's values
+// from `first` on, pair pi of them) and leaves its output.
+template <bool COH> struct PlainRows
+{
+  __device__ __forceinline__ int
+  thread () const
+  {
+    return (int)threadIdx.x;
+  }
+  __device__ __forceinline__ uint32_t
+  pair (const Params &p, bool is_k, bool is_v, int first, int pi) const
+  {
+    const int dim = p.m.dim;
+    const uint16_t *kin = p.s.kqv + first, *qin = p.s.kqv + dim + first, *vin = p.s.kqv + 2 * dim + first;
+    return ld_u32<COH> ((const uint32_t *)(is_k ? kin : (is_v ? vin : qin)) + pi);
+  }
+  // column `at` has the value o and its right neighbour `next`; four lanes
+  // call for each column, `lane` numbers the eight of a pair of columns
+  __device__ __forceinline__ void
+  put (const Params &p, int at, int lane, float o, float next) const
+  {
+    if (lane == 0)
+      st_u32<COH> ((uint32_t *)(p.s.att + at), (uint32_t)f2h (o) | ((uint32_t)f2h (next) << 16));
+  }
+  __device__ __forceinline__ bool
+  live () const
+  {
+    return true;
+  }
+};
+
 // EARLY: the cached rows are requested first, then `wait` is called (it waits
 // for the producers of this token's q, k and v inside the same launch; false:
 // give up, nothing is stored), then q, k and v are read.
-template <int HD, bool COH, bool EARLY = false, typename Wait = NoWait>
+template <int HD, bool COH, bool EARLY = false, typename Wait = NoWait, typename Rows = PlainRows<COH> >
 __device__ __forceinline__ void
 attention_head (const Params &p, const vkl_layer_weights &lw, int head,
-                uint8_t *lds, unsigned long long *tr = nullptr, Wait wait = Wait ())
+                uint8_t *lds, unsigned long long *tr = nullptr, Wait wait = Wait (),
+                const Rows rows = Rows ())
 {
 #ifdef VKL_TRACE
 #define VKL_TRA(slot)                                                         \
@@ -203,7 +264,7 @@ attention_head (const Params &p, const vkl_layer_weights &lw, int head,
   constexpr int LPR = HD / 8;            // lanes per cache row (16 B each)
   constexpr int RPB = kDecThreads / LPR; // cache rows per sweep
   constexpr int PRE = 8;                 // sweeps prefetched up front
-  const int dim = p.m.dim, maxlen = p.m.maxlen;
+  const int maxlen = p.m.maxlen;
   const uint32_t pos = step_pos (p);
   const int L = (int)pos + 1;
   uint16_t *qk = (uint16_t *)lds;    // [3*HD]
@@ -212,10 +273,7 @@ attention_head (const Params &p, const vkl_layer_weights &lw, int head,
   float *red = part + RPB * HD;           // [2*kDecWaves]
   uint16_t *kc = (uint16_t *)lw.kcache + (size_t)head * maxlen * HD;
   uint16_t *vc = (uint16_t *)lw.vcache + (size_t)head * maxlen * HD;
-  const uint16_t *kin = p.s.kqv + head * HD;
-  const uint16_t *qin = p.s.kqv + dim + head * HD;
-  const uint16_t *vin = p.s.kqv + 2 * dim + head * HD;
-  const int tid = threadIdx.x;
+  const int tid = rows.thread ();
   const int sub = tid % LPR, grp = tid / LPR;
 
   // This token's q, k, v and its rotation factors are requested first and
@@ -232,7 +290,7 @@ attention_head (const Params &p, const vkl_layer_weights &lw, int head,
   float fc = 0.f, fs = 0.f;
   if (!EARLY)
     {
-      inw = ld_u32<COH> ((const uint32_t *)(is_k ? kin : (is_v ? vin : qin)) + pi);
+      inw = rows.pair (p, is_k, is_v, head * HD, pi);
       fc = ldg (p.m.freqc + (size_t)pos * (HD / 2) + pi);
       fs = ldg (p.m.freqs + (size_t)pos * (HD / 2) + pi);
       // (the scheduler must not move the cache rows ahead of these)
@@ -253,7 +311,7 @@ attention_head (const Params &p, const vkl_layer_weights &lw, int head,
       fs = ldg (p.m.freqs + (size_t)pos * (HD / 2) + pi);
       if (!wait ())
         return;
-      inw = ld_u32<COH> ((const uint32_t *)(is_k ? kin : (is_v ? vin : qin)) + pi);
+      inw = rows.pair (p, is_k, is_v, head * HD, pi);
     }
 
   // RoPE on adjacent pairs at position pos.  The new K and V rows are used
@@ -406,11 +464,12 @@ attention_head (const Params &p, const vkl_layer_weights &lw, int head,
       }
     o = row_sum<4> (o);
     const float onext = dpp_get<0x104> (o); // row_shl:4: the lane four up
-    if (c < HD && (tid & 7) == 0)
-      st_u32<COH> ((uint32_t *)(p.s.att + head * HD) + (c >> 1),
-                   (uint32_t)f2h (o) | ((uint32_t)f2h (onext) << 16));
+    if (c < HD)
+      rows.put (p, head * HD + c, tid & 7, o, onext);
   }
   __syncthreads ();
+  if (!rows.live ())
+    return;
   if (is_k)
     stg ((uint32_t *)(kc + (size_t)pos * HD) + pi, rot);
   if (is_v)
@@ -571,6 +630,10 @@ flags_equal_scalar (const uint32_t *flag, int nflags, uint32_t want)
 // a layer has little weight) that must all be resident at once.
 bool layer_launch_supported (const vkl_decode_model &m, int G);
 int launch_layer (const Params &p, const vkl_layer_weights &lw, int layer, int G, hipStream_t s);
+// Layers first .. first + count - 1 in one launch (vkl_decode_layers.hip): narrow rows, whose
+// layers are bound by their hand-overs.  At most one workgroup per compute unit, all resident.
+bool layers_launch_supported (const vkl_decode_model &m, int n_cu);
+int launch_layers (const Params &p, int first, int count, hipStream_t s);
 // the token's embedding row -> residual stream (one small launch in front of layer 0)
 int launch_embed_row (const Params &p, hipStream_t s);
 } // namespace dec

@@ -19,9 +19,25 @@ pytestmark = pytest.mark.gpu
     (1792, 5408, 14, 8, 3, 64),    # more than three pairs for a wave: a launch per layer
 ])
 def test_all_layers_in_one_launch(dim, ffn, heads, wtype, prompt, maxlen):
-    cfg = dict(dim=dim, n_layers=3, n_heads=heads, ffn=ffn, vocab=642, maxlen=maxlen, eps=1e-5, wtype=wtype)
+    compare(dim, ffn, heads, wtype, prompt, maxlen, 642)
+
+
+@pytest.mark.parametrize("dim,wtype,vocab", [
+    (64, 8, 2),             # one wave has the vocabulary
+    (64, 1, 95234),         # two rounds of what the waves hold, of no round number
+    (512, 8, 32000),
+    (512, 1, 70654),        # one row of each in every load, two rounds
+    (1024, 8, 43006),       # as many as the one launch takes
+    (1024, 8, 43012),       # more: a launch of its own
+])
+def test_whole_step_in_one_launch(dim, wtype, vocab):
+    compare(dim, 3 * dim // 64 * 32, max(1, dim // 128), wtype, 3, 64, vocab)
+
+
+def compare(dim, ffn, heads, wtype, prompt, maxlen, vocab):
+    cfg = dict(dim=dim, n_layers=3, n_heads=heads, ffn=ffn, vocab=vocab, maxlen=maxlen, eps=1e-5, wtype=wtype)
     m = M.Llama2(cfg, M.synth_weights(cfg, seed=dim))
-    ids0 = np.random.default_rng(dim).integers(3, 642, prompt).astype(np.uint32)
+    ids0 = np.random.default_rng(dim).integers(0, vocab, prompt).astype(np.uint32)
     runs = []
     for mode in (0, 1):
         m.set_option("decode_mode", mode)

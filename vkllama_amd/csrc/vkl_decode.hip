@@ -1022,6 +1022,12 @@ launch_step (const Params &p, const vkl_decode_model *m, int mode, int n_cu, int
   // the split attention take the launches per phase)
   const bool per_layer = mode == 1 && layer_launch_supported (*m, G)
                          && (int)p.pos + 1 < attn_split_min (*m);
+  if (per_layer && !g_timer.on && whole_step_supported (*m, n_cu))
+    {
+      if (int e = launch_step_whole (p, n_cu, s))
+        return e;
+      return p.loop && p.sample ? sample_loop_launch (p.logits32, m->vocab, p.sample, (uint32_t *)p.loop, p.ids, s) : 0;
+    }
   // (in a replayed greedy loop the previous step's lm_head launch has left the
   // row; the loop launches this once in front of its first step)
   if (per_layer && !(p.loop && !p.sample))
@@ -1364,6 +1370,16 @@ decode_loop (const vkl_decode_model *m, uint32_t *ids, uint32_t pos0, int n_step
       int upto = n_steps;
       if (!long_ctx)
         upto = (int)std::min<long long> (n_steps, (long long)attn_split_min (*m) - 1 - (long long)pos0);
+      // A step of one or a few launches needs no graph: with graphs of one node the GPU had 17 us
+      // without work between tokens (512 wide, 8 layers: 108 us per token, 103 launched), and
+      // the capture goes as well.
+      if (!long_ctx && mode == 1 && layer_launch_supported (*m, G) && layers_launch_supported (*m, n_cu))
+        {
+          p.pos = (uint32_t)std::min (attn_split_min (*m) - 2, m->maxlen - 1);
+          for (; done < upto && !err; ++done)
+            err = launch_step (p, m, mode, n_cu, G, lds, s);
+          continue;
+        }
       StepGraph *g = nullptr, *lru = &g_graphs[0];
       for (StepGraph &c : g_graphs)
         {

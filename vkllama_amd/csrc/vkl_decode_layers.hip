@@ -10,7 +10,8 @@
 // Us per layer at 512 values: 21.5 with a launch per layer, 14.4 in this form with a head on
 // some of the row workgroups and weights requested a phase ahead, 12.6 as below, 11.6 with a
 // workgroup's results as 32-byte stores (words of single waves: memory takes the partial
-// lines one by one), 11.1 with k, q and v gathered too and one SiLU for a wave's three pairs.
+// lines one by one), 11.1 with k, q and v gathered too and one SiLU for a wave's three pairs,
+// 9.9 with two rows of up to 512 bytes side by side in a wave.
 //
 // Rows: dim / 8 workgroups of eight waves, a wave owns row g of each of the square matrices
 // (k, q, v, o, down) and two or three up/gate pairs, g its number among dim waves; all its
@@ -45,7 +46,7 @@ static_assert ((kLsTags + 32) * 4 <= kLayerSyncBytes, "layer-sync area too small
 constexpr int kSyncErr = 1;   // word of Scratch::sync: a wait gave up
 constexpr int kTagSpinLimit = 1 << 14;
 constexpr int kPairs = 3;     // up/gate pairs of a wave, at most
-enum Stage { ST_KQV = 0, ST_ATT, ST_WO, ST_UP, ST_DOWN };
+enum Stage { ST_KQV = 0, ST_ATT, ST_WO, ST_UP, ST_DOWN, ST_HEAD };
 
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 
@@ -134,13 +135,13 @@ row_in (uint32_t *base, int n, uint32_t tag, const Wait &w, uint32_t stage, uint
   __syncthreads ();
 }
 
-// a row that is normalised first (at most 4096 values, eight per thread): the row itself ->
-// xr, y = fp16 (x * g * (1 / sqrt (mean (x^2) + eps))) -> xl.  The sums are those of
-// stage_row, thread for thread.
-template <bool TAGGED>
+// a row that is normalised first (at most 4096 values, eight per thread; fetch (c) brings
+// values 8 c .. 8 c + 7): the row itself -> xr,
+// y = fp16 (x * g * (1 / sqrt (mean (x^2) + eps))) -> xl.  The sums are those of stage_row,
+// thread for thread.
+template <typename Fetch>
 __device__ __forceinline__ void
-row_in_norm (uint32_t *base, const uint16_t *plain, int n, uint32_t tag, const Wait &w, uint32_t stage,
-             const uint4 (&g)[2], float eps, uint16_t *xr, uint16_t *xl, float *red)
+row_in_norm (Fetch fetch, int n, const uint4 (&g)[2], float eps, uint16_t *xr, uint16_t *xl, float *red)
 {
   const int c = (int)threadIdx.x;
   const bool in = c * 8 < n;
@@ -148,10 +149,7 @@ row_in_norm (uint32_t *base, const uint16_t *plain, int n, uint32_t tag, const W
   float s = 0.f;
   if (in)
     {
-      if (!TAGGED)
-        v = ldg4 (plain + c * 8);
-      else if (!poll8 (tagged_row (base, n), c * 8, tag, polls (w), v))
-        give_up (w, stage);
+      v = fetch (c);
       ((uint4 *)xr)[c] = v;
     }
   const uint32_t x[4] = { v.x, v.y, v.z, v.w };
@@ -187,6 +185,16 @@ row_in_norm (uint32_t *base, const uint16_t *plain, int n, uint32_t tag, const W
   __syncthreads ();
 }
 
+// values 8 c .. of a row of tagged words (0 where the wait gave up)
+__device__ __forceinline__ uint4
+tagged8 (uint32_t *base, int n, int c, uint32_t tag, const Wait &w, uint32_t stage)
+{
+  uint4 v = make_uint4 (0, 0, 0, 0);
+  if (!poll8 (tagged_row (base, n), c * 8, tag, polls (w), v))
+    give_up (w, stage);
+  return v;
+}
+
 __device__ __forceinline__ void
 load_norm_weights (const float *g, int n, uint4 (&v)[2])
 {
@@ -194,26 +202,55 @@ load_norm_weights (const float *g, int n, uint4 (&v)[2])
   v[0] = ldg4 (g + c), v[1] = ldg4 (g + c + 4);
 }
 
-// One row of a matrix in a wave's registers: S steps of 1024 bytes, 16 per lane.  The sums
-// are those of Gemv (vkl_decode_gemv.h), so the results are too.  No branches: a lane past the
-// end of the row requests its start and adds nothing.
+// The part of a product that a lane adds in one step: 16 bytes of a row.  The sums over a row
+// are those of Gemv (vkl_decode_gemv.h), term for term, so the results are too.
+template <int WT>
+__device__ __forceinline__ float
+add16 (float acc, const uint4 w, uint16_t d, const uint16_t *xl, int at)
+{
+  if (WT != 8)
+    return dot8_f16 (w, *(const uint4 *)(xl + (at >> 1)), acc);
+  const uint4 *xp = (const uint4 *)(xl + at);
+  const uint4 x0 = xp[0], x1 = xp[1];
+  const h16x2 xv[8] = { __builtin_bit_cast (h16x2, x0.x), __builtin_bit_cast (h16x2, x0.y),
+                        __builtin_bit_cast (h16x2, x0.z), __builtin_bit_cast (h16x2, x0.w),
+                        __builtin_bit_cast (h16x2, x1.x), __builtin_bit_cast (h16x2, x1.y),
+                        __builtin_bit_cast (h16x2, x1.z), __builtin_bit_cast (h16x2, x1.w) };
+  return acc + dot16_q8 (w, xv, 0.f) * h2f (d);
+}
+
+// a [N, K] matrix
+template <int WT> struct Matrix
+{
+  const uint8_t *q;
+  const uint16_t *d;
+  int bytes, nb; // of a row
+
+  __device__ __forceinline__
+  Matrix (const void *base, int N, int K)
+      : q ((const uint8_t *)base), d ((const uint16_t *)((const uint8_t *)base + (size_t)N * K)),
+        bytes (WT == 8 ? K : 2 * K), nb (K >> 5)
+  {
+  }
+};
+
+// One row in a wave's registers: S steps of 1024 bytes, 16 per lane.  No branches: a lane
+// past the end of the row requests its start and adds nothing.
 template <int WT, bool NT, int S> struct Row
 {
   uint4 w[S];
   uint16_t d[S];
 
-  // the row of a [N, K] matrix
   __device__ __forceinline__ void
-  request (const void *matrix, int N, int K, int row, int lane)
+  request (const Matrix<WT> m, int row, int lane)
   {
-    const int bytes = WT == 8 ? K : 2 * K, nb = K >> 5;
-    const uint8_t *q = (const uint8_t *)matrix + (size_t)row * bytes;
-    const uint16_t *sc = (const uint16_t *)((const uint8_t *)matrix + (size_t)N * K) + (size_t)row * nb;
+    const uint8_t *q = m.q + (size_t)row * m.bytes;
+    const uint16_t *sc = m.d + (size_t)row * m.nb;
 #pragma unroll
     for (int s = 0; s < S; ++s)
       {
         const int kk = s * 1024 + lane * 16;
-        const uint32_t kc = kk < bytes ? (uint32_t)kk : 0u;
+        const uint32_t kc = kk < m.bytes ? (uint32_t)kk : 0u;
         w[s] = NT ? ldg4_stream (q + kc) : ldg4 (q + kc);
         if (WT == 8)
           d[s] = ldg (sc + (kc >> 5));
@@ -231,24 +268,58 @@ template <int WT, bool NT, int S> struct Row
       {
         const int kk = s * 1024 + lane * 16;
         const bool in = kk < bytes;
-        const int kc = in ? kk : 0;
-        float sum;
-        if (WT != 8)
-          sum = dot8_f16 (w[s], *(const uint4 *)(xl + (kc >> 1)), acc);
-        else
-          {
-            const uint4 *xp = (const uint4 *)(xl + kc);
-            const uint4 x0 = xp[0], x1 = xp[1];
-            const h16x2 xv[8]
-                = { __builtin_bit_cast (h16x2, x0.x), __builtin_bit_cast (h16x2, x0.y),
-                    __builtin_bit_cast (h16x2, x0.z), __builtin_bit_cast (h16x2, x0.w),
-                    __builtin_bit_cast (h16x2, x1.x), __builtin_bit_cast (h16x2, x1.y),
-                    __builtin_bit_cast (h16x2, x1.z), __builtin_bit_cast (h16x2, x1.w) };
-            sum = acc + dot16_q8 (w[s], xv, 0.f) * h2f (d[s]);
-          }
+        const float sum = add16<WT> (acc, w[s], d[s], xl, in ? kk : 0);
         acc = in ? sum : acc;
       }
     return wave_sum (acc);
+  }
+};
+
+// Two rows.  SD = 0: rows of up to 512 bytes, the halves of a wave take one each (half the
+// loads, conversions and sums; the half that a row of its own would leave idle adds zeros).
+template <int WT, bool NT, int SD> struct Duo
+{
+  Row<WT, NT, SD> a, b;
+
+  __device__ __forceinline__ void
+  request (const Matrix<WT> ma, int ra, const Matrix<WT> mb, int rb, int lane)
+  {
+    a.request (ma, ra, lane), b.request (mb, rb, lane);
+  }
+  __device__ __forceinline__ void
+  dot (const uint16_t *xl, int K, int lane, float &ya, float &yb) const
+  {
+    ya = a.dot (xl, K, lane), yb = b.dot (xl, K, lane);
+  }
+};
+
+template <int WT, bool NT> struct Duo<WT, NT, 0>
+{
+  uint4 w;
+  uint16_t d;
+
+  __device__ __forceinline__ void
+  request (const Matrix<WT> ma, int ra, const Matrix<WT> mb, int rb, int lane)
+  {
+    const int kk = (lane & 31) * 16;
+    const uint32_t kc = kk < ma.bytes ? (uint32_t)kk : 0u;
+    const uint8_t *qa = ma.q + (size_t)ra * ma.bytes, *qb = mb.q + (size_t)rb * mb.bytes;
+    const uint8_t *q = (lane < 32 ? qa : qb) + kc;
+    w = NT ? ldg4_stream (q) : ldg4 (q);
+    if (WT == 8)
+      {
+        const uint16_t *da = ma.d + (size_t)ra * ma.nb, *db = mb.d + (size_t)rb * mb.nb;
+        d = ldg ((lane < 32 ? da : db) + (kc >> 5));
+      }
+  }
+  __device__ __forceinline__ void
+  dot (const uint16_t *xl, int K, int lane, float &ya, float &yb) const
+  {
+    const int kk = (lane & 31) * 16;
+    const bool in = kk < (WT == 8 ? K : 2 * K);
+    const float sum = add16<WT> (0.f, w, d, xl, in ? kk : 0);
+    const float v = row_sum<16> (in ? sum : 0.f);
+    ya = lane_value (v, 0) + lane_value (v, 16), yb = lane_value (v, 32) + lane_value (v, 48);
   }
 };
 
@@ -334,22 +405,199 @@ lds_map (int dim, int ffn, int maxlen, int hd)
 }
 
 // What a wave multiplies in a layer; the entry's part is on its way a layer ahead.
+// SD: steps of 1024 bytes in a row of dim values, 0 where it takes half of one
 template <int WT, int SD, bool NT> struct Entry
 {
-  Row<WT, NT, SD> k, q, v;
+  Duo<WT, NT, SD> kq;
+  Row<WT, NT, SD ? SD : 1> v;
   uint4 g[2]; // norm weights
 };
 
 template <int WT, int SD, bool NT> struct Rest
 {
-  Row<WT, NT, SD> o, up[kPairs], gate[kPairs];
-  Row<WT, NT, 3 * SD> down; // (SD: steps of 1024 bytes in a row of dim values)
+  Row<WT, NT, SD ? SD : 1> o;
+  Duo<WT, NT, SD> ug[kPairs];
+  Row<WT, NT, SD ? 3 * SD : 2> down;
   uint4 g[2];
 };
 
+// Where the step's token comes from and goes to, by scalar loads: nothing of it is written
+// before every workgroup has read it.
+typedef const __attribute__ ((address_space (4))) uint32_t *ScalarWord;
+
+__device__ __forceinline__ uint32_t
+this_token (const Params &p)
+{
+  const uint32_t t = p.loop ? ((ScalarWord)p.ids)[((ScalarWord)p.loop)[0]] : *(ScalarWord)p.tok;
+  return t < (uint32_t)p.m.vocab ? t : 0u;
+}
+
+// values 8 c .. of the token's embedding row (the arithmetic of embed_row)
+template <int WT>
+__device__ __forceinline__ uint4
+embedding8 (const Params &p, uint32_t tok, int c)
+{
+  const int dim = p.m.dim;
+  if (WT != 8)
+    return ldg4 ((const uint16_t *)p.m.tok_embd + (size_t)tok * dim + c * 8);
+  const Matrix<8> t (p.m.tok_embd, p.m.vocab, dim);
+  const unsigned long long q = ldg ((const unsigned long long *)(t.q + (size_t)tok * dim + c * 8));
+  const float sc = h2f (ldg (t.d + (size_t)tok * (dim >> 5) + (c >> 2)));
+  uint32_t o[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    o[j] = (uint32_t)f2h ((float)(int8_t)(q >> (16 * j)) * sc)
+           | ((uint32_t)f2h ((float)(int8_t)(q >> (16 * j + 8)) * sc) << 16);
+  return make_uint4 (o[0], o[1], o[2], o[3]);
+}
+
+// The vocabulary: the workgroups that have neither rows nor a head request their part of the
+// output matrix when the launch begins and hold it in registers until the last layer's row
+// arrives; each leaves its arg-max for workgroup 0.  From the last row to the next token 8.5 us
+// (512 wide, 17 MB) where the lm_head launch, its arg-max and two launch boundaries took 33
+// of 120 us per token.
+constexpr int kVocabLoads = 24; // loads of 16 bytes per lane that a wave holds of it
+
+template <int WT, int SD, bool NT>
+__device__ __forceinline__ void
+vocabulary (const Params &p, int part, int parts, uint32_t tag, int layers, const Wait &w, uint32_t *x,
+            uint32_t *best, uint16_t *xr, uint16_t *xa, float *red)
+{
+  constexpr int kDuos = kVocabLoads / (SD ? 2 * SD : 1);
+  const vkl_decode_model &m = p.m;
+  const int dim = m.dim, V = m.vocab;
+  const int lane = (int)threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane ((int)(threadIdx.x >> 6));
+  const Matrix<WT> out (m.output, V, dim);
+  const int waves = parts * kDecWaves, mine = part * kDecWaves + wave;
+  // (vocab is even: a wave's rows come in twos)
+  const int lo = 2 * (int)((long)(V / 2) * mine / waves), hi = 2 * (int)((long)(V / 2) * (mine + 1) / waves);
+  Duo<WT, NT, SD> r[kDuos];
+  uint4 g[2];
+  load_norm_weights (m.output_norm, dim, g);
+  auto request = [&] (int row) {
+#pragma unroll
+    for (int i = 0; i < kDuos; ++i)
+      {
+        const int at = min (row + 2 * i, V - 2);
+        r[i].request (out, at, out, at + 1, lane);
+      }
+  };
+  request (lo);
+  // Until the row of the layer before the last is there: seldom and one word, so that these
+  // many workgroups stay out of the way of those that poll the row for its values.
+  if (layers > 1)
+    for (long spin = 0; spin < (long)w.limit * layers; ++spin)
+      {
+        if ((tag - (ld_coherent_u32 (x) & 0xffff0000u)) >> 16 <= 1u)
+          break;
+        __builtin_amdgcn_s_sleep (32);
+      }
+  row_in_norm ([&] (int c) { return tagged8 (x, dim, c, tag, w, ST_DOWN); }, dim, g, m.final_eps, xr, xa, red);
+  float top = -INFINITY;
+  uint32_t top_at = 0xffffffffu;
+  for (int row = lo; row < hi; row += 2 * kDuos)
+    {
+      if (row != lo)
+        request (row);
+      // lane j takes row j of them
+      float mine_v = 0.f;
+#pragma unroll
+      for (int i = 0; i < kDuos; ++i)
+        {
+          float a, b;
+          r[i].dot (xa, dim, lane, a, b);
+          mine_v = lane == 2 * i ? a : (lane == 2 * i + 1 ? b : mine_v);
+        }
+      const uint16_t h = f2h (mine_v);
+      const float v = h2f (h);
+      const int n = min (hi - row, 2 * kDuos);
+      const bool in = lane < n;
+      if (in && *w.dead == 0u)
+        {
+          stg (p.s.logits16 + row + lane, h);
+          stg (p.logits32 + row + lane, v);
+        }
+      // the first of the largest (a NaN is never the largest)
+      const float mx = wave_max (in ? v : -INFINITY);
+      const unsigned long long at = __ballot (in && v == mx);
+      if (at && better (mx, (uint32_t)(row + __builtin_ctzll (at)), top, top_at))
+        top = mx, top_at = (uint32_t)(row + __builtin_ctzll (at));
+    }
+  uint32_t *idx = (uint32_t *)red + kDecWaves; // (red itself is not read any more: barriers since)
+  if (lane == 0)
+    red[wave] = top, idx[wave] = top_at;
+  __syncthreads ();
+  if (threadIdx.x == 0 && *w.dead == 0u)
+    {
+      for (int i = 1; i < kDecWaves; ++i)
+        if (better (red[i], idx[i], red[0], idx[0]))
+          red[0] = red[i], idx[0] = idx[i];
+      const unsigned long long word = (unsigned long long)idx[0] << 32 | tag | f2h (red[0]);
+      __hip_atomic_store ((unsigned long long *)best + part, word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+// workgroup 0, last: the token from the `parts` arg-maxima
+__device__ __forceinline__ void
+pick_token (const Params &p, int parts, uint32_t tag, const Wait &w, uint32_t *best, uint8_t *lds)
+{
+  float v = -INFINITY;
+  uint32_t at = 0xffffffffu;
+  if ((int)threadIdx.x < parts)
+    {
+      const rsrc_t row = tagged_row (best, 2 * parts);
+      const int limit = polls (w);
+      bool ok = false;
+      for (int spin = 0; spin < limit && !ok; ++spin)
+        {
+          asm volatile ("" ::: "memory");
+          typedef uint32_t u32x2 __attribute__ ((ext_vector_type (2)));
+          const u32x2 b = __builtin_bit_cast (
+              u32x2, __builtin_amdgcn_raw_buffer_load_b64 (row, (int)threadIdx.x * 8, 0, kPastL2));
+          ok = ((b.x ^ tag) >> 16) == 0;
+          v = h2f ((uint16_t)(b.x & 0xffff)), at = b.y;
+        }
+      if (!ok)
+        give_up (w, ST_HEAD);
+    }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+    {
+      const float ov = __shfl_xor (v, o, 64);
+      const uint32_t oi = __shfl_xor (at, o, 64);
+      if (better (ov, oi, v, at))
+        v = ov, at = oi;
+    }
+  float *bv = (float *)lds;
+  uint32_t *bi = (uint32_t *)(lds + 64);
+  if ((threadIdx.x & 63) == 0)
+    bv[threadIdx.x >> 6] = v, bi[threadIdx.x >> 6] = at;
+  __syncthreads ();
+  if (threadIdx.x == 0 && *w.dead == 0u)
+    {
+      for (int i = 1; i < kDecWaves; ++i)
+        if (better (bv[i], bi[i], v, at))
+          v = bv[i], at = bi[i];
+      const uint32_t id = at == 0xffffffffu ? 0u : at;
+      if (p.loop && !p.sample)
+        {
+          // to the next replay of the step
+          const uint32_t i = ldg (p.loop), ps = ldg (p.loop + 1);
+          stg (p.ids + i + 1, id);
+          stg ((uint32_t *)p.loop, i + 1);
+          stg ((uint32_t *)p.loop + 1, ps + 1);
+        }
+      else if (p.next_tok)
+        stg (p.next_tok, id);
+    }
+}
+
+// whole: a step from its token to the logits and the next token (the grid has workgroups for
+// the vocabulary); otherwise the layers alone, from Scratch::x to Scratch::x
 template <int WT, int SD, bool NT>
 __global__ __launch_bounds__ (kDecThreads) __attribute__ ((amdgpu_waves_per_eu (2, 2))) void
-decode_layers_kernel (const Params p, int first, int count)
+decode_layers_kernel (const Params p, int first, int count, bool whole)
 {
   extern __shared__ __align__ (16) uint8_t lds[];
   const vkl_decode_model &m = p.m;
@@ -362,6 +610,7 @@ decode_layers_kernel (const Params p, int first, int count)
   uint32_t *rows = p.s.tagged;
   uint32_t *err = p.s.sync + kSyncErr;
   uint32_t *counter = p.s.lsync + kLsTags;
+  const int copy = (int)(__builtin_amdgcn_s_getreg (20 | (0 << 6) | (3 << 11)) & 7u); // the XCD's number
   const uint32_t done = ld_coherent_u32 (counter);
   // (once a wait has given up the step is lost anyway)
   const Wait w = { err, dead, ld_coherent_u32 (err) != 0u ? 1 : (m.wait_polls > 0 ? m.wait_polls : kTagSpinLimit) };
@@ -371,9 +620,21 @@ decode_layers_kernel (const Params p, int first, int count)
   // the table of layers is not written while a step runs: scalar loads
   typedef const __attribute__ ((address_space (4))) vkl_layer_weights *Table;
   const Table table = (Table)m.layers + first;
+  uint16_t *xa = (uint16_t *)(lds + map.xa), *xb = (uint16_t *)(lds + map.xb), *xc = (uint16_t *)(lds + map.xc);
+  uint16_t *xr = (uint16_t *)(lds + map.xr), *xd = (uint16_t *)(lds + map.xd);
+  const int G = dim / kDecWaves;
+  const int parts = (int)gridDim.x - G - m.n_heads; // workgroups of the vocabulary
+  const uint32_t last_tag = (done + (uint32_t)count) << 16;
+  uint32_t *best = rows + tr.best;
+
+  if ((int)blockIdx.x >= G + m.n_heads)
+    {
+      vocabulary<WT, SD, NT> (p, (int)blockIdx.x - G - m.n_heads, parts, last_tag, count, w,
+                              rows + tr.x + copy * tr.copy_d, best, xr, xa, red);
+      return;
+    }
 
   // ---- the workgroups behind those of the rows: a head of the attention each -------------
-  const int G = dim / kDecWaves;
   if ((int)blockIdx.x >= G)
     {
       for (int l = 0; l < count; ++l)
@@ -392,8 +653,6 @@ decode_layers_kernel (const Params p, int first, int count)
       return;
     }
 
-  uint16_t *xa = (uint16_t *)(lds + map.xa), *xb = (uint16_t *)(lds + map.xb), *xc = (uint16_t *)(lds + map.xc);
-  uint16_t *xr = (uint16_t *)(lds + map.xr), *xd = (uint16_t *)(lds + map.xd);
   const int wave = __builtin_amdgcn_readfirstlane ((int)(threadIdx.x >> 6));
   const int g = (int)blockIdx.x * kDecWaves + wave; // number of the wave: dim of them
   const int first_row = (int)blockIdx.x * kDecWaves;
@@ -401,17 +660,16 @@ decode_layers_kernel (const Params p, int first, int count)
   const int end_pair = (int)((unsigned)ffn * (unsigned)(first_row + kDecWaves) / (unsigned)dim);
   const int lo = (int)((unsigned)ffn * (unsigned)g / (unsigned)dim);
   const int pairs = (int)((unsigned)ffn * (unsigned)(g + 1) / (unsigned)dim) - lo;
-  const int copy = (int)(__builtin_amdgcn_s_getreg (20 | (0 << 6) | (3 << 11)) & 7u); // the XCD's number
   int lane = (int)threadIdx.x & 63;
 
   auto request_entry = [&] (const void *wk, const void *wq, const void *wv, const float *norm) {
     Entry<WT, SD, NT> n;
-    n.k.request (wk, dim, dim, g, lane);
-    n.q.request (wq, dim, dim, g, lane);
-    n.v.request (wv, dim, dim, g, lane);
+    n.kq.request (Matrix<WT> (wk, dim, dim), g, Matrix<WT> (wq, dim, dim), g, lane);
+    n.v.request (Matrix<WT> (wv, dim, dim), g, lane);
     load_norm_weights (norm, dim, n.g);
     return n;
   };
+  const uint32_t tok = whole ? this_token (p) : 0u;
   Entry<WT, SD, NT> in = request_entry (table[0].wk, table[0].wq, table[0].wv, table[0].attn_norm);
 
   for (int l = 0;; ++l)
@@ -427,13 +685,17 @@ decode_layers_kernel (const Params p, int first, int count)
       const uint32_t tag = (done + (uint32_t)l + 1u) << 16;
 
       // ---- RMSNorm + K/Q/V ------------------------------------------------------
-      if (l == 0)
-        row_in_norm<false> (nullptr, p.s.x, dim, 0, w, ST_DOWN, in.g, m.eps, xr, xa, red);
-      else
-        row_in_norm<true> (rows + tr.x + copy * tr.copy_d, nullptr, dim, tag - 0x10000u, w, ST_DOWN, in.g, m.eps, xr,
-                           xa, red);
+      row_in_norm (
+          [&] (int c) {
+            if (l > 0)
+              return tagged8 (rows + tr.x + copy * tr.copy_d, dim, c, tag - 0x10000u, w, ST_DOWN);
+            return whole ? embedding8<WT> (p, tok, c) : ldg4 (p.s.x + c * 8);
+          },
+          dim, in.g, m.eps, xr, xa, red);
       {
-        const float a = in.k.dot (xa, dim, lane), b = in.q.dot (xa, dim, lane), c = in.v.dot (xa, dim, lane);
+        float a, b;
+        in.kq.dot (xa, dim, lane, a, b);
+        const float c = in.v.dot (xa, dim, lane);
         uint32_t *ok = out + kDecWaves * (2 + kPairs);
         if (lane < 3)
           ok[lane * kDecWaves + wave] = tag | f2h (lane == 0 ? a : (lane == 1 ? b : c));
@@ -447,17 +709,16 @@ decode_layers_kernel (const Params p, int first, int count)
       // (a poll returns behind the weights requested before it, and any of the later
       // hand-overs is shorter than their way from memory)
       Rest<WT, SD, NT> r;
-      r.o.request (wo, dim, dim, g, lane);
+      r.o.request (Matrix<WT> (wo, dim, dim), g, lane);
 #pragma unroll
       for (int j = 0; j < kPairs; ++j)
         {
           // (a wave with fewer pairs repeats its last)
           const int u = min (lo + j, max (lo + pairs - 1, 0));
-          r.up[j].request (w_up, ffn, dim, u, lane);
-          r.gate[j].request (w_gate, ffn, dim, u, lane);
+          r.ug[j].request (Matrix<WT> (w_up, ffn, dim), u, Matrix<WT> (w_gate, ffn, dim), u, lane);
         }
       load_norm_weights (ffn_norm, dim, r.g);
-      r.down.request (w_down, dim, ffn, g, lane);
+      r.down.request (Matrix<WT> (w_down, dim, ffn), g, lane);
       in = request_entry (wk, wq, wv, attn_norm);
 
       // ---- Wo + residual ------------------------------------------------------------
@@ -470,8 +731,8 @@ decode_layers_kernel (const Params p, int first, int count)
       }
 
       // ---- RMSNorm + up/gate with SiLU -------------------------------------------------
-      row_in_norm<true> (rows + tr.xm + copy * tr.copy_d, nullptr, dim, tag, w, ST_WO, r.g, m.eps, xr, xc,
-                         red + kDecWaves);
+      row_in_norm ([&] (int c) { return tagged8 (rows + tr.xm + copy * tr.copy_d, dim, c, tag, w, ST_WO); }, dim,
+                   r.g, m.eps, xr, xc, red + kDecWaves);
       {
         uint32_t *ot = out + kDecWaves;
         // (lane j ends pair j)
@@ -479,7 +740,8 @@ decode_layers_kernel (const Params p, int first, int count)
 #pragma unroll
         for (int j = 0; j < kPairs; ++j)
           {
-            const float uj = r.up[j].dot (xc, dim, lane), aj = r.gate[j].dot (xc, dim, lane);
+            float uj, aj;
+            r.ug[j].dot (xc, dim, lane, uj, aj);
             u = lane == j ? uj : u, a = lane == j ? aj : a;
           }
         if (lane < pairs)
@@ -490,52 +752,82 @@ decode_layers_kernel (const Params p, int first, int count)
       // ---- down + residual --------------------------------------------------------------
       row_in<2> (rows + tr.t + copy * tr.copy_f, ffn, tag, w, ST_UP, xd);
       const uint32_t y = f2h (h2f (f2h (r.down.dot (xd, ffn, lane))) + h2f (xr[g]));
-      if (l + 1 == count)
+      uint32_t *ox = out + kDecWaves * (1 + kPairs);
+      if (l + 1 == count && !whole)
         {
           if (lane == 0 && *dead == 0u)
             stg (p.s.x + g, (uint16_t)y);
           break;
         }
-      uint32_t *ox = out + kDecWaves * (1 + kPairs);
       if (lane == 0)
         ox[wave] = tag | y;
       publish (rows + tr.x, tr.copy_d, first_row, ox, kDecWaves, wave, lane, dead);
+      if (l + 1 == count)
+        break;
+    }
+  if (blockIdx.x != 0)
+    return;
+  if (whole)
+    {
+      __syncthreads ();
+      pick_token (p, parts, last_tag, w, best, lds + map.attn);
     }
   // (every workgroup has read the counter before it published its first word, and this one
   // has seen words of all)
-  if (blockIdx.x == 0 && threadIdx.x == 0)
+  if (threadIdx.x == 0)
     st_coherent_u32 (counter, done + (uint32_t)count);
 }
 
 template <int WT, int SD, bool NT>
 int
-launch_layers_t (const Params &p, int first, int count, hipStream_t s)
+launch_layers_t (const Params &p, int first, int count, int groups, hipStream_t s)
 {
   const size_t lds = (size_t)lds_map (p.m.dim, p.m.ffn, p.m.maxlen, p.m.head_dim).bytes;
   static LdsLimit limit;
   if (int e = limit.raise ((const void *)decode_layers_kernel<WT, SD, NT>, lds))
     return e;
+  const int own = p.m.dim / kDecWaves + p.m.n_heads;
   decode_layers_kernel<WT, SD, NT>
-      <<<dim3 ((unsigned)(p.m.dim / kDecWaves + p.m.n_heads)), dim3 (kDecThreads), lds, s>>> (p, first, count);
+      <<<dim3 ((unsigned)std::max (own, groups)), dim3 (kDecThreads), lds, s>>> (p, first, count, groups > own);
   return 0;
 }
 
 template <int WT, int SD>
 int
-launch_layers_nt (const Params &p, int first, int count, hipStream_t s)
+launch_layers_nt (const Params &p, int first, int count, int groups, hipStream_t s)
 {
-  return p.stream_once ? launch_layers_t<WT, SD, true> (p, first, count, s)
-                       : launch_layers_t<WT, SD, false> (p, first, count, s);
+  return p.stream_once ? launch_layers_t<WT, SD, true> (p, first, count, groups, s)
+                       : launch_layers_t<WT, SD, false> (p, first, count, groups, s);
+}
+
+int
+row_bytes (const vkl_decode_model &m)
+{
+  return m.wtype == 8 ? m.dim : 2 * m.dim;
+}
+
+int
+launch_any (const Params &p, int first, int count, int groups, hipStream_t s)
+{
+  const int bytes = row_bytes (p.m);
+  if (p.m.wtype == 8)
+    return bytes <= 512    ? launch_layers_nt<8, 0> (p, first, count, groups, s)
+           : bytes <= 1024 ? launch_layers_nt<8, 1> (p, first, count, groups, s)
+                           : launch_layers_nt<8, 2> (p, first, count, groups, s);
+  return bytes <= 512    ? launch_layers_nt<1, 0> (p, first, count, groups, s)
+         : bytes <= 1024 ? launch_layers_nt<1, 1> (p, first, count, groups, s)
+                         : launch_layers_nt<1, 2> (p, first, count, groups, s);
 }
 } // namespace
 
 // Where dim waves have at most three up/gate pairs each, a layer's weights fit the registers
 // and all workgroups have a compute unit of their own.  Us per token, a launch per layer / this
-// form (greedy, 64 or 48 tokens, the lm_head launch included): 256 wide Q8_0, 6 layers 137 /
-// 93; 512 wide, 8 layers 182 / 120, fp16 171 / 107; 4 layers: 1024 wide 112 / 83, fp16 110 /
-// 82; 1536 wide 123 / 98.  2048 wide (all 256 compute units for the rows, the heads beside
-// them, weights a phase ahead) it was slower: 144 / 158, fp16 160 / 212; there a layer is
-// bound by its weights, and polls behind them come late.
+// form with an lm_head launch / the whole step in one launch (greedy, 64 or 48 tokens): 256
+// wide Q8_0, 6 layers 137 / 93 / 77; 512 wide, 8 layers 182 / 120 / 102, fp16 171 / 107 / 95; 4
+// layers: 1024 wide 112 / 83 / 76, fp16 110 / 79 / -; 1536 wide 123 / 93 / -.  2048 wide (all
+// 256 compute units for the rows, the heads beside them, weights a phase ahead) it was slower:
+// 144 / 158, fp16 160 / 212; there a layer is bound by its weights, and polls behind them come
+// late.
 bool
 layers_launch_supported (const vkl_decode_model &m, int n_cu)
 {
@@ -548,10 +840,27 @@ layers_launch_supported (const vkl_decode_model &m, int n_cu)
 int
 launch_layers (const Params &p, int first, int count, hipStream_t s)
 {
-  const int steps = ((p.m.wtype == 8 ? p.m.dim : 2 * p.m.dim) + 1023) / 1024;
-  if (p.m.wtype == 8)
-    return steps == 1 ? launch_layers_nt<8, 1> (p, first, count, s) : launch_layers_nt<8, 2> (p, first, count, s);
-  return steps == 1 ? launch_layers_nt<1, 1> (p, first, count, s) : launch_layers_nt<1, 2> (p, first, count, s);
+  return launch_any (p, first, count, 0, s);
+}
+
+// The workgroups left over hold the output matrix in their registers, or at most twice that.
+bool
+whole_step_supported (const vkl_decode_model &m, int n_cu)
+{
+  if (!layers_launch_supported (m, n_cu))
+    return false;
+  const long parts = n_cu - m.dim / kDecWaves - m.n_heads;
+  if (parts < 1 || parts > kDecThreads || parts > kMaxParts)
+    return false;
+  const int steps = (row_bytes (m) + 1023) / 1024;
+  const long held = row_bytes (m) <= 512 ? 2 * kVocabLoads : kVocabLoads / steps; // rows of a wave
+  return m.vocab <= 2 * held * parts * kDecWaves;
+}
+
+int
+launch_step_whole (const Params &p, int n_cu, hipStream_t s)
+{
+  return launch_any (p, 0, p.m.n_layers, n_cu, s);
 }
 } // namespace dec
 } // namespace vkl

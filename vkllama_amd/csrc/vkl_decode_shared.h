@@ -43,8 +43,9 @@ constexpr int kTaggedMaxDim = 2048; // rows of up to so many (and three times as
 struct TaggedRows
 {
   // words from Scratch::tagged: rows, and from copy to copy
-  int kqv, att, xm, x, t, copy_d, copy_f, words;
+  int kqv, att, xm, x, t, best, copy_d, copy_f, words;
 };
+constexpr int kMaxParts = 512; // arg-maxima of parts of the vocabulary, two words each
 
 __host__ __device__ inline TaggedRows
 tagged_rows (int dim, int ffn)
@@ -55,7 +56,8 @@ tagged_rows (int dim, int ffn)
   r.xm = r.att + kTagCopies * r.copy_d;
   r.x = r.xm + kTagCopies * r.copy_d;
   r.t = r.x + kTagCopies * r.copy_d;
-  r.words = r.t + kTagCopies * r.copy_f;
+  r.best = r.t + kTagCopies * r.copy_f;
+  r.words = r.best + 2 * kMaxParts;
   return r;
 }
 
@@ -634,6 +636,10 @@ int launch_layer (const Params &p, const vkl_layer_weights &lw, int layer, int G
 // layers are bound by their hand-overs.  At most one workgroup per compute unit, all resident.
 bool layers_launch_supported (const vkl_decode_model &m, int n_cu);
 int launch_layers (const Params &p, int first, int count, hipStream_t s);
+// a whole step, from the token to the logits and the next token, where the compute units left
+// over can hold the output matrix
+bool whole_step_supported (const vkl_decode_model &m, int n_cu);
+int launch_step_whole (const Params &p, int n_cu, hipStream_t s);
 // the token's embedding row -> residual stream (one small launch in front of layer 0)
 int launch_embed_row (const Params &p, hipStream_t s);
 } // namespace dec

@@ -316,6 +316,10 @@ int vkl_stack_supported (const vkl_stack_model *m);
 int vkl_stack_step (const vkl_stack_model *m, const uint32_t *tok,
                     uint32_t pos, float *logits32, uint32_t *next_tok,
                     void *stream);
+/* The step's last launch by itself: logits32 [vocab] of one row x [width_p] of the
+ * residual stream (final norm, output matrix, soft cap), all in fp32. */
+int vkl_stack_logits (const vkl_stack_model *m, const float *x, float *logits32,
+                      void *stream);
 /* vkl_decode_loop / vkl_decode_loop_sampled for such a stack */
 int vkl_stack_loop (const vkl_stack_model *m, uint32_t *ids, uint32_t pos0,
                     int n_steps, float *logits32, void *stream);

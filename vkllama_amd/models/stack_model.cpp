@@ -301,17 +301,30 @@ StackModel::wait_all_ ()
   return command_->wait ();
 }
 
-// S tokens through every layer; leaves the residual stream in x_
+// the tokens of a call, where its passes read them: host memory that the GPU sees
 absl::Status
-StackModel::pass_ (const uint32_t *toks, int S, size_t offset, std::vector<float> *streams)
+StackModel::put_tokens_ (std::vector<uint32_t> const &toks)
+{
+  // (nothing of a call before may still read there)
+  VKLLAMA_STATUS_OK (launched ("waiting for the stream", vkl_stream_sync (gpu_->stream ())));
+  if (toks_.width () < toks.size ())
+    {
+      toks_ = Tensor (1, 1, (int)toks.size (), gpu_, UINT32, true);
+      VKLLAMA_STATUS_OK (toks_.create ());
+    }
+  std::copy (toks.begin (), toks.end (), (uint32_t *)toks_.host ());
+  return toks_.flush ();
+}
+
+// S tokens from number `first` of the call on through every layer; leaves the residual stream in x_
+absl::Status
+StackModel::pass_ (size_t first, int S, size_t offset, std::vector<float> *streams)
 {
   void *s = gpu_->stream ();
   VKLLAMA_STATUS_OK (reserve (x_, S, width_p_, gpu_, FP32));
   VKLLAMA_STATUS_OK (reserve (buf_.h, S, width_p_, gpu_, dtype_));
   VKLLAMA_STATUS_OK (reserve (buf_.cat, S, buf_.cat_stride, gpu_, dtype_));
-  VKLLAMA_STATUS_OK (reserve (toks_, 1, S, gpu_, UINT32));
-  VKLLAMA_STATUS_OK (command_->upload (toks, (size_t)S, toks_));
-  const uint32_t *ids = (const uint32_t *)toks_.data ();
+  const uint32_t *ids = (const uint32_t *)toks_.data () + first;
   float *xp = (float *)x_.data ();
   VKLLAMA_STATUS_OK (launched (
       "embedding", cfg_.embed_norm ? vkl_embed_norm_bf16 (embed_.data (), (uint32_t)vocab_, width_p_, cfg_.width, ids,
@@ -342,6 +355,9 @@ StackModel::logits_ (const std::vector<uint32_t> &rows, float *out)
 {
   const int type = dtype_ == FP32 ? VKL_TYPE_F32 : VKL_TYPE_BF16, n = (int)rows.size ();
   void *s = gpu_->stream ();
+  if (n == 1 && plan_->usable ())
+    return launched ("output product", vkl_stack_logits (&plan_->desc (),
+                                                         (const float *)x_.data () + (size_t)rows[0] * width_p_, out, s));
   VKLLAMA_STATUS_OK (reserve (rows_, 1, n, gpu_, UINT32));
   VKLLAMA_STATUS_OK (reserve (out_h_, n, width_p_, gpu_, dtype_));
   VKLLAMA_STATUS_OK (command_->upload (rows.data (), rows.size (), rows_));
@@ -362,10 +378,11 @@ StackModel::forward_ (std::vector<uint32_t> const &toks, const size_t offset, st
   VKLLAMA_STATUS_OK (check_span_ (toks.size (), offset));
   Tensor out (1, (int)std::max<size_t> (rows.size (), 1), (int)vocab_, gpu_, FP32);
   VKLLAMA_STATUS_OK (out.create ());
+  VKLLAMA_STATUS_OK (put_tokens_ (toks));
   for (size_t at = 0; at < toks.size (); at += kPortion)
     {
       const int S = (int)std::min<size_t> (kPortion, toks.size () - at);
-      VKLLAMA_STATUS_OK (pass_ (toks.data () + at, S, offset + at, nullptr));
+      VKLLAMA_STATUS_OK (pass_ (at, S, offset + at, nullptr));
       // runs of wanted rows that fall into this portion (in the order asked for)
       for (size_t i = 0; i < rows.size ();)
         {
@@ -392,7 +409,8 @@ StackModel::residual_streams (std::vector<uint32_t> const &toks, size_t offset)
     return absl::InvalidArgumentError ("residual streams: one portion at most");
   std::vector<float> out;
   VKLLAMA_STATUS_OK (begin_pass_ (offset));
-  VKLLAMA_STATUS_OK (pass_ (toks.data (), (int)toks.size (), offset, &out));
+  VKLLAMA_STATUS_OK (put_tokens_ (toks));
+  VKLLAMA_STATUS_OK (pass_ (0, (int)toks.size (), offset, &out));
   end_pass_ (offset + toks.size ());
   return out;
 }

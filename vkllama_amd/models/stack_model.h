@@ -130,7 +130,8 @@ protected:
 private:
   absl::StatusOr<Tensor> forward_ (std::vector<uint32_t> const &toks, const size_t offset,
                                    std::vector<uint32_t> const &rows) override;
-  absl::Status pass_ (const uint32_t *toks, int S, size_t offset, std::vector<float> *streams);
+  absl::Status put_tokens_ (std::vector<uint32_t> const &toks);
+  absl::Status pass_ (size_t first, int S, size_t offset, std::vector<float> *streams);
   absl::Status logits_ (const std::vector<uint32_t> &rows, float *out);
   absl::Status wait_all_ () override;
   StepPlan *plan_ptr_ () override { return plan_.get (); }

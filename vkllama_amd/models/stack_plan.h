@@ -15,6 +15,7 @@ public:
   // desc: everything but layers_h and scratch; one layer entry per run
   absl::Status build (GPUDevice *gpu, const vkl_stack_model &desc, std::vector<vkl_stack_layer> layers);
   bool usable () const override { return usable_; }
+  const vkl_stack_model &desc () const { return desc_; }
   absl::Status step_device_token (const uint32_t *tok, size_t offset, uint32_t *next_tok = nullptr) override;
   absl::Status loop (uint32_t *ids, size_t pos0, size_t n_steps) override;
   absl::Status loop_sampled (uint32_t *ids, size_t pos0, size_t n_steps, int topk, float topp,

@@ -487,7 +487,7 @@ wide_f32_again (const GemmSegArgs &a, float16v (&acc)[TM][WTN], int lane, int mr
 }
 
 // BM: token rows of a tile, 256 or (where 256-row tiles would be too few to
-// occupy the compute units) 128, i.e. 64 x 64 per wave.
+// occupy the compute units) 128, i.e. 64 x 64 per wave; of bf16 products also 64.
 // PLANES > 1: x holds PLANES values for every weight, in blocks of 64 (one k-step of
 // each plane in turn): see the 32-bit product below.
 template <int BM, bool UPGATE, class Args, int PLANES>
@@ -1215,42 +1215,63 @@ wide_reduce_seg_kernel (const GemmSegArgs a, const float *ws, int parts)
 // to 2048 rows in every plan (microseconds: a round of 256-row tiles 0.67 per k-step + 8.8, of
 // 128-row tiles 0.60 + 5.1, cut tiles likewise; where a segment's sums are parked in LDS 9.6 and
 // 5.6 more per round, which parts leave to the reduction; that launch 3.6 + its bytes at 1.7
-// TB/s).  The plan is 0.3 % slower than the best one in the mean, 18 % at worst.  With the
-// constants of the planes of a 32-bit operand, whose weights come from the L2 two times of three, it
-// was 2.8 and 54 %, and divided too little where few tiles stream the weights: 128 x 8064 x 2048
-// 26 us, 28 with GELU, in one part and 22 in two, 160 x 5504 x 2048 23 and 21, 512 x 2048 x 2048
-// with GELU 28 and 21.
+// TB/s).  With the constants of the planes of a 32-bit operand, whose weights come from the L2 two
+// times of three, it was 2.8 and 54 % slower than the best plan, in the mean and at worst, and
+// divided too little where few tiles stream the weights: 128 x 8064 x 2048 26 us, 28 with GELU, in
+// one part and 22 in two, 160 x 5504 x 2048 23 and 21, 512 x 2048 x 2048 with GELU 28 and 21.
+// Tiles of 64 rows have two workgroups to a compute unit: up to 256 of them take 0.54 per k-step +
+// 2.6, up to 512 0.81 + 3.7 (planes 0.37 + 1.7 and 0.47 + 6.3).  They win where rows are few or half
+// of a taller tile is empty; us without / with them, bf16: 40 x 8064 x 2048 16.3 / 14.5, 128 x
+// 2048 x 7552 21.0 / 18.1, 12 x 16128 x 4096 35.3 / 30.2; planes: 12 x 16128 x
+// 4096 54.7 / 43.5, 300 x 5504 x 2048 50.1 / 41.9.  Over 198 products of 2 to 2048 rows (114 of
+// planes) the plan is 1.1 % (0.7) slower than the best in the mean; without these tiles it was 4.7
+// (6.6).  Not yet for bf16 operands of more than 128 rows, where they are faster too, but whole where
+// products are held to be in parts (160 x 5504 x 2048 18.4 us, 128-row tiles in two parts 20.3).
 WidePlan
 wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
 {
   struct Fit
   {
     double step256, round256, step128, round128, reduce, rate, park256, park128;
+    double one64, first64, two64, round64; // 64-row tiles: one and two workgroups per compute unit
   };
-  const Fit f = a.xf ? Fit{ 0.79, 5, 0.47, 4, 5, 2.5e6, 0, 0 } : Fit{ 0.67, 8.8, 0.60, 5.1, 3.6, 1.7e6, 9.6, 5.6 };
+  const Fit f = a.xf ? Fit{ 0.79, 5, 0.47, 4, 5, 2.5e6, 0, 0, 0.37, 1.7, 0.47, 6.3 }
+                     : Fit{ 0.67, 8.8, 0.60, 5.1, 3.6, 1.7e6, 9.6, 5.6, 0.54, 2.6, 0.81, 3.7 };
   WidePlan best = { 0, 1 };
   double best_cost = 0;
   const int nk = a.K / WBK;
   bool parked = false; // see WideSimple
   for (int i = 0; i < a.nseg; ++i)
     parked = parked || !a.seg[i].vec || a.seg[i].cap > 0.f || (a.seg[i].act != VKL_ACT_NONE && a.seg[i].act != VKL_ACT_RELU2);
-  for (int bm = 128; bm <= WBM; bm *= 2)
+  for (int bm = 64; bm <= WBM; bm *= 2)
     for (int ks = 1; ks <= 16; ks *= 2)
       {
-        if (a.M < bm && bm > 128)
+        if ((a.M < bm && bm > 128) || (bm == 64 && !a.xf && a.M > 128))
           continue;
         if (ks > 1
             && (nk / ks < 4 || (size_t)ks * a.M * a.N * sizeof (float) > scratch))
           continue;
         const WideGrid tiles ((a.M + bm - 1) / bm, (a.N + WBN - 1) / WBN, 1, ks, bm == WBM);
-        const int whole = (tiles.whole + WideGrid::kUnits - 1) / WideGrid::kUnits;
         const double steps = (double)nk / ks;
-        const double park = parked && ks == 1 ? std::min (1.0, a.M / 64.0) : 0; // (a wave walks 64 or 128 rows)
-        const double half = f.step128 * steps + f.round128 + park * f.park128;
-        const double round = bm == WBM ? f.step256 * steps + f.round256 + park * f.park256 : half;
-        const double cut = tiles.whole < tiles.tiles () ? half : 0;
         const double reduce = ks > 1 ? f.reduce + (double)ks * a.M * a.N * sizeof (float) / f.rate : 0;
-        const double cost = whole * round + cut + reduce;
+        double cost = reduce;
+        if (bm == 64)
+          {
+            const double park = parked && ks == 1 ? std::min (1.0, a.M / 32.0) * f.park128 / 2 : 0;
+            const int two = tiles.tiles () / (2 * WideGrid::kUnits), rest = tiles.tiles () % (2 * WideGrid::kUnits);
+            const double round = f.two64 * steps + f.round64 + park;
+            cost += two * round;
+            if (rest > 0)
+              cost += rest <= WideGrid::kUnits ? f.one64 * steps + f.first64 + park : round;
+          }
+        else
+          {
+            const int whole = (tiles.whole + WideGrid::kUnits - 1) / WideGrid::kUnits;
+            const double park = parked && ks == 1 ? std::min (1.0, a.M / 64.0) : 0; // (a wave walks 64 or 128 rows)
+            const double half = f.step128 * steps + f.round128 + park * f.park128;
+            const double round = bm == WBM ? f.step256 * steps + f.round256 + park * f.park256 : half;
+            cost += whole * round + (tiles.whole < tiles.tiles () ? half : 0);
+          }
         if (!best.bm || cost < best_cost)
           best = { bm, ks }, best_cost = cost;
       }
@@ -1279,6 +1300,15 @@ launch_wide_bf16 (const GemmSegArgs &a, int ksplit, float *ws, hipStream_t s)
       wide_reduce_seg_kernel<PLANES><<<dim3 ((unsigned)((total + kSegReduce - 1) / kSegReduce)), dim3 (kSegReduce), 0, s>>> (a, ws, ksplit);
     }
   return (int)hipGetLastError ();
+}
+
+template <int PLANES>
+int
+launch_wide_bf16_any (const GemmSegArgs &a, const WidePlan &p, float *ws, hipStream_t s)
+{
+  return p.bm == WBM   ? launch_wide_bf16<WBM, PLANES> (a, p.ksplit, ws, s)
+         : p.bm == 128 ? launch_wide_bf16<128, PLANES> (a, p.ksplit, ws, s)
+                       : launch_wide_bf16<64, PLANES> (a, p.ksplit, ws, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1348,7 +1378,7 @@ int
 gemm_wide_bf16_launch (const GemmSegArgs &a, hipStream_t s)
 {
   const WidePlan p = wide_plan_bf16 (a, StreamScratch::bytes ());
-  return p.bm == WBM ? launch_wide_bf16<WBM> (a, p.ksplit, nullptr, s) : launch_wide_bf16<128> (a, p.ksplit, nullptr, s);
+  return launch_wide_bf16_any<1> (a, p, nullptr, s);
 }
 
 bool
@@ -1405,8 +1435,7 @@ gemm_wide_f32_launch (const GemmSegArgs &a, hipStream_t s, int &err)
         }
       const WidePlan p = wide_plan_bf16 (b, half);
       float *parts = ws + half / sizeof (float);
-      err = p.bm == WBM ? launch_wide_bf16<WBM, kPlanes> (b, p.ksplit, parts, s)
-                        : launch_wide_bf16<128, kPlanes> (b, p.ksplit, parts, s);
+      err = launch_wide_bf16_any<kPlanes> (b, p, parts, s);
       if (err)
         return true;
     }

@@ -84,7 +84,8 @@ enum Phase
   PH_HEAD,
   PH_ARGMAX,
   PH_GEMV, // a stand-alone y = W x (+ residual) on the down projection's path
-  PH_LAYER // a whole layer in one launch (vkl_decode_layer.hip)
+  PH_LAYER, // a whole layer in one launch (vkl_decode_layer.hip)
+  PH_UPROW, // up/gate with SiLU of one row that is multiplied as it is
 };
 
 // ---------------------------------------------------------------------------
@@ -314,6 +315,16 @@ run_phase_direct (const Params &p, const vkl_layer_weights &lw, int layer,
         GV::begin (ps, A, B, 2, up, gate, up, ffn, dim, wg, G, 1, nullptr, true);
         stage_row<true, XCH> (x, dim, xl, nw, m.eps, red, VKL_TRP);
         VKL_TR (2);
+        e.y[0] = p.s.t;
+        break;
+      }
+    case PH_UPROW:
+      {
+        const QMat up = wmat<WT> (lw.w_up, ffn, dim), gate = wmat<WT> (lw.w_gate, ffn, dim);
+        load_row<XCH> (p.s.x, dim, x);
+        __builtin_amdgcn_sched_barrier (0);
+        GV::begin (ps, A, B, 2, up, gate, up, ffn, dim, wg, G, 1, nullptr, true);
+        stage_row<false, XCH> (x, dim, xl, nw, 0.f, red, VKL_TRP);
         e.y[0] = p.s.t;
         break;
       }
@@ -821,7 +832,7 @@ launch_phase_wt (const Params &p, const vkl_layer_weights &lw, int layer,
                  int grid, int G, size_t lds, hipStream_t s)
 {
   if (PHASE == PH_WO || PHASE == PH_UPGATE || PHASE == PH_DOWN || PHASE == PH_HEAD
-      || PHASE == PH_GEMV || (PHASE == PH_KQV && layer > 0))
+      || PHASE == PH_GEMV || PHASE == PH_UPROW || (PHASE == PH_KQV && layer > 0))
     return launch_direct<PHASE, WT> (p, lw, layer, grid, G, lds, s);
   static LdsLimit limit;
   if (int e = limit.raise ((const void *)decode_phase_kernel<PHASE, WT>, lds))
@@ -1120,6 +1131,29 @@ decode_gemv_launch (const void *x, const void *w, int wtype, int N, int K,
   const size_t lds = (size_t)K * 2 + 256 + 64;
   if (int e = wtype == 8 ? launch_phase_wt<PH_GEMV, 8> (p, lw, 0, G, G, lds, s)
                          : launch_phase_wt<PH_GEMV, 1> (p, lw, 0, G, G, lds, s))
+    return e;
+  return vkl_launch_status ();
+}
+
+// y[N] = silu (Wgate x) * (Wup x) for one token row on the decode step's up/gate kernel, planar
+// Q8_0 weights
+int
+decode_uprow_launch (const void *x, const void *up, const void *gate, int N, int K, void *y, hipStream_t s)
+{
+  if (!decode_gemv_supported (N, K, 8))
+    return (int)hipErrorInvalidValue;
+  int dev = 0, n_cu = 0;
+  VKL_HIP (hipGetDevice (&dev));
+  VKL_HIP (hipDeviceGetAttribute (&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
+  Params p = {};
+  p.m.dim = K, p.m.ffn = N, p.m.wtype = 8;
+  p.s.x = (uint16_t *)x, p.s.t = (uint16_t *)y;
+  p.stream_once = 2.0 * N * K * 34.0 / 32.0 > (double)kCacheResidentBytes;
+  vkl_layer_weights lw = {};
+  lw.w_up = up, lw.w_gate = gate;
+  const int G = n_cu * 2;
+  const size_t lds = (size_t)K * 2 + 256 + 64;
+  if (int e = launch_phase_wt<PH_UPROW, 8> (p, lw, 0, G, G, lds, s))
     return e;
   return vkl_launch_status ();
 }

@@ -156,5 +156,7 @@ float *gemm_static_scratch (size_t *bytes);
 bool decode_gemv_supported (int N, int K, int wtype);
 int decode_gemv_launch (const void *x, const void *w, int wtype, int N, int K,
                         const void *residual, void *y, hipStream_t s);
+// y[N] = silu (Wgate x) * (Wup x), planar Q8_0 weights, where decode_gemv_supported
+int decode_uprow_launch (const void *x, const void *up, const void *gate, int N, int K, void *y, hipStream_t s);
 }
 #endif

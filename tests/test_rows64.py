@@ -8,9 +8,9 @@ torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (12, 16136, 512), (31, 264, 2048), (33, 2048, 2048), (64, 5504, 512),
+@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (12, 16136, 512), (31, 264, 2048), (63, 136, 576), (33, 2048, 2048), (64, 5504, 512),
                                    (65, 136, 5504), (128, 8064, 512), (192, 2048, 2048), (300, 5512, 1088),
-                                   (520, 2048, 2048)])
+                                   (520, 2048, 2048), (640, 16128, 576)])
 @pytest.mark.parametrize("xtype", [stack.BF16, stack.F32])
 def test_rows_in_tiles_of_64(dev, M, N, K, xtype):
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
@@ -29,7 +29,7 @@ def test_rows_in_tiles_of_64(dev, M, N, K, xtype):
     dev.sync()
     xd, wd = x.double(), w.double()
     want, mag = xd @ wd.t(), xd.abs() @ wd.abs().t()
-    # exact products, K (planes: 3 K) of them added sixteen at a time, the 32-bit instructions two: 2^-23 of the sum of
+    # exact products, K (planes: and 2 K small ones) of them added sixteen at a time, the 32-bit instructions two: 2^-23 of the sum of
     # magnitudes each; a square doubles that
     bound = K / 2 * 2.0 ** -23 * mag + 2.0 ** -23
     assert bool(((a - res - want[:, :cut]).abs() <= bound[:, :cut] + 2.0 ** -23 * (res.abs() + mag[:, :cut])).all())

@@ -652,6 +652,176 @@ wide_f16_tile (const Args &a, const WidePlace &at, int vec, int ksplit, float *w
   wide_epilogue<UPGATE, TM, WTN> (a, acc, wide_lds, wave, lane, m0 + wm * TM * 32, n0 + (UPGATE ? wn * 32 : wn * 64), zmat, vec, part);
 }
 
+// The planes of a 32-bit operand (see there) in tiles of 64 rows: x holds three values for
+// every weight, [plane 0 | plane 1 | plane 2] of 64 columns next to each other, and a k-step is
+// 64 columns of the weights with those of all three planes.  Walked as a row of 3 K values, the
+// weights came from the L2 and went through LDS three times: for 64 rows 72 KB into LDS and 144
+// out of it per 64 columns, 1730 cycles at 128 bytes for 770 of products; now 40 + 80 KB.  Two
+// stages are 80 KB, two workgroups to a compute unit, each of which multiplies where the other
+// one waits.  Tiles of 128 rows (128 KB, one workgroup) were slower (800 x 16128 x 4096 362 us for
+// 315); of 256 they do not fit, and those of wide_f16_tile (144 + 288 KB for 3070 cycles of products)
+// stay the better ones where they fill the chip (wide_plan_planes).  us before / now: 12 x 12288 x
+// 4096 39.9 / 33.0, 300 x 2048 x 2048 27.8 / 25.2, 300 x 5504 x 2048 41.9 / 37.1, 300 x 12288 x 4096
+// 120 / 96, 700 x 11008 x 4096 236 / 188.
+constexpr int kPlanes = 3, kPlaneRows = 64;
+
+constexpr size_t
+wide_lds_planes ()
+{
+  const size_t stages = (size_t)2 * (kPlanes * kPlaneRows + WBN) * WROWB, park = (size_t)kPlaneRows * 2 * kWideParkLd * 4;
+  return stages > park ? stages : park;
+}
+
+__global__ __launch_bounds__ (WWAVES * 64) void
+gemm_wide_planes_kernel (const GemmSegArgs a, WideGrid grid, int ksplit, float *ws)
+{
+  WidePlace at;
+  if (grid.place<kPlaneRows> (a.M, at) != WIDE_TILE)
+    return;
+  constexpr int BM = kPlaneRows;
+  typedef WideElem<GemmSegArgs>::v8 v8;
+  constexpr int TM = BM / 2 / 32;
+  constexpr int A_BYTES = BM * WROWB, STAGE_BYTES = kPlanes * A_BYTES + WBN * WROWB;
+  constexpr int AG = BM / 8 / WWAVES, BG = WBN / 8 / WWAVES, LOADS = kPlanes * AG + BG;
+  extern __shared__ __align__ (16) uint8_t wide_lds[];
+  const int ks = at.ks, nk_all = a.K / WBK / kPlanes;
+  const int kbase = (int)((long)nk_all * ks / ksplit);
+  const int nk = (int)((long)nk_all * (ks + 1) / ksplit) - kbase;
+  float *part = ksplit > 1 ? ws + (size_t)ks * a.M * a.N : nullptr;
+  const int m0 = at.m0, n0 = at.tn * WBN;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane (threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+
+  // rows and chunks as in wide_f16_tile
+  const int lr = lane >> 3;
+  const int chunk = (lane & 7) ^ lr ^ (wave & 1);
+  const uint16_t *srca[AG], *srcb[BG];
+#pragma unroll
+  for (int i = 0; i < AG; ++i)
+    srca[i] = a.x + (size_t)min (m0 + (wave + WWAVES * i) * 8 + lr, a.M - 1) * a.K + (size_t)kbase * kPlanes * WBK
+              + chunk * 8;
+#pragma unroll
+  for (int i = 0; i < BG; ++i)
+    srcb[i] = a.wh[0] + (size_t)min (n0 + (wave + WWAVES * i) * 8 + lr, a.N - 1) * a.ws + (size_t)kbase * WBK + chunk * 8;
+  const int fsw = (lane & 7) ^ ((lane >> 3) & 1);
+  uint32_t aoff[4], boff[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    {
+      const int ko = ((2 * q + (lane >> 5)) ^ fsw) << 4;
+      aoff[q] = (wm * (BM / 2) + (lane & 31)) * WROWB + ko;
+      boff[q] = kPlanes * A_BYTES + (wn * 64 + (lane & 31)) * WROWB + ko;
+    }
+
+  // the two lower planes' sums are kept apart: added to the large ones they would round those
+  // two times more per sixteen products
+  float16v acc[TM][WTN], low[TM][WTN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int jn = 0; jn < WTN; ++jn)
+#pragma unroll
+      for (int q = 0; q < 16; ++q)
+        acc[i][jn][q] = 0.f, low[i][jn][q] = 0.f;
+
+  // loads [i0, i1) of a k-step: the weights, then the planes
+  auto issue = [&] (int kt, int st, int i0, int i1) {
+#pragma unroll
+    for (int i = i0; i < i1; ++i)
+      {
+        uint8_t *base = wide_lds + st * STAGE_BYTES;
+        if (i < BG)
+          __builtin_amdgcn_global_load_lds ((const VKL_GLOBAL void *)(srcb[i] + (size_t)kt * WBK),
+                                            (VKL_LDS void *)(base + kPlanes * A_BYTES + (wave + WWAVES * i) * 1024), 16,
+                                            0, 0);
+        else
+          {
+            const int p = (i - BG) / AG, g = (i - BG) % AG;
+            __builtin_amdgcn_global_load_lds (
+                (const VKL_GLOBAL void *)(srca[g] + (size_t)kt * kPlanes * WBK + p * WBK),
+                (VKL_LDS void *)(base + p * A_BYTES + (wave + WWAVES * g) * 1024), 16, 0, 0);
+          }
+      }
+  };
+  v8 af[2][kPlanes][TM], bf[2][WTN];
+  auto read_frags = [&] (int st, int q, int buf) {
+    const uint8_t *sb = wide_lds + st * STAGE_BYTES;
+#pragma unroll
+    for (int jn = 0; jn < WTN; ++jn)
+      bf[buf][jn] = *(const v8 *)(sb + boff[q] + jn * 32 * WROWB);
+#pragma unroll
+    for (int p = 0; p < kPlanes; ++p)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+        af[buf][p][i] = *(const v8 *)(sb + aoff[q] + p * A_BYTES + i * 32 * WROWB);
+  };
+  constexpr int NP = kPlanes * TM * WTN, NR = kPlanes * TM + WTN;
+  issue (0, 0, 0, LOADS);
+  __builtin_amdgcn_s_waitcnt (0x0f70); // vmcnt(0)
+  __builtin_amdgcn_s_barrier ();
+  issue (nk > 1 ? 1 : 0, 1, 0, LOADS);
+  read_frags (0, 0, 0);
+  __builtin_amdgcn_sched_barrier (0);
+  // One k-step: on entry tile kt is in stage ST, the fragments of its first quarter are on
+  // their way and tile kt + 1 is on its way into the other stage.
+  auto step = [&] (int kt, auto stc) {
+    constexpr int ST = decltype (stc)::value;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      {
+        if (q < 3)
+          read_frags (ST, q + 1, (q + 1) & 1);
+        else
+          {
+            // tile kt + 1 is there and nobody reads tile kt any more: its stage takes tile
+            // kt + 2 (past the end the last tile again, which nothing reads)
+            __builtin_amdgcn_s_waitcnt (0x0070); // vmcnt(0) lgkmcnt(0)
+            __builtin_amdgcn_s_barrier ();
+            __builtin_amdgcn_sched_barrier (0);
+            read_frags (ST ^ 1, 0, 0);
+            issue (kt + 2 < nk ? kt + 2 : nk - 1, ST, 0, LOADS);
+          }
+#pragma unroll
+        for (int p = 0; p < kPlanes; ++p)
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int jn = 0; jn < WTN; ++jn)
+              {
+                float16v &sum = p ? low[i][jn] : acc[i][jn];
+                sum = WideElem<GemmSegArgs>::mfma (bf[q & 1][jn], af[q & 1][p][i], sum);
+              }
+        if (q < 3)
+          WideOrder<0, NP, NR, 0>::run ();
+        else
+          WideOrder<0, NP, NR, LOADS>::run ();
+        __builtin_amdgcn_sched_barrier (0);
+      }
+  };
+  int kt = 0;
+  for (; kt + 2 <= nk; kt += 2)
+    {
+      step (kt, WideInt<0> ());
+      step (kt + 1, WideInt<1> ());
+    }
+  if (kt < nk)
+    step (kt, WideInt<0> ());
+  __builtin_amdgcn_s_waitcnt (0x0f70); // no load may outlive the workgroup's LDS
+  __builtin_amdgcn_s_barrier ();       // (nor a fragment read the parked sums)
+
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int jn = 0; jn < WTN; ++jn)
+#pragma unroll
+      for (int q = 0; q < 16; ++q)
+        acc[i][jn][q] += low[i][jn][q];
+  if (!part) // (of parts the sum is looked at)
+    wide_f32_again<TM> (a, acc, lane, m0 + wm * TM * 32, n0 + wn * 64, a.K / kPlanes);
+  wide_epilogue<false, TM, WTN> (a, acc, wide_lds, wave, lane, m0 + wm * TM * 32, n0 + wn * 64, 0, 1, part);
+}
+
 template <int BM, bool UPGATE, class Args = GemmArgs, int PLANES = 1>
 __global__ __launch_bounds__ (WWAVES * 64) void
 gemm_wide_f16_kernel (const Args a, WideGrid grid, int vec, int ksplit, float *ws)
@@ -1155,9 +1325,9 @@ seg_f32_again (const GemmSegArgs &a, float (&v)[8], int m, int n, int lane, int 
 }
 
 // adds the parts of a split k range in order and applies the segments' epilogue; the
-// values of four parts are requested at a time.  PLANES: as for the product.
+// values of four parts are requested at a time.  PLANES: a product of planes.
 constexpr int kSegReduce = 64; // threads: few values, spread over many compute units
-template <int PLANES>
+template <bool PLANES>
 __global__ __launch_bounds__ (kSegReduce) void
 wide_reduce_seg_kernel (const GemmSegArgs a, const float *ws, int parts)
 {
@@ -1165,7 +1335,7 @@ wide_reduce_seg_kernel (const GemmSegArgs a, const float *ws, int parts)
   const size_t all = (size_t)a.M * n8;
   size_t i = (size_t)blockIdx.x * kSegReduce + threadIdx.x;
   const bool live = i < all;
-  if (PLANES == 1 && !live)
+  if (!PLANES && !live)
     return;
   i = live ? i : all - 1;
   const int m = (int)(i / n8), n = (int)(i % n8) * 8;
@@ -1200,9 +1370,9 @@ wide_reduce_seg_kernel (const GemmSegArgs a, const float *ws, int parts)
         for (int e = 0; e < 8; ++e)
           v[e] += ldg (src + min (n + e, a.N - 1));
       }
-  if (PLANES > 1)
+  if (PLANES)
     {
-      seg_f32_again (a, v, m, n, (int)threadIdx.x, a.K / PLANES);
+      seg_f32_again (a, v, m, n, (int)threadIdx.x, a.K / kPlanes);
       if (!live)
         return;
     }
@@ -1216,17 +1386,16 @@ wide_reduce_seg_kernel (const GemmSegArgs a, const float *ws, int parts)
 // 128-row tiles 0.60 + 5.1, cut tiles likewise; where a segment's sums are parked in LDS 9.6 and
 // 5.6 more per round, which parts leave to the reduction; that launch 3.6 + its bytes at 1.7
 // TB/s).  With the constants of the planes of a 32-bit operand, whose weights come from the L2 two
-// times of three, it was 2.8 and 54 % slower than the best plan, in the mean and at worst, and
+// times of three then, it was 2.8 and 54 % slower than the best plan, in the mean and at worst, and
 // divided too little where few tiles stream the weights: 128 x 8064 x 2048 26 us, 28 with GELU, in
 // one part and 22 in two, 160 x 5504 x 2048 23 and 21, 512 x 2048 x 2048 with GELU 28 and 21.
 // Tiles of 64 rows have two workgroups to a compute unit: up to 256 of them take 0.54 per k-step +
-// 2.6, up to 512 0.81 + 3.7 (planes 0.37 + 1.7 and 0.47 + 6.3).  They win where rows are few or half
-// of a taller tile is empty; us without / with them, bf16: 40 x 8064 x 2048 16.3 / 14.5, 128 x
-// 2048 x 7552 21.0 / 18.1, 12 x 16128 x 4096 35.3 / 30.2; planes: 12 x 16128 x
-// 4096 54.7 / 43.5, 300 x 5504 x 2048 50.1 / 41.9.  Over 198 products of 2 to 2048 rows (114 of
-// planes) the plan is 1.1 % (0.7) slower than the best in the mean; without these tiles it was 4.7
-// (6.6).  Not yet for bf16 operands of more than 128 rows, where they are faster too, but whole where
-// products are held to be in parts (160 x 5504 x 2048 18.4 us, 128-row tiles in two parts 20.3).
+// 2.6, up to 512 0.81 + 3.7.  They win where rows are few or half of a taller tile is empty; us
+// without / with them: 40 x 8064 x 2048 16.3 / 14.5, 128 x 2048 x 7552 21.0 / 18.1, 12 x 16128 x
+// 4096 35.3 / 30.2.  Over 198 products of 2 to 2048 rows the plan is 1.1 % slower than the best in
+// the mean; without these tiles it was 4.7.  Not yet for operands of more than 128 rows, where they
+// are faster too, but whole where products are held to be in parts (160 x 5504 x 2048 18.4 us,
+// 128-row tiles in two parts 20.3).
 WidePlan
 wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
 {
@@ -1235,8 +1404,7 @@ wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
     double step256, round256, step128, round128, reduce, rate, park256, park128;
     double one64, first64, two64, round64; // 64-row tiles: one and two workgroups per compute unit
   };
-  const Fit f = a.xf ? Fit{ 0.79, 5, 0.47, 4, 5, 2.5e6, 0, 0, 0.37, 1.7, 0.47, 6.3 }
-                     : Fit{ 0.67, 8.8, 0.60, 5.1, 3.6, 1.7e6, 9.6, 5.6, 0.54, 2.6, 0.81, 3.7 };
+  const Fit f = { 0.67, 8.8, 0.60, 5.1, 3.6, 1.7e6, 9.6, 5.6, 0.54, 2.6, 0.81, 3.7 };
   WidePlan best = { 0, 1 };
   double best_cost = 0;
   const int nk = a.K / WBK;
@@ -1246,7 +1414,7 @@ wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
   for (int bm = 64; bm <= WBM; bm *= 2)
     for (int ks = 1; ks <= 16; ks *= 2)
       {
-        if ((a.M < bm && bm > 128) || (bm == 64 && !a.xf && a.M > 128))
+        if ((a.M < bm && bm > 128) || (bm == 64 && a.M > 128))
           continue;
         if (ks > 1
             && (nk / ks < 4 || (size_t)ks * a.M * a.N * sizeof (float) > scratch))
@@ -1278,22 +1446,44 @@ wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
   return best;
 }
 
-// ws: scratch for the parts of a split k range (null: the stream's)
-template <int BM, int PLANES = 1>
-int
-launch_wide_bf16 (const GemmSegArgs &a, int ksplit, float *ws, hipStream_t s)
+// The tiles of a product of planes: 64 rows in up to 16 parts of the k range (one and two
+// workgroups to a compute unit, as above), or wide_f16_tile's 256 rows, the last of which may be
+// cut.  Fitted to 160 products of 2 to 2048 rows in 1 to 16 parts and 151 of 192 to 2048 rows in
+// both forms: 0.5 % slower than the best plan in the mean, 7 at worst; without 256 rows 2.5 % and 22
+// (2048 x 8064 x 2048 187 us with them, 229 without; 512 x 16128 x 4096 175, 199).
+WidePlan
+wide_plan_planes (const GemmSegArgs &a, size_t scratch)
 {
-  static LdsLimit limit;
-  constexpr size_t lds = wide_lds_f16<BM> ();
-  const auto kernel = gemm_wide_f16_kernel<BM, false, GemmSegArgs, PLANES>;
-  if (int e = limit.raise ((const void *)kernel, lds))
-    return e;
-  StreamScratch own;
-  if (ksplit > 1 && !ws && !(ws = own.take (s)))
-    ksplit = 1;
-  const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + WBN - 1) / WBN;
-  const WideGrid tiles (tiles_m, tiles_n, 1, ksplit, BM == WBM);
-  kernel<<<dim3 ((unsigned)tiles.groups ()), dim3 (WWAVES * 64), lds, s>>> (a, tiles, 1, ksplit, ws);
+  const int nk = a.K / WBK / kPlanes, tiles_n = (a.N + WBN - 1) / WBN;
+  WidePlan best = { kPlaneRows, 1 };
+  double best_cost = 0;
+  for (int ks = 1; ks <= 16; ks *= 2)
+    {
+      if (ks > 1 && (nk / ks < 4 || (size_t)ks * a.M * a.N * sizeof (float) > scratch))
+        continue;
+      const int tiles = (a.M + kPlaneRows - 1) / kPlaneRows * tiles_n * ks;
+      const int two = tiles / (2 * WideGrid::kUnits), rest = tiles % (2 * WideGrid::kUnits);
+      const double steps = (double)nk / ks, round = 1.14 * steps + 6.4;
+      double cost = two * round + (ks > 1 ? 4.2 + (double)ks * a.M * a.N * sizeof (float) / 3.8e6 : 0);
+      if (rest > 0)
+        cost += rest <= WideGrid::kUnits ? 0.935 * steps + 1.6 : round;
+      if (ks == 1 || cost < best_cost)
+        best.ksplit = ks, best_cost = cost;
+    }
+  if (a.M >= WBM)
+    {
+      const WideGrid tiles ((a.M + WBM - 1) / WBM, tiles_n, 1, 1, true);
+      const int whole = (tiles.whole + WideGrid::kUnits - 1) / WideGrid::kUnits;
+      if (whole * (1.97 * nk + 9.6) + (tiles.whole < tiles.tiles () ? 1.44 * nk + 6.6 : 0) < best_cost)
+        best = { WBM, 1 };
+    }
+  return best;
+}
+
+template <bool PLANES>
+int
+launch_reduce_seg (const GemmSegArgs &a, int ksplit, const float *ws, hipStream_t s)
+{
   if (ksplit > 1)
     {
       const size_t total = (size_t)a.M * ((a.N + 7) / 8);
@@ -1302,13 +1492,35 @@ launch_wide_bf16 (const GemmSegArgs &a, int ksplit, float *ws, hipStream_t s)
   return (int)hipGetLastError ();
 }
 
-template <int PLANES>
+template <int BM, int PLANES = 1>
 int
-launch_wide_bf16_any (const GemmSegArgs &a, const WidePlan &p, float *ws, hipStream_t s)
+launch_wide_bf16 (const GemmSegArgs &a, int ksplit, hipStream_t s)
 {
-  return p.bm == WBM   ? launch_wide_bf16<WBM, PLANES> (a, p.ksplit, ws, s)
-         : p.bm == 128 ? launch_wide_bf16<128, PLANES> (a, p.ksplit, ws, s)
-                       : launch_wide_bf16<64, PLANES> (a, p.ksplit, ws, s);
+  static LdsLimit limit;
+  constexpr size_t lds = wide_lds_f16<BM> ();
+  const auto kernel = gemm_wide_f16_kernel<BM, false, GemmSegArgs, PLANES>;
+  if (int e = limit.raise ((const void *)kernel, lds))
+    return e;
+  StreamScratch own;
+  float *ws = nullptr;
+  if (ksplit > 1 && !(ws = own.take (s)))
+    ksplit = 1;
+  const WideGrid tiles ((a.M + BM - 1) / BM, (a.N + WBN - 1) / WBN, 1, ksplit, BM == WBM);
+  kernel<<<dim3 ((unsigned)tiles.groups ()), dim3 (WWAVES * 64), lds, s>>> (a, tiles, 1, ksplit, ws);
+  return launch_reduce_seg<false> (a, ksplit, ws, s);
+}
+
+// ws: scratch for the parts of the k range
+int
+launch_wide_planes (const GemmSegArgs &a, int ksplit, float *ws, hipStream_t s)
+{
+  static LdsLimit limit;
+  constexpr size_t lds = wide_lds_planes ();
+  if (int e = limit.raise ((const void *)gemm_wide_planes_kernel, lds))
+    return e;
+  const WideGrid tiles ((a.M + kPlaneRows - 1) / kPlaneRows, (a.N + WBN - 1) / WBN, 1, ksplit, false);
+  gemm_wide_planes_kernel<<<dim3 ((unsigned)tiles.groups ()), dim3 (WWAVES * 64), lds, s>>> (a, tiles, ksplit, ws);
+  return launch_reduce_seg<true> (a, ksplit, ws, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1320,21 +1532,19 @@ launch_wide_bf16_any (const GemmSegArgs &a, const WidePlan &p, float *ws, hipStr
 // without any rounding that the 32-bit matrix instructions would not do (they add
 // one product at a time, these sixteen before they round).  The matrix cores do
 // three such products in a fifth of the time of one in fp32.  Against 64 bits the
-// result is closer than that of the 32-bit instructions: relative error 2e-7 to 7e-7
-// instead of 8e-7 to 1.4e-6 over K = 2048 to 5504 (1.4e-7 / 4e-7 at K = 512).
+// result is closer than that of the 32-bit instructions: relative error 1.3e-7 to 4e-7
+// (1.6e-7 to 7e-7 where the lower planes share the first one's accumulators) instead
+// of 8e-7 to 1.4e-6 over K = 2048 to 7552.
 //
 // What this does not hold for: an infinite weight meets zeros in the lower planes, and
 // of values below 2^-110 the last bits lie below the smallest bf16 number, 2^-133 (the
 // matrix cores take numbers below the smallest normal one as they are).  Such a value gets
 // a NaN for its third plane, and sums that are not finite are formed again by the 32-bit
-// instructions (wide_f32_again; sums of parts of a split k range, which may divide a step's
-// planes, by seg_f32_again).
+// instructions (wide_f32_again; sums of parts of a split k range by seg_f32_again).
 //
-// Planes lie in blocks of 64 columns, [plane 0 | plane 1 | plane 2] of a block next
-// to each other, so that the wide kernel walks them as one row of 3 K values and
-// takes every k-step of the weights three times (the second and third time from
-// the L2).
-constexpr int kPlanes = 3;
+// Planes lie in blocks of 64 columns, [plane 0 | plane 1 | plane 2] of a block next to
+// each other: one k-step of gemm_wide_planes_kernel, three of wide_f16_tile, which walks
+// them as one row of 3 K values and takes every k-step of the weights three times.
 
 __global__ __launch_bounds__ (256) void
 split_planes_kernel (const float *x, size_t xs, int M, int K, uint16_t *out)
@@ -1378,7 +1588,9 @@ int
 gemm_wide_bf16_launch (const GemmSegArgs &a, hipStream_t s)
 {
   const WidePlan p = wide_plan_bf16 (a, StreamScratch::bytes ());
-  return launch_wide_bf16_any<1> (a, p, nullptr, s);
+  return p.bm == WBM   ? launch_wide_bf16<WBM> (a, p.ksplit, s)
+         : p.bm == 128 ? launch_wide_bf16<128> (a, p.ksplit, s)
+                       : launch_wide_bf16<64> (a, p.ksplit, s);
 }
 
 bool
@@ -1387,8 +1599,8 @@ gemm_wide_f32_launch (const GemmSegArgs &a, hipStream_t s, int &err)
   // Short rows of few values are over in the time of two more launches.  Measured, us,
   // 32-bit instructions / planes: K = 256, N = 2048, 300 rows 10 / 16, 4000 rows 48 / 36;
   // K = 512, N = 512, 1000 rows 15.5 / 20; K = 768, N = 128, 1 row 20 / 13; K = 2048,
-  // N = 2048, 1 row 47 / 14, 2000 rows 162 / 65; K = 2048, N = 8064, 300 rows 121 / 51;
-  // K = 5504, N = 2048, 300 rows 161 / 43; K = 4096, N = 11008, 2000 rows 1530 / 628.
+  // N = 2048, 1 row 47 / 14, 2000 rows 162 / 60; K = 2048, N = 8064, 300 rows 121 / 48;
+  // K = 5504, N = 2048, 300 rows 161 / 42; K = 4096, N = 11008, 2000 rows 1530 / 570.
   if (a.K <= 512 && (size_t)a.M * a.N * a.K <= (size_t)1 << 30)
     return false;
   // Where their 64 x 64 tiles just fill the compute units once, the 32-bit instructions need
@@ -1433,9 +1645,9 @@ gemm_wide_f32_launch (const GemmSegArgs &a, hipStream_t s, int &err)
           if (a.seg[i].residual)
             b.seg[i].residual = a.seg[i].residual + (size_t)m0 * a.seg[i].ys;
         }
-      const WidePlan p = wide_plan_bf16 (b, half);
-      float *parts = ws + half / sizeof (float);
-      err = launch_wide_bf16_any<kPlanes> (b, p, parts, s);
+      const WidePlan p = wide_plan_planes (b, half);
+      err = p.bm == WBM ? launch_wide_bf16<WBM, kPlanes> (b, 1, s)
+                        : launch_wide_planes (b, p.ksplit, ws + half / sizeof (float), s);
       if (err)
         return true;
     }

@@ -440,12 +440,17 @@ def main():
         per = 34.0 / 32.0 if cfg["wtype"] == 8 else 2.0
         wbytes = (cfg["n_layers"] * (4.0 * cfg["dim"] ** 2 + 3.0 * cfg["dim"] * cfg["ffn"])
                   + cfg["vocab"] * cfg["dim"]) * per
+        # rows that a step hands over inside one launch: see layers_launch_supported
+        narrow = (cfg["dim"] // 8 + cfg["n_heads"] <= 256 and cfg["dim"] <= (2048 if cfg["wtype"] == 8 else 1024)
+                  and cfg["ffn"] <= 3 * cfg["dim"])
         if dom == "layer":
             # (row chunks of 4096 values as the library picks them: see launch_layer_wt)
             xd, xf = (cfg["dim"] + 4095) // 4096, (cfg["ffn"] + 4095) // 4096
             xd, xf = (1, 1) if (xd, xf) == (1, 1) else ((1, 3) if xd == 1 and xf <= 3 else (2, 4))
             dom_kernel = "decode_layer_kernel<%d, %d, %d, %s> (the five phases of a layer in one launch)" % (
                 8 if cfg["wtype"] == 8 else 1, xd, xf, "true" if wbytes > (288 << 20) else "false")
+            if narrow:
+                dom_kernel = "decode_layers_kernel (one layer of the step's only launch, by itself)"
         elif dom == "attention+wo":
             dom_kernel = "decode_attn_wo_kernel<%d, %d> (attention + Wo)" % (8 if cfg["wtype"] == 8 else 1,
                                                                             min(4, (cfg["dim"] + 4095) // 4096))
@@ -489,7 +494,8 @@ def main():
         "data": "synthetic: random-init N(0,0.02) weights" + (" quantised to Q8_0" if cfg["wtype"] == 8 else " in FP16")
                 + ", random prompt ids",
         "config": {"workload": args.workload, "prompt_tokens": n_prompt, "decode_tokens": steps,
-                   "decode_mode": ("one launch per layer" if "layer" in per_phase else "one launch per phase")
+                   "decode_mode": "one launch per step or all layers" if narrow and "layer" in per_phase else
+                                  ("one launch per layer" if "layer" in per_phase else "one launch per phase")
                                   + (", replayed from a HIP graph" if args.decode_graph else ""),
                    "dims": {k: cfg[k] for k in ("dim", "n_layers", "n_heads", "ffn", "vocab", "maxlen")}},
         "decode_tokens_per_second_host_interface": round(host_tok_s, 1),

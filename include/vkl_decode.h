@@ -135,8 +135,9 @@ const uint32_t *vkl_decode_status_word (const vkl_decode_model *m);
  * ids[i] (device memory) at position pos0 + i and writes its arg-max id to
  * ids[i + 1], the loop of app/llama2_infer.cpp:140-177 with the sampler on the
  * device.  The launches of one step are captured once in a HIP graph (per
- * model / buffers / attention form) and replayed; results are identical to
- * n_steps calls of vkl_decode_step in the same mode.  logits32 (optional)
+ * model / buffers / attention form) and replayed (a step of one launch is
+ * launched as it is); results are identical to n_steps calls of
+ * vkl_decode_step in the same mode.  logits32 (optional)
  * receives the logits of the last step.  The stream must not be capturing. */
 int vkl_decode_loop (const vkl_decode_model *m, uint32_t *ids, uint32_t pos0,
                      int n_steps, int mode, float *logits32, void *stream);

@@ -206,8 +206,9 @@ typedef struct
 int vkl_recurrence (const vkl_recurrence_args *a, int S, uint32_t pos0,
                     int form, void *scratch, size_t scratch_bytes,
                     void *stream);
-/* whether VKL_RECUR_AUTO takes the chunked form (it needs scratch memory then; below 24 tokens it
- * takes the other one, which needs z, where there is none) */
+/* whether VKL_RECUR_AUTO takes the chunked form (the delta rule from 5 tokens on, decaying sums from
+ * 24; it needs scratch memory then; below 24 tokens it takes the other one, which needs z, where
+ * there is none) */
 int vkl_recurrence_chunked (const vkl_recurrence_args *a, int S);
 /* what the chunked form needs for S tokens at once (it takes them in pieces if
  * there is less, at least what 64 tokens need) */

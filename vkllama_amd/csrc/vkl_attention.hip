@@ -83,7 +83,8 @@ struct AttnArgs
   const float *gate;  // optional [S, gs]: head h's output times sigmoid (gate[s, h])
   size_t gs;
   int chunk, sink;    // CHUNKED kernels: see vkl_attn_prefill_chunked_bf16
-  int parts;          // workgroups that share the keys of a query tile
+  int parts;          // workgroups that share the keys of a query tile (at most, with a span)
+  int span;           // != 0: tiles of keys to a part, at most
   float *ws;          // parts > 1: their results, see part_row
 };
 
@@ -521,6 +522,13 @@ template <int KIND, int PER, int N, int AHEAD> struct Alternate
   }
 };
 
+// parts of a query tile that sees n tiles of keys
+__host__ __device__ __forceinline__ int
+parts_of (const AttnArgs &a, int n)
+{
+  return a.span ? (n + a.span - 1) / a.span : a.parts;
+}
+
 template <int HD, class E, bool CHUNKED, bool PARTS>
 __global__ __launch_bounds__ (kThreads, 2) void
 attn_tiles_kernel (const AttnArgs a)
@@ -557,8 +565,10 @@ attn_tiles_kernel (const AttnArgs a)
   int t0 = CHUNKED ? chunk_start (q0) / kBKey : 0, t1 = (kmax + kBKey - 1) / kBKey;
   if (PARTS)
     {
-      const int n = t1 - t0, first = t0;
-      t0 = first + n * part / a.parts, t1 = first + n * (part + 1) / a.parts;
+      const int n = t1 - t0, first = t0, parts = parts_of (a, n);
+      if (part >= parts)
+        return;
+      t0 = first + n * part / parts, t1 = first + n * (part + 1) / parts;
     }
   const int kvh = head / a.rep;
   const uint16_t *kb = a.k + (size_t)kvh * a.kcs;
@@ -812,9 +822,12 @@ attn_parts_kernel (const AttnArgs a)
   const int row = i / a.H, head = i - row * a.H;
   if (row >= a.S)
     return;
+  const int q0 = row / kBQ * kBQ, shift = a.L - a.S;
+  const int parts = parts_of (a, (min (a.L, q0 + kBQ + shift) + kBKey - 1) / kBKey
+                                     - (a.chunk ? (q0 + shift) / a.chunk * a.chunk : 0) / kBKey);
   // lane p looks at part p
   float pm = -3.0e38f, ps = 0.f;
-  if (lane < a.parts)
+  if (lane < parts)
     {
       const float *pr = part_row<HD> (a, lane, head, row);
       pm = vkl::ldg (pr + HD), ps = vkl::ldg (pr + HD + 1);
@@ -823,7 +836,7 @@ attn_parts_kernel (const AttnArgs a)
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1)
     top = fmaxf (top, __shfl_xor (top, d, 64));
-  const float w = lane < a.parts ? __builtin_amdgcn_exp2f (pm - top) : 0.f;
+  const float w = lane < parts ? __builtin_amdgcn_exp2f (pm - top) : 0.f;
   float total = w * ps;
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1)
@@ -832,7 +845,7 @@ attn_parts_kernel (const AttnArgs a)
 #pragma unroll
   for (int e = 0; e < VPL; ++e)
     o[e] = 0.f;
-  for (int p = 0; p < a.parts; ++p)
+  for (int p = 0; p < parts; ++p)
     {
       const float wp = __shfl (w, p, 64);
       const float *pr = part_row<HD> (a, p, head, row) + lane * VPL;
@@ -887,11 +900,47 @@ key_parts (const AttnArgs &a, int hd)
   return best;
 }
 
+// How many tiles of keys a part gets where query tiles get different numbers of parts (0: all
+// get the same).  Where two parts each leave a quarter of the 512 places empty or more (up to 200
+// groups), the longest rows get three: the smallest span that needs no more than 500 places
+// (of 512, as of 528, some cases took the time of three workgroups on a compute unit) and
+// three parts.  A compute unit takes 1.1 us per tile however many workgroups it holds, and two
+// long halves on one are what a launch waits for.  16 heads of 128, 1500 rows behind 300 / 600 /
+// 1200 / 2400 keys, us: in two 42 / 46 / 55 / 72, as here 37 / 40 / 48 / 66; 24 heads, 1000
+// behind 1200 50 / 47; 32 heads, 700 behind 2400 61.8 / 61.0.  With more groups (16 heads, 2000 rows
+// behind 1200: 69 / 71) and where all get three (24 heads, 700 rows: 35.4 / 36.5) even parts stay.
+int
+key_span (const AttnArgs &a)
+{
+  const int groups = a.ntq * a.H, shift = a.L - a.S;
+  if (a.parts != 2 || groups > 200)
+    return 0;
+  auto tiles = [&] (int q0) {
+    return (std::min (a.L, q0 + kBQ + shift) + kBKey - 1) / kBKey
+           - (a.chunk ? (q0 + shift) / a.chunk * a.chunk : 0) / kBKey;
+  };
+  int most = 0;
+  for (int q0 = 0; q0 < a.S; q0 += kBQ)
+    most = std::max (most, tiles (q0));
+  for (int span = (most + 2) / 3; 2 * span < most; ++span)
+    {
+      int places = 0;
+      for (int q0 = 0; q0 < a.S; q0 += kBQ)
+        places += (tiles (q0) + span - 1) / span * a.H;
+      if (places <= 500)
+        return span;
+    }
+  return 0;
+}
+
 template <int HD, class E, bool CHUNKED>
 int
 launch_tiles (AttnArgs a, hipStream_t s)
 {
   a.parts = key_parts (a, HD);
+  const size_t part = (size_t)a.H * a.S * (HD + 4) * sizeof (float);
+  if ((a.span = HD == 128 && 3 * part <= vkl::StreamScratch::bytes () ? key_span (a) : 0))
+    a.parts = 3;
   vkl::StreamScratch own;
   if (a.parts > 1)
     {
@@ -900,13 +949,13 @@ launch_tiles (AttnArgs a, hipStream_t s)
       if (hipStreamIsCapturing (s, &capture) != hipSuccess)
         (void)hipGetLastError (); // (the default stream while another one is captured)
       else if (capture == hipStreamCaptureStatusNone
-               && (size_t)a.parts * a.H * a.S * (HD + 4) * sizeof (float) <= vkl::StreamScratch::bytes ())
+               && a.parts * part <= vkl::StreamScratch::bytes ())
         a.ws = own.take (s);
     }
   const int groups = a.ntq * a.H;
   if (!a.ws)
     {
-      a.parts = 1;
+      a.parts = 1, a.span = 0;
       attn_tiles_kernel<HD, E, CHUNKED, false><<<dim3 ((unsigned)groups), dim3 (kThreads), 0, s>>> (a);
       return vkl_launch_status ();
     }

@@ -34,3 +34,30 @@ def test_up_gate_q8_0(dev, N, K):
     want = gate / (1 + np.exp(-gate)) * up
     # sums of order one: fp32 roundings of some 1e-6 of them, one rounding to fp16
     assert (np.abs(got - want) <= 2.0 ** -11 * np.abs(want) + 2e-5).all()
+
+
+@pytest.mark.parametrize("N", [(1 << 23) - 2, 1 << 23, (1 << 23) + 4096])   # on either side of what the step's kernel deals
+@pytest.mark.parametrize("fused", [False, True])
+def test_more_rows_than_32_bits_deal(dev, N, fused):
+    """N rows times 512 workgroups no longer fit 32 bits: every row is written all the same."""
+    K, P = 32, 4094
+    rng = np.random.default_rng(N)
+    x = rng.standard_normal(K).astype(np.float16)
+    ws, want = [], []
+    for _ in range(2):
+        q = rng.integers(-127, 128, (P, K), dtype=np.int8)
+        d = rng.uniform(0.5, 1.5, (P, 1)).astype(np.float16) * np.float16(K ** -0.5 / 64)
+        ws.append(dev.upload_q8_0(np.resize(blocks(q, d), (N, 34)), N, K))
+        want.append((q.astype(np.float64) * d.astype(np.float64)) @ x.astype(np.float64))
+    y, dx = dev.alloc(N * 2), dev.upload(x)
+    y.write(np.full(N, 0x7E00, np.uint16))
+    if fused:
+        capi.check(capi.lib().vkl_ffn_upgate_q8_0(dx.ptr, ws[0].ptr, ws[1].ptr, 1, N, K, y.ptr, dev.stream))
+        want = want[1] / (1 + np.exp(-want[1])) * want[0]
+    else:
+        capi.check(capi.lib().vkl_matmul_q8_0(dx.ptr, ws[0].ptr, 1, N, K, K, N, 1.0, 0.0, 0, None, y.ptr, None, dev.stream))
+        want = want[0]
+    dev.sync()
+    got = y.read(np.uint16, (N,)).view(np.float16).astype(np.float64)
+    want = np.resize(want, N)
+    assert (np.abs(got - want) <= 2.0 ** -11 * np.abs(want) + 2e-5).all()

@@ -1095,11 +1095,13 @@ namespace vkl
 {
 // One token row times a matrix on the decode step's down-projection kernel:
 // y[N] = W[N, K] x[K] (+ residual), W planar Q8_0 (wtype 8) or dense fp16.
+// N: up to 512 workgroups (two per compute unit) share up to N units, by products of the two in
+// 32 bits (dealt_units).
 bool
 decode_gemv_supported (int N, int K, int wtype)
 {
   return (wtype == 8 || wtype == 1) && N > 0 && (N % 2) == 0 && K > 0
-         && (K % 32) == 0 && K <= 16384 && N <= (1 << 24)
+         && (K % 32) == 0 && K <= 16384 && N < (1 << 23)
          && lds_bytes_needed (0, K, 1, 64) <= 160 * 1024;
 }
 

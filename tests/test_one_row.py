@@ -61,3 +61,32 @@ def test_more_rows_than_32_bits_deal(dev, N, fused):
     got = y.read(np.uint16, (N,)).view(np.float16).astype(np.float64)
     want = np.resize(want, N)
     assert (np.abs(got - want) <= 2.0 ** -11 * np.abs(want) + 2e-5).all()
+
+
+@pytest.mark.parametrize("N,K", [(2, 32), (2, 64), (6, 96), (14, 64)])      # less than 1 KiB
+@pytest.mark.parametrize("fused", [False, True])
+def test_matrices_at_the_end_of_their_memory(dev, N, K, fused):
+    """Waves without rows of their own request nothing behind a small matrix."""
+    rng = np.random.default_rng(N * K)
+    x, room = rng.standard_normal(K).astype(np.float16), 1 << 21
+    bufs, ptrs, want = [], [], []
+    for _ in range(2):
+        q = rng.integers(-127, 128, (N, K), dtype=np.int8)
+        d = rng.uniform(0.5, 1.5, (N, K // 32)).astype(np.float16) * np.float16(K ** -0.5 / 64)
+        planar = q.tobytes() + d.tobytes()
+        at = (room - len(planar)) // 16 * 16
+        whole = np.zeros(room, np.uint8)
+        whole[at:at + len(planar)] = np.frombuffer(planar, np.uint8)
+        bufs.append(dev.upload(whole))
+        ptrs.append(bufs[-1].ptr.value + at)
+        want.append((q.reshape(N, -1, 32) * d.astype(np.float64)[:, :, None]).reshape(N, K) @ x.astype(np.float64))
+    y, dx = dev.alloc(N * 2), dev.upload(x)
+    if fused:
+        capi.check(capi.lib().vkl_ffn_upgate_q8_0(dx.ptr, ptrs[0], ptrs[1], 1, N, K, y.ptr, dev.stream))
+        want = want[1] / (1 + np.exp(-want[1])) * want[0]
+    else:
+        capi.check(capi.lib().vkl_matmul_q8_0(dx.ptr, ptrs[0], 1, N, K, K, N, 1.0, 0.0, 0, None, y.ptr, None, dev.stream))
+        want = want[0]
+    dev.sync()
+    got = y.read(np.uint16, (N,)).view(np.float16).astype(np.float64)
+    assert (np.abs(got - want) <= 2.0 ** -11 * np.abs(want) + 2e-5).all()

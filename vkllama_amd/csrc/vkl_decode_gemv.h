@@ -506,8 +506,10 @@ template <int WT = 8, bool NT = false, int RU = 2> struct Gemv
       b.res = ldg ((const uint32_t *)(rp + (2 * u + 1 < ps.N ? 2 * u : 0)));
     // an item past the wave's last (requested all the same when begin ()
     // issues unconditionally) reads one and the same KiB for every load, so
-    // that it adds nothing to the traffic
+    // that it adds nothing to the traffic: the first of row 0, or the row where
+    // it is shorter (a small matrix need not have a KiB)
     const bool none = it >= ps.nit;
+    const int idle = min (ps.lane * 16, ps.Kp - 16);
     if (none)
       {
 #pragma unroll
@@ -518,7 +520,7 @@ template <int WT = 8, bool NT = false, int RU = 2> struct Gemv
     for (int s = 0; s < S; ++s)
       {
         const int kk = c * CHUNK + s * (VKL_WAVE * 16) + ps.lane * 16;
-        const int kc = none ? ps.lane * 16 : (kk < ps.Kp ? kk : 0);
+        const int kc = none ? idle : (kk < ps.Kp ? kk : 0);
 #pragma unroll
         for (int r = 0; r < R; ++r)
           {

@@ -123,9 +123,12 @@ int vkl_decode_step (const vkl_decode_model *m, const uint32_t *tok,
  * the workgroup concerned drops its results instead of storing them, and the
  * step's results are invalid.  This call synchronises the stream and returns
  * 0 if nothing of the kind happened since the last call,
- * hipErrorLaunchFailure otherwise (the mark is cleared); the caller then
- * repeats the step with mode 0 and separate_attn_wo = 1, which wait for
- * nothing.  No counterpart in the reference, which has no such kernels. */
+ * hipErrorLaunchFailure otherwise (the mark is cleared, and with it all that
+ * the workgroups of lost launches have left for one another in scratch and
+ * flags); the caller then repeats the step with mode 0 and
+ * separate_attn_wo = 1, which wait for nothing, and may return to the other
+ * forms afterwards.  No counterpart in the reference, which has no such
+ * kernels. */
 int vkl_decode_status (const vkl_decode_model *m, void *stream);
 /* the device word that vkl_decode_status looks at: zero if nothing of the kind
  * happened (null for a model without scratch) */

@@ -1283,7 +1283,16 @@ vkl_decode_status (const vkl_decode_model *m, void *stream)
     return 0;
   if (getenv ("VKL_DECODE_VERBOSE"))
     fprintf (stderr, "vkl_decode_status: error word 0x%x\n", gave_up);
+  // Everything that workgroups leave for one another starts anew.  A workgroup that became
+  // resident only after workgroup 0 had given up (the usual reason for a wait to give up) has read
+  // the number of the NEXT launch and may have left words, flags and tickets of it, which that
+  // launch would take for its own.  All launches have ended here, the late ones too.
   VKL_HIP (hipMemsetAsync (sc.sync + 1, 0, sizeof (uint32_t), s));
+  VKL_HIP (hipMemsetAsync (sc.lsync, 0, kLayerSyncBytes, s));
+  if (sc.tagged)
+    VKL_HIP (hipMemsetAsync (sc.tagged, 0, (size_t)tagged_rows (m->dim, m->ffn).words * 4, s));
+  if (m->flags)
+    VKL_HIP (hipMemsetAsync (m->flags, 0, kFlagBytes, s));
   VKL_HIP (hipStreamSynchronize (s));
   return (int)hipErrorLaunchFailure;
 }

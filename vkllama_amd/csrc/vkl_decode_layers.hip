@@ -31,7 +31,8 @@
 // a row holds before is always an older tag.  A row is not overwritten while somebody still
 // waits for it: the next layer's needs a row that all workgroups have contributed to since.
 // Waits are bounded and a wait that gave up is reported as in the layer launch; its
-// workgroup publishes nothing from then on.
+// workgroup publishes nothing from then on.  vkl_decode_status clears counter and rows with
+// the error word.
 #include "vkl_decode_shared.h"
 #include <algorithm>
 
@@ -773,7 +774,8 @@ decode_layers_kernel (const Params p, int first, int count, bool whole)
       pick_token (p, parts, last_tag, w, best, lds + map.attn);
     }
   // (every workgroup has read the counter before it published its first word, and this one
-  // has seen words of all)
+  // has seen words of all, unless it gave up: what a workgroup that starts later leaves then is
+  // cleared with the error word)
   if (threadIdx.x == 0)
     st_coherent_u32 (counter, done + (uint32_t)count);
 }

@@ -34,6 +34,7 @@ class Llama:
     def __init__(self, dev, dim, heads, ffn, vocab, layers, maxlen=64, seed=1):
         rng = np.random.default_rng(seed)
         self.dev, self.keep, m = dev, [], Model()
+        self.stream = dev.stream
 
         def up(a):
             self.keep.append(dev.upload(a))
@@ -62,14 +63,17 @@ class Llama:
         m.flags, self.m = flags, m
         self.tok, self.logits = dev.upload(np.zeros(1, np.uint32)), dev.alloc(vocab * 4)
 
+    def launch(self, pos, mode):
+        capi.check(lib().vkl_decode_step(C.byref(self.m), self.tok.ptr, pos, mode, self.logits.ptr, None, self.stream))
+
     def step(self, tok, pos, mode):
         """logits of one token; (nothing waits for them to be right: see status)"""
         self.tok.write(np.array([tok], np.uint32))
-        capi.check(lib().vkl_decode_step(C.byref(self.m), self.tok.ptr, pos, mode, self.logits.ptr, None, self.dev.stream))
+        self.launch(pos, mode)
         return self.logits.read(np.float32, (self.m.vocab,))
 
     def status(self):
-        return lib().vkl_decode_status(C.byref(self.m), self.dev.stream)
+        return lib().vkl_decode_status(C.byref(self.m), self.stream)
 
     def close(self):
         lib().vkl_decode_flags_release(self.m.flags)

@@ -16,6 +16,7 @@ pytestmark = pytest.mark.gpu
     (1024, 3072, 8, 1, 3, 64),     # fp16: the widest
     (1088, 2912, 17, 8, 3, 64),    # Q8_0: a second step of loads in part
     (1792, 4768, 28, 8, 3, 64),    # Q8_0: workgroups for all but four compute units
+    (64, 192, 1, 8, 3, 15900),     # as many positions as half the LDS of a compute unit takes
     (1792, 5408, 14, 8, 3, 64),    # more than three pairs for a wave: a launch per layer
 ])
 def test_all_layers_in_one_launch(dim, ffn, heads, wtype, prompt, maxlen):
@@ -26,9 +27,12 @@ def test_all_layers_in_one_launch(dim, ffn, heads, wtype, prompt, maxlen):
     (64, 8, 2),             # one wave has the vocabulary
     (64, 1, 95234),         # two rounds of what the waves hold, of no round number
     (512, 8, 32000),
-    (512, 1, 70654),        # one row of each in every load, two rounds
-    (1024, 8, 43006),       # as many as the one launch takes
-    (1024, 8, 43012),       # more: a launch of its own
+    (512, 1, 40002),        # one row of each in every load, two rounds
+    (512, 1, 70654),        # more than two rounds: a launch of its own
+    (1024, 8, 30720),       # as many as the one launch takes
+    (1024, 8, 30722),       # more: a launch of its own
+    (1024, 8, 43006),
+    (1024, 8, 43012),
 ])
 def test_whole_step_in_one_launch(dim, wtype, vocab):
     compare(dim, 3 * dim // 64 * 32, max(1, dim // 128), wtype, 3, 64, vocab)

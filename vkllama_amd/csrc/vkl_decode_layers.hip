@@ -22,9 +22,16 @@
 // q and v arrive.
 //
 // The memory path of a compute unit returns loads in order, so a poll returns behind all
-// weights requested before it: everything up to the next layer's K/Q/V is requested at the one
-// point of the layer where the wait is longer than the way from memory, while the heads are
-// computed.
+// weights requested before it: as much as the registers hold is requested at the one point of
+// the layer where the wait is longer than the way from memory, while the heads are computed.
+//
+// Two launches have to fit the GPU at once, as two launches per layer of narrow rows do (two
+// models on two streams would each wait for workgroups that the other one keeps out): a
+// workgroup takes one of two places of its compute unit, 128 registers and at most 80 KB of
+// LDS.  Rows of more than 512 bytes therefore request the down projection's, of more than 1024
+// the next layer's K/Q/V too, only when the up/gate product has left its registers.  With 256
+// registers and all of it requested at the one point above it was no faster, us per token: 512
+// wide Q8_0 97 / now 88, 1024 68 / 66, 1536 83 / 82, 768 wide fp16 87 / 82.
 //
 // The tags of a step follow on those of the step before (a counter in the sync area,
 // advanced at the end of a launch), and every word of a row is written once per layer: what
@@ -397,11 +404,14 @@ lds_map (int dim, int ffn, int maxlen, int hd)
 {
   LdsMap m;
   const int row = (dim * 2 + 15) & ~15;
-  m.xa = 0, m.xb = row, m.xc = 2 * row, m.xr = 3 * row, m.xd = 4 * row;
-  m.words = m.xd + ((ffn * 2 + 15) & ~15);
-  m.attn = m.words + 128 + (5 + kPairs) * kDecWaves * 4;
+  m.words = 0;
+  // rows, or what a head needs: a workgroup has one or the other (the token is picked in a head's
+  // place, behind the last row)
+  m.attn = 128 + (5 + kPairs) * kDecWaves * 4;
+  m.xa = m.attn, m.xb = m.xa + row, m.xc = m.xb + row, m.xr = m.xc + row, m.xd = m.xr + row;
   const int rpb = kDecThreads / (hd / 8);
-  m.bytes = m.attn + 1024 + ((maxlen + 3) & ~3) * 4 + rpb * hd * 4 + 256;
+  const int rows = m.xd + ((ffn * 2 + 15) & ~15), head = m.attn + 1024 + ((maxlen + 3) & ~3) * 4 + rpb * hd * 4 + 256;
+  m.bytes = rows > head ? rows : head;
   return m;
 }
 
@@ -457,7 +467,7 @@ embedding8 (const Params &p, uint32_t tok, int c)
 // arrives; each leaves its arg-max for workgroup 0.  From the last row to the next token 8.5 us
 // (512 wide, 17 MB) where the lm_head launch, its arg-max and two launch boundaries took 33
 // of 120 us per token.
-constexpr int kVocabLoads = 24; // loads of 16 bytes per lane that a wave holds of it
+constexpr int kVocabLoads = 16; // loads of 16 bytes per lane that a wave holds of it (24 do not fit 128 registers)
 
 template <int WT, int SD, bool NT>
 __device__ __forceinline__ void
@@ -597,7 +607,7 @@ pick_token (const Params &p, int parts, uint32_t tag, const Wait &w, uint32_t *b
 // whole: a step from its token to the logits and the next token (the grid has workgroups for
 // the vocabulary); otherwise the layers alone, from Scratch::x to Scratch::x
 template <int WT, int SD, bool NT>
-__global__ __launch_bounds__ (kDecThreads) __attribute__ ((amdgpu_waves_per_eu (2, 2))) void
+__global__ __launch_bounds__ (kDecThreads) __attribute__ ((amdgpu_waves_per_eu (4, 4))) void
 decode_layers_kernel (const Params p, int first, int count, bool whole)
 {
   extern __shared__ __align__ (16) uint8_t lds[];
@@ -654,6 +664,8 @@ decode_layers_kernel (const Params p, int first, int count, bool whole)
       return;
     }
 
+  // (what is requested behind the up/gate product, see above)
+  constexpr bool kLateDown = SD > 0, kLateEntry = SD > 1;
   const int wave = __builtin_amdgcn_readfirstlane ((int)(threadIdx.x >> 6));
   const int g = (int)blockIdx.x * kDecWaves + wave; // number of the wave: dim of them
   const int first_row = (int)blockIdx.x * kDecWaves;
@@ -706,9 +718,10 @@ decode_layers_kernel (const Params p, int first, int count, bool whole)
           st_coherent_u32 (rows + tr.kqv + (lane >> 3) * tr.copy_d + first_row + (lane & 7), ok[lane]);
       }
 
-      // ---- while the heads are computed: all weights up to the next layer's K/Q/V -------------
+      // ---- while the heads are computed: the weights up to the next layer's K/Q/V -------------
       // (a poll returns behind the weights requested before it, and any of the later
-      // hand-overs is shorter than their way from memory)
+      // hand-overs is shorter than their way from memory; kLateDown and kLateEntry: what the
+      // registers do not hold beside up/gate)
       Rest<WT, SD, NT> r;
       r.o.request (Matrix<WT> (wo, dim, dim), g, lane);
 #pragma unroll
@@ -719,8 +732,10 @@ decode_layers_kernel (const Params p, int first, int count, bool whole)
           r.ug[j].request (Matrix<WT> (w_up, ffn, dim), u, Matrix<WT> (w_gate, ffn, dim), u, lane);
         }
       load_norm_weights (ffn_norm, dim, r.g);
-      r.down.request (Matrix<WT> (w_down, dim, ffn), g, lane);
-      in = request_entry (wk, wq, wv, attn_norm);
+      if (!kLateDown)
+        r.down.request (Matrix<WT> (w_down, dim, ffn), g, lane);
+      if (!kLateEntry)
+        in = request_entry (wk, wq, wv, attn_norm);
 
       // ---- Wo + residual ------------------------------------------------------------
       row_in<1> (rows + tr.att + copy * tr.copy_d, dim, tag, w, ST_ATT, xb);
@@ -748,6 +763,10 @@ decode_layers_kernel (const Params p, int first, int count, bool whole)
         if (lane < pairs)
           ot[lo + lane - first_pair] = tag | f2h (silu (a) * u);
         publish (rows + tr.t, tr.copy_f, first_pair, ot, end_pair - first_pair, wave, lane, dead);
+        if (kLateDown)
+          r.down.request (Matrix<WT> (w_down, dim, ffn), g, lane);
+        if (kLateEntry)
+          in = request_entry (wk, wq, wv, attn_norm);
       }
 
       // ---- down + residual --------------------------------------------------------------
@@ -823,10 +842,11 @@ launch_any (const Params &p, int first, int count, int groups, hipStream_t s)
 } // namespace
 
 // Where dim waves have at most three up/gate pairs each, a layer's weights fit the registers
-// and all workgroups have a compute unit of their own.  Us per token, a launch per layer / this
-// form with an lm_head launch / the whole step in one launch (greedy, 64 or 48 tokens): 256
-// wide Q8_0, 6 layers 137 / 93 / 77; 512 wide, 8 layers 182 / 120 / 102, fp16 171 / 107 / 95; 4
-// layers: 1024 wide 112 / 83 / 76, fp16 110 / 79 / -; 1536 wide 123 / 93 / -.  2048 wide (all
+// and all workgroups have a compute unit of their own, of which they take half.  Us per token
+// of a greedy loop, 32000 ids, a launch per layer / this form with an lm_head launch / the whole
+// step in one launch: 256 wide Q8_0, 6 layers 131 / 74 / 65; 512 wide, 8 layers 173 / 100 / 88,
+// fp16 167 / 94 / 88; 768 wide, 6 layers 141 / 86 / 80, fp16 134 / 82 / -; 4 layers: 1024 wide
+// 102 / 67 / -, fp16 102 / 68 / -; 1536 wide 116 / 82 / -; 1792 wide 122 / 88 / -.  2048 wide (all
 // 256 compute units for the rows, the heads beside them, weights a phase ahead) it was slower:
 // 144 / 158, fp16 160 / 212; there a layer is bound by its weights, and polls behind them come
 // late.
@@ -836,7 +856,7 @@ layers_launch_supported (const vkl_decode_model &m, int n_cu)
   return m.flags != nullptr && m.layers != nullptr && m.dim <= (m.wtype == 8 ? kTaggedMaxDim : kTaggedMaxDim / 2)
          && (m.dim % 64) == 0 && m.dim / kDecWaves + m.n_heads <= n_cu && m.ffn <= kPairs * m.dim
          && (m.ffn % 32) == 0 && m.ffn >= m.dim / kDecWaves
-         && lds_map (m.dim, m.ffn, m.maxlen, m.head_dim).bytes <= 160 * 1024;
+         && 2 * lds_map (m.dim, m.ffn, m.maxlen, m.head_dim).bytes <= 160 * 1024;
 }
 
 int

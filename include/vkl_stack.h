@@ -151,11 +151,15 @@ int vkl_attn_prefill_chunked_bf16 (const void *q, const void *k, const void *v,
                                    size_t qhs, size_t khs, size_t vhs,
                                    float scale, int chunk, int sink, void *out,
                                    size_t ors, void *stream);
-/* Into how many parts the attention of many query rows divides the keys of a query
- * tile (heads of 64 or 128 values; others and wrong arguments: 1); more than one
- * go through the stream's scratch and a second launch.  Host arithmetic only: what
- * a test can pin. */
+/* Into how many parts at most the attention of many query rows divides the keys of a
+ * query tile (heads of 64 or 128 values; others and wrong arguments: 1); more than
+ * one go through the stream's scratch and a second launch, and without that scratch
+ * there is one.  Host arithmetic only: what a test can pin. */
 int vkl_attn_prefill_parts (int H, int S, int L, int hd, int chunk);
+/* the same of the query tile (128 rows) that `row` lies in: tiles behind more keys may
+ * get more parts than others */
+int vkl_attn_prefill_tile_parts (int H, int S, int L, int hd, int chunk,
+                                 int row);
 
 /* ---- linear recurrences ---------------------------------------------------- */
 /* Causal convolution over time per channel, then SiLU: out[s, c] = silu (sum_j

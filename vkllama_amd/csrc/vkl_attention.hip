@@ -522,6 +522,14 @@ template <int KIND, int PER, int N, int AHEAD> struct Alternate
   }
 };
 
+// tiles of keys that the query tile from row q0 on sees
+__host__ __device__ __forceinline__ int
+key_tiles (const AttnArgs &a, int q0)
+{
+  const int shift = a.L - a.S, end = q0 + kBQ + shift;
+  return ((end < a.L ? end : a.L) + kBKey - 1) / kBKey - (a.chunk ? (q0 + shift) / a.chunk * a.chunk : 0) / kBKey;
+}
+
 // parts of a query tile that sees n tiles of keys
 __host__ __device__ __forceinline__ int
 parts_of (const AttnArgs &a, int n)
@@ -822,9 +830,7 @@ attn_parts_kernel (const AttnArgs a)
   const int row = i / a.H, head = i - row * a.H;
   if (row >= a.S)
     return;
-  const int q0 = row / kBQ * kBQ, shift = a.L - a.S;
-  const int parts = parts_of (a, (min (a.L, q0 + kBQ + shift) + kBKey - 1) / kBKey
-                                     - (a.chunk ? (q0 + shift) / a.chunk * a.chunk : 0) / kBKey);
+  const int parts = parts_of (a, key_tiles (a, row / kBQ * kBQ));
   // lane p looks at part p
   float pm = -3.0e38f, ps = 0.f;
   if (lane < parts)
@@ -912,35 +918,39 @@ key_parts (const AttnArgs &a, int hd)
 int
 key_span (const AttnArgs &a)
 {
-  const int groups = a.ntq * a.H, shift = a.L - a.S;
+  const int groups = a.ntq * a.H;
   if (a.parts != 2 || groups > 200)
     return 0;
-  auto tiles = [&] (int q0) {
-    return (std::min (a.L, q0 + kBQ + shift) + kBKey - 1) / kBKey
-           - (a.chunk ? (q0 + shift) / a.chunk * a.chunk : 0) / kBKey;
-  };
   int most = 0;
   for (int q0 = 0; q0 < a.S; q0 += kBQ)
-    most = std::max (most, tiles (q0));
+    most = std::max (most, key_tiles (a, q0));
   for (int span = (most + 2) / 3; 2 * span < most; ++span)
     {
       int places = 0;
       for (int q0 = 0; q0 < a.S; q0 += kBQ)
-        places += (tiles (q0) + span - 1) / span * a.H;
+        places += (key_tiles (a, q0) + span - 1) / span * a.H;
       if (places <= 500)
         return span;
     }
   return 0;
 }
 
+// parts of the keys (at most, with a span) and the span
+void
+plan_parts (AttnArgs &a, int hd)
+{
+  a.parts = key_parts (a, hd);
+  const size_t part = (size_t)a.H * a.S * (hd + 4) * sizeof (float);
+  if ((a.span = hd == 128 && 3 * part <= vkl::StreamScratch::bytes () ? key_span (a) : 0))
+    a.parts = 3;
+}
+
 template <int HD, class E, bool CHUNKED>
 int
 launch_tiles (AttnArgs a, hipStream_t s)
 {
-  a.parts = key_parts (a, HD);
+  plan_parts (a, HD);
   const size_t part = (size_t)a.H * a.S * (HD + 4) * sizeof (float);
-  if ((a.span = HD == 128 && 3 * part <= vkl::StreamScratch::bytes () ? key_span (a) : 0))
-    a.parts = 3;
   vkl::StreamScratch own;
   if (a.parts > 1)
     {
@@ -1137,7 +1147,19 @@ vkl_attn_prefill_parts (int H, int S, int L, int hd, int chunk)
     return 1;
   AttnArgs a = {};
   a.H = H, a.S = S, a.L = L, a.ntq = (S + kBQ - 1) / kBQ, a.chunk = chunk;
-  return key_parts (a, hd);
+  plan_parts (a, hd);
+  return a.parts;
+}
+
+extern "C" int
+vkl_attn_prefill_tile_parts (int H, int S, int L, int hd, int chunk, int row)
+{
+  if (H <= 0 || S <= 0 || L < S || chunk < 0 || (hd != 64 && hd != 128) || row < 0 || row >= S)
+    return 1;
+  AttnArgs a = {};
+  a.H = H, a.S = S, a.L = L, a.ntq = (S + kBQ - 1) / kBQ, a.chunk = chunk;
+  plan_parts (a, hd);
+  return parts_of (a, key_tiles (a, row / kBQ * kBQ));
 }
 
 extern "C" int

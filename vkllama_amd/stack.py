@@ -46,6 +46,7 @@ SIGNATURES = {
     "vkl_attn_kv_rows_scratch_bytes": (sz, [i32, i32, i32, i32, i32]),
     "vkl_attn_prefill_chunked_bf16": (i32, [vp, vp, vp, i32, i32, i32, i32, i32, sz, sz, sz, f32, i32, i32, vp, sz, vp]),
     "vkl_attn_prefill_parts": (i32, [i32, i32, i32, i32, i32]),
+    "vkl_attn_prefill_tile_parts": (i32, [i32, i32, i32, i32, i32, i32]),
     "vkl_short_conv_silu": (i32, [vp, i32, sz, vp, i32, i32, vp, u32, i32, vp, sz, vp]),
     "vkl_recurrence": (i32, [C.POINTER(RecurrenceArgs), i32, u32, i32, vp, sz, vp]),
     "vkl_recurrence_scratch_bytes": (sz, [C.POINTER(RecurrenceArgs), i32]),

@@ -16,7 +16,7 @@ def parts(H, S, L, chunk=0, hd=128):
 
 # 12, 8 and 6 query tiles, two and three parts; 24 x 7: a last tile of one row
 PLAIN = [(16, 1500, 1800), (16, 1500, 2700), (24, 1000, 2200), (24, 897, 2097), (32, 700, 3100), (32, 700, 1900), (40, 600, 3000),
-         (17, 1300, 2500)]
+         (7, 3200, 3201), (10, 2177, 2477)]
 # rows whose chunk begins behind the first key, tiles that a chunk's end divides
 CHUNKED = [(16, 4, 1500, 4400, 2500, 1), (16, 16, 1411, 5600, 2500, 0), (24, 8, 1000, 5200, 3000, 1), (8, 2, 2946, 5946, 3500, 1)]
 UNEVEN = PLAIN + [(H, S, L, c) for H, _, S, L, c, _ in CHUNKED]
@@ -34,8 +34,9 @@ def test_longer_rows_have_more_parts(shape):
     assert sum(each) * H <= 500
 
 
-# too many groups; heads of 64 values
-@pytest.mark.parametrize("H,S,L,hd", [(16, 2000, 3200, 128), (16, 1500, 2100, 64)])
+# too many groups; 192 groups of heads that are not dealt to XCDs; too many heads; heads of 64 values; 198 groups of heads that are not dealt
+@pytest.mark.parametrize("H,S,L,hd", [(16, 2000, 3200, 128), (12, 2018, 3000, 128), (6, 3969, 6369, 128), (48, 448, 3648, 128),
+                                      (96, 192, 3392, 128), (16, 1500, 2100, 64), (18, 1408, 2608, 128)])
 def test_even_parts(H, S, L, hd):
     assert set(parts(H, S, L, 0, hd)) == {2}
 

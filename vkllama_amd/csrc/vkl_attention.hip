@@ -912,14 +912,22 @@ key_parts (const AttnArgs &a, int hd)
 // (of 512, as of 528, some cases took the time of three workgroups on a compute unit) and
 // three parts.  A compute unit takes 1.1 us per tile however many workgroups it holds, and two
 // long halves on one are what a launch waits for.  16 heads of 128, 1500 rows behind 300 / 600 /
-// 1200 / 2400 keys, us: in two 42 / 46 / 55 / 72, as here 37 / 40 / 48 / 66; 24 heads, 1000
-// behind 1200 50 / 47; 32 heads, 700 behind 2400 61.8 / 61.0.  With more groups (16 heads, 2000 rows
-// behind 1200: 69 / 71) and where all get three (24 heads, 700 rows: 35.4 / 36.5) even parts stay.
+// 1200 / 2400 keys, us: in two 42 / 46 / 55 / 72, as here 37 / 40 / 48 / 66.
+// Over 700 shapes of 163 (fewer groups do not get two parts) to 255 groups, time as here / in two:
+// heads that are dealt to XCDs (multiples of 8), 171 to 200 groups: 8 heads 0.86-0.96, 16 0.85-0.94,
+// 24 0.93-0.97, 32 0.93-0.97, 40 0.93-0.99, but 48 1.05-1.09, 64 0.97-1.01, 88 and 96 1.09-1.19.
+// Other numbers of heads: workgroups go to XCDs in turn, and what third parts add does not reach
+// all alike.  With up to 440 places (55 of an XCD's 64) it was 0.74-0.93 for up to 5 heads, 0.78-1.02
+// for more in up to 183 groups; 6 and 17 heads in 186 and 187 up to 1.11, 12 heads in 444 places
+// 1.05, in 480 places and 198 groups up to 1.19 (18 heads, 1408 rows behind 1200), 192 groups (a
+// tile's parts on one XCD) 1.07-1.26.  With more than 200 groups it was 0.81 to 1.15 (240 groups of 8
+// heads 0.82-0.99, of 16 0.90-1.15): even parts.
 int
 key_span (const AttnArgs &a)
 {
   const int groups = a.ntq * a.H;
-  if (a.parts != 2 || groups > 200)
+  const bool dealt = a.H % 8 == 0;
+  if (a.parts != 2 || groups > (dealt || a.H <= 5 ? 200 : 183) || (dealt ? a.H > 40 : groups % 8 == 0))
     return 0;
   int most = 0;
   for (int q0 = 0; q0 < a.S; q0 += kBQ)
@@ -929,7 +937,7 @@ key_span (const AttnArgs &a)
       int places = 0;
       for (int q0 = 0; q0 < a.S; q0 += kBQ)
         places += (key_tiles (a, q0) + span - 1) / span * a.H;
-      if (places <= 500)
+      if (places <= (dealt ? 500 : 440))
         return span;
     }
   return 0;

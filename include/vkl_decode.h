@@ -90,7 +90,7 @@ void vkl_decode_flags_release (void *flags);
  * No counterpart in the reference. */
 int vkl_decode_default_mode (const vkl_decode_model *m);
 
-/* bytes of device scratch a model of these dimensions needs */
+/* bytes of device scratch a model of these dimensions and matrix type needs */
 size_t vkl_decode_scratch_bytes (const vkl_decode_model *m);
 
 /* One token at KV position `pos` (context length becomes pos + 1).

@@ -1000,8 +1000,7 @@ vkl_decode_scratch_bytes (const vkl_decode_model *m)
 {
   if (!m)
     return 0;
-  return carve (nullptr, m->dim, m->ffn, m->vocab, m->n_heads, m->maxlen, m->head_dim,
-                m->n_layers).bytes;
+  return carve (*m).bytes;
 }
 
 extern "C" const void *
@@ -1009,8 +1008,7 @@ vkl_decode_logits_f16 (const vkl_decode_model *m)
 {
   if (!m || !m->scratch)
     return nullptr;
-  return carve (m->scratch, m->dim, m->ffn, m->vocab, m->n_heads, m->maxlen, m->head_dim,
-                m->n_layers).logits16;
+  return carve (*m).logits16;
 }
 
 #ifdef VKL_TRACE
@@ -1181,8 +1179,7 @@ vkl_decode_step (const vkl_decode_model *m, const uint32_t *tok, uint32_t pos,
       = lds_bytes_needed (m->dim, m->ffn, m->maxlen, m->head_dim);
   Params p = {};
   p.m = *m;
-  p.s = carve (m->scratch, m->dim, m->ffn, m->vocab, m->n_heads, m->maxlen, m->head_dim,
-                m->n_layers);
+  p.s = carve (*m);
   p.tok = tok;
   p.pos = pos;
   p.logits32 = logits32 ? logits32 : p.s.logits32;
@@ -1266,15 +1263,14 @@ vkl_decode_status_word (const vkl_decode_model *m)
 {
   if (!m || !m->scratch)
     return nullptr;
-  return carve (m->scratch, m->dim, m->ffn, m->vocab, m->n_heads, m->maxlen, m->head_dim, m->n_layers).sync + 1;
+  return carve (*m).sync + 1;
 }
 
 extern "C" int
 vkl_decode_status (const vkl_decode_model *m, void *stream)
 {
   VKL_CHECK_ARG (m != nullptr && m->scratch != nullptr);
-  const Scratch sc = carve (m->scratch, m->dim, m->ffn, m->vocab, m->n_heads, m->maxlen,
-                            m->head_dim, m->n_layers);
+  const Scratch sc = carve (*m);
   hipStream_t s = (hipStream_t)stream;
   uint32_t gave_up = 0;
   VKL_HIP (hipMemcpyAsync (&gave_up, sc.sync + 1, sizeof (gave_up), hipMemcpyDeviceToHost, s));
@@ -1380,8 +1376,7 @@ decode_loop (const vkl_decode_model *m, uint32_t *ids, uint32_t pos0, int n_step
   hipStream_t s = (hipStream_t)stream;
   Params p = {};
   p.m = *m;
-  p.s = carve (m->scratch, m->dim, m->ffn, m->vocab, m->n_heads, m->maxlen, m->head_dim,
-                m->n_layers);
+  p.s = carve (*m);
   p.tok = nullptr;
   p.logits32 = logits32 ? logits32 : p.s.logits32;
   p.next_tok = nullptr;
@@ -1530,8 +1525,7 @@ vkl_decode_phase_replay (const vkl_decode_model *m, int kind, uint32_t pos,
   const size_t lds = lds_bytes_needed (m->dim, m->ffn, m->maxlen, m->head_dim);
   Params p = {};
   p.m = *m;
-  p.s = carve (m->scratch, m->dim, m->ffn, m->vocab, m->n_heads, m->maxlen, m->head_dim,
-                m->n_layers);
+  p.s = carve (*m);
   p.tok = (const uint32_t *)p.s.amax_idx; // any device word: ids >= vocab read row 0
   p.pos = pos;
   p.logits32 = p.s.logits32;

@@ -53,7 +53,7 @@ constexpr int kLsTags = 2048; // word of the layer-sync area: layers done so far
 static_assert ((kLsTags + 32) * 4 <= kLayerSyncBytes, "layer-sync area too small");
 constexpr int kSyncErr = 1;   // word of Scratch::sync: a wait gave up
 constexpr int kTagSpinLimit = 1 << 14;
-constexpr int kPairs = 3;     // up/gate pairs of a wave, at most
+constexpr int kPairs = kTaggedPairs;
 enum Stage { ST_KQV = 0, ST_ATT, ST_WO, ST_UP, ST_DOWN, ST_HEAD };
 
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
@@ -853,9 +853,7 @@ launch_any (const Params &p, int first, int count, int groups, hipStream_t s)
 bool
 layers_launch_supported (const vkl_decode_model &m, int n_cu)
 {
-  return m.flags != nullptr && m.layers != nullptr && m.dim <= (m.wtype == 8 ? kTaggedMaxDim : kTaggedMaxDim / 2)
-         && (m.dim % 64) == 0 && m.dim / kDecWaves + m.n_heads <= n_cu && m.ffn <= kPairs * m.dim
-         && (m.ffn % 32) == 0 && m.ffn >= m.dim / kDecWaves
+  return m.flags != nullptr && m.layers != nullptr && tagged_shape (m) && m.dim / kDecWaves + m.n_heads <= n_cu
          && 2 * lds_map (m.dim, m.ffn, m.maxlen, m.head_dim).bytes <= 160 * 1024;
 }
 

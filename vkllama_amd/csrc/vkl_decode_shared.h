@@ -39,7 +39,9 @@ struct Scratch
 // reader knows by the tag that a word has arrived.  k | q | v are read by one workgroup per
 // head; the others by all, from one copy per XCD.
 constexpr int kTagCopies = 8;
-constexpr int kTaggedMaxDim = 2048; // rows of up to so many (and three times as many) values
+constexpr int kTaggedUnits = 256;     // compute units: one for eight of the row's values and one per head
+constexpr int kTaggedPairs = 3;       // up/gate pairs of a wave, at most
+constexpr int kTaggedMaxDim16 = 1024; // widest fp16 row (two steps of loads)
 struct TaggedRows
 {
   // words from Scratch::tagged: rows, and from copy to copy
@@ -74,12 +76,21 @@ align256 (size_t v)
   return (v + 255) & ~(size_t)255;
 }
 
-__host__ __device__ inline Scratch
-carve (void *base, int dim, int ffn, int vocab, int heads, int maxlen, int hd,
-       int n_layers)
+// Shapes whose layers can share one launch (layers_launch_supported asks for more): the only ones
+// that have tagged rows.
+inline bool
+tagged_shape (const vkl_decode_model &m)
+{
+  return (m.wtype != 1 || m.dim <= kTaggedMaxDim16) && (m.dim % 64) == 0 && m.dim / kDecWaves + m.n_heads <= kTaggedUnits
+         && m.ffn <= kTaggedPairs * m.dim && (m.ffn % 32) == 0 && m.ffn >= m.dim / kDecWaves;
+}
+
+inline Scratch
+carve (const vkl_decode_model &m)
 {
   Scratch s;
-  uint8_t *p = (uint8_t *)base;
+  const int dim = m.dim, ffn = m.ffn, vocab = m.vocab, heads = m.n_heads, hd = m.head_dim;
+  uint8_t *p = (uint8_t *)m.scratch;
   size_t o = 0;
   s.x = (uint16_t *)(p + o), o += align256 ((size_t)dim * 2);
   s.kqv = (uint16_t *)(p + o), o += align256 ((size_t)dim * 6);
@@ -97,7 +108,7 @@ carve (void *base, int dim, int ffn, int vocab, int heads, int maxlen, int hd,
   s.part_sum = (float *)(p + o), o += align256 ((size_t)heads * kAttnChunks * 4);
   s.part_out = (float *)(p + o), o += align256 ((size_t)heads * kAttnChunks * hd * 4);
   s.attn_cnt = (uint32_t *)(p + o), o += align256 ((size_t)heads * 4);
-  const bool tagged = dim <= kTaggedMaxDim && ffn <= 3 * dim;
+  const bool tagged = tagged_shape (m);
   s.tagged = tagged ? (uint32_t *)(p + o) : nullptr;
   o += tagged ? align256 ((size_t)tagged_rows (dim, ffn).words * 4) : 0;
   s.bytes = o;

@@ -408,6 +408,7 @@ def main():
     m.set_option("decode_graph", args.decode_graph)
     phases = m.phase_times()
     L_mid = int(ctx[len(ctx) // 2])
+    form = m.decode_form(L_mid - 1)
     per_phase = {}
     for name, (ms, n) in phases.items():
         if n:
@@ -435,22 +436,22 @@ def main():
         # the kernel's name as a profiler prints it: phase number, weight type,
         # 4096-value chunks of the staged activation row
         phase_no = {"kqv": 0, "attention": 1, "attention+wo": 1, "wo": 2, "upgate": 3, "down": 4, "lm_head": 5,
-                    "layer": 8}[dom]
+                    "step": 6, "layers": 7, "layer": 8}[dom]
         kstage = cfg["ffn"] if dom == "down" else cfg["dim"]
         per = 34.0 / 32.0 if cfg["wtype"] == 8 else 2.0
         wbytes = (cfg["n_layers"] * (4.0 * cfg["dim"] ** 2 + 3.0 * cfg["dim"] * cfg["ffn"])
                   + cfg["vocab"] * cfg["dim"]) * per
-        # rows that a step hands over inside one launch: see layers_launch_supported
-        narrow = (cfg["dim"] // 8 + cfg["n_heads"] <= 256 and cfg["dim"] <= (2048 if cfg["wtype"] == 8 else 1024)
-                  and cfg["ffn"] <= 3 * cfg["dim"])
-        if dom == "layer":
+        if dom in ("step", "layers"):
+            row = cfg["dim"] * (1 if cfg["wtype"] == 8 else 2)
+            dom_kernel = "decode_layers_kernel<%d, %d, %s> (%s in one launch)" % (
+                8 if cfg["wtype"] == 8 else 1, 0 if row <= 512 else (row + 1023) // 1024,
+                "true" if wbytes > (288 << 20) else "false", "a whole step" if dom == "step" else "all layers")
+        elif dom == "layer":
             # (row chunks of 4096 values as the library picks them: see launch_layer_wt)
             xd, xf = (cfg["dim"] + 4095) // 4096, (cfg["ffn"] + 4095) // 4096
             xd, xf = (1, 1) if (xd, xf) == (1, 1) else ((1, 3) if xd == 1 and xf <= 3 else (2, 4))
             dom_kernel = "decode_layer_kernel<%d, %d, %d, %s> (the five phases of a layer in one launch)" % (
                 8 if cfg["wtype"] == 8 else 1, xd, xf, "true" if wbytes > (288 << 20) else "false")
-            if narrow:
-                dom_kernel = "decode_layers_kernel (one layer of the step's only launch, by itself)"
         elif dom == "attention+wo":
             dom_kernel = "decode_attn_wo_kernel<%d, %d> (attention + Wo)" % (8 if cfg["wtype"] == 8 else 1,
                                                                             min(4, (cfg["dim"] + 4095) // 4096))
@@ -494,9 +495,10 @@ def main():
         "data": "synthetic: random-init N(0,0.02) weights" + (" quantised to Q8_0" if cfg["wtype"] == 8 else " in FP16")
                 + ", random prompt ids",
         "config": {"workload": args.workload, "prompt_tokens": n_prompt, "decode_tokens": steps,
-                   "decode_mode": "one launch per step or all layers" if narrow and "layer" in per_phase else
-                                  ("one launch per layer" if "layer" in per_phase else "one launch per phase")
-                                  + (", replayed from a HIP graph" if args.decode_graph else ""),
+                   "decode_mode": {"phases": "one launch per phase", "layer": "one launch per layer",
+                                   "layers": "one launch for all layers", "step": "one launch per step"}[form]
+                                  + (", replayed from a HIP graph" if args.decode_graph and form in ("phases", "layer")
+                                     else ""),
                    "dims": {k: cfg[k] for k in ("dim", "n_layers", "n_heads", "ffn", "vocab", "maxlen")}},
         "decode_tokens_per_second_host_interface": round(host_tok_s, 1),
         "prefill_tokens_per_second": round(n_prompt / (prefill_ms * 1e-3), 1),

@@ -89,6 +89,15 @@ void vkl_decode_flags_release (void *flags);
  * Either value may be passed for any model that the form supports.
  * No counterpart in the reference. */
 int vkl_decode_default_mode (const vkl_decode_model *m);
+/* How vkl_decode_step runs at position `pos` in that mode on the current device: a launch per
+ * phase, a launch per layer, one launch for all layers (embedding row and lm_head have their
+ * own), or the whole step, from the token to the logits and the next token, in one launch.
+ * (A model that vkl_decode_step refuses: VKL_DECODE_FORM_PHASES.) */
+#define VKL_DECODE_FORM_PHASES 0
+#define VKL_DECODE_FORM_LAYER 1
+#define VKL_DECODE_FORM_LAYERS 2
+#define VKL_DECODE_FORM_STEP 3
+int vkl_decode_form (const vkl_decode_model *m, uint32_t pos, int mode);
 
 /* bytes of device scratch a model of these dimensions and matrix type needs */
 size_t vkl_decode_scratch_bytes (const vkl_decode_model *m);
@@ -96,8 +105,9 @@ size_t vkl_decode_scratch_bytes (const vkl_decode_model *m);
 /* One token at KV position `pos` (context length becomes pos + 1).
  *  tok      device-visible uint32: the input token id (ids >= vocab -> 0)
  *  mode     0 = one launch per phase (attention and Wo share one below the
- *           split length); 1 = one launch per layer, or for all layers where
- *           rows are narrow (up to about 1792 values): all workgroups stay
+ *           split length); 1 = one launch per layer, for all layers or for the
+ *           whole step where rows are narrow (see vkl_decode_form; Q8_0 rows of
+ *           up to 1920 values, fp16 of up to 1024): all workgroups stay
  *           resident through the five phases, hand activations over through
  *           memory with bounded waits for one another, and have the next
  *           phase's weights on the way meanwhile.  Results are bit for bit
@@ -138,9 +148,9 @@ const uint32_t *vkl_decode_status_word (const vkl_decode_model *m);
  * ids[i] (device memory) at position pos0 + i and writes its arg-max id to
  * ids[i + 1], the loop of app/llama2_infer.cpp:140-177 with the sampler on the
  * device.  The launches of one step are captured once in a HIP graph (per
- * model / buffers / attention form) and replayed (a step of one launch is
- * launched as it is); results are identical to n_steps calls of
- * vkl_decode_step in the same mode.  logits32 (optional)
+ * model / buffers / attention form) and replayed (steps of
+ * VKL_DECODE_FORM_LAYERS and _STEP are launched as they are); results are
+ * identical to n_steps calls of vkl_decode_step in the same mode.  logits32 (optional)
  * receives the logits of the last step.  The stream must not be capturing. */
 int vkl_decode_loop (const vkl_decode_model *m, uint32_t *ids, uint32_t pos0,
                      int n_steps, int mode, float *logits32, void *stream);
@@ -173,23 +183,25 @@ int vkl_argmax_f32 (const float *x, int n, uint32_t *out, void *stream);
  * phase launch with a pair of HIP events on the launch stream and
  * synchronises the stream before it returns.  vkl_decode_phase_times adds up,
  * per phase kind (0 K/Q/V, 1 attention, 2 Wo, 3 up/gate, 4 down, 5 lm_head
- * with the arg-max its last workgroup forms, 8 a whole layer in one launch as
- * mode 1 runs it; 6 and 7 are not used), the elapsed milliseconds and the
+ * with the arg-max its last workgroup forms; as mode 1 runs them, 6 a whole
+ * step, 7 all layers, 8 a layer in one launch), the elapsed milliseconds and the
  * number of launches since the last call, and clears both.  The timer is one
  * per process: use it from one host thread, with no other decode call in
  * flight. */
 #define VKL_DECODE_PHASES 9
+#define VKL_DECODE_PHASE_STEP 6
+#define VKL_DECODE_PHASE_LAYERS 7
 #define VKL_DECODE_PHASE_LAYER 8
 int vkl_decode_phase_timing (int enable);
 int vkl_decode_phase_times (double ms_sum[VKL_DECODE_PHASES],
                             uint64_t launches[VKL_DECODE_PHASES]);
-/* Launches phase `kind` (0..4 and 8: of every layer in turn; 5: lm_head) `rounds`
- * times back to back on `stream` between ONE pair of events and returns the
+/* Launches phase `kind` (0..4 and 8: of every layer in turn; 5: lm_head; 6 and 7 where
+ * steps at `pos` take that form in mode 1) `rounds` times back to back on `stream` between ONE pair of events and returns the
  * average milliseconds per launch: the kernel's duration without the cost of
  * an event pair per launch.  The phase's outputs in scratch are overwritten
  * (a following vkl_decode_step recomputes them); the KV cache is not touched
- * for kinds other than 1, and kind 1 rewrites the rows of position `pos` with
- * what scratch currently holds, so call it before, not between, real steps of
+ * for kinds other than 1 and 6 to 8, which rewrite the rows of position `pos`
+ * with what scratch currently holds, so call it before, not between, real steps of
  * a sequence you still need. */
 int vkl_decode_phase_replay (const vkl_decode_model *m, int kind, uint32_t pos,
                              int rounds, void *stream, double *avg_ms,

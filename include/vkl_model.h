@@ -127,6 +127,9 @@ int vkl_model_write_kv_cache (vkl_model *m, size_t layer, int value,
                               const uint16_t *rows_h, size_t n);
 /* algorithmic bytes of one decode step at context length L */
 size_t vkl_model_decode_step_bytes (const vkl_model *m, size_t L);
+/* VKL_DECODE_FORM_* of a decode step at position pos (vkl_decode_form); 0 without the
+ * fused step */
+int vkl_model_decode_form (const vkl_model *m, size_t pos);
 /* per-phase measurements of the fused decode step: option "phase_timing"
  * switches them on; see vkl_decode_phase_times / vkl_decode_phase_bytes */
 int vkl_model_phase_times (vkl_model *m, double ms_sum[9], uint64_t launches[9]);

@@ -82,7 +82,7 @@ enum Phase
   PH_UPGATE,
   PH_DOWN,
   PH_HEAD,
-  PH_ARGMAX,
+  PH_ARGMAX, // (the numbers of this and the next are VKL_DECODE_PHASE_STEP and _LAYERS to the timer)
   PH_GEMV, // a stand-alone y = W x (+ residual) on the down projection's path
   PH_LAYER, // a whole layer in one launch (vkl_decode_layer.hip)
   PH_UPROW, // up/gate with SiLU of one row that is multiplied as it is
@@ -1022,38 +1022,57 @@ vkl_debug_set_trace (void *buf)
 
 namespace
 {
-// the launches of one token: one per phase (mode 0) or one per layer (mode 1)
+// VKL_DECODE_FORM_*: how a step at position `pos` runs
+int
+step_form (const vkl_decode_model &m, int pos, int mode, int n_cu)
+{
+  // (one head per workgroup inside the launches of a layer and more: contexts long enough for
+  // the split attention take the launches per phase)
+  if (mode != 1 || !layer_launch_supported (m, 2 * n_cu) || pos + 1 >= attn_split_min (m))
+    return VKL_DECODE_FORM_PHASES;
+  return whole_step_supported (m, n_cu)      ? VKL_DECODE_FORM_STEP
+         : layers_launch_supported (m, n_cu) ? VKL_DECODE_FORM_LAYERS
+                                             : VKL_DECODE_FORM_LAYER;
+}
+
+// the launches of one token
 int
 launch_step (const Params &p, const vkl_decode_model *m, int mode, int n_cu, int G,
              size_t lds, hipStream_t s)
 {
-  // (one head per workgroup inside the layer launch: contexts long enough for
-  // the split attention take the launches per phase)
-  const bool per_layer = mode == 1 && layer_launch_supported (*m, G)
-                         && (int)p.pos + 1 < attn_split_min (*m);
-  if (per_layer && !g_timer.on && whole_step_supported (*m, n_cu))
+  const int form = step_form (*m, (int)p.pos, mode, n_cu);
+  if (form == VKL_DECODE_FORM_STEP)
     {
+      if (int e = timer_mark (VKL_DECODE_PHASE_STEP, false, s))
+        return e;
       if (int e = launch_step_whole (p, n_cu, s))
+        return e;
+      if (int e = timer_mark (VKL_DECODE_PHASE_STEP, true, s))
         return e;
       return p.loop && p.sample ? sample_loop_launch (p.logits32, m->vocab, p.sample, (uint32_t *)p.loop, p.ids, s) : 0;
     }
-  // (in a replayed greedy loop the previous step's lm_head launch has left the
-  // row; the loop launches this once in front of its first step)
-  if (per_layer && !(p.loop && !p.sample))
+  // (in a greedy loop the previous step's lm_head launch has left the row; the
+  // loop launches this once in front of its first step)
+  if (form != VKL_DECODE_FORM_PHASES && !(p.loop && !p.sample))
     if (int e = launch_embed_row (p, s))
       return e;
-  const bool many = per_layer && layers_launch_supported (*m, n_cu);
-  if (many && !g_timer.on)
-    if (int e = launch_layers (p, 0, m->n_layers, s))
-      return e;
-  for (int l = 0; l < m->n_layers && !(many && !g_timer.on); ++l)
+  if (form == VKL_DECODE_FORM_LAYERS)
+    {
+      if (int e = timer_mark (VKL_DECODE_PHASE_LAYERS, false, s))
+        return e;
+      if (int e = launch_layers (p, s))
+        return e;
+      if (int e = timer_mark (VKL_DECODE_PHASE_LAYERS, true, s))
+        return e;
+    }
+  for (int l = 0; l < m->n_layers && form != VKL_DECODE_FORM_LAYERS; ++l)
     {
       const vkl_layer_weights &lw = m->layers_h[l];
-      if (per_layer)
+      if (form == VKL_DECODE_FORM_LAYER)
         {
           if (int e = timer_mark (PH_LAYER, false, s))
             return e;
-          if (int e = many ? launch_layers (p, l, 1, s) : launch_layer (p, lw, l, G, s))
+          if (int e = launch_layer (p, lw, l, G, s))
             return e;
           if (int e = timer_mark (PH_LAYER, true, s))
             return e;
@@ -1243,6 +1262,16 @@ vkl_decode_default_mode (const vkl_decode_model *m)
   return m && m->flags && m->dim <= 4096 && m->ffn <= 12288 ? 1 : 0;
 }
 
+extern "C" int
+vkl_decode_form (const vkl_decode_model *m, uint32_t pos, int mode)
+{
+  int dev = 0, n_cu = 0;
+  if (!m || check_model (m) != 0 || pos >= (uint32_t)m->maxlen || hipGetDevice (&dev) != hipSuccess
+      || hipDeviceGetAttribute (&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return VKL_DECODE_FORM_PHASES;
+  return step_form (*m, (int)pos, mode, n_cu);
+}
+
 extern "C" void
 vkl_decode_flags_release (void *flags)
 {
@@ -1413,9 +1442,9 @@ decode_loop (const vkl_decode_model *m, uint32_t *ids, uint32_t pos0, int n_step
       // A step of one or a few launches needs no graph: with graphs of one node the GPU had 17 us
       // without work between tokens (512 wide, 8 layers: 108 us per token, 103 launched), and
       // the capture goes as well.
-      if (!long_ctx && mode == 1 && layer_launch_supported (*m, G) && layers_launch_supported (*m, n_cu))
+      p.pos = (uint32_t)std::min (attn_split_min (*m) - 2, m->maxlen - 1);
+      if (!long_ctx && step_form (*m, (int)p.pos, mode, n_cu) >= VKL_DECODE_FORM_LAYERS)
         {
-          p.pos = (uint32_t)std::min (attn_split_min (*m) - 2, m->maxlen - 1);
           for (; done < upto && !err; ++done)
             err = launch_step (p, m, mode, n_cu, G, lds, s);
           continue;
@@ -1516,7 +1545,7 @@ vkl_decode_phase_replay (const vkl_decode_model *m, int kind, uint32_t pos,
 {
   if (int e = check_model (m))
     return e;
-  VKL_CHECK_ARG (((kind >= PH_KQV && kind <= PH_HEAD) || kind == PH_LAYER) && rounds > 0 && avg_ms);
+  VKL_CHECK_ARG (kind >= PH_KQV && kind < VKL_DECODE_PHASES && rounds > 0 && avg_ms);
   VKL_CHECK_ARG (pos < (uint32_t)m->maxlen);
   int dev = 0, n_cu = 0;
   VKL_HIP (hipGetDevice (&dev));
@@ -1535,8 +1564,12 @@ vkl_decode_phase_replay (const vkl_decode_model *m, int kind, uint32_t pos,
   p.stream_once = step_weight_bytes (*m) > kCacheResidentBytes;
   hipStream_t s = (hipStream_t)stream;
   const int G = n_cu * 2;
-  VKL_CHECK_ARG (kind != PH_LAYER
-                 || (layer_launch_supported (*m, G) && (int)pos + 1 < attn_split_min (*m)));
+  const int form = step_form (*m, (int)pos, 1, n_cu);
+  VKL_CHECK_ARG (kind != PH_LAYER || form != VKL_DECODE_FORM_PHASES);
+  // (all layers or the whole step in one launch: in the form that steps take, whose every launch
+  // writes all the tagged rows that the next one reads)
+  VKL_CHECK_ARG (kind != VKL_DECODE_PHASE_LAYERS || form == VKL_DECODE_FORM_LAYERS);
+  VKL_CHECK_ARG (kind != VKL_DECODE_PHASE_STEP || form == VKL_DECODE_FORM_STEP);
   const bool was_on = g_timer.on;
   g_timer.on = false;
   hipEvent_t e0, e1;
@@ -1551,6 +1584,11 @@ vkl_decode_phase_replay (const vkl_decode_model *m, int kind, uint32_t pos,
         {
           const vkl_layer_weights none = {};
           err = launch_phase<PH_HEAD> (p, none, 0, G, G, lds, s), ++n;
+          continue;
+        }
+      if (kind == VKL_DECODE_PHASE_LAYERS || kind == VKL_DECODE_PHASE_STEP)
+        {
+          err = kind == VKL_DECODE_PHASE_STEP ? launch_step_whole (p, n_cu, s) : launch_layers (p, s), ++n;
           continue;
         }
       for (int l = 0; l < m->n_layers && !err; ++l, ++n)
@@ -1574,7 +1612,7 @@ vkl_decode_phase_replay (const vkl_decode_model *m, int kind, uint32_t pos,
               err = launch_phase<PH_UPGATE> (p, lw, l, G, G, lds, s);
               break;
             case PH_LAYER:
-              err = layers_launch_supported (*m, n_cu) ? launch_layers (p, l, 1, s) : launch_layer (p, lw, l, G, s);
+              err = launch_layer (p, lw, l, G, s);
               break;
             default:
               err = launch_phase<PH_DOWN> (p, lw, l, G, G, lds, s);
@@ -1629,8 +1667,10 @@ vkl_decode_phase_bytes (const vkl_decode_model *m, int kind, size_t L)
       return vkl_decode_phase_bytes (m, PH_KQV, L) + vkl_decode_phase_bytes (m, PH_ATTN, L)
              + vkl_decode_phase_bytes (m, PH_WO, L) + vkl_decode_phase_bytes (m, PH_UPGATE, L)
              + vkl_decode_phase_bytes (m, PH_DOWN, L);
-    default:
-      return (size_t)1024 * 8;
+    case VKL_DECODE_PHASE_LAYERS:
+      return (size_t)m->n_layers * vkl_decode_phase_bytes (m, PH_LAYER, L);
+    default: // VKL_DECODE_PHASE_STEP: the layers, the output matrix and the token's embedding row
+      return vkl_decode_phase_bytes (m, VKL_DECODE_PHASE_LAYERS, L) + vkl_decode_phase_bytes (m, PH_HEAD, L) + mat (1, dim);
     }
 }
 

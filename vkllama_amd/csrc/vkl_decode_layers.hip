@@ -34,8 +34,9 @@
 // wide Q8_0 97 / now 88, 1024 68 / 66, 1536 83 / 82, 768 wide fp16 87 / 82.
 //
 // The tags of a step follow on those of the step before (a counter in the sync area,
-// advanced at the end of a launch), and every word of a row is written once per layer: what
-// a row holds before is always an older tag.  A row is not overwritten while somebody still
+// advanced at the end of a launch), and every word of a row is written once per layer, of the
+// last layer's row and of the arg-maxima once per launch (a model's launches are all of one
+// form): what a row holds before is always an older tag, of 2^16.  A row is not overwritten while somebody still
 // waits for it: the next layer's needs a row that all workgroups have contributed to since.
 // Waits are bounded and a wait that gave up is reported as in the layer launch; its
 // workgroup publishes nothing from then on.  vkl_decode_status clears counter and rows with
@@ -608,7 +609,7 @@ pick_token (const Params &p, int parts, uint32_t tag, const Wait &w, uint32_t *b
 // the vocabulary); otherwise the layers alone, from Scratch::x to Scratch::x
 template <int WT, int SD, bool NT>
 __global__ __launch_bounds__ (kDecThreads) __attribute__ ((amdgpu_waves_per_eu (4, 4))) void
-decode_layers_kernel (const Params p, int first, int count, bool whole)
+decode_layers_kernel (const Params p, bool whole)
 {
   extern __shared__ __align__ (16) uint8_t lds[];
   const vkl_decode_model &m = p.m;
@@ -630,7 +631,8 @@ decode_layers_kernel (const Params p, int first, int count, bool whole)
   __syncthreads ();
   // the table of layers is not written while a step runs: scalar loads
   typedef const __attribute__ ((address_space (4))) vkl_layer_weights *Table;
-  const Table table = (Table)m.layers + first;
+  const Table table = (Table)m.layers;
+  const int count = m.n_layers;
   uint16_t *xa = (uint16_t *)(lds + map.xa), *xb = (uint16_t *)(lds + map.xb), *xc = (uint16_t *)(lds + map.xc);
   uint16_t *xr = (uint16_t *)(lds + map.xr), *xd = (uint16_t *)(lds + map.xd);
   const int G = dim / kDecWaves;
@@ -801,7 +803,7 @@ decode_layers_kernel (const Params p, int first, int count, bool whole)
 
 template <int WT, int SD, bool NT>
 int
-launch_layers_t (const Params &p, int first, int count, int groups, hipStream_t s)
+launch_layers_t (const Params &p, int groups, hipStream_t s)
 {
   const size_t lds = (size_t)lds_map (p.m.dim, p.m.ffn, p.m.maxlen, p.m.head_dim).bytes;
   static LdsLimit limit;
@@ -809,16 +811,16 @@ launch_layers_t (const Params &p, int first, int count, int groups, hipStream_t 
     return e;
   const int own = p.m.dim / kDecWaves + p.m.n_heads;
   decode_layers_kernel<WT, SD, NT>
-      <<<dim3 ((unsigned)std::max (own, groups)), dim3 (kDecThreads), lds, s>>> (p, first, count, groups > own);
+      <<<dim3 ((unsigned)std::max (own, groups)), dim3 (kDecThreads), lds, s>>> (p, groups > own);
   return 0;
 }
 
 template <int WT, int SD>
 int
-launch_layers_nt (const Params &p, int first, int count, int groups, hipStream_t s)
+launch_layers_nt (const Params &p, int groups, hipStream_t s)
 {
-  return p.stream_once ? launch_layers_t<WT, SD, true> (p, first, count, groups, s)
-                       : launch_layers_t<WT, SD, false> (p, first, count, groups, s);
+  return p.stream_once ? launch_layers_t<WT, SD, true> (p, groups, s)
+                       : launch_layers_t<WT, SD, false> (p, groups, s);
 }
 
 int
@@ -828,16 +830,16 @@ row_bytes (const vkl_decode_model &m)
 }
 
 int
-launch_any (const Params &p, int first, int count, int groups, hipStream_t s)
+launch_any (const Params &p, int groups, hipStream_t s)
 {
   const int bytes = row_bytes (p.m);
   if (p.m.wtype == 8)
-    return bytes <= 512    ? launch_layers_nt<8, 0> (p, first, count, groups, s)
-           : bytes <= 1024 ? launch_layers_nt<8, 1> (p, first, count, groups, s)
-                           : launch_layers_nt<8, 2> (p, first, count, groups, s);
-  return bytes <= 512    ? launch_layers_nt<1, 0> (p, first, count, groups, s)
-         : bytes <= 1024 ? launch_layers_nt<1, 1> (p, first, count, groups, s)
-                         : launch_layers_nt<1, 2> (p, first, count, groups, s);
+    return bytes <= 512    ? launch_layers_nt<8, 0> (p, groups, s)
+           : bytes <= 1024 ? launch_layers_nt<8, 1> (p, groups, s)
+                           : launch_layers_nt<8, 2> (p, groups, s);
+  return bytes <= 512    ? launch_layers_nt<1, 0> (p, groups, s)
+         : bytes <= 1024 ? launch_layers_nt<1, 1> (p, groups, s)
+                         : launch_layers_nt<1, 2> (p, groups, s);
 }
 } // namespace
 
@@ -858,9 +860,9 @@ layers_launch_supported (const vkl_decode_model &m, int n_cu)
 }
 
 int
-launch_layers (const Params &p, int first, int count, hipStream_t s)
+launch_layers (const Params &p, hipStream_t s)
 {
-  return launch_any (p, first, count, 0, s);
+  return launch_any (p, 0, s);
 }
 
 // The workgroups left over hold the output matrix in their registers, or at most twice that.
@@ -880,7 +882,7 @@ whole_step_supported (const vkl_decode_model &m, int n_cu)
 int
 launch_step_whole (const Params &p, int n_cu, hipStream_t s)
 {
-  return launch_any (p, 0, p.m.n_layers, n_cu, s);
+  return launch_any (p, n_cu, s);
 }
 } // namespace dec
 } // namespace vkl

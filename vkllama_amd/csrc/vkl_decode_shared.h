@@ -643,10 +643,10 @@ flags_equal_scalar (const uint32_t *flag, int nflags, uint32_t want)
 // a layer has little weight) that must all be resident at once.
 bool layer_launch_supported (const vkl_decode_model &m, int G);
 int launch_layer (const Params &p, const vkl_layer_weights &lw, int layer, int G, hipStream_t s);
-// Layers first .. first + count - 1 in one launch (vkl_decode_layers.hip): narrow rows, whose
-// layers are bound by their hand-overs.  At most one workgroup per compute unit, all resident.
+// All layers in one launch (vkl_decode_layers.hip): narrow rows, whose layers are bound by their
+// hand-overs.  At most one workgroup per compute unit, all resident.
 bool layers_launch_supported (const vkl_decode_model &m, int n_cu);
-int launch_layers (const Params &p, int first, int count, hipStream_t s);
+int launch_layers (const Params &p, hipStream_t s);
 // a whole step, from the token to the logits and the next token, where the compute units left
 // over can hold the output matrix
 bool whole_step_supported (const vkl_decode_model &m, int n_cu);

@@ -368,6 +368,12 @@ vkl_model_decode_step_bytes (const vkl_model *m, size_t L)
 }
 
 extern "C" int
+vkl_model_decode_form (const vkl_model *m, size_t pos)
+{
+  return m && m->llama () ? m->llama ()->decode_form (pos) : VKL_DECODE_FORM_PHASES;
+}
+
+extern "C" int
 vkl_model_phase_times (vkl_model *m, double ms_sum[VKL_DECODE_PHASES],
                        uint64_t launches[VKL_DECODE_PHASES])
 {

@@ -43,6 +43,7 @@ SIGNATURES = {
     "vkl_model_write_kv_cache": (i32, [vp, sz, i32, vp, sz]),
     "vkl_model_read_kv_cache": (i32, [vp, sz, i32, vp, sz]),
     "vkl_model_decode_step_bytes": (sz, [vp, sz]),
+    "vkl_model_decode_form": (i32, [vp, sz]),
     "vkl_model_phase_times": (i32, [vp, vp, vp]),
     "vkl_model_phase_bytes": (sz, [vp, i32, sz]),
     "vkl_model_phase_replay": (i32, [vp, i32, sz, i32, C.POINTER(C.c_double), C.POINTER(C.c_uint64)]),
@@ -318,7 +319,12 @@ class Llama2(CausalModel):
         self._check(lib().vkl_model_write_kv_cache(self._h, layer, int(value), rows.ctypes.data, rows.size),
                     "vkl_model_write_kv_cache")
 
-    PHASES = ("kqv", "attention", "wo", "upgate", "down", "lm_head", "argmax", "unused", "layer")
+    FORMS = ("phases", "layer", "layers", "step")
+    PHASES = ("kqv", "attention", "wo", "upgate", "down", "lm_head", "step", "layers", "layer")
+
+    def decode_form(self, pos):
+        """What one launch of a decode step at this position holds: one of FORMS."""
+        return self.FORMS[lib().vkl_model_decode_form(self._h, pos)]
 
     def phase_times(self):
         """{phase: (milliseconds summed, launches)} since the last call; filled

@@ -511,6 +511,14 @@ Model::decode_step_bytes (size_t L) const
   return wbytes + norm + emb + kv * L + kv;
 }
 
+int
+Model::decode_form (size_t pos) const
+{
+  if (!plan_ || !plan_->usable ())
+    return VKL_DECODE_FORM_PHASES;
+  return vkl_decode_form (&plan_->desc (), (uint32_t)pos, plan_->mode ());
+}
+
 size_t
 Model::decode_phase_bytes (int kind, size_t L) const
 {

@@ -176,6 +176,8 @@ public:
                                size_t n);
   size_t block_count () const { return blocks_.size (); }
   size_t decode_step_bytes (size_t L) const override;
+  // how a decode step at this position is launched (vkl_decode_form)
+  int decode_form (size_t pos) const;
   // algorithmic bytes of one launch of a decode phase (see vkl_decode.h)
   size_t decode_phase_bytes (int kind, size_t L) const;
   absl::Status decode_phase_replay (int kind, size_t pos, int rounds,

@@ -1439,9 +1439,10 @@ decode_loop (const vkl_decode_model *m, uint32_t *ids, uint32_t pos0, int n_step
       int upto = n_steps;
       if (!long_ctx)
         upto = (int)std::min<long long> (n_steps, (long long)attn_split_min (*m) - 1 - (long long)pos0);
-      // A step of one or a few launches needs no graph: with graphs of one node the GPU had 17 us
-      // without work between tokens (512 wide, 8 layers: 108 us per token, 103 launched), and
-      // the capture goes as well.
+      // A step of one to four launches (VKL_DECODE_FORM_STEP and _LAYERS) needs no graph: between
+      // graphs of so few nodes the GPU idles some 5 us longer than between launches (us per
+      // token, replayed / launched, 512 wide, 8 layers 97 / 92, fp16 88 / 84, 1024 wide 70 / 66, 1536
+      // 88 / 83), and the capture goes as well.
       p.pos = (uint32_t)std::min (attn_split_min (*m) - 2, m->maxlen - 1);
       if (!long_ctx && step_form (*m, (int)p.pos, mode, n_cu) >= VKL_DECODE_FORM_LAYERS)
         {

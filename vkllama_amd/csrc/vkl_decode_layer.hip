@@ -577,7 +577,7 @@ layer_launch_supported (const vkl_decode_model &m, int G)
 // Workgroups of a layer launch out of the G that fit (two per compute unit).  A layer of
 // little weight is bound by its hand-overs, not by the bytes in flight: half the workgroups
 // are half the arrivals to count and half the copies of the row to stage (most of the models up
-// to 1792 wide run all layers in one launch, vkl_decode_layers.hip).  us per token, G /
+// to 1920 wide run all layers in one launch, vkl_decode_layers.hip).  us per token, G /
 // G / 2, 8 layers, by MB of weights per layer: 3 (512 wide) 185 / 169, 14 197 / 182, 54 (2048
 // Q8_0) 261 / 236, 84 290 / 277, 101 (2048 fp16) 277 / 263, 120 321 / 317, 158 346 / 371, 215
 // (4096 Q8_0, 4 layers) 222 / 235.  Heads that take more than an eighth of the half leave the

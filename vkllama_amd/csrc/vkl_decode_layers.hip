@@ -27,8 +27,8 @@
 //
 // Two launches have to fit the GPU at once, as two launches per layer of narrow rows do (two
 // models on two streams would each wait for workgroups that the other one keeps out): a
-// workgroup takes one of two places of its compute unit, 128 registers and at most 80 KB of
-// LDS.  Rows of more than 512 bytes therefore request the down projection's, of more than 1024
+// workgroup takes one of two places of its compute unit, 128 registers (Q8_0 rows of more than
+// 1024 values spill nine) and at most 80 KB of LDS.  Rows of more than 512 bytes therefore request the down projection's, of more than 1024
 // the next layer's K/Q/V too, only when the up/gate product has left its registers.  With 256
 // registers and all of it requested at the one point above it was no faster, us per token: 512
 // wide Q8_0 97 / now 88, 1024 68 / 66, 1536 83 / 82, 768 wide fp16 87 / 82.

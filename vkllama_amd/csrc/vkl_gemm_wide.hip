@@ -1392,10 +1392,13 @@ wide_reduce_seg_kernel (const GemmSegArgs a, const float *ws, int parts)
 // Tiles of 64 rows have two workgroups to a compute unit: up to 256 of them take 0.54 per k-step +
 // 2.6, up to 512 0.81 + 3.7.  They win where rows are few or half of a taller tile is empty; us
 // without / with them: 40 x 8064 x 2048 16.3 / 14.5, 128 x 2048 x 7552 21.0 / 18.1, 12 x 16128 x
-// 4096 35.3 / 30.2.  Over 198 products of 2 to 2048 rows the plan is 1.1 % slower than the best in
-// the mean; without these tiles it was 4.7.  Not yet for operands of more than 128 rows, where they
-// are faster too, but whole where products are held to be in parts (160 x 5504 x 2048 18.4 us,
-// 128-row tiles in two parts 20.3).
+// 4096 35.3 / 30.2.  Over 198 products of 2 to 2048 rows the plan is 2.1 % slower than the best in
+// the mean (1.5 up to 128 rows, 2.7 above); without these tiles it was 4.7.  The line at 128 rows
+// is not where they stop to gain: over 140 products of 129 to 2000 rows the plan with them takes
+// 0.95 of the time in the mean up to 256 rows, 0.98 up to 640 and 0.99 above, 0.74 at best (448 x 2048
+// x 2048 21.3 / 15.7 us, 160 x 5504 x 2048 19.0 / 15.9) and 1.03 at worst (448 x 12544 x 4096 56.5 /
+// 58.0), but products of 160 and 512 rows are held to be in parts (tests/test_gemm_f32.py), which
+// 64-row tiles would not be.
 WidePlan
 wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
 {

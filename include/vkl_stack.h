@@ -203,7 +203,9 @@ typedef struct
   size_t os;
 } vkl_recurrence_args;
 /* form: VKL_RECUR_TOKENS one token after the other; VKL_RECUR_CHUNKS 64 at a time
- * as matrix products (dim up to 128); VKL_RECUR_AUTO by S and dim */
+ * as matrix products (dim up to 128); VKL_RECUR_AUTO by S and dim.  A key or value that
+ * is not finite reaches its token and those behind it, in chunks also those before it
+ * in the same sixteen of the call (it meets the zeros of their products) */
 #define VKL_RECUR_AUTO 0
 #define VKL_RECUR_TOKENS 1
 #define VKL_RECUR_CHUNKS 2

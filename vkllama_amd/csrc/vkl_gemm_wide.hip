@@ -1,28 +1,22 @@
 // y[M,N] = x[M,K] W[N,K]^T for many token rows (prompt passes of 128 tokens
 // and more), fp16 activations and dense fp16 or planar Q8_0 weights, fp32
-// accumulation on the matrix cores (v_mfma_f32_32x32x16_f16).  First the
-// kernel for fp16 weights; the one for Q8_0 weights follows it.
+// accumulation on the matrix cores; bf16 and 32-bit activations with bf16 weights.
 //
-// One workgroup of four waves per compute unit owns a 256 x 128 output tile;
-// each wave a 128 x 64 quarter (4 x 2 accumulators of 32 x 32).  A k-step is 64
-// wide, so a tile row is one 128-byte cache line.  The tiles of x and W do not
-// pass through registers on their way in: global_load_lds_dwordx4 writes them
-// straight into LDS, three k-steps deep (3 x 48 KiB), one 1 KiB instruction
+// A k-step is 64 wide, so a tile row is one 128-byte cache line.  The tiles of x and W do
+// not pass through registers on their way in: global_load_lds_dwordx4 writes them
+// straight into LDS, two to four k-steps deep, one 1 KiB instruction
 // per 8 tile rows.  Such an instruction writes its 64 x 16 bytes to consecutive
 // LDS addresses, so rows cannot be padded against bank conflicts; instead every
 // lane fetches the 16-byte chunk (slot ^ f(row)) of its row, which stores the
 // row XOR-swizzled, and the fragment reads apply the same f.
 //
-// The k loop is scheduled by hand (sched_group_barrier): the products of one
-// quarter of a k-step are issued alternately with the fragment reads of the
-// next quarter and with a share of the loads for the k-step after next, so the
-// single wave of a SIMD keeps the matrix core fed.  The barrier that hands over
-// the next k-step sits before the last quarter, whose products then overlap
-// with the first fragment reads of that step.
+// The k loop is scheduled by hand (sched_group_barrier): products alternate with the
+// fragment reads of the next part of a k-step and with a share of the loads for a later
+// k-step.  The barrier that hands over the next k-step sits inside a step, whose
+// remaining products then overlap with the first fragment reads of the next one.
 //
-// Measured on the 7B shapes at 2048 rows: matrix cores busy 63 % of the cycles
-// (the tile kernel of vkl_gemm_mfma.hip, which stages through registers:
-// 30-39 %).
+// Tiles of up to 256 x 256 (gemm_mix_kernel) multiply fp16 and bf16; those of 32 x 32
+// products (wide_bf16_tile) are left for 64 rows of bf16 and for 32-bit operands.
 #include "../../include/vkl_stack.h"
 #include "vkl_common.h"
 #include "vkl_gemm.h"
@@ -35,6 +29,7 @@ namespace
 {
 typedef _Float16 half8 __attribute__ ((ext_vector_type (8)));
 typedef __bf16 bf8 __attribute__ ((ext_vector_type (8)));
+typedef float float4v __attribute__ ((ext_vector_type (4)));
 typedef float float16v __attribute__ ((ext_vector_type (16)));
 #define VKL_LDS __attribute__ ((address_space (3)))
 
@@ -45,20 +40,25 @@ constexpr int WTN = WBN / 2 / 32;
 constexpr int WROWB = WBK * 2;                  // bytes of a tile row
 
 
-// element type of the dense kernel by its argument block: fp16 for the products
+// element type of the dense kernels by their argument block: fp16 for the products
 // with one plain epilogue, bf16 for those with segments
 template <class Args> struct WideElem
 {
   typedef half8 v8;
-  static __device__ __forceinline__ float16v
-  mfma (v8 a, v8 b, float16v c)
+  static __device__ __forceinline__ float4v
+  mfma (v8 a, v8 b, float4v c)
   {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16 (a, b, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16 (a, b, c, 0, 0, 0);
   }
 };
 template <> struct WideElem<GemmSegArgs>
 {
   typedef bf8 v8;
+  static __device__ __forceinline__ float4v
+  mfma (v8 a, v8 b, float4v c)
+  {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16 (a, b, c, 0, 0, 0);
+  }
   static __device__ __forceinline__ float16v
   mfma (v8 a, v8 b, float16v c)
   {
@@ -283,23 +283,22 @@ template <bool UPGATE> struct WideSimple<UPGATE, GemmSegArgs>
   }
 };
 
-// TN: 32-column accumulators of a wave, of the fused pair the first half up, the second
-// gate; mrow, ncol: the first row and output column of the wave's block
-template <bool UPGATE, int TM, int TN, class Args>
+// TN: 32-column accumulators of a wave; mrow, ncol: the first row and output column of the
+// wave's block
+template <int TM, int TN>
 __device__ __forceinline__ void
-wide_epilogue (const Args &a, const float16v (&acc)[TM][TN], uint8_t *wide_lds, int wave, int lane, int mrow, int ncol,
-               int zmat, int vec, float *part)
+wide_epilogue (const GemmSegArgs &a, const float16v (&acc)[TM][TN], uint8_t *wide_lds, int wave, int lane, int mrow, int ncol,
+               float *part)
 {
-  constexpr int NB = UPGATE ? TN / 2 : TN; // blocks of 32 output columns
-  const WideSimple<UPGATE, Args> simple (a, ncol, NB * 32, zmat, vec, part);
+  const WideSimple<false, GemmSegArgs> simple (a, ncol, TN * 32, 0, 1, part);
   if (simple.ok)
     {
       const int m0 = mrow + (lane & 31);
       auto walk = [&] (auto with) {
         constexpr bool RES = decltype (with)::value != 0;
-        constexpr int NR = WideSimple<UPGATE, Args>::NR;
+        constexpr int NR = WideSimple<false, GemmSegArgs>::NR;
 #pragma unroll
-        for (int jn = 0; jn < NB; ++jn)
+        for (int jn = 0; jn < TN; ++jn)
           {
             uint4 res[TM][2][NR];
             if (RES)
@@ -319,8 +318,6 @@ wide_epilogue (const Args &a, const float16v (&acc)[TM][TN], uint8_t *wide_lds, 
                     {
                       half_swap (acc[i][jn][8 * p + e], acc[i][jn][8 * p + 4 + e], v[e], v[4 + e]);
                       g[e] = g[4 + e] = 0.f;
-                      if (UPGATE)
-                        half_swap (acc[i][NB + jn][8 * p + e], acc[i][NB + jn][8 * p + 4 + e], g[e], g[4 + e]);
                     }
                   if (m0 + i * 32 < a.M)
                     simple.store ((size_t)(m0 + i * 32), jn * 32 + p * 16 + (lane >> 5) * 8, v, g, RES ? res[i][p] : nullptr);
@@ -343,8 +340,7 @@ wide_epilogue (const Args &a, const float16v (&acc)[TM][TN], uint8_t *wide_lds, 
 #pragma unroll
       for (int c = 0; c < 2; ++c)
         {
-          // of the fused pair a block of up, then its gate
-          const int jn = UPGATE ? c * NB + half : 2 * half + c;
+          const int jn = 2 * half + c;
 #pragma unroll
           for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -353,10 +349,10 @@ wide_epilogue (const Args &a, const float16v (&acc)[TM][TN], uint8_t *wide_lds, 
                   = make_float4 (acc[i][jn][q], acc[i][jn][q + 1], acc[i][jn][q + 2], acc[i][jn][q + 3]);
         }
       // (a wave reads back only what it wrote itself: no barrier)
-      constexpr int CPR = UPGATE ? 4 : 8;   // lanes per row
+      constexpr int CPR = 8;                // lanes per row
       constexpr int RPI = 64 / CPR;         // rows per iteration
       const int er = lane / CPR, ec = (lane % CPR) * 8;
-      const FinishRows<UPGATE, Args> fin (a, ncol + half * (UPGATE ? 32 : 64) + ec, zmat, vec, part);
+      const FinishRows<false, GemmSegArgs> fin (a, ncol + half * 64 + ec, 0, 1, part);
       for (int it = 0; it < ROWS / RPI; ++it)
         {
           const int row = it * RPI + er;
@@ -365,12 +361,7 @@ wide_epilogue (const Args &a, const float16v (&acc)[TM][TN], uint8_t *wide_lds, 
           const float *pr = park + row * LD + ec;
           const float4 p0 = *(const float4 *)pr, p1 = *(const float4 *)(pr + 4);
           float v[8] = { p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w };
-          float g[8] = { 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f };
-          if (UPGATE)
-            {
-              const float4 g0 = *(const float4 *)(pr + 32), g1 = *(const float4 *)(pr + 36);
-              g[0] = g0.x, g[1] = g0.y, g[2] = g0.z, g[3] = g0.w, g[4] = g1.x, g[5] = g1.y, g[6] = g1.z, g[7] = g1.w;
-            }
+          const float g[8] = { 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f };
           fin.store (mrow + row, v, g, res);
         }
     }
@@ -424,7 +415,7 @@ wide_epilogue_tile (const GemmArgs &a, const float16v (&acc)[TM][1], uint8_t *wi
 
 template <int BM>
 constexpr size_t
-wide_lds_f16 ()
+wide_lds_bf16 ()
 {
   const size_t stages = (size_t)WSTAGES * (BM + WBN) * WROWB, park = (size_t)BM * 2 * kWideParkLd * 4;
   return stages > park ? stages : park;
@@ -486,26 +477,26 @@ wide_f32_again (const GemmSegArgs &a, float16v (&acc)[TM][WTN], int lane, int mr
       }
 }
 
-// BM: token rows of a tile, 256 or (where 256-row tiles would be too few to
-// occupy the compute units) 128, i.e. 64 x 64 per wave; of bf16 products also 64.
+// A BM x 128 tile by four waves of BM / 2 x 64, three k-steps of it in LDS: 64 rows of bf16
+// products (two workgroups share a compute unit then), and 256 and 128 rows of 32-bit ones.
 // PLANES > 1: x holds PLANES values for every weight, in blocks of 64 (one k-step of
 // each plane in turn): see the 32-bit product below.
-template <int BM, bool UPGATE, class Args, int PLANES>
+template <int BM, int PLANES>
 __device__ __forceinline__ void
-wide_f16_tile (const Args &a, const WidePlace &at, int vec, int ksplit, float *ws)
+wide_bf16_tile (const GemmSegArgs &a, const WidePlace &at, int ksplit, float *ws)
 {
-  typedef typename WideElem<Args>::v8 v8;
+  typedef WideElem<GemmSegArgs>::v8 v8;
   constexpr int TM = BM / 2 / 32;                    // 32-row accumulators per wave
   constexpr int STAGE_BYTES = (BM + WBN) * WROWB;
   constexpr int GPW = (BM + WBN) / 8 / WWAVES;       // 1 KiB load instructions per wave and k-step
   constexpr int AG = BM / 8 / WWAVES;                // of which rows of x
   extern __shared__ __align__ (16) uint8_t wide_lds[];
-  const int ks = at.ks, zmat = at.zmat;
+  const int ks = at.ks;
   const int nk_all = a.K / WBK;
   const int kbase = (int)((long)nk_all * ks / ksplit);
   const int nk = (int)((long)nk_all * (ks + 1) / ksplit) - kbase; // k-steps of this workgroup
   float *part = ksplit > 1 ? ws + (size_t)ks * a.M * a.N : nullptr;
-  const int m0 = at.m0, n0 = at.tn * (UPGATE ? WBN / 2 : WBN); // weight rows per matrix and tile
+  const int m0 = at.m0, n0 = at.tn * WBN;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane (threadIdx.x >> 6);
   const int wm = wave >> 1, wn = wave & 1;
@@ -528,10 +519,7 @@ wide_f16_tile (const Args &a, const WidePlace &at, int vec, int ksplit, float *w
   for (int i = AG; i < GPW; ++i)
     {
       const int v = (wave + WWAVES * (i - AG)) * 8 + lr; // row of the weight tile
-      const int mat = UPGATE ? v >> 6 : zmat;
-      const int n = min (UPGATE ? n0 + (v & 63) : n0 + v, a.N - 1);
-      const uint16_t *w = pick3 (a.wh[0], a.wh[1], a.wh[2], mat);
-      src[i] = w + (size_t)n * a.ws + chunk * 8 + (PLANES > 1 ? 0 : (size_t)kbase * WBK);
+      src[i] = a.wh[0] + (size_t)min (n0 + v, a.N - 1) * a.ws + chunk * 8 + (PLANES > 1 ? 0 : (size_t)kbase * WBK);
     }
 
   // fragment reads: lane l holds row l%32 of a 32-row block, k = 16 ks + 8 (l/32) .. +7
@@ -542,9 +530,9 @@ wide_f16_tile (const Args &a, const WidePlace &at, int vec, int ksplit, float *w
     {
       const int ko = ((2 * ks + (lane >> 5)) ^ fsw) << 4;
       aoff[ks] = (wm * (BM / 2) + (lane & 31)) * WROWB + ko;
-      boff[ks] = BM * WROWB + ((UPGATE ? wn * 32 : wn * 64) + (lane & 31)) * WROWB + ko;
+      boff[ks] = BM * WROWB + (wn * 64 + (lane & 31)) * WROWB + ko;
     }
-  constexpr int BJ = (UPGATE ? 64 : 32) * WROWB; // from a wave's first to its second column block
+  constexpr int BJ = 32 * WROWB; // from a wave's first to its second column block
 
   float16v acc[TM][WTN];
 #pragma unroll
@@ -617,7 +605,7 @@ wide_f16_tile (const Args &a, const WidePlace &at, int vec, int ksplit, float *w
         for (int i = 0; i < TM; ++i)
 #pragma unroll
           for (int jn = 0; jn < WTN; ++jn)
-            acc[i][jn] = WideElem<Args>::mfma (bf[ks & 1][jn], af[ks & 1][i], acc[i][jn]);
+            acc[i][jn] = WideElem<GemmSegArgs>::mfma (bf[ks & 1][jn], af[ks & 1][i], acc[i][jn]);
         if (ks == 0)
           WideOrder<0, NP, NR, LB1>::run ();
         else if (ks == 1)
@@ -649,7 +637,7 @@ wide_f16_tile (const Args &a, const WidePlace &at, int vec, int ksplit, float *w
   if constexpr (PLANES > 1)
     if (!part) // (of parts the sum is looked at)
       wide_f32_again<TM> (a, acc, lane, m0 + wm * TM * 32, n0 + wn * 64, a.K / PLANES);
-  wide_epilogue<UPGATE, TM, WTN> (a, acc, wide_lds, wave, lane, m0 + wm * TM * 32, n0 + (UPGATE ? wn * 32 : wn * 64), zmat, vec, part);
+  wide_epilogue<TM, WTN> (a, acc, wide_lds, wave, lane, m0 + wm * TM * 32, n0 + wn * 64, part);
 }
 
 // The planes of a 32-bit operand (see there) in tiles of 64 rows: x holds three values for
@@ -659,7 +647,7 @@ wide_f16_tile (const Args &a, const WidePlace &at, int vec, int ksplit, float *w
 // out of it per 64 columns, 1730 cycles at 128 bytes for 770 of products; now 40 + 80 KB.  Two
 // stages are 80 KB, two workgroups to a compute unit, each of which multiplies where the other
 // one waits.  Tiles of 128 rows (128 KB, one workgroup) were slower (800 x 16128 x 4096 362 us for
-// 315); of 256 they do not fit, and those of wide_f16_tile (144 + 288 KB for 3070 cycles of products)
+// 315); of 256 they do not fit, and those of wide_bf16_tile (144 + 288 KB for 3070 cycles of products)
 // stay the better ones where they fill the chip (wide_plan_planes).  us before / now: 12 x 12288 x
 // 4096 39.9 / 33.0, 300 x 2048 x 2048 27.8 / 25.2, 300 x 5504 x 2048 41.9 / 37.1, 300 x 12288 x 4096
 // 120 / 96, 700 x 11008 x 4096 236 / 188.
@@ -693,7 +681,7 @@ gemm_wide_planes_kernel (const GemmSegArgs a, WideGrid grid, int ksplit, float *
   const int wave = __builtin_amdgcn_readfirstlane (threadIdx.x >> 6);
   const int wm = wave >> 1, wn = wave & 1;
 
-  // rows and chunks as in wide_f16_tile
+  // rows and chunks as in wide_bf16_tile
   const int lr = lane >> 3;
   const int chunk = (lane & 7) ^ lr ^ (wave & 1);
   const uint16_t *srca[AG], *srcb[BG];
@@ -819,12 +807,12 @@ gemm_wide_planes_kernel (const GemmSegArgs a, WideGrid grid, int ksplit, float *
         acc[i][jn][q] += low[i][jn][q];
   if (!part) // (of parts the sum is looked at)
     wide_f32_again<TM> (a, acc, lane, m0 + wm * TM * 32, n0 + wn * 64, a.K / kPlanes);
-  wide_epilogue<false, TM, WTN> (a, acc, wide_lds, wave, lane, m0 + wm * TM * 32, n0 + wn * 64, 0, 1, part);
+  wide_epilogue<TM, WTN> (a, acc, wide_lds, wave, lane, m0 + wm * TM * 32, n0 + wn * 64, part);
 }
 
-template <int BM, bool UPGATE, class Args = GemmArgs, int PLANES = 1>
+template <int BM, int PLANES>
 __global__ __launch_bounds__ (WWAVES * 64) void
-gemm_wide_f16_kernel (const Args a, WideGrid grid, int vec, int ksplit, float *ws)
+gemm_wide_bf16_kernel (const GemmSegArgs a, WideGrid grid, int ksplit, float *ws)
 {
   WidePlace at;
   switch (grid.place<BM> (a.M, at))
@@ -832,10 +820,494 @@ gemm_wide_f16_kernel (const Args a, WideGrid grid, int vec, int ksplit, float *w
     case WIDE_NONE:
       return;
     case WIDE_TILE:
-      return wide_f16_tile<BM, UPGATE, Args, PLANES> (a, at, vec, ksplit, ws);
+      return wide_bf16_tile<BM, PLANES> (a, at, ksplit, ws);
     case WIDE_HALF:
       if constexpr (BM == WBM)
-        return wide_f16_tile<BM / 2, UPGATE, Args, PLANES> (a, at, vec, ksplit, ws);
+        return wide_bf16_tile<BM / 2, PLANES> (a, at, ksplit, ws);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// tiles of up to 256 x 256
+// ---------------------------------------------------------------------------
+constexpr int MWAVES = 8;
+
+// What the tiles of gemm_mix_kernel take, us: of bm token rows and 256 columns, of 128 columns,
+// and of half the rows.  Fitted (with wide_plan_bf16's other constants) to 195 bf16 products of
+// 130 to 2200 rows, K = 512 to 15104, weights that no cache holds, in up to 24 plans each.
+struct MixTime
+{
+  double step, start, parked; // per k-step; per tile; more where its sums are parked in LDS
+};
+inline MixTime
+mix_time (int bm, int kind)
+{
+  constexpr MixTime t256[3] = { { 1.42, 5.5, 15.5 }, { 0.76, 6.9, 8.3 }, { 0.54, 5.6, 4.4 } };
+  constexpr MixTime t128[3] = { { 0.80, 6.3, 7.6 }, { 0.52, 5.9, 4.6 }, { 0.52, 5.9, 4.6 } };
+  return bm == WBM ? t256[kind] : t128[kind];
+}
+
+// When the compute units are done with tiles dealt in turn to whichever is free first.
+struct MixSpan
+{
+  double at[4] = { 0, 0, 0, 0 };
+  int units[4] = { WideGrid::kUnits, 0, 0, 0 }, n = 1; // each kind of tile adds at most one level
+  double last = 0;
+
+  void
+  deal (int tiles, double time)
+  {
+    while (tiles > 0)
+      {
+        if (n == 1 && tiles >= units[0])
+          {
+            at[0] += tiles / units[0] * time, tiles %= units[0];
+            last = at[0];
+            continue;
+          }
+        int f = 0;
+        for (int i = 1; i < n; ++i)
+          if (at[i] < at[f])
+            f = i;
+        const double end = at[f] + time;
+        const int take = tiles < units[f] ? tiles : units[f];
+        last = end > last ? end : last, tiles -= take;
+        int same = 0;
+        while (same < n && at[same] != end)
+          ++same;
+        if (take == units[f] && same == n)
+          at[f] = end; // the level moves
+        else
+          {
+            if (same < n)
+              units[same] += take;
+            else
+              at[n] = end, units[n++] = take;
+            units[f] -= take;
+            if (!units[f])
+              --n, at[f] = at[n], units[f] = units[n];
+          }
+      }
+  }
+};
+
+// The tiles of a launch: pairs of 128-column tiles as one of 256 columns, then tiles of 128
+// columns, of which the last may be cut in two by their rows.  Each kind is dealt to the XCDs
+// in contiguous ranges of pairs, row tile fastest in groups of eight: the 32 pairs that an XCD
+// multiplies at a time are then 8 x 4 and not 32 x 1, and share their rows in its L2 (8192 x
+// 8192 x 8192 1023 us with 32 x 1, 823 with 8 x 4, 256 x 128 tiles).
+//
+// A tile of 256 columns takes 0.92 of two of 128 (every fragment that is read from LDS goes into
+// twice the products), but fewer of them fill a round over the 256 compute units.  So either no
+// pair, as many as fill whole rounds, or all go into one tile, whichever is done first: 2048 x
+// 12288 columns (1.5 rounds of pairs) 182 us with one round of pairs and 256 tiles, 198 without pairs,
+// 211 of pairs alone; 1500 x 8064, K = 2048 59 / 59 / 55.
+struct WideMix
+{
+  int tiles_m, tiles_n, nmat, ksplit;
+  int wide;  // pairs in one tile
+  int whole; // tiles of 128 columns that are not cut
+
+  __host__ __device__ int
+  pairs () const
+  {
+    return tiles_m * (tiles_n / 2) * nmat * ksplit;
+  }
+  __host__ __device__ int
+  narrow () const // tiles of 128 columns, cut or not
+  {
+    return tiles_m * tiles_n * nmat * ksplit - 2 * wide;
+  }
+  // bm: token rows of a tile, 256 (which may be cut) or 128; steps: of the k range of a part;
+  // park: how much of the time for parked sums a tile takes; us: the time of the launch's tiles
+  __host__
+  WideMix (int bm, int tm, int tn, int mats, int parts, double steps, double park, double *us = nullptr)
+      : tiles_m (tm), tiles_n (tn), nmat (mats), ksplit (parts)
+  {
+    constexpr int U = WideGrid::kUnits;
+    double t[3];
+    for (int k = 0; k < 3; ++k)
+      {
+        const MixTime m = mix_time (bm, k);
+        t[k] = m.step * steps + m.start + park * m.parked;
+      }
+    const int options[3] = { 0, pairs () / U * U, pairs () };
+    int best_wide = 0, best_whole = 0;
+    double best = -1;
+    for (int o = 0; o < 3; ++o)
+      {
+        if (o && options[o] == options[o - 1])
+          continue;
+        wide = options[o];
+        const int rest = narrow () % U;
+        whole = bm == WBM && wide % U == 0 && rest > 0 && rest <= U / 2 ? narrow () - rest : narrow ();
+        MixSpan span;
+        span.deal (wide, t[0]);
+        span.deal (whole, t[1]);
+        span.deal (2 * (narrow () - whole), t[2]);
+        if (best < 0 || span.last < best)
+          best = span.last, best_wide = wide, best_whole = whole;
+      }
+    wide = best_wide, whole = best_whole;
+    if (us)
+      *us = best;
+  }
+  static __host__ __device__ int
+  eight (int n)
+  {
+    return (n + 7) / 8 * 8;
+  }
+  __host__ int
+  groups () const
+  {
+    return eight (wide) + eight (whole) + eight (2 * (narrow () - whole));
+  }
+  __device__ __forceinline__ void
+  pair_at (int p, WidePlace &at, int BM) const
+  {
+    const int cols = tiles_n / 2, mats = tiles_m * cols * nmat, grp = 8 * cols * nmat;
+    at.ks = p / mats;
+    p -= at.ks * mats;
+    const int g = p / grp, gm = min (8, tiles_m - 8 * g);
+    p -= g * grp;
+    at.m0 = (8 * g + p % gm) * BM;
+    p /= gm;
+    at.tn = 2 * (p % cols);
+    at.zmat = p / cols;
+  }
+  // 0: nothing to do, 1: a pair, 2: one tile, 3: half a tile
+  __device__ __forceinline__ int
+  place (int M, int BM, WidePlace &at) const
+  {
+    const int g0 = eight (wide), g1 = g0 + eight (whole);
+    int id = (int)blockIdx.x;
+    const int kind = id < g0 ? 1 : id < g1 ? 2 : 3;
+    id -= kind == 1 ? 0 : kind == 2 ? g0 : g1;
+    const int count = kind == 1 ? wide : kind == 2 ? whole : 2 * (narrow () - whole);
+    const int per_xcd = (count + 7) / 8, j = id >> 3;
+    int i = (id & 7) * per_xcd + j;
+    if (j >= per_xcd || i >= count)
+      return 0;
+    if (kind == 1)
+      {
+        pair_at (i, at, BM);
+        return 1;
+      }
+    int half = 0;
+    if (kind == 3)
+      half = i & 1, i = whole + (i >> 1);
+    const int left = 2 * (pairs () - wide);
+    if (i < left)
+      {
+        pair_at (wide + (i >> 1), at, BM);
+        at.tn += i & 1;
+      }
+    else
+      {
+        // the last column of an odd number
+        i -= left;
+        at.m0 = i % tiles_m * BM;
+        i /= tiles_m;
+        at.tn = tiles_n - 1, at.zmat = i % nmat, at.ks = i / nmat;
+      }
+    at.m0 += half * (BM / 2);
+    return at.m0 < M ? kind : 0;
+  }
+};
+
+// Issue order of half a k-step: after each product an even share of its fragment reads and loads
+template <int Q, int NP, int NR, int NL> struct MixOrder
+{
+  static __device__ __forceinline__ void
+  run ()
+  {
+    __builtin_amdgcn_sched_group_barrier (0x008, 1, 0); // one MFMA
+    constexpr int nr = NR * (Q + 1) / NP - NR * Q / NP, nl = NL * (Q + 1) / NP - NL * Q / NP;
+    if constexpr (nr > 0)
+      __builtin_amdgcn_sched_group_barrier (0x100, nr, 0); // LDS reads
+    if constexpr (nl > 0)
+      __builtin_amdgcn_sched_group_barrier (0x020, nl, 0); // loads
+    if constexpr (Q + 1 < NP)
+      MixOrder<Q + 1, NP, NR, NL>::run ();
+  }
+};
+
+// acc[i][j]: 16 token rows by 16 weight rows; blocks 2 b and 2 b + 1 of a wave hold, in lane l,
+// columns 8 (l / 16) .. + 3 and + 4 .. + 7 of its 32 columns b (see mix_tile): eight neighbours
+// of token row l % 16.  Of the fused pair blocks 0, 1 are up and 2, 3 gate.
+template <bool UPGATE, int TM, class Args>
+__device__ __forceinline__ void
+mix_epilogue (const Args &a, const float4v (&acc)[TM][4], uint8_t *wide_lds, int wave, int lane, int mrow, int ncol,
+              int zmat, int vec, float *part)
+{
+  constexpr int NB = UPGATE ? 1 : 2; // 32-column blocks of outputs, each by itself
+  bool parked = false;
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+    {
+      const WideSimple<UPGATE, Args> simple (a, ncol + b * 32, 32, zmat, vec, part);
+      if (!simple.ok)
+        {
+          parked = true;
+          continue;
+        }
+      const int m0 = mrow + (lane & 15), col = (lane >> 4) * 8;
+      auto walk = [&] (auto with) {
+        constexpr bool RES = decltype (with)::value != 0;
+        constexpr int NR = WideSimple<UPGATE, Args>::NR;
+        uint4 res[TM][NR];
+        if (RES)
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+            simple.request ((size_t)min (m0 + i * 16, a.M - 1), col, res[i]);
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+          {
+            float v[8], g[8];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              {
+                v[e] = acc[i][2 * b][e], v[4 + e] = acc[i][2 * b + 1][e];
+                g[e] = UPGATE ? acc[i][2][e] : 0.f, g[4 + e] = UPGATE ? acc[i][3][e] : 0.f;
+              }
+            if (m0 + i * 16 < a.M)
+              simple.store ((size_t)(m0 + i * 16), col, v, g, RES ? res[i] : nullptr);
+          }
+      };
+      if (simple.r)
+        walk (WideInt<1> ());
+      else
+        walk (WideInt<0> ());
+    }
+  if (!parked)
+    return;
+  __builtin_amdgcn_s_barrier (); // every wave (that is left) has read its last fragments
+  // through LDS: a block of 32 columns of all rows, of the fused pair both blocks of 64 rows
+  constexpr int PM = UPGATE && TM > 4 ? 4 : TM, ROWS = PM * 16, LD = UPGATE ? 68 : 36;
+  float *park = (float *)(wide_lds + wave * (ROWS * LD * 4));
+  constexpr int RPI = 16; // rows per iteration, four lanes each
+  const int er = lane >> 2, ec = (lane & 3) * 8;
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+    {
+      if (WideSimple<UPGATE, Args> (a, ncol + b * 32, 32, zmat, vec, part).ok)
+        continue;
+      const FinishRows<UPGATE, Args> fin (a, ncol + b * 32 + ec, zmat, vec, part);
+#pragma unroll
+      for (int i0 = 0; i0 < TM; i0 += PM)
+        {
+#pragma unroll
+          for (int i = 0; i < PM; ++i)
+#pragma unroll
+            for (int j = 0; j < (UPGATE ? 4 : 2); ++j)
+              *(float4v *)(park + (i * 16 + (lane & 15)) * LD + (j >> 1) * 32 + (lane >> 4) * 8 + (j & 1) * 4)
+                  = acc[i0 + i][2 * b + j];
+          // (a wave reads back only what it wrote itself: no barrier)
+#pragma unroll 1
+          for (int it = 0; it < ROWS / RPI; ++it)
+            {
+              const int row = it * RPI + er, m = mrow + i0 * 16 + row;
+              uint4 res[2];
+              fin.request (m, res);
+              const float *pr = park + row * LD + ec;
+              const float4v p0 = *(const float4v *)pr, p1 = *(const float4v *)(pr + 4);
+              float v[8] = { p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w };
+              float g[8] = { 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f };
+              if (UPGATE)
+                {
+                  const float4v g0 = *(const float4v *)(pr + 32), g1 = *(const float4v *)(pr + 36);
+                  g[0] = g0.x, g[1] = g0.y, g[2] = g0.z, g[3] = g0.w, g[4] = g1.x, g[5] = g1.y, g[6] = g1.z, g[7] = g1.w;
+                }
+              fin.store (m, v, g, res);
+            }
+        }
+    }
+}
+
+// A BM x BN tile by WM x WN waves of (BM / WM) x 64, ST k-steps of 64 in LDS: one workgroup
+// of eight waves to a compute unit, so that one wave of a SIMD multiplies where the other one
+// waits for a barrier or its fragments.
+//
+// Products of 16 x 16 x 32 (rather than 32 x 32 x 16) and 256 x 256 tiles: bound by the chip's
+// power under matrix load (at 8192 x 8192 x 8192 matrix cores busy 71 % of the cycles at 1.81
+// GHz, 56 % at 1.87 in 256 x 128 tiles of four waves with 32 x 32 x 16; the vendor library's kernel 88 %
+// at 1.64), so less data per product out of LDS and L2 is what makes it faster.  The loads of a k-step are
+// issued when its stage has just been read, not a quarter later: two stages of 64 KB are enough then.
+// Tried on the way, 4096 x 4096 x 4096, us: 107 as it is, 123 with 32 x 32 x 16, 147 with four waves
+// of 128 x 128 (AGPR moves), 117 with raised wave priority around the products, 114 with four stages of
+// 32 columns, 111 with two reads per product.
+// Same call before / now, us, fp16, one box: 4096 x 4096 x 4096 132 / 110, 2048 x 12288 x 4096 191 / 174,
+// 2048 x 22016 x 4096 366 / 318, 3967 x 5120 x 5120 256 / 192, 8192 x 8192 x 8192 1250 / 822, 300 x 4096 x
+// 4096 28.8 / 27.2, 77 x 4096 x 4096 18.1 / 16.5, 2048 x 4096 x 4096 64.4 / 62.7.
+template <int BM, int BN, int WM, int ST, bool UPGATE, class Args>
+__device__ __forceinline__ void
+mix_tile (const Args &a, const WidePlace &at, int vec, int ksplit, float *ws)
+{
+  typedef typename WideElem<Args>::v8 v8;
+  constexpr int WN = MWAVES / WM, TM = BM / WM / 16, TN = 4;
+  static_assert (BN / WN == 64 && BM % (MWAVES * 8) == 0 && BN % (MWAVES * 8) == 0, "");
+  constexpr int STAGE_BYTES = (BM + BN) * WROWB;
+  constexpr int AG = BM / 8 / MWAVES, LOADS = (BM + BN) / 8 / MWAVES; // 1 KiB instructions per wave and k-step
+  extern __shared__ __align__ (16) uint8_t wide_lds[];
+  const int nk_all = a.K / WBK;
+  const int kbase = (int)((long)nk_all * at.ks / ksplit);
+  const int nk = (int)((long)nk_all * (at.ks + 1) / ksplit) - kbase;
+  float *part = ksplit > 1 ? ws + (size_t)at.ks * a.M * a.N : nullptr;
+  const int m0 = at.m0, n0 = at.tn * (UPGATE ? WBN / 2 : WBN);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane (threadIdx.x >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+
+  // Load addresses.  Instruction i of a wave covers eight tile rows 8 g .. 8 g + 7, g = wave +
+  // 8 i; slot l % 8 of row 8 g + l / 8 receives the row's chunk (l % 8) ^ f (row).  Sixteen
+  // lanes read 16 bytes at a time, 0-3, 12-15, 20-27 and their complement of a half wave: of a
+  // fragment eight rows at one chunk and eight others at the next.  With f = row / 2 of the
+  // token rows, and of the weight rows, whose fragments are rows 8 (r / 4) + r % 4 (+ 4), bit 1
+  // below bits 3 and 4, these lie in different banks (no conflicts by the counters; half of
+  // the read cycles with the order of the 32 x 32 products).  Rows beyond M or N repeat the
+  // last row (never stored).
+  const int lr = lane >> 3;
+  const int fa = (wave & 1) * 4 + (lane >> 4), fb = ((lr >> 1) & 1) | ((wave & 3) << 1);
+  const uint16_t *src[LOADS];
+#pragma unroll
+  for (int i = 0; i < AG; ++i)
+    src[i] = a.x + (size_t)min (m0 + (wave + MWAVES * i) * 8 + lr, a.M - 1) * a.xs + ((lane & 7) ^ fa) * 8
+             + (size_t)kbase * WBK;
+#pragma unroll
+  for (int i = AG; i < LOADS; ++i)
+    {
+      const int v = (wave + MWAVES * (i - AG)) * 8 + lr;
+      const int mat = UPGATE ? v / (BN / 2) : at.zmat;
+      const int n = min (n0 + (UPGATE ? v % (BN / 2) : v), a.N - 1);
+      src[i] = pick3 (a.wh[0], a.wh[1], a.wh[2], mat) + (size_t)n * a.ws + ((lane & 7) ^ fb) * 8 + (size_t)kbase * WBK;
+    }
+  // fragment reads: lane l holds row l % 16 of a fragment, k = 32 h + 8 (l / 16) .. + 7
+  const int r = lane & 15, brow = (r >> 2) * 8 + (r & 3);
+  const int ga = (r >> 1) & 7, gb = ((brow >> 1) & 1) | (((brow >> 3) & 3) << 1);
+  uint32_t aoff[2], boff[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    {
+      const int c = 4 * h + (lane >> 4);
+      aoff[h] = (wm * (BM / WM) + r) * WROWB + ((c ^ ga) << 4);
+      boff[h] = (BM + wn * (UPGATE ? 32 : 64) + brow) * WROWB + ((c ^ gb) << 4);
+    }
+  constexpr int BJ = (UPGATE ? BN / 2 : 32) * WROWB; // from a wave's first to its second 32 weight rows
+
+  float4v acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      acc[i][j] = float4v{ 0.f, 0.f, 0.f, 0.f };
+
+  auto issue = [&] (int kt, int st) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i)
+      {
+        const int g = i < AG ? wave + MWAVES * i : BM / 8 + wave + MWAVES * (i - AG);
+        __builtin_amdgcn_global_load_lds ((const VKL_GLOBAL void *)(src[i] + (size_t)kt * WBK),
+                                          (VKL_LDS void *)(wide_lds + st * STAGE_BYTES + g * 1024), 16, 0, 0);
+      }
+  };
+#pragma unroll
+  for (int p = 0; p < ST; ++p)
+    issue (p < nk ? p : nk - 1, p);
+  v8 af[2][TM], bf[2][TN];
+  auto read_frags = [&] (int st, int h, int buf) {
+    const uint8_t *sb = wide_lds + st * STAGE_BYTES;
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      bf[buf][j] = *(const v8 *)(sb + boff[h] + (j >> 1) * BJ + (j & 1) * 4 * WROWB);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+      af[buf][i] = *(const v8 *)(sb + aoff[h] + i * 16 * WROWB);
+  };
+  // s_waitcnt immediates: vmcnt = the loads of so many k-steps may stay in flight
+  constexpr int V0 = (ST - 1) * LOADS, V1 = (ST - 2) * LOADS;
+  static_assert (V0 < 64, "");
+  constexpr int WAIT0 = 0x0f70 | (V0 & 15) | ((V0 >> 4) << 14), WAIT1 = 0x0070 | (V1 & 15) | ((V1 >> 4) << 14);
+  // One k-step.  On entry tile kt is in stage S and the fragments of its first half are on
+  // their way.  Between its halves tile kt + 1 has landed (this wave's part; the barrier covers
+  // the others') and nobody reads tile kt any more, whose last fragments are in registers: its
+  // stage takes tile kt + ST, a whole step and more before it is wanted (past the end the last
+  // tile again, which nothing reads).
+  auto step = [&] (int kt, auto stc) {
+    constexpr int S = decltype (stc)::value;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      {
+        if (h == 0)
+          read_frags (S, 1, 1);
+        else
+          {
+            __builtin_amdgcn_s_waitcnt (WAIT1); // also for the wave's own LDS reads
+            __builtin_amdgcn_s_barrier ();
+            __builtin_amdgcn_sched_barrier (0);
+            issue (kt + ST < nk ? kt + ST : nk - 1, S);
+            read_frags ((S + 1) % ST, 0, 0);
+          }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            acc[i][j] = WideElem<Args>::mfma (bf[h][j], af[h][i], acc[i][j]);
+        if (h)
+          MixOrder<0, TM * TN, TM + TN, LOADS>::run ();
+        else
+          MixOrder<0, TM * TN, TM + TN, 0>::run ();
+        __builtin_amdgcn_sched_barrier (0);
+      }
+  };
+  __builtin_amdgcn_s_waitcnt (WAIT0);
+  __builtin_amdgcn_s_barrier ();
+  read_frags (0, 0, 0);
+  __builtin_amdgcn_sched_barrier (0);
+  int kt = 0;
+  for (; kt + ST <= nk; kt += ST)
+    {
+      step (kt, WideInt<0> ());
+      step (kt + 1, WideInt<1 % ST> ());
+      if constexpr (ST > 2)
+        step (kt + 2, WideInt<2 % ST> ());
+      if constexpr (ST > 3)
+        step (kt + 3, WideInt<3 % ST> ());
+    }
+  if (kt < nk)
+    step (kt, WideInt<0> ());
+  if (ST > 2 && kt + 1 < nk)
+    step (kt + 1, WideInt<1> ());
+  if (ST > 3 && kt + 2 < nk)
+    step (kt + 2, WideInt<2 % ST> ());
+  __builtin_amdgcn_s_waitcnt (0x0070); // no load may outlive the workgroup's LDS (nor a fragment read the parked sums)
+  mix_epilogue<UPGATE, TM, Args> (a, acc, wide_lds, wave, lane, m0 + wm * (BM / WM), n0 + wn * (UPGATE ? 32 : 64), at.zmat,
+                                  vec, part);
+}
+
+template <int BM>
+constexpr size_t
+mix_lds ()
+{
+  constexpr size_t wide = (size_t)(BM == WBM ? 2 : 3) * (BM + 256) * WROWB;
+  constexpr size_t narrow = (size_t)(BM == WBM ? 3 : 4) * (BM + WBN) * WROWB;
+  constexpr size_t park = (size_t)MWAVES * std::max (BM / 2 * 36, 64 * 68) * 4; // see mix_epilogue
+  return std::max (std::max (wide, narrow), park);
+}
+
+template <int BM, bool UPGATE, class Args>
+__global__ __launch_bounds__ (MWAVES * 64) void
+gemm_mix_kernel (const Args a, WideMix grid, int vec, int ksplit, float *ws)
+{
+  WidePlace at;
+  switch (grid.place (a.M, BM, at))
+    {
+    case 1:
+      return mix_tile<BM, 256, 2, BM == WBM ? 2 : 3, UPGATE, Args> (a, at, vec, ksplit, ws);
+    case 2:
+      return mix_tile<BM, WBN, 4, BM == WBM ? 3 : 4, UPGATE, Args> (a, at, vec, ksplit, ws);
+    case 3:
+      if constexpr (BM == WBM)
+        return mix_tile<BM / 2, WBN, 4, 4, UPGATE, Args> (a, at, vec, ksplit, ws);
     }
 }
 
@@ -1116,6 +1588,8 @@ gemm_wide_q8_kernel (const GemmArgs a, WideGrid grid, int vec, int ksplit, float
 // three fp16 matrices of one launch: their 2.25 rounds came out level with 4.5 of 128-row tiles,
 // which took longer than the matrices apart (4096 x 4096, 1300 / 1500 rows: 1.07 / 1.12 of that;
 // in 256-row tiles 0.91 / 0.94, 158 / 164 us).
+// (The fp16 tiles have become faster since, those of 256 rows more than those of 128; the
+// choices for the 7B and 13B shapes are held by tests/test_gemm_plan.py.)
 // Below kWideMinGroups workgroups the tile kernel of vkl_gemm_mfma.hip does
 // better.
 constexpr int kWideMinRows = 128;
@@ -1212,15 +1686,15 @@ gemm_wide_workspace_bytes (const GemmArgs &a)
 int
 gemm_wide_launch (const GemmArgs &a, hipStream_t s)
 {
-  constexpr size_t lds256 = wide_lds_f16<256> (), lds128 = wide_lds_f16<128> ();
+  constexpr size_t m256 = mix_lds<256> (), m128 = mix_lds<128> ();
   constexpr size_t q256 = wide_lds_q8<256> (), q128 = wide_lds_q8<128> ();
   static LdsLimit limits[8];
   const void *const kernels[8]
-      = { (const void *)gemm_wide_f16_kernel<256, false>,       (const void *)gemm_wide_f16_kernel<256, true>,
-          (const void *)gemm_wide_f16_kernel<128, false>,       (const void *)gemm_wide_f16_kernel<128, true>,
+      = { (const void *)gemm_mix_kernel<256, false, GemmArgs>, (const void *)gemm_mix_kernel<256, true, GemmArgs>,
+          (const void *)gemm_mix_kernel<128, false, GemmArgs>, (const void *)gemm_mix_kernel<128, true, GemmArgs>,
           (const void *)gemm_wide_q8_kernel<256, false>, (const void *)gemm_wide_q8_kernel<256, true>,
           (const void *)gemm_wide_q8_kernel<128, false>, (const void *)gemm_wide_q8_kernel<128, true> };
-  const size_t need[8] = { lds256, lds256, lds128, lds128, q256, q256, q128, q128 };
+  const size_t need[8] = { m256, m256, m128, m128, q256, q256, q128, q128 };
   for (int i = 0; i < 8; ++i)
     if (int e = limits[i].raise (kernels[i], need[i]))
       return e;
@@ -1236,8 +1710,9 @@ gemm_wide_launch (const GemmArgs &a, hipStream_t s)
   const int tiles_m = (a.M + bm - 1) / bm;
   const int tiles_n = (a.N + (a.upgate ? 63 : 127)) / (a.upgate ? 64 : 128);
   const WideGrid tiles (tiles_m, tiles_n, a.upgate ? 1 : a.nmat, ksplit, bm == WBM);
-  const dim3 grid ((unsigned)tiles.groups ());
-  const dim3 block ((a.wtype == 8 ? QWAVES : WWAVES) * 64);
+  const WideMix mix (bm, tiles_m, tiles_n, a.upgate ? 1 : a.nmat, ksplit, (double)(a.K / WBK) / ksplit, 0);
+  const dim3 grid ((unsigned)(a.wtype == 8 ? tiles.groups () : mix.groups ()));
+  const dim3 block ((a.wtype == 8 ? QWAVES : MWAVES) * 64);
   // 16-byte accesses to the outputs (and the residual) where their rows allow it
   int vec = (a.ys % 8) == 0 && (!a.residual || ((uintptr_t)a.residual % 16) == 0)
             && (!a.y32 || ((a.N % 4) == 0 && ((uintptr_t)a.y32 % 16) == 0));
@@ -1260,14 +1735,14 @@ gemm_wide_launch (const GemmArgs &a, hipStream_t s)
   else if (bm == 256)
     {
       if (a.upgate)
-        gemm_wide_f16_kernel<256, true><<<grid, block, lds256, s>>> (a, tiles, vec, ksplit, ws);
+        gemm_mix_kernel<256, true, GemmArgs><<<grid, block, m256, s>>> (a, mix, vec, ksplit, ws);
       else
-        gemm_wide_f16_kernel<256, false><<<grid, block, lds256, s>>> (a, tiles, vec, ksplit, ws);
+        gemm_mix_kernel<256, false, GemmArgs><<<grid, block, m256, s>>> (a, mix, vec, ksplit, ws);
     }
   else if (a.upgate)
-    gemm_wide_f16_kernel<128, true><<<grid, block, lds128, s>>> (a, tiles, vec, ksplit, ws);
+    gemm_mix_kernel<128, true, GemmArgs><<<grid, block, m128, s>>> (a, mix, vec, ksplit, ws);
   else
-    gemm_wide_f16_kernel<128, false><<<grid, block, lds128, s>>> (a, tiles, vec, ksplit, ws);
+    gemm_mix_kernel<128, false, GemmArgs><<<grid, block, m128, s>>> (a, mix, vec, ksplit, ws);
   if (ksplit > 1)
     return gemm_reduce_parts (a, ws, ksplit, a.M, s);
   return (int)hipGetLastError ();
@@ -1381,68 +1856,66 @@ wide_reduce_seg_kernel (const GemmSegArgs a, const float *ws, int parts)
 
 // As wide_plan, with every row count allowed and, where the tiles are few, up to 16 parts
 // of at least 4 k-steps: with few token rows the workgroups exist to stream the weights.
-// The model is fitted to the products of this form with weights that no cache holds, 968 of 2
-// to 2048 rows in every plan (microseconds: a round of 256-row tiles 0.67 per k-step + 8.8, of
-// 128-row tiles 0.60 + 5.1, cut tiles likewise; where a segment's sums are parked in LDS 9.6 and
-// 5.6 more per round, which parts leave to the reduction; that launch 3.6 + its bytes at 1.7
-// TB/s).  With the constants of the planes of a 32-bit operand, whose weights come from the L2 two
-// times of three then, it was 2.8 and 54 % slower than the best plan, in the mean and at worst, and
-// divided too little where few tiles stream the weights: 128 x 8064 x 2048 26 us, 28 with GELU, in
-// one part and 22 in two, 160 x 5504 x 2048 23 and 21, 512 x 2048 x 2048 with GELU 28 and 21.
-// Tiles of 64 rows have two workgroups to a compute unit: up to 256 of them take 0.54 per k-step +
-// 2.6, up to 512 0.81 + 3.7.  They win where rows are few or half of a taller tile is empty; us
-// without / with them: 40 x 8064 x 2048 16.3 / 14.5, 128 x 2048 x 7552 21.0 / 18.1, 12 x 16128 x
-// 4096 35.3 / 30.2.  Over 198 products of 2 to 2048 rows the plan is 2.1 % slower than the best in
-// the mean (1.5 up to 128 rows, 2.7 above); without these tiles it was 4.7.  The line at 128 rows
-// is not where they stop to gain: over 140 products of 129 to 2000 rows the plan with them takes
-// 0.95 of the time in the mean up to 256 rows, 0.98 up to 640 and 0.99 above, 0.74 at best (448 x 2048
-// x 2048 21.3 / 15.7 us, 160 x 5504 x 2048 19.0 / 15.9) and 1.03 at worst (448 x 12544 x 4096 56.5 /
-// 58.0), but products of 160 and 512 rows are held to be in parts (tests/test_gemm_f32.py), which
-// 64-row tiles would not be.
-WidePlan
-wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
+// The model is the time of the tiles (WideMix) and that of the reduction, 4.5 us + its bytes at 2.6
+// TB/s.  Tiles of 64 rows have two workgroups to a compute unit: up to 128 rows, up to 256 of them take
+// 0.54 per k-step + 2.6, up to 512 0.81 + 3.7 (fitted to 968 products of 2 to 2048 rows).
+// Where a segment's sums are parked in LDS a tile takes longer (MixTime), which parts leave to the
+// reduction.  With weights that no cache holds the plan is 1.4 % slower than the best one in the mean over
+// 195 products of 130 to 2200 rows, 2.6 % with GELU, 1.7 to 3.2 over 91 of 2 to 128 rows.
+// Beyond 128 rows, 64-row tiles in one part where no sums are parked: us without / with them 512
+// x 2048 x 2048 17.4 / 13.0, 300 x 2048 x 2048 17.7 / 12.9, 300 x 4096 x 512 9.0 / 6.7, 192 x 2048 x 2048 15.1 /
+// 12.8.  With GELU they would gain as much (600 x 2048 x 2048 20.3 / 17.4), and up to 192 rows with more
+// than 128 tiles a tenth (192 x 5504 x 2048 20.3 / 18.8), but a product of either kind is held to be in
+// parts (tests/test_gemm_f32.py), which these tiles are not.
+// (a tile's waves walk 64 parked rows at a time)
+double
+mix_park (const GemmSegArgs &a)
 {
-  struct Fit
-  {
-    double step256, round256, step128, round128, reduce, rate, park256, park128;
-    double one64, first64, two64, round64; // 64-row tiles: one and two workgroups per compute unit
-  };
-  const Fit f = { 0.67, 8.8, 0.60, 5.1, 3.6, 1.7e6, 9.6, 5.6, 0.54, 2.6, 0.81, 3.7 };
-  WidePlan best = { 0, 1 };
-  double best_cost = 0;
-  const int nk = a.K / WBK;
   bool parked = false; // see WideSimple
   for (int i = 0; i < a.nseg; ++i)
     parked = parked || !a.seg[i].vec || a.seg[i].cap > 0.f || (a.seg[i].act != VKL_ACT_NONE && a.seg[i].act != VKL_ACT_RELU2);
+  return parked ? std::min (1.0, a.M / 64.0) : 0;
+}
+
+WidePlan
+wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
+{
+  // 64-row tiles, one and two workgroups per compute unit: one or two rows of them stream the
+  // weights, more share them in the L2; the reduction
+  const bool few = a.M <= 128;
+  const double one64 = few ? 0.54 : 0.42, first64 = few ? 2.6 : 2.7, two64 = few ? 0.81 : 0.9, round64 = few ? 3.7 : 2.7;
+  constexpr double park64 = 3.9, reduce0 = 4.5, rate = 2.6e6;
+  WidePlan best = { 0, 1 };
+  double best_cost = 0;
+  const int nk = a.K / WBK, tiles_n = (a.N + WBN - 1) / WBN;
+  const double parked = mix_park (a);
   for (int bm = 64; bm <= WBM; bm *= 2)
     for (int ks = 1; ks <= 16; ks *= 2)
       {
-        if ((a.M < bm && bm > 128) || (bm == 64 && a.M > 128))
+        const int tiles_m = (a.M + bm - 1) / bm, tiles = tiles_m * tiles_n * ks;
+        if (a.M < bm && bm > 128)
           continue;
+        if (bm == 64 && !few && (ks > 1 || parked > 0 || (a.M <= 192 && tiles > 128)))
+          continue;
+        // (parts that fill the compute units four times gain nothing)
         if (ks > 1
-            && (nk / ks < 4 || (size_t)ks * a.M * a.N * sizeof (float) > scratch))
+            && (nk / ks < 4 || (size_t)ks * a.M * a.N * sizeof (float) > scratch || tiles > 4 * 2 * WideGrid::kUnits))
           continue;
-        const WideGrid tiles ((a.M + bm - 1) / bm, (a.N + WBN - 1) / WBN, 1, ks, bm == WBM);
-        const double steps = (double)nk / ks;
-        const double reduce = ks > 1 ? f.reduce + (double)ks * a.M * a.N * sizeof (float) / f.rate : 0;
-        double cost = reduce;
+        const double steps = (double)nk / ks, park = ks == 1 ? parked : 0;
+        double cost = 0;
         if (bm == 64)
           {
-            const double park = parked && ks == 1 ? std::min (1.0, a.M / 32.0) * f.park128 / 2 : 0;
-            const int two = tiles.tiles () / (2 * WideGrid::kUnits), rest = tiles.tiles () % (2 * WideGrid::kUnits);
-            const double round = f.two64 * steps + f.round64 + park;
-            cost += two * round;
+            const double p = ks == 1 && parked > 0 ? std::min (1.0, a.M / 32.0) * park64 : 0;
+            const int two = tiles / (2 * WideGrid::kUnits), rest = tiles % (2 * WideGrid::kUnits);
+            const double round = two64 * steps + round64 + p;
+            cost = two * round;
             if (rest > 0)
-              cost += rest <= WideGrid::kUnits ? f.one64 * steps + f.first64 + park : round;
+              cost += rest <= WideGrid::kUnits ? one64 * steps + first64 + p : round;
           }
         else
-          {
-            const int whole = (tiles.whole + WideGrid::kUnits - 1) / WideGrid::kUnits;
-            const double park = parked && ks == 1 ? std::min (1.0, a.M / 64.0) : 0; // (a wave walks 64 or 128 rows)
-            const double half = f.step128 * steps + f.round128 + park * f.park128;
-            const double round = bm == WBM ? f.step256 * steps + f.round256 + park * f.park256 : half;
-            cost += whole * round + (tiles.whole < tiles.tiles () ? half : 0);
-          }
+          WideMix (bm, tiles_m, tiles_n, 1, ks, steps, park, &cost);
+        if (ks > 1)
+          cost += reduce0 + (double)ks * a.M * a.N * sizeof (float) / rate;
         if (!best.bm || cost < best_cost)
           best = { bm, ks }, best_cost = cost;
       }
@@ -1450,7 +1923,7 @@ wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
 }
 
 // The tiles of a product of planes: 64 rows in up to 16 parts of the k range (one and two
-// workgroups to a compute unit, as above), or wide_f16_tile's 256 rows, the last of which may be
+// workgroups to a compute unit, as above), or wide_bf16_tile's 256 rows, the last of which may be
 // cut.  Fitted to 160 products of 2 to 2048 rows in 1 to 16 parts and 151 of 192 to 2048 rows in
 // both forms: 0.5 % slower than the best plan in the mean, 7 at worst; without 256 rows 2.5 % and 22
 // (2048 x 8064 x 2048 187 us with them, 229 without; 512 x 16128 x 4096 175, 199).
@@ -1495,13 +1968,34 @@ launch_reduce_seg (const GemmSegArgs &a, int ksplit, const float *ws, hipStream_
   return (int)hipGetLastError ();
 }
 
+// 256 and 128 rows
+template <int BM>
+int
+launch_mix_bf16 (const GemmSegArgs &a, int ksplit, hipStream_t s)
+{
+  static LdsLimit limit;
+  constexpr size_t lds = mix_lds<BM> ();
+  const auto kernel = gemm_mix_kernel<BM, false, GemmSegArgs>;
+  if (int e = limit.raise ((const void *)kernel, lds))
+    return e;
+  StreamScratch own;
+  float *ws = nullptr;
+  if (ksplit > 1 && !(ws = own.take (s)))
+    ksplit = 1;
+  const WideMix tiles (BM, (a.M + BM - 1) / BM, (a.N + WBN - 1) / WBN, 1, ksplit, (double)(a.K / WBK) / ksplit,
+                       ksplit == 1 ? mix_park (a) : 0);
+  kernel<<<dim3 ((unsigned)tiles.groups ()), dim3 (MWAVES * 64), lds, s>>> (a, tiles, 1, ksplit, ws);
+  return launch_reduce_seg<false> (a, ksplit, ws, s);
+}
+
+// 64 rows, and planes in 256
 template <int BM, int PLANES = 1>
 int
 launch_wide_bf16 (const GemmSegArgs &a, int ksplit, hipStream_t s)
 {
   static LdsLimit limit;
-  constexpr size_t lds = wide_lds_f16<BM> ();
-  const auto kernel = gemm_wide_f16_kernel<BM, false, GemmSegArgs, PLANES>;
+  constexpr size_t lds = wide_lds_bf16<BM> ();
+  const auto kernel = gemm_wide_bf16_kernel<BM, PLANES>;
   if (int e = limit.raise ((const void *)kernel, lds))
     return e;
   StreamScratch own;
@@ -1509,7 +2003,7 @@ launch_wide_bf16 (const GemmSegArgs &a, int ksplit, hipStream_t s)
   if (ksplit > 1 && !(ws = own.take (s)))
     ksplit = 1;
   const WideGrid tiles ((a.M + BM - 1) / BM, (a.N + WBN - 1) / WBN, 1, ksplit, BM == WBM);
-  kernel<<<dim3 ((unsigned)tiles.groups ()), dim3 (WWAVES * 64), lds, s>>> (a, tiles, 1, ksplit, ws);
+  kernel<<<dim3 ((unsigned)tiles.groups ()), dim3 (WWAVES * 64), lds, s>>> (a, tiles, ksplit, ws);
   return launch_reduce_seg<false> (a, ksplit, ws, s);
 }
 
@@ -1546,7 +2040,7 @@ launch_wide_planes (const GemmSegArgs &a, int ksplit, float *ws, hipStream_t s)
 // instructions (wide_f32_again; sums of parts of a split k range by seg_f32_again).
 //
 // Planes lie in blocks of 64 columns, [plane 0 | plane 1 | plane 2] of a block next to
-// each other: one k-step of gemm_wide_planes_kernel, three of wide_f16_tile, which walks
+// each other: one k-step of gemm_wide_planes_kernel, three of wide_bf16_tile, which walks
 // them as one row of 3 K values and takes every k-step of the weights three times.
 
 __global__ __launch_bounds__ (256) void
@@ -1591,8 +2085,8 @@ int
 gemm_wide_bf16_launch (const GemmSegArgs &a, hipStream_t s)
 {
   const WidePlan p = wide_plan_bf16 (a, StreamScratch::bytes ());
-  return p.bm == WBM   ? launch_wide_bf16<WBM> (a, p.ksplit, s)
-         : p.bm == 128 ? launch_wide_bf16<128> (a, p.ksplit, s)
+  return p.bm == WBM   ? launch_mix_bf16<WBM> (a, p.ksplit, s)
+         : p.bm == 128 ? launch_mix_bf16<128> (a, p.ksplit, s)
                        : launch_wide_bf16<64> (a, p.ksplit, s);
 }
 

@@ -125,3 +125,76 @@ def test_bf16_segments(dev, M, N, K, act):
     assert bool(((b[:, :n1 - n0] - v[:, n0:n1]).abs() <= off[:, n0:n1] + rounded(v[:, n0:n1], 8)).all())
     want = v[:, n1:] + r
     assert bool(((c - want).abs() <= off[:, n1:] + 2.0 ** -23 * want.abs()).all())
+
+
+class Q8:
+    """A Q8_0 matrix of random quants and scales, in the library's layout and in 64 bits"""
+
+    def __init__(self, dev, seed, n, k):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        q = torch.randint(-127, 128, (n, k // 32, 32), generator=g, device="cuda", dtype=torch.int8)
+        d = (torch.rand((n, k // 32, 1), generator=g, device="cuda") * 0.01 + 0.001).half()
+        raw = torch.cat([d.view(torch.uint8).view(n, k // 32, 2), q.view(torch.uint8)], -1)
+        self.wide = (q.double() * d.double()).view(n, k)
+        self.buf = dev.upload_q8_0(raw.view(n, -1).cpu().numpy(), n, k)
+
+
+# (2049, 8200): 256 pairs of columns, then cut tiles and the odd column; (2300, 8320): the same with more k-steps than
+# stages; (1025, 16390): pairs, then whole tiles of 128 columns; the last two: tiles of 128 rows
+@pytest.mark.parametrize("M,N,K", [(2049, 8200, 64), (2300, 8320, 320), (1025, 16390, 192), (770, 16500, 128), (512, 4096, 256)])
+def test_q8_0(dev, M, N, K):
+    x, w = numbers(1, M, K), Q8(dev, 2, N, K)
+    ys = (N + 7) // 8 * 8 + 8
+    y = torch.full((M, ys), 7.0, device="cuda", dtype=torch.float16)
+    torch.cuda.synchronize()
+    capi.check(capi.lib().vkl_matmul_q8_0(x.data_ptr(), w.buf.ptr, M, N, K, K, ys, 1.0, 0.0, 0, None, y.data_ptr(), None, dev.stream))
+    dev.sync()
+    want, off = sums(x, w.wide)
+    assert bool((y[:, N:] == 7.0).all())
+    assert bool(((y[:, :N] - want).abs() <= off + rounded(want, 11)).all())
+
+
+# with and without what is parked in LDS
+@pytest.mark.parametrize("M,N,K,scale,act,copy", [(2049, 8200, 64, 1.0, 0, False), (2049, 8200, 128, 0.25, 1, False), (1030, 16384, 64, 1.0, 0, True)])
+def test_q8_0_with_a_residual(dev, M, N, K, scale, act, copy):
+    x, w, r = numbers(1, M, K), Q8(dev, 2, N, K), numbers(3, M, N)
+    y, y32 = torch.empty((M, N), device="cuda", dtype=torch.float16), torch.empty((M, N), device="cuda")
+    torch.cuda.synchronize()
+    capi.check(capi.lib().vkl_matmul_q8_0(x.data_ptr(), w.buf.ptr, M, N, K, K, N, scale, 0.0, act, r.data_ptr(), y.data_ptr(),
+                                          y32.data_ptr() if copy else None, dev.stream))
+    dev.sync()
+    v, off = sums(x, w.wide)
+    v, off = v * scale, off * scale + 2.0 ** -22 * v.abs()
+    if act:
+        v = v * torch.sigmoid(v)
+        off = 1.1 * off + 2.0 ** -20 * v.abs()
+    off = off + rounded(v, 11)
+    want = v + r.double()
+    assert bool(((y - want).abs() <= off + rounded(want, 11)).all())
+    assert not copy or torch.equal(y32, y.float())
+
+
+@pytest.mark.parametrize("M,N,K", [(2049, 4104, 64), (1300, 4096, 192)])
+def test_q8_0_three_matrices(dev, M, N, K):
+    x, ws = numbers(1, M, K), [Q8(dev, 2 + i, N, K) for i in range(3)]
+    ys = [torch.empty((M, N), device="cuda", dtype=torch.float16) for _ in range(3)]
+    torch.cuda.synchronize()
+    capi.check(capi.lib().vkl_kqv_q8_0(x.data_ptr(), *[w.buf.ptr for w in ws], M, N, K, *[y.data_ptr() for y in ys], dev.stream))
+    dev.sync()
+    for w, y in zip(ws, ys):
+        want, off = sums(x, w.wide)
+        assert bool(((y - want).abs() <= off + rounded(want, 11)).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(2051, 5504, 192), (2300, 6208, 128), (1030, 8212, 64)])
+def test_q8_0_up_and_gate(dev, M, N, K):
+    x, up, gate = numbers(1, M, K), Q8(dev, 2, N, K), Q8(dev, 3, N, K)
+    y = torch.empty((M, N), device="cuda", dtype=torch.float16)
+    torch.cuda.synchronize()
+    capi.check(capi.lib().vkl_ffn_upgate_q8_0(x.data_ptr(), up.buf.ptr, gate.buf.ptr, M, N, K, y.data_ptr(), dev.stream))
+    dev.sync()
+    (u, uo), (g, go) = sums(x, up.wide), sums(x, gate.wide)
+    s = g * torch.sigmoid(g)
+    want = s * u
+    off = 1.1 * go * u.abs() + s.abs() * uo + go * uo + 2.0 ** -20 * want.abs() + rounded(want, 11)
+    assert bool(((y - want).abs() <= off).all())

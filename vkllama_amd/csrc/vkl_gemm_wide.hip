@@ -840,8 +840,12 @@ struct MixTime
   double step, start, parked; // per k-step; per tile; more where its sums are parked in LDS
 };
 inline MixTime
-mix_time (int bm, int kind)
+mix_time (int bm, int kind, bool q8)
 {
+  // (Q8_0 weights: 256 rows only, and no parked sums to weigh; from the products named at mix_q8_tile)
+  constexpr MixTime tq8[3] = { { 2.20, 10.0, 0 }, { 1.30, 8.0, 0 }, { 0.70, 6.0, 0 } };
+  if (q8)
+    return tq8[kind];
   constexpr MixTime t256[3] = { { 1.42, 5.5, 15.5 }, { 0.76, 6.9, 8.3 }, { 0.54, 5.6, 4.4 } };
   constexpr MixTime t128[3] = { { 0.80, 6.3, 7.6 }, { 0.52, 5.9, 4.6 }, { 0.52, 5.9, 4.6 } };
   return bm == WBM ? t256[kind] : t128[kind];
@@ -921,14 +925,14 @@ struct WideMix
   // bm: token rows of a tile, 256 (which may be cut) or 128; steps: of the k range of a part;
   // park: how much of the time for parked sums a tile takes; us: the time of the launch's tiles
   __host__
-  WideMix (int bm, int tm, int tn, int mats, int parts, double steps, double park, double *us = nullptr)
+  WideMix (int bm, int tm, int tn, int mats, int parts, double steps, double park, double *us = nullptr, bool q8 = false)
       : tiles_m (tm), tiles_n (tn), nmat (mats), ksplit (parts)
   {
     constexpr int U = WideGrid::kUnits;
     double t[3];
     for (int k = 0; k < 3; ++k)
       {
-        const MixTime m = mix_time (bm, k);
+        const MixTime m = mix_time (bm, k, q8);
         t[k] = m.step * steps + m.start + park * m.parked;
       }
     const int options[3] = { 0, pairs () / U * U, pairs () };
@@ -1560,6 +1564,316 @@ wide_q8_tile (const GemmArgs &a, const WidePlace &at, int vec, int ksplit, float
   wide_epilogue_tile<BM, UPGATE, QTM> (a, acc, wide_lds, wave, lane, m0, n0, zmat, vec, part);
 }
 
+// A 256 x 256 tile of Q8_0 weights: eight waves of 128 x 64, three k-steps in LDS, products of
+// 16 x 16 x 32, one for each block of a weight row, scaled in fp32 as above.
+//
+// Bound by the issue of vector instructions: 64 products, 256 scaling FMAs, 80 for the conversion
+// of the weights and 20 more per wave and k-step fill 71 % of the cycles of a SIMD (matrix cores 37 %, LDS
+// 20 %); a tile of 256 x 128 by the waves above spends as much on half of the products' reads.
+// Each fragment of x is replaced by that of the next half step as soon as its four products are
+// issued, so they need one set of registers.  The weight rows are dealt to fragments so that a
+// lane ends with four neighbouring columns (of the fused pair two of up and of gate); the
+// order of LDS is that of the fragments, its swizzle (row / 4) % 4.
+// Same call before / now, us: 4096 x 4096 x 4096 181 / 154, 3967 rows: 13824 x 5120 768 / 668, 5120 x 13824 756 /
+// 660, up/gate 13824 x 5120 1542 / 1325, three of 5120 x 5120 855 / 734; 1500 rows, up/gate 5120 x 5120 210 / 187; 1100 x
+// 11008 x 4096 159 / 136.  Tried: 256 x 32 per wave (half the conversions) 151 for 153 at 4096 x 4096 x 4096,
+// loads and reads dealt among the products 158, conversions of the next half step among them 153 to 162, the
+// same with 256 x 128 tiles 186.
+template <bool UPGATE>
+__device__ __forceinline__ void
+mix_q8_epilogue (const GemmArgs &a, const float4v (&acc)[8][4], uint8_t *wide_lds, int wave, int lane, int mrow, int ncol,
+                 int zmat, int vec, float *part)
+{
+  constexpr int TM = 8, TN = 4, C = UPGATE ? 2 : 4; // columns of a lane
+  const int row = (lane >> 4) * 4, col = (lane & 15) * C;
+  const WideSimple<UPGATE, GemmArgs> simple (a, ncol, 16 * C, zmat, vec, part);
+  if (simple.ok)
+    {
+      auto walk = [&] (auto with) {
+        constexpr bool RES = decltype (with)::value != 0;
+        constexpr int HALF = TM / 2;
+#pragma unroll
+        for (int i0 = 0; i0 < TM; i0 += HALF)
+          {
+            u32x2 res[HALF][4];
+            if (RES)
+#pragma unroll
+              for (int i = 0; i < HALF; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                  res[i][e] = *(const VKL_GLOBAL u32x2 *)(simple.r + (size_t)min (mrow + (i0 + i) * 16 + row + e, a.M - 1) * simple.ys + col);
+#pragma unroll
+            for (int i = 0; i < HALF; ++i)
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                {
+                  const int m = mrow + (i0 + i) * 16 + row + e;
+                  uint16_t h[C];
+#pragma unroll
+                  for (int c = 0; c < C; ++c)
+                    {
+                      const float v = acc[i0 + i][c][e];
+                      h[c] = f2h (UPGATE ? silu (acc[i0 + i][2 + c % 2][e]) * v : v);
+                      if (RES)
+                        h[c] = f2h (h2f (h[c]) + h2f ((uint16_t)(res[i][e][c / 2] >> ((c & 1) * 16))));
+                    }
+                  if (m < a.M)
+                    {
+                      uint16_t *o = simple.y + (size_t)m * simple.ys + col;
+                      if constexpr (UPGATE)
+                        *(VKL_GLOBAL uint32_t *)o = h[0] | ((uint32_t)h[1] << 16);
+                      else
+                        *(VKL_GLOBAL u32x2 *)o = u32x2{ h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16) };
+                    }
+                }
+          }
+      };
+      if (simple.r)
+        walk (WideInt<1> ());
+      else
+        walk (WideInt<0> ());
+      return;
+    }
+  // through LDS, 64 rows of a wave at a time
+  constexpr int PM = 4, ROWS = PM * 16, LD = kWideParkLd;
+  float *park = (float *)(wide_lds + wave * (ROWS * LD * 4));
+  __builtin_amdgcn_s_barrier (); // every wave (that is left) has read its last fragments
+  constexpr int CPR = UPGATE ? 4 : 8, RPI = 64 / CPR; // lanes per row, rows per iteration
+  const int er = lane / CPR, ec = (lane % CPR) * 8;
+  const FinishRows<UPGATE, GemmArgs> fin (a, ncol + ec, zmat, vec, part);
+#pragma unroll
+  for (int i0 = 0; i0 < TM; i0 += PM)
+    {
+#pragma unroll
+      for (int i = 0; i < PM; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int j = 0; j < TN; j += C)
+            {
+              float *dst = park + (i * 16 + row + e) * LD + (j / C) * 32 + col;
+#pragma unroll
+              for (int c = 0; c < C; ++c)
+                dst[c] = acc[i0 + i][j + c][e];
+            }
+      // (a wave reads back only what it wrote itself: no barrier)
+#pragma unroll 1
+      for (int it = 0; it < ROWS / RPI; ++it)
+        {
+          const int r = it * RPI + er, m = mrow + i0 * 16 + r;
+          uint4 res[2];
+          fin.request (m, res);
+          const float *pr = park + r * LD + ec;
+          const float4v p0 = *(const float4v *)pr, p1 = *(const float4v *)(pr + 4);
+          float v[8] = { p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w };
+          float g[8] = { 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f };
+          if (UPGATE)
+            {
+              const float4v g0 = *(const float4v *)(pr + 32), g1 = *(const float4v *)(pr + 36);
+              g[0] = g0.x, g[1] = g0.y, g[2] = g0.z, g[3] = g0.w, g[4] = g1.x, g[5] = g1.y, g[6] = g1.z, g[7] = g1.w;
+            }
+          fin.store (m, v, g, res);
+        }
+    }
+}
+
+constexpr int kMixQ8Cols = 256;
+
+constexpr size_t
+mix_lds_q8 ()
+{
+  constexpr size_t wide = (size_t)QSTAGES * (WBM * WROWB + kMixQ8Cols * (WBK + 4)), park = (size_t)QWAVES * 64 * kWideParkLd * 4;
+  return std::max (std::max (wide, park), wide_lds_q8<WBM> ());
+}
+
+template <bool UPGATE>
+__device__ __forceinline__ void
+mix_q8_tile (const GemmArgs &a, const WidePlace &at, int vec, int ksplit, float *ws)
+{
+  constexpr int BM = WBM, BN = kMixQ8Cols, WN = 4, TM = 8, TN = 4, ST = QSTAGES;
+  constexpr int A_BYTES = BM * WROWB, Q_BYTES = BN * WBK, S_BYTES = BN * 4; // of a stage; laid out by kind
+  constexpr int Q_BASE = ST * A_BYTES, S_BASE = Q_BASE + ST * Q_BYTES;
+  constexpr int AG = BM / 8 / QWAVES, QG = BN / 16 / QWAVES, LOADS = AG + QG + 1; // per wave and k-step
+  extern __shared__ __align__ (16) uint8_t wide_lds[];
+  const int nk_all = a.K / WBK;
+  const int kbase = (int)((long)nk_all * at.ks / ksplit);
+  const int nk = (int)((long)nk_all * (at.ks + 1) / ksplit) - kbase;
+  float *part = ksplit > 1 ? ws + (size_t)at.ks * a.M * a.N : nullptr;
+  const int m0 = at.m0, n0 = at.tn * (UPGATE ? WBN / 2 : WBN);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane (threadIdx.x >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+
+  // load addresses: x as in mix_tile
+  const int lr = lane >> 3, fa = (wave & 1) * 4 + (lane >> 4);
+  const uint8_t *src[LOADS];
+#pragma unroll
+  for (int i = 0; i < AG; ++i)
+    src[i] = (const uint8_t *)(a.x + (size_t)min (m0 + (wave + QWAVES * i) * 8 + lr, a.M - 1) * a.xs + ((lane & 7) ^ fa) * 8
+                               + (size_t)kbase * WBK);
+  // slot s of the tile holds, of wave s / 64, row s % 16 of fragment (s / 16) % 4: columns 4 (s % 16)
+  // + fragment, of the fused pair 2 (s % 16) + fragment % 2 of up (fragments 0, 1) or gate
+  auto weight = [&] (int s, int &n) {
+    const int f = (s >> 4) & 3, r = s & 15;
+    n = min (n0 + (UPGATE ? (s >> 6) * 32 + 2 * r + (f & 1) : (s >> 6) * 64 + 4 * r + f), a.N - 1);
+    return UPGATE ? f >> 1 : at.zmat;
+  };
+  // quants: an instruction covers slots 16 g .. + 15, g = wave + 8 i; lane l fetches chunk (l % 4) ^
+  // (slot / 4) % 4 of slot 16 g + l / 4
+#pragma unroll
+  for (int i = 0; i < QG; ++i)
+    {
+      const int s = (wave + QWAVES * i) * 16 + (lane >> 2);
+      int n;
+      const int mat = weight (s, n);
+      src[AG + i] = pick3 (a.wq[0], a.wq[1], a.wq[2], mat) + (size_t)n * a.Kp + ((lane & 3) ^ ((s >> 2) & 3)) * 16 + (size_t)kbase * WBK;
+    }
+  // scales: the two of a row are one dword; a wave fetches 64 of the 256 rows (two waves the same)
+  {
+    int n;
+    const int mat = weight ((wave & 3) * 64 + lane, n);
+    src[AG + QG] = (const uint8_t *)(pick3 (a.wd[0], a.wd[1], a.wd[2], mat) + (size_t)n * (a.Kp >> 5) + (size_t)kbase * 2);
+  }
+  // fragment reads
+  const int r = lane & 15;
+  uint32_t aoff[2], qoff[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    {
+      aoff[h] = (wm * (BM / 2) + r) * WROWB + (((4 * h + (lane >> 4)) ^ ((r >> 1) & 7)) << 4);
+      qoff[h] = Q_BASE + (wn * 64 + r) * WBK + (((2 * h + (lane >> 5)) ^ ((r >> 2) & 3)) << 4) + ((lane >> 4) & 1) * 8;
+    }
+  const uint32_t soff = S_BASE + (wn * 64 + r) * 4;
+
+  float4v acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      acc[i][j] = float4v{ 0.f, 0.f, 0.f, 0.f };
+
+  auto issue = [&] (int kt, int st) {
+#pragma unroll
+    for (int i = 0; i < AG; ++i)
+      __builtin_amdgcn_global_load_lds ((const VKL_GLOBAL void *)(src[i] + (size_t)kt * WROWB),
+                                        (VKL_LDS void *)(wide_lds + st * A_BYTES + (wave + QWAVES * i) * 1024), 16, 0, 0);
+#pragma unroll
+    for (int i = 0; i < QG; ++i)
+      __builtin_amdgcn_global_load_lds ((const VKL_GLOBAL void *)(src[AG + i] + (size_t)kt * WBK),
+                                        (VKL_LDS void *)(wide_lds + Q_BASE + st * Q_BYTES + (wave + QWAVES * i) * 1024), 16, 0,
+                                        0);
+    __builtin_amdgcn_global_load_lds ((const VKL_GLOBAL void *)(src[AG + QG] + (size_t)kt * 4),
+                                      (VKL_LDS void *)(wide_lds + S_BASE + st * S_BYTES + (wave & 3) * 256), 4, 0, 0);
+  };
+#pragma unroll
+  for (int p = 0; p < ST; ++p)
+    issue (p < nk ? p : nk - 1, p);
+
+  half8 af[TM], bf[TN];
+  u32x2 raw[TN];         // the next weight fragments as they lie
+  uint32_t scales[TN];   // the next k-step's
+  auto read_x = [&] (int st, int h, int i) { af[i] = *(const half8 *)(wide_lds + st * A_BYTES + aoff[h] + i * 16 * WROWB); };
+  auto read_w = [&] (int st, int h) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      raw[j] = *(const u32x2 *)(wide_lds + st * Q_BYTES + qoff[h] + j * 16 * WBK);
+  };
+  auto read_scales = [&] (int st) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      scales[j] = *(const uint32_t *)(wide_lds + st * S_BYTES + soff + j * 16 * 4);
+  };
+  auto convert = [&] {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      bf[j] = q8_frag (raw[j]);
+  };
+  // the products of half a k-step, each scaled behind the second one after it; the fragments of
+  // x become those of half h of the k-step in stage st
+  auto multiply = [&] (const float (&d)[TN], int st, int h) {
+    constexpr int NP = TM * TN, BEHIND = 2;
+    float4v sum[BEHIND + 1];
+#pragma unroll
+    for (int p = 0; p < NP + BEHIND; ++p)
+      {
+        if (p < NP)
+          {
+            sum[p % (BEHIND + 1)] = __builtin_amdgcn_mfma_f32_16x16x32_f16 (af[p / TN], bf[p % TN],
+                                                                            float4v{ 0.f, 0.f, 0.f, 0.f }, 0, 0, 0);
+            if (p % TN == TN - 1)
+              read_x (st, h, p / TN);
+          }
+        if (p >= BEHIND)
+          {
+            const int q = p - BEHIND;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              acc[q / TN][q % TN][e] = __builtin_fmaf (sum[q % (BEHIND + 1)][e], d[q % TN], acc[q / TN][q % TN][e]);
+          }
+      }
+  };
+  // s_waitcnt immediates as in mix_tile
+  constexpr int V0 = (ST - 1) * LOADS, V1 = (ST - 2) * LOADS;
+  constexpr int WAIT0 = 0x0f70 | (V0 & 15) | ((V0 >> 4) << 14), WAIT1 = 0x0070 | (V1 & 15) | ((V1 >> 4) << 14);
+  __builtin_amdgcn_s_waitcnt (WAIT0);
+  __builtin_amdgcn_s_barrier ();
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+    read_x (0, 0, i);
+  read_w (0, 0);
+  read_scales (0);
+  __builtin_amdgcn_sched_barrier (0);
+  // One k-step per turn, as in mix_tile: between its halves tile kt + 1 has landed and the stage of
+  // tile kt, whose last fragments are in registers, takes tile kt + 3.
+  int st = 0;
+  for (int kt = 0; kt < nk; ++kt)
+    {
+      const int s1 = st == ST - 1 ? 0 : st + 1;
+      float d0[TN], d1[TN];
+      convert ();
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        {
+          d0[j] = h2f ((uint16_t)(scales[j] & 0xffff)), d1[j] = h2f ((uint16_t)(scales[j] >> 16));
+          // (keeps the conversion out of the scaling products, see wide_q8_tile)
+          asm volatile ("" : "+v"(d0[j]), "+v"(d1[j]));
+        }
+      read_w (st, 1);
+      multiply (d0, st, 1);
+      __builtin_amdgcn_sched_barrier (0);
+      __builtin_amdgcn_s_waitcnt (WAIT1); // also for the wave's own LDS reads
+      __builtin_amdgcn_s_barrier ();
+      __builtin_amdgcn_sched_barrier (0);
+      issue (kt + ST < nk ? kt + ST : nk - 1, st);
+      convert ();
+      read_w (s1, 0);
+      read_scales (s1);
+      multiply (d1, s1, 0);
+      __builtin_amdgcn_sched_barrier (0);
+      st = s1;
+    }
+  __builtin_amdgcn_s_waitcnt (0x0070); // no load may outlive the workgroup's LDS (nor a fragment read the parked sums)
+  mix_q8_epilogue<UPGATE> (a, acc, wide_lds, wave, lane, m0 + wm * (BM / 2), n0 + wn * (UPGATE ? 32 : 64), at.zmat, vec, part);
+}
+
+template <bool UPGATE>
+__global__ __launch_bounds__ (QWAVES * 64) void
+gemm_mix_q8_kernel (const GemmArgs a, WideMix grid, int vec, int ksplit, float *ws)
+{
+  WidePlace at;
+  switch (grid.place (a.M, WBM, at))
+    {
+    case 1:
+      return mix_q8_tile<UPGATE> (a, at, vec, ksplit, ws);
+    case 2:
+      return wide_q8_tile<WBM, UPGATE> (a, at, vec, ksplit, ws);
+    case 3:
+      return wide_q8_tile<WBM / 2, UPGATE> (a, at, vec, ksplit, ws);
+    }
+}
+
+// no pairs: tiles of 256 (or, the last, 128) rows and 128 columns, or of 128 rows.  (Beside the
+// wide tile the compiler orders the k loop of these less well: 2048 x 4096 x 4096 99 us there, 93 here.)
 template <int BM, bool UPGATE>
 __global__ __launch_bounds__ (QWAVES * 64) void
 gemm_wide_q8_kernel (const GemmArgs a, WideGrid grid, int vec, int ksplit, float *ws)
@@ -1687,15 +2001,17 @@ int
 gemm_wide_launch (const GemmArgs &a, hipStream_t s)
 {
   constexpr size_t m256 = mix_lds<256> (), m128 = mix_lds<128> ();
-  constexpr size_t q256 = wide_lds_q8<256> (), q128 = wide_lds_q8<128> ();
-  static LdsLimit limits[8];
-  const void *const kernels[8]
+  constexpr size_t qmix = mix_lds_q8 (), q256 = wide_lds_q8<256> (), q128 = wide_lds_q8<128> ();
+  constexpr int NK = 10;
+  static LdsLimit limits[NK];
+  const void *const kernels[NK]
       = { (const void *)gemm_mix_kernel<256, false, GemmArgs>, (const void *)gemm_mix_kernel<256, true, GemmArgs>,
           (const void *)gemm_mix_kernel<128, false, GemmArgs>, (const void *)gemm_mix_kernel<128, true, GemmArgs>,
+          (const void *)gemm_mix_q8_kernel<false>, (const void *)gemm_mix_q8_kernel<true>,
           (const void *)gemm_wide_q8_kernel<256, false>, (const void *)gemm_wide_q8_kernel<256, true>,
           (const void *)gemm_wide_q8_kernel<128, false>, (const void *)gemm_wide_q8_kernel<128, true> };
-  const size_t need[8] = { m256, m256, m128, m128, q256, q256, q128, q128 };
-  for (int i = 0; i < 8; ++i)
+  const size_t need[NK] = { m256, m256, m128, m128, qmix, qmix, q256, q256, q128, q128 };
+  for (int i = 0; i < NK; ++i)
     if (int e = limits[i].raise (kernels[i], need[i]))
       return e;
   const WidePlan plan = wide_plan (a);
@@ -1709,23 +2025,32 @@ gemm_wide_launch (const GemmArgs &a, hipStream_t s)
     ksplit = 1;
   const int tiles_m = (a.M + bm - 1) / bm;
   const int tiles_n = (a.N + (a.upgate ? 63 : 127)) / (a.upgate ? 64 : 128);
+  const bool q8 = a.wtype == 8;
   const WideGrid tiles (tiles_m, tiles_n, a.upgate ? 1 : a.nmat, ksplit, bm == WBM);
-  const WideMix mix (bm, tiles_m, tiles_n, a.upgate ? 1 : a.nmat, ksplit, (double)(a.K / WBK) / ksplit, 0);
-  const dim3 grid ((unsigned)(a.wtype == 8 ? tiles.groups () : mix.groups ()));
-  const dim3 block ((a.wtype == 8 ? QWAVES : MWAVES) * 64);
+  const WideMix mix (bm, tiles_m, tiles_n, a.upgate ? 1 : a.nmat, ksplit, (double)(a.K / WBK) / ksplit, 0, nullptr, q8);
+  const bool pairs = !q8 || (bm == WBM && mix.wide > 0);
+  const dim3 grid ((unsigned)(pairs ? mix.groups () : tiles.groups ()));
+  const dim3 block ((q8 ? QWAVES : MWAVES) * 64);
   // 16-byte accesses to the outputs (and the residual) where their rows allow it
   int vec = (a.ys % 8) == 0 && (!a.residual || ((uintptr_t)a.residual % 16) == 0)
             && (!a.y32 || ((a.N % 4) == 0 && ((uintptr_t)a.y32 % 16) == 0));
   for (int t = 0; t < (a.upgate ? 1 : a.nmat); ++t)
     vec = vec && ((uintptr_t)a.y[t] % 16) == 0;
-  if (a.wtype == 8 && bm == 256)
+  if (q8 && pairs)
+    {
+      if (a.upgate)
+        gemm_mix_q8_kernel<true><<<grid, block, qmix, s>>> (a, mix, vec, ksplit, ws);
+      else
+        gemm_mix_q8_kernel<false><<<grid, block, qmix, s>>> (a, mix, vec, ksplit, ws);
+    }
+  else if (q8 && bm == 256)
     {
       if (a.upgate)
         gemm_wide_q8_kernel<256, true><<<grid, block, q256, s>>> (a, tiles, vec, ksplit, ws);
       else
         gemm_wide_q8_kernel<256, false><<<grid, block, q256, s>>> (a, tiles, vec, ksplit, ws);
     }
-  else if (a.wtype == 8)
+  else if (q8)
     {
       if (a.upgate)
         gemm_wide_q8_kernel<128, true><<<grid, block, q128, s>>> (a, tiles, vec, ksplit, ws);

@@ -61,6 +61,32 @@ typedef struct
 int vkl_project_bf16w (const void *x, int xtype, size_t xs, const void *w,
                        int M, int N, int K, const vkl_out_seg *segs, int nseg,
                        void *stream);
+/* What stands between two products of a layer, and the second one: y += x W^T
+ * (x null: nothing is added), h = rms_norm (y) * norm, and the product of h.  The
+ * same as vkl_project_bf16w with the residual y in place, vkl_rmsnorm_f32 and
+ * vkl_project_bf16w, bit for bit, in fewer launches where that is possible.
+ * `type`: of x and h. */
+typedef struct
+{
+  const void *x; /* [M, K], row stride xs */
+  size_t xs;
+  const void *w; /* [W, K] */
+  int K;
+  float *y; /* [M, W], row stride ys */
+  size_t ys;
+  int W;
+  const float *norm; /* [W] */
+  float eps;
+  void *h; /* [M, Wp], row stride hs; columns W .. Wp-1 are set to zero */
+  size_t hs;
+  int Wp;
+  const void *w_next; /* [N, Wp] */
+  int N;
+  const vkl_out_seg *segs;
+  int nseg;
+} vkl_add_norm_project;
+int vkl_add_norm_project_bf16w (const vkl_add_norm_project *p, int type, int M,
+                                void *stream);
 /* out[i, :W] = rms_norm (table[toks[i]]) * w (w null: the plain rows), fp32 rows
  * of stride os; table bf16 [VH, K] of which the first W columns are valid;
  * ids >= VH read row 0.  Columns W .. os-1 are not written. */

@@ -133,6 +133,8 @@ public:
   ~StreamScratch ();
   // the buffer, allocated on first use (null if that fails); at most once per object
   float *take (hipStream_t s);
+  // before the object ends, where the launches that follow take it themselves
+  void give ();
   static size_t bytes ();
   // see vkl_debug_refuse_scratch
   static bool refuse (hipStream_t s);

@@ -1297,10 +1297,17 @@ StreamScratch::refuse (hipStream_t s)
   return true;
 }
 
-StreamScratch::~StreamScratch ()
+void
+StreamScratch::give ()
 {
   if (held_)
     held_->in_use.unlock ();
+  held_ = nullptr;
+}
+
+StreamScratch::~StreamScratch ()
+{
+  give ();
 }
 
 size_t

@@ -18,6 +18,7 @@
 // Tiles of up to 256 x 256 (gemm_mix_kernel) multiply fp16 and bf16; those of 32 x 32
 // products (wide_bf16_tile) are left for 64 rows of bf16 and for 32-bit operands.
 #include "../../include/vkl_stack.h"
+#include "vkl_stack_dev.h"
 #include "vkl_common.h"
 #include "vkl_gemm.h"
 #include <algorithm>
@@ -2078,15 +2079,16 @@ gemm_wide_launch (const GemmArgs &a, hipStream_t s)
 // ---------------------------------------------------------------------------
 namespace
 {
-// wide_f32_again for sums of parts: v the sums of eight columns from n on of row m, in every
+// wide_f32_again for sums of parts: v the sums of E columns from n on of row m, in every
 // lane of a wave others.  The wave forms the sums of a lane that has one that is not finite
 // together, 512 values of k at a time.
+template <int E>
 __device__ __forceinline__ void
-seg_f32_again (const GemmSegArgs &a, float (&v)[8], int m, int n, int lane, int K)
+seg_f32_again (const GemmSegArgs &a, float (&v)[E], int m, int n, int lane, int K)
 {
   float t = 0.f;
 #pragma unroll
-  for (int e = 0; e < 8; ++e)
+  for (int e = 0; e < E; ++e)
     t = __builtin_fmaf (v[e], 0.f, t);
   uint64_t bad = __builtin_amdgcn_ballot_w64 (t != 0.f);
 #pragma unroll 1
@@ -2096,14 +2098,17 @@ seg_f32_again (const GemmSegArgs &a, float (&v)[8], int m, int n, int lane, int 
       bad &= bad - 1;
       const float *x = a.xf + (size_t)__builtin_amdgcn_readlane (m, who) * a.xs;
       const int n0 = __builtin_amdgcn_readlane (n, who);
-      float sum[8] = { 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f };
+      float sum[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        sum[e] = 0.f;
 #pragma unroll 1
       for (int k = lane * 8; k < K; k += 64 * 8)
         {
           const uint4 x0 = ldg4 (x + k), x1 = ldg4 (x + k + 4);
           const uint32_t xw[8] = { x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w };
 #pragma unroll
-          for (int e = 0; e < 8; ++e)
+          for (int e = 0; e < E; ++e)
             {
               const uint4 w0 = ldg4 (a.wh[0] + (size_t)min (n0 + e, a.N - 1) * a.ws + k);
               const uint32_t ww[4] = { w0.x, w0.y, w0.z, w0.w };
@@ -2113,7 +2118,7 @@ seg_f32_again (const GemmSegArgs &a, float (&v)[8], int m, int n, int lane, int 
             }
         }
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
+      for (int e = 0; e < E; ++e)
         {
 #pragma unroll
           for (int d = 32; d > 0; d >>= 1)
@@ -2281,6 +2286,60 @@ wide_plan_planes (const GemmSegArgs &a, size_t scratch)
   return best;
 }
 
+// ws: scratch for the parts of the k range, whose sums the caller adds
+template <int BM>
+int
+launch_mix_parts (const GemmSegArgs &a, int ksplit, float *ws, hipStream_t s)
+{
+  static LdsLimit limit;
+  constexpr size_t lds = mix_lds<BM> ();
+  const auto kernel = gemm_mix_kernel<BM, false, GemmSegArgs>;
+  if (int e = limit.raise ((const void *)kernel, lds))
+    return e;
+  const WideMix tiles (BM, (a.M + BM - 1) / BM, (a.N + WBN - 1) / WBN, 1, ksplit, (double)(a.K / WBK) / ksplit,
+                       ksplit == 1 ? mix_park (a) : 0);
+  kernel<<<dim3 ((unsigned)tiles.groups ()), dim3 (MWAVES * 64), lds, s>>> (a, tiles, 1, ksplit, ws);
+  return (int)hipGetLastError ();
+}
+
+template <int BM, int PLANES = 1>
+int
+launch_wide_parts (const GemmSegArgs &a, int ksplit, float *ws, hipStream_t s)
+{
+  static LdsLimit limit;
+  constexpr size_t lds = wide_lds_bf16<BM> ();
+  const auto kernel = gemm_wide_bf16_kernel<BM, PLANES>;
+  if (int e = limit.raise ((const void *)kernel, lds))
+    return e;
+  const WideGrid tiles ((a.M + BM - 1) / BM, (a.N + WBN - 1) / WBN, 1, ksplit, BM == WBM);
+  kernel<<<dim3 ((unsigned)tiles.groups ()), dim3 (WWAVES * 64), lds, s>>> (a, tiles, ksplit, ws);
+  return (int)hipGetLastError ();
+}
+
+// the tiles of a bf16 product
+int
+launch_bf16_tiles (const GemmSegArgs &a, const WidePlan &p, float *ws, hipStream_t s)
+{
+  return p.bm == WBM   ? launch_mix_parts<WBM> (a, p.ksplit, ws, s)
+         : p.bm == 128 ? launch_mix_parts<128> (a, p.ksplit, ws, s)
+                       : launch_wide_parts<64> (a, p.ksplit, ws, s);
+}
+
+// the tiles of a product of planes
+int
+launch_planes_tiles (const GemmSegArgs &a, const WidePlan &p, float *ws, hipStream_t s)
+{
+  if (p.bm == WBM)
+    return launch_wide_parts<WBM, kPlanes> (a, 1, nullptr, s);
+  static LdsLimit limit;
+  constexpr size_t lds = wide_lds_planes ();
+  if (int e = limit.raise ((const void *)gemm_wide_planes_kernel, lds))
+    return e;
+  const WideGrid tiles ((a.M + kPlaneRows - 1) / kPlaneRows, (a.N + WBN - 1) / WBN, 1, p.ksplit, false);
+  gemm_wide_planes_kernel<<<dim3 ((unsigned)tiles.groups ()), dim3 (WWAVES * 64), lds, s>>> (a, tiles, p.ksplit, ws);
+  return (int)hipGetLastError ();
+}
+
 template <bool PLANES>
 int
 launch_reduce_seg (const GemmSegArgs &a, int ksplit, const float *ws, hipStream_t s)
@@ -2293,56 +2352,14 @@ launch_reduce_seg (const GemmSegArgs &a, int ksplit, const float *ws, hipStream_
   return (int)hipGetLastError ();
 }
 
-// 256 and 128 rows
-template <int BM>
+// a product of planes and, if it is in parts, their sum; ws: scratch for the parts
 int
-launch_mix_bf16 (const GemmSegArgs &a, int ksplit, hipStream_t s)
+launch_planes (const GemmSegArgs &a, size_t bytes, float *ws, hipStream_t s)
 {
-  static LdsLimit limit;
-  constexpr size_t lds = mix_lds<BM> ();
-  const auto kernel = gemm_mix_kernel<BM, false, GemmSegArgs>;
-  if (int e = limit.raise ((const void *)kernel, lds))
+  const WidePlan p = wide_plan_planes (a, bytes);
+  if (int e = launch_planes_tiles (a, p, ws, s))
     return e;
-  StreamScratch own;
-  float *ws = nullptr;
-  if (ksplit > 1 && !(ws = own.take (s)))
-    ksplit = 1;
-  const WideMix tiles (BM, (a.M + BM - 1) / BM, (a.N + WBN - 1) / WBN, 1, ksplit, (double)(a.K / WBK) / ksplit,
-                       ksplit == 1 ? mix_park (a) : 0);
-  kernel<<<dim3 ((unsigned)tiles.groups ()), dim3 (MWAVES * 64), lds, s>>> (a, tiles, 1, ksplit, ws);
-  return launch_reduce_seg<false> (a, ksplit, ws, s);
-}
-
-// 64 rows, and planes in 256
-template <int BM, int PLANES = 1>
-int
-launch_wide_bf16 (const GemmSegArgs &a, int ksplit, hipStream_t s)
-{
-  static LdsLimit limit;
-  constexpr size_t lds = wide_lds_bf16<BM> ();
-  const auto kernel = gemm_wide_bf16_kernel<BM, PLANES>;
-  if (int e = limit.raise ((const void *)kernel, lds))
-    return e;
-  StreamScratch own;
-  float *ws = nullptr;
-  if (ksplit > 1 && !(ws = own.take (s)))
-    ksplit = 1;
-  const WideGrid tiles ((a.M + BM - 1) / BM, (a.N + WBN - 1) / WBN, 1, ksplit, BM == WBM);
-  kernel<<<dim3 ((unsigned)tiles.groups ()), dim3 (WWAVES * 64), lds, s>>> (a, tiles, ksplit, ws);
-  return launch_reduce_seg<false> (a, ksplit, ws, s);
-}
-
-// ws: scratch for the parts of the k range
-int
-launch_wide_planes (const GemmSegArgs &a, int ksplit, float *ws, hipStream_t s)
-{
-  static LdsLimit limit;
-  constexpr size_t lds = wide_lds_planes ();
-  if (int e = limit.raise ((const void *)gemm_wide_planes_kernel, lds))
-    return e;
-  const WideGrid tiles ((a.M + kPlaneRows - 1) / kPlaneRows, (a.N + WBN - 1) / WBN, 1, ksplit, false);
-  gemm_wide_planes_kernel<<<dim3 ((unsigned)tiles.groups ()), dim3 (WWAVES * 64), lds, s>>> (a, tiles, ksplit, ws);
-  return launch_reduce_seg<true> (a, ksplit, ws, s);
+  return launch_reduce_seg<true> (a, p.ksplit, ws, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -2368,6 +2385,22 @@ launch_wide_planes (const GemmSegArgs &a, int ksplit, float *ws, hipStream_t s)
 // each other: one k-step of gemm_wide_planes_kernel, three of wide_bf16_tile, which walks
 // them as one row of 3 K values and takes every k-step of the weights three times.
 
+// the planes of one value
+__device__ __forceinline__ void
+split_value (uint32_t in, uint32_t (&p)[kPlanes])
+{
+  // truncation: no plane overflows, and each remainder is exact.  Infinities and
+  // NaN go into the first plane alone.  A last remainder (of the smallest values)
+  // marks the third.
+  const bool finite = (in & 0x7f800000u) != 0x7f800000u;
+  const float v = __uint_as_float (in);
+  p[0] = finite ? in >> 16 : (uint32_t)f2bf (v);
+  const float r = finite ? v - __uint_as_float (in & 0xffff0000u) : 0.f;
+  p[1] = __float_as_uint (r) >> 16;
+  const uint32_t last = __float_as_uint (r - __uint_as_float (__float_as_uint (r) & 0xffff0000u));
+  p[2] = (last & 0xffffu) ? 0x7fc0u : last >> 16;
+}
+
 __global__ __launch_bounds__ (256) void
 split_planes_kernel (const float *x, size_t xs, int M, int K, uint16_t *out)
 {
@@ -2383,16 +2416,11 @@ split_planes_kernel (const float *x, size_t xs, int M, int K, uint16_t *out)
 #pragma unroll
   for (int e = 0; e < 8; ++e)
     {
-      // truncation: no plane overflows, and each remainder is exact.  Infinities and
-      // NaN go into the first plane alone.  A last remainder (of the smallest values)
-      // marks the third.
-      const bool finite = (in[e] & 0x7f800000u) != 0x7f800000u;
-      const float v = __uint_as_float (in[e]);
-      p[0][e] = finite ? in[e] >> 16 : (uint32_t)f2bf (v);
-      const float r = finite ? v - __uint_as_float (in[e] & 0xffff0000u) : 0.f;
-      p[1][e] = __float_as_uint (r) >> 16;
-      const uint32_t last = __float_as_uint (r - __uint_as_float (__float_as_uint (r) & 0xffff0000u));
-      p[2][e] = (last & 0xffffu) ? 0x7fc0u : last >> 16;
+      uint32_t one[kPlanes];
+      split_value (in[e], one);
+#pragma unroll
+      for (int q = 0; q < kPlanes; ++q)
+        p[q][e] = one[q];
     }
   uint16_t *dst = out + (size_t)m * kPlanes * K + (size_t)(c / WBK) * kPlanes * WBK + c % WBK;
 #pragma unroll
@@ -2409,14 +2437,21 @@ split_planes_kernel (const float *x, size_t xs, int M, int K, uint16_t *out)
 int
 gemm_wide_bf16_launch (const GemmSegArgs &a, hipStream_t s)
 {
-  const WidePlan p = wide_plan_bf16 (a, StreamScratch::bytes ());
-  return p.bm == WBM   ? launch_mix_bf16<WBM> (a, p.ksplit, s)
-         : p.bm == 128 ? launch_mix_bf16<128> (a, p.ksplit, s)
-                       : launch_wide_bf16<64> (a, p.ksplit, s);
+  WidePlan p = wide_plan_bf16 (a, StreamScratch::bytes ());
+  StreamScratch own;
+  float *ws = nullptr;
+  if (p.ksplit > 1 && !(ws = own.take (s)))
+    p.ksplit = 1;
+  if (int e = launch_bf16_tiles (a, p, ws, s))
+    return e;
+  return launch_reduce_seg<false> (a, p.ksplit, ws, s);
 }
 
+namespace
+{
+// whether the 32-bit instructions would take longer than planes
 bool
-gemm_wide_f32_launch (const GemmSegArgs &a, hipStream_t s, int &err)
+planes_pay (const GemmSegArgs &a)
 {
   // Short rows of few values are over in the time of two more launches.  Measured, us,
   // 32-bit instructions / planes: K = 256, N = 2048, 300 rows 10 / 16, 4000 rows 48 / 36;
@@ -2432,21 +2467,54 @@ gemm_wide_f32_launch (const GemmSegArgs &a, hipStream_t s, int &err)
   // 23.4, 896 24.3 / 24.2, 256 x 4096, K = 768 21.4 / 25.2; fewer outputs, 130 x 2048, K = 640
   // 18.1 / 15.1).
   const size_t outputs = (size_t)a.M * a.N, tiles = (size_t)((a.M + 63) / 64) * ((a.N + 63) / 64);
-  if (tiles <= 256 && ((a.K <= 640 && outputs >= 600000) || (a.K <= 768 && outputs >= 800000)))
-    return false;
-  // nothing is allocated while the stream is captured
+  return !(tiles <= 256 && ((a.K <= 640 && outputs >= 600000) || (a.K <= 768 && outputs >= 800000)));
+}
+
+// nothing is allocated while the stream is captured
+bool
+capturing (hipStream_t s)
+{
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing (s, &capture) != hipSuccess)
     {
       (void)hipGetLastError (); // (the default stream while another one is captured)
-      return false;
+      return true;
     }
-  if (capture != hipStreamCaptureStatusNone)
+  return capture != hipStreamCaptureStatusNone;
+}
+
+// rows whose planes half of the scratch holds
+size_t
+plane_rows (int K)
+{
+  return StreamScratch::bytes () / 2 / ((size_t)kPlanes * K * sizeof (uint16_t));
+}
+
+void
+launch_split (const float *x, size_t xs, int M, int K, float *ws, hipStream_t s)
+{
+  const size_t total = (size_t)M * (K / 8);
+  split_planes_kernel<<<dim3 ((unsigned)((total + 255) / 256)), dim3 (256), 0, s>>> (x, xs, M, K, (uint16_t *)ws);
+}
+
+// a with the planes of its x in ws
+GemmSegArgs
+with_planes (const GemmSegArgs &a, float *ws)
+{
+  GemmSegArgs b = a;
+  b.x = (const uint16_t *)ws, b.K = kPlanes * a.K;
+  return b;
+}
+} // namespace
+
+bool
+gemm_wide_f32_launch (const GemmSegArgs &a, hipStream_t s, int &err)
+{
+  if (!planes_pay (a) || capturing (s))
     return false;
   // the planes of as many rows as half of the scratch holds at a time, the parts of
   // a split k range behind them
-  const size_t row = (size_t)kPlanes * a.K * sizeof (uint16_t), half = StreamScratch::bytes () / 2;
-  const size_t most = half / row;
+  const size_t half = StreamScratch::bytes () / 2, most = plane_rows (a.K);
   const int rows = most >= (size_t)a.M ? a.M : (int)(most / WBM * WBM);
   StreamScratch own;
   float *ws = rows > 0 ? own.take (s) : nullptr;
@@ -2454,37 +2522,209 @@ gemm_wide_f32_launch (const GemmSegArgs &a, hipStream_t s, int &err)
     return false;
   for (int m0 = 0; m0 < a.M; m0 += rows)
     {
-      GemmSegArgs b = a;
+      GemmSegArgs b = with_planes (a, ws);
       b.M = a.M - m0 < rows ? a.M - m0 : rows, b.xf = a.xf + (size_t)m0 * a.xs;
-      const size_t total = (size_t)b.M * (a.K / 8);
-      split_planes_kernel<<<dim3 ((unsigned)((total + 255) / 256)), dim3 (256), 0, s>>> (b.xf, a.xs, b.M, a.K,
-                                                                                         (uint16_t *)ws);
-      b.x = (const uint16_t *)ws;
-      b.K = kPlanes * a.K;
+      launch_split (b.xf, a.xs, b.M, a.K, ws, s);
       for (int i = 0; i < a.nseg; ++i)
         {
           b.seg[i].y = (char *)a.seg[i].y + (size_t)m0 * a.seg[i].ys * (a.seg[i].f32 ? 4 : 2);
           if (a.seg[i].residual)
             b.seg[i].residual = a.seg[i].residual + (size_t)m0 * a.seg[i].ys;
         }
-      const WidePlan p = wide_plan_planes (b, half);
-      err = p.bm == WBM ? launch_wide_bf16<WBM, kPlanes> (b, 1, s)
-                        : launch_wide_planes (b, p.ksplit, ws + half / sizeof (float), s);
-      if (err)
+      if ((err = launch_planes (b, half, ws + half / sizeof (float), s)))
         return true;
     }
   return true;
 }
-} // namespace vkl
 
-extern "C" int
-vkl_project_bf16w (const void *x, int xtype, size_t xs, const void *w, int M, int N, int K,
-                   const vkl_out_seg *segs, int nseg, void *stream)
+// ---------------------------------------------------------------------------
+// between two products: the sum into the residual rows and its norm
+// ---------------------------------------------------------------------------
+// A launch costs 4.5 to 5 us behind another one whatever it does, so one does what three did:
+// it adds the parts of a product and the residual row (wide_reduce_seg_kernel), norms the row
+// (rmsnorm_f32_kernel) and, in 32 bits, writes the planes that the next product reads
+// (split_planes_kernel).  A workgroup has one row in registers; the sums and the norm are formed in
+// the order of those kernels, bit for bit.  us before / now: 300 rows of 2048 in four parts 15.4 / 6.1,
+// in bf16 (1500 rows, two parts) 15.0 / 11.2.
+namespace
+{
+struct RowNorm
+{
+  const float *w;
+  float eps;
+  int Wp; // values of a row of h, zeros beyond N
+  void *h;
+  size_t hs;
+  int f32;
+  uint16_t *planes; // optional: rows of 3 Wp
+};
+
+// NV: float4 of a row per thread.  a: the product, one segment; parts 0: its sum stands in y.
+template <int NV, bool PLANES>
+__global__ __launch_bounds__ (256) void
+sum_norm_kernel (const GemmSegArgs a, const float *ws, int parts, const RowNorm r)
+{
+  __shared__ float red[4];
+  const int m = blockIdx.x, tid = threadIdx.x;
+  float *y = (float *)a.seg[0].y + (size_t)m * a.seg[0].ys;
+  const size_t at = (size_t)m * a.N, part = (size_t)a.M * a.N;
+  float v[NV][4];
+  float ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < NV; ++j)
+    {
+      // (N is a multiple of 4: a load is all inside or all padding)
+      const int c = (tid + j * 256) * 4, cc = min (c, a.N - 4);
+      const float4v res = __builtin_bit_cast (float4v, ldg4 (y + cc));
+      if (parts > 0)
+        {
+          float t[4] = { 0.f, 0.f, 0.f, 0.f };
+          for (int p0 = 0; p0 < parts; p0 += 4)
+            {
+              float4v x[4];
+#pragma unroll
+              for (int p = 0; p < 4; ++p)
+                x[p] = __builtin_bit_cast (float4v, ldg4 (ws + (size_t)min (p0 + p, parts - 1) * part + at + cc));
+#pragma unroll
+              for (int p = 0; p < 4; ++p)
+                if (p0 + p < parts)
+#pragma unroll
+                  for (int e = 0; e < 4; ++e)
+                    t[e] += x[p][e];
+            }
+          if (PLANES)
+            seg_f32_again<4> (a, t, m, cc, tid & 63, a.K / kPlanes);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            v[j][e] = t[e] + res[e];
+          if (c < a.N)
+            *(VKL_GLOBAL float4v *)(y + c) = float4v{ v[j][0], v[j][1], v[j][2], v[j][3] };
+        }
+      else
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          v[j][e] = res[e];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        {
+          v[j][e] = c < a.N ? v[j][e] : 0.f;
+          ss = __builtin_fmaf (v[j][e], v[j][e], ss);
+        }
+    }
+  const float alpha = 1.0f / sqrtf (group_sum (ss, red) / (float)a.N + r.eps);
+#pragma unroll
+  for (int j = 0; j < NV; ++j)
+    {
+      const int c = (tid + j * 256) * 4;
+      if (c >= r.Wp)
+        continue;
+      const float4v w = __builtin_bit_cast (float4v, ldg4 (r.w + min (c, a.N - 4)));
+      float o[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        o[e] = v[j][e] * alpha * w[e];
+      const size_t to = (size_t)m * r.hs + c;
+      if (r.f32)
+        *(VKL_GLOBAL float4v *)((float *)r.h + to) = float4v{ o[0], o[1], o[2], o[3] };
+      else
+        stg ((unsigned long long *)((uint16_t *)r.h + to),
+             (unsigned long long)f2bf (o[0]) | ((unsigned long long)f2bf (o[1]) << 16)
+                 | ((unsigned long long)f2bf (o[2]) << 32) | ((unsigned long long)f2bf (o[3]) << 48));
+      if (r.planes)
+        {
+          uint32_t p[4][kPlanes];
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            split_value (__float_as_uint (o[e]), p[e]);
+          uint16_t *dst = r.planes + (size_t)m * kPlanes * r.Wp + (size_t)(c / WBK) * kPlanes * WBK + c % WBK;
+#pragma unroll
+          for (int q = 0; q < kPlanes; ++q)
+            stg ((unsigned long long *)(dst + q * WBK),
+                 (unsigned long long)(p[0][q] | (p[1][q] << 16)) | ((unsigned long long)(p[2][q] | (p[3][q] << 16)) << 32));
+        }
+    }
+}
+
+template <bool PLANES>
+int
+launch_sum_norm (const GemmSegArgs &a, const float *ws, int parts, const RowNorm &r, hipStream_t s)
+{
+  const dim3 grid ((unsigned)a.M), block (256);
+  if (r.Wp <= 1024)
+    sum_norm_kernel<1, PLANES><<<grid, block, 0, s>>> (a, ws, parts, r);
+  else if (r.Wp <= 2048)
+    sum_norm_kernel<2, PLANES><<<grid, block, 0, s>>> (a, ws, parts, r);
+  else if (r.Wp <= 4096)
+    sum_norm_kernel<4, PLANES><<<grid, block, 0, s>>> (a, ws, parts, r);
+  else
+    sum_norm_kernel<8, PLANES><<<grid, block, 0, s>>> (a, ws, parts, r);
+  return (int)hipGetLastError ();
+}
+
+constexpr int kSumNormWidth = 8192;
+
+// y += x W^T (add null: nothing is added), h = norm (y), the product of h; the arguments are
+// checked.  False where no launch would be saved (nothing has been launched then).
+bool
+add_norm_project (const GemmSegArgs *add, const GemmSegArgs &rows, RowNorm r, const GemmSegArgs &next, hipStream_t s, int &err)
+{
+  const GemmSegArgs &y = add ? *add : rows;
+  if (r.Wp > kSumNormWidth || (y.N % 8) != 0 || (y.seg[0].ys % 4) != 0 || (r.hs % 4) != 0 || ((uintptr_t)y.seg[0].y % 16) != 0
+      || ((uintptr_t)r.w % 16) != 0 || ((uintptr_t)r.h % 16) != 0 || capturing (s))
+    return false;
+  StreamScratch own;
+  if (!r.f32)
+    {
+      // only parts are added here: a sum without parts is formed by the tiles
+      const WidePlan p = add ? wide_plan_bf16 (*add, StreamScratch::bytes ()) : WidePlan{ 0, 1 };
+      float *ws = p.ksplit > 1 ? own.take (s) : nullptr;
+      if (!ws)
+        return false;
+      if ((err = launch_bf16_tiles (*add, p, ws, s)))
+        return true;
+      err = launch_sum_norm<false> (*add, ws, p.ksplit, r, s);
+      own.give ();
+      if (!err)
+        err = gemm_wide_bf16_launch (next, s);
+      return true;
+    }
+  // planes of all rows at once, of both products or the next one
+  const bool first = add && planes_pay (*add) && plane_rows (add->K) >= (size_t)add->M;
+  if ((add && !first) || !planes_pay (next) || plane_rows (next.K) < (size_t)next.M)
+    return false;
+  float *ws = own.take (s);
+  if (!ws)
+    return false;
+  const size_t half = StreamScratch::bytes () / 2;
+  float *parts = ws + half / sizeof (float);
+  r.planes = (uint16_t *)ws; // (those of the first product have been read by then)
+  int n = 0;
+  if (add)
+    {
+      launch_split (add->xf, add->xs, add->M, add->K, ws, s);
+      const GemmSegArgs b = with_planes (*add, ws);
+      const WidePlan p = wide_plan_planes (b, half);
+      if ((err = launch_planes_tiles (b, p, parts, s)))
+        return true;
+      n = p.ksplit > 1 ? p.ksplit : 0;
+      err = launch_sum_norm<true> (b, parts, n, r, s);
+    }
+  else
+    err = launch_sum_norm<false> (rows, nullptr, 0, r, s);
+  if (!err)
+    err = launch_planes (with_planes (next, ws), half, parts, s);
+  return true;
+}
+
+// the arguments of a product, checked
+int
+seg_args (const void *x, int xtype, size_t xs, const void *w, int M, int N, int K, const vkl_out_seg *segs, int nseg,
+          GemmSegArgs &a)
 {
   VKL_CHECK_ARG (x && w && segs && M > 0 && N > 0 && K > 0 && (K % 64) == 0 && xs >= (size_t)K);
-  VKL_CHECK_ARG (nseg > 0 && nseg <= vkl::kGemmSegs && (xtype == VKL_TYPE_F32 || xtype == VKL_TYPE_BF16));
+  VKL_CHECK_ARG (nseg > 0 && nseg <= kGemmSegs && (xtype == VKL_TYPE_F32 || xtype == VKL_TYPE_BF16));
   VKL_CHECK_ARG ((xs % 8) == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0);
-  vkl::GemmSegArgs a = {};
+  a = {};
   if (xtype == VKL_TYPE_F32)
     a.xf = (const float *)x;
   else
@@ -2501,12 +2741,54 @@ vkl_project_bf16w (const void *x, int xtype, size_t xs, const void *w, int M, in
       VKL_CHECK_ARG (i > 0 || o.n0 == 0);
       VKL_CHECK_ARG (o.act >= VKL_ACT_NONE && o.act <= VKL_ACT_GELU);
       VKL_CHECK_ARG (o.type == VKL_TYPE_F32 || (o.type == VKL_TYPE_BF16 && !o.residual));
-      vkl::GemmSeg &g = a.seg[i];
+      GemmSeg &g = a.seg[i];
       g.n0 = o.n0, g.n = o.n, g.y = o.y, g.ys = o.ys, g.f32 = o.type == VKL_TYPE_F32;
       g.act = o.act, g.residual = o.residual, g.cap = o.cap;
       g.vec = (o.ys % 8) == 0 && ((uintptr_t)o.y % 16) == 0 && (!o.residual || ((uintptr_t)o.residual % 16) == 0);
       end = o.n0 + o.n;
     }
-  return xtype == VKL_TYPE_F32 ? vkl::gemm_f32_launch (a, (hipStream_t)stream)
-                               : vkl::gemm_wide_bf16_launch (a, (hipStream_t)stream);
+  return 0;
+}
+
+int
+project (const GemmSegArgs &a, hipStream_t s)
+{
+  return a.xf ? gemm_f32_launch (a, s) : gemm_wide_bf16_launch (a, s);
+}
+} // namespace
+} // namespace vkl
+
+extern "C" int
+vkl_project_bf16w (const void *x, int xtype, size_t xs, const void *w, int M, int N, int K,
+                   const vkl_out_seg *segs, int nseg, void *stream)
+{
+  vkl::GemmSegArgs a;
+  if (int e = vkl::seg_args (x, xtype, xs, w, M, N, K, segs, nseg, a))
+    return e;
+  return vkl::project (a, (hipStream_t)stream);
+}
+
+extern "C" int
+vkl_add_norm_project_bf16w (const vkl_add_norm_project *p, int type, int M, void *stream)
+{
+  VKL_CHECK_ARG (p && p->y && p->norm && p->h && p->W > 0 && p->Wp >= p->W && p->ys >= (size_t)p->W && p->hs >= (size_t)p->Wp);
+  const vkl_out_seg back = { 0, p->W, p->y, p->ys, VKL_TYPE_F32, VKL_ACT_NONE, p->y, 0.f };
+  vkl::GemmSegArgs add = {}, rows = {}, next;
+  if (p->x)
+    if (int e = vkl::seg_args (p->x, type, p->xs, p->w, M, p->W, p->K, &back, 1, add))
+      return e;
+  if (int e = vkl::seg_args (p->h, type, p->hs, p->w_next, M, p->N, p->Wp, p->segs, p->nseg, next))
+    return e;
+  rows.M = M, rows.N = p->W, rows.seg[0].y = p->y, rows.seg[0].ys = p->ys;
+  const vkl::RowNorm r = { p->norm, p->eps, p->Wp, p->h, p->hs, type == VKL_TYPE_F32, nullptr };
+  hipStream_t s = (hipStream_t)stream;
+  int err = 0;
+  if (vkl::add_norm_project (p->x ? &add : nullptr, rows, r, next, s, err))
+    return err;
+  if (p->x)
+    if (int e = vkl::project (add, s))
+      return e;
+  if (int e = vkl_rmsnorm_f32 (p->y, p->ys, nullptr, M, p->W, p->norm, p->eps, p->h, type, p->hs, p->Wp, stream))
+    return e;
+  return vkl::project (next, s);
 }

@@ -53,24 +53,31 @@ StackBlock::norm_weights_ (const WeightSource &w, const std::string &name)
 }
 
 absl::Status
-StackBlock::norm_input_ (Tensor &x, int S, Tensor &w, Buffers &b)
+StackBlock::norm_product_ (const char *what, Tensor &x, int S, Tensor &norm, Tensor &w, int n,
+                           std::vector<vkl_out_seg> const &segs, Buffers &b)
 {
-  const int type = dtype_ == FP32 ? VKL_TYPE_F32 : VKL_TYPE_BF16;
-  return launched ("layer norm",
-                   vkl_rmsnorm_f32 ((const float *)x.data (), (size_t)width_p_, nullptr, S, width_,
-                                    (const float *)w.data (), eps_, b.h.data (), type, (size_t)width_p_, width_p_,
-                                    dev_->stream ()));
+  vkl_add_norm_project p = {};
+  if (b.back)
+    p.x = b.cat.data (), p.xs = (size_t)b.cat_stride, p.w = b.back->data (), p.K = b.back_k;
+  b.back = nullptr;
+  p.y = (float *)x.data (), p.ys = (size_t)width_p_, p.W = width_;
+  p.norm = (const float *)norm.data (), p.eps = eps_, p.h = b.h.data (), p.hs = (size_t)width_p_, p.Wp = width_p_;
+  p.w_next = w.data (), p.N = n, p.segs = segs.data (), p.nseg = (int)segs.size ();
+  return launched (what, vkl_add_norm_project_bf16w (&p, dtype_ == FP32 ? VKL_TYPE_F32 : VKL_TYPE_BF16, S, dev_->stream ()));
 }
 
 absl::Status
-StackBlock::add_product_ (Tensor &x, int S, Tensor &w, int k, Buffers &b)
+StackBlock::finish (Tensor &x, int S, Buffers &b)
 {
+  if (!b.back)
+    return absl::OkStatus ();
   const int type = dtype_ == FP32 ? VKL_TYPE_F32 : VKL_TYPE_BF16;
   float *xp = (float *)x.data ();
   const vkl_out_seg back = { 0, width_, xp, (size_t)width_p_, VKL_TYPE_F32, VKL_ACT_NONE, xp, 0.f };
-  return launched ("layer output product",
-                   vkl_project_bf16w (b.cat.data (), type, (size_t)b.cat_stride, w.data (), S, width_, k, &back, 1,
-                                      dev_->stream ()));
+  const void *w = b.back->data ();
+  b.back = nullptr;
+  return launched ("layer output product", vkl_project_bf16w (b.cat.data (), type, (size_t)b.cat_stride, w, S, width_,
+                                                              b.back_k, &back, 1, dev_->stream ()));
 }
 
 ParallelBlock::ParallelBlock (GPUDevice *dev, Command *command, const std::string &name,
@@ -112,17 +119,15 @@ ParallelBlock::operator() (Tensor &x, int S, size_t offset, int run, Buffers &b)
 {
   const int type = dtype_ == FP32 ? VKL_TYPE_F32 : VKL_TYPE_BF16;
   const size_t esize = dtype_ == FP32 ? 4 : 2, cs = (size_t)b.cat_stride;
-  VKLLAMA_STATUS_OK (norm_input_ (x, S, norm_, b));
   auto segs = mixer_->segments (S, offset, run);
   VKLLAMA_STATUS_OK (segs);
   if (ff_.ff)
     segs->push_back ({ up_row_, ff_.ff, (uint8_t *)b.cat.data () + (size_t)ff_col_ * esize, cs, type, ff_.act, nullptr,
                        0.f });
-  VKLLAMA_STATUS_OK (launched ("layer input product",
-                               vkl_project_bf16w (b.h.data (), type, (size_t)width_p_, w_in_.data (), S, n_in_,
-                                                  width_p_, segs->data (), (int)segs->size (), dev_->stream ())));
+  VKLLAMA_STATUS_OK (norm_product_ ("layer input product", x, S, norm_, w_in_, n_in_, *segs, b));
   VKLLAMA_STATUS_OK (mixer_->mix (S, offset, run, b.cat.data (), cs));
-  return add_product_ (x, S, w_out_, k_out_, b);
+  b.back = &w_out_, b.back_k = k_out_;
+  return absl::OkStatus ();
 }
 
 void
@@ -179,22 +184,17 @@ SequentialBlock::operator() (Tensor &x, int S, size_t offset, int run, Buffers &
 {
   const int type = dtype_ == FP32 ? VKL_TYPE_F32 : VKL_TYPE_BF16;
   const size_t cs = (size_t)b.cat_stride;
-  VKLLAMA_STATUS_OK (norm_input_ (x, S, norm1_, b));
   auto segs = mixer_->segments (S, offset, run);
   VKLLAMA_STATUS_OK (segs);
-  VKLLAMA_STATUS_OK (launched ("mixer input product",
-                               vkl_project_bf16w (b.h.data (), type, (size_t)width_p_, w_in_.data (), S, n_in_,
-                                                  width_p_, segs->data (), (int)segs->size (), dev_->stream ())));
+  VKLLAMA_STATUS_OK (norm_product_ ("mixer input product", x, S, norm1_, w_in_, n_in_, *segs, b));
   VKLLAMA_STATUS_OK (mixer_->mix (S, offset, run, b.cat.data (), cs));
-  VKLLAMA_STATUS_OK (add_product_ (x, S, w_out_, k_out_, b));
+  b.back = &w_out_, b.back_k = k_out_;
   if (!ff_.ff)
     return absl::OkStatus ();
-  VKLLAMA_STATUS_OK (norm_input_ (x, S, norm2_, b));
-  const vkl_out_seg up = { 0, ff_p_, b.cat.data (), cs, type, ff_.act, nullptr, 0.f };
-  VKLLAMA_STATUS_OK (launched ("feed-forward product",
-                               vkl_project_bf16w (b.h.data (), type, (size_t)width_p_, w_up_.data (), S, ff_p_,
-                                                  width_p_, &up, 1, dev_->stream ())));
-  return add_product_ (x, S, w_down_, ff_p_, b);
+  VKLLAMA_STATUS_OK (norm_product_ ("feed-forward product", x, S, norm2_, w_up_, ff_p_,
+                                    { { 0, ff_p_, b.cat.data (), cs, type, ff_.act, nullptr, 0.f } }, b));
+  b.back = &w_down_, b.back_k = ff_p_;
+  return absl::OkStatus ();
 }
 
 void
@@ -333,9 +333,13 @@ StackModel::pass_ (size_t first, int S, size_t offset, std::vector<float> *strea
                                    : vkl_embed_rows_bf16 (embed_.data (), (uint32_t)vocab_, width_p_, cfg_.width, ids,
                                                           (uint32_t)S, cfg_.embed_scale, xp, (size_t)width_p_, s)));
   std::vector<int> seen (blocks_.size (), 0);
-  for (int i : cfg_.order)
+  buf_.back = nullptr; // (of a pass that failed)
+  for (size_t n = 0; n < cfg_.order.size (); ++n)
     {
-      VKLLAMA_STATUS_OK ((*blocks_[(size_t)i]) (x_, S, offset, seen[(size_t)i]++, buf_));
+      const size_t i = (size_t)cfg_.order[n];
+      VKLLAMA_STATUS_OK ((*blocks_[i]) (x_, S, offset, seen[i]++, buf_));
+      if (streams || n + 1 == cfg_.order.size ())
+        VKLLAMA_STATUS_OK (blocks_[i]->finish (x_, S, buf_));
       if (streams)
         {
           std::vector<float> rows ((size_t)S * width_p_);

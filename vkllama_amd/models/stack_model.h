@@ -33,14 +33,19 @@ public:
     Tensor h;   // a normed input, [rows, width_p]
     Tensor cat; // what a product back into the residual stream reads, [rows, widest]
     int cat_stride = 0;
+    // the product back that the next norm adds first (x += cat W^T over k columns of cat), if any
+    Tensor *back = nullptr;
+    int back_k = 0;
   };
   // name: "l0." etc.; mixer: made from parameters with the model's width, eps, ...
   StackBlock (GPUDevice *dev, Command *command, const std::string &name, std::unique_ptr<TokenMixer> mixer,
               const MixerParams &mp, const FeedForwardParams &ff);
   virtual ~StackBlock () {}
   virtual absl::Status load (const WeightSource &w) = 0;
-  // x [S, width_p] fp32, in place
+  // x [S, width_p] fp32, in place; the last product back may be left to the next block or finish ()
   virtual absl::Status operator() (Tensor &x, int S, size_t offset, int run, Buffers &b) = 0;
+  // the product back that is left
+  absl::Status finish (Tensor &x, int S, Buffers &b);
   virtual void describe (vkl_stack_layer &l, int run) = 0;
   // columns of `cat` the block needs
   virtual int cat_width () const = 0;
@@ -49,10 +54,9 @@ public:
 
 protected:
   absl::StatusOr<Tensor> norm_weights_ (const WeightSource &w, const std::string &name);
-  // h = rms_norm (x) w
-  absl::Status norm_input_ (Tensor &x, int S, Tensor &w, Buffers &b);
-  // x += cat W^T over the first k columns of cat
-  absl::Status add_product_ (Tensor &x, int S, Tensor &w, int k, Buffers &b);
+  // the product back that is left, h = rms_norm (x) norm, and the product of h with the n rows of w
+  absl::Status norm_product_ (const char *what, Tensor &x, int S, Tensor &norm, Tensor &w, int n,
+                              std::vector<vkl_out_seg> const &segs, Buffers &b);
   GPUDevice *dev_;
   Command *command_;
   std::string prefix_;

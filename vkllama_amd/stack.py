@@ -14,6 +14,12 @@ class OutSeg(C.Structure):
                 ("cap", f32)]
 
 
+class AddNormProject(C.Structure):
+    """vkl_add_norm_project"""
+    _fields_ = [("x", vp), ("xs", sz), ("w", vp), ("K", i32), ("y", vp), ("ys", sz), ("W", i32), ("norm", vp), ("eps", f32),
+                ("h", vp), ("hs", sz), ("Wp", i32), ("w_next", vp), ("N", i32), ("segs", C.POINTER(OutSeg)), ("nseg", i32)]
+
+
 class AttnRowsPrep(C.Structure):
     """vkl_attn_rows_prep"""
     _fields_ = [("H", i32), ("G", i32), ("dim", i32), ("n", i32), ("npair", i32), ("freq", vp), ("eps", f32),
@@ -34,6 +40,7 @@ ACT_NONE, ACT_SILU, ACT_RELU2, ACT_GELU = 0, 1, 2, 3
 
 SIGNATURES = {
     "vkl_project_bf16w": (i32, [vp, i32, sz, vp, i32, i32, i32, C.POINTER(OutSeg), i32, vp]),
+    "vkl_add_norm_project_bf16w": (i32, [C.POINTER(AddNormProject), i32, i32, vp]),
     "vkl_embed_norm_bf16": (i32, [vp, u32, i32, i32, vp, u32, vp, f32, vp, sz, vp]),
     "vkl_rmsnorm_f32": (i32, [vp, sz, vp, i32, i32, vp, f32, vp, i32, sz, i32, vp]),
     "vkl_attn_prefill_causal_bf16": (i32, [vp, vp, vp, i32, i32, i32, i32, i32, sz, sz, sz, f32, f32, i32, vp, sz, vp, sz,

@@ -165,6 +165,76 @@ template <int V> struct WideInt
   static constexpr int value = V;
 };
 
+// The k-steps of a tile of ST stages whose loads are issued D steps ahead: step (kt, stage, left) for
+// kt = 0 .. nk - 1.  left: how many k-steps stand behind it, D for D and more, where it issues the loads of
+// kt + D; the last D steps issue none, so that no tile waits for loads that nothing reads (with stages
+// for a whole compute unit, see one_round, us before / now, weights that no cache holds: 300 x 2048 x 2048
+// 32-bit 28.2 / 25.8, 500 x 3072 x 2048 39.3 / 32.8, 128 x 8192 x 2048 bf16 18.2 / 17.0).  Their stage is
+// a variable, which spares copies of them.
+template <int D, int ST, int I = 0, class F>
+__device__ __forceinline__ void
+wide_steps_some (int kt, int n, F &step)
+{
+  if constexpr (I < ST)
+    if (I < n)
+      {
+        step (kt + I, I, WideInt<D> ());
+        wide_steps_some<D, ST, I + 1> (kt, n, step);
+      }
+}
+template <int D, int ST, int I = 0, class F>
+__device__ __forceinline__ void
+wide_steps_round (int kt, F &step)
+{
+  if constexpr (I < ST)
+    {
+      step (kt + I, I, WideInt<D> ());
+      wide_steps_round<D, ST, I + 1> (kt, step);
+    }
+}
+template <int D, int ST, int LEFT, class F>
+__device__ __forceinline__ void
+wide_steps_last (int nk, int st, F &step)
+{
+  if (nk > LEFT)
+    {
+      step (nk - 1 - LEFT, st, WideInt<LEFT> ());
+      st = st == ST - 1 ? 0 : st + 1;
+    }
+  if constexpr (LEFT > 0)
+    wide_steps_last<D, ST, LEFT - 1> (nk, st, step);
+}
+// every one as if D stood behind it, for tiles without the registers for more copies of a step
+template <int D, int ST, class F>
+__device__ __forceinline__ void
+wide_steps_alike (int nk, F &step)
+{
+  int kt = 0;
+  for (; kt + ST <= nk; kt += ST)
+    wide_steps_round<D, ST> (kt, step);
+  wide_steps_some<D, ST> (kt, nk - kt, step);
+}
+template <int D, int ST, class F>
+__device__ __forceinline__ void
+wide_steps (int nk, F &step)
+{
+  int kt = 0;
+  for (; kt + ST <= nk - D; kt += ST)
+    wide_steps_round<D, ST> (kt, step);
+  const int n = nk - D - kt > 0 ? nk - D - kt : 0; // 0 .. ST - 1
+  wide_steps_some<D, ST> (kt, n, step);
+  wide_steps_last<D, ST, D - 1> (nk, n, step);
+}
+
+// waits until at most V loads are in flight; LDS: and the wave's own LDS reads are back
+template <int V, bool LDS>
+__device__ __forceinline__ void
+wait_loads ()
+{
+  constexpr int imm = (LDS ? 0x0070 : 0x0f70) | (V & 15) | ((V >> 4) << 14);
+  __builtin_amdgcn_s_waitcnt (imm);
+}
+
 // The products are formed transposed (the weights are the first operand): of a 32 x 32
 // block lane l holds token row l%32, and register q output column 8 (q/4) + 4 (l/32) +
 // q%4.  After exchanging half waves between the registers of two groups of four
@@ -414,11 +484,11 @@ wide_epilogue_tile (const GemmArgs &a, const float16v (&acc)[TM][1], uint8_t *wi
     }
 }
 
-template <int BM>
+template <int BM, int ST>
 constexpr size_t
 wide_lds_bf16 ()
 {
-  const size_t stages = (size_t)WSTAGES * (BM + WBN) * WROWB, park = (size_t)BM * 2 * kWideParkLd * 4;
+  const size_t stages = (size_t)ST * (BM + WBN) * WROWB, park = (size_t)BM * 2 * kWideParkLd * 4;
   return stages > park ? stages : park;
 }
 
@@ -482,7 +552,7 @@ wide_f32_again (const GemmSegArgs &a, float16v (&acc)[TM][WTN], int lane, int mr
 // products (two workgroups share a compute unit then), and 256 and 128 rows of 32-bit ones.
 // PLANES > 1: x holds PLANES values for every weight, in blocks of 64 (one k-step of
 // each plane in turn): see the 32-bit product below.
-template <int BM, int PLANES>
+template <int BM, int PLANES, int ST_>
 __device__ __forceinline__ void
 wide_bf16_tile (const GemmSegArgs &a, const WidePlace &at, int ksplit, float *ws)
 {
@@ -555,8 +625,9 @@ wide_bf16_tile (const GemmSegArgs &a, const WidePlace &at, int ksplit, float *ws
       }
   };
 #pragma unroll
-  for (int p = 0; p < WSTAGES - 1; ++p)
-    issue_part (p < nk ? p : nk - 1, p, 0, GPW);
+  for (int p = 0; p < ST_ - 1; ++p)
+    if (p < nk)
+      issue_part (p, p, 0, GPW);
 
   v8 af[2][TM], bf[2][WTN];
   // in the order the products need them
@@ -570,70 +641,60 @@ wide_bf16_tile (const GemmSegArgs &a, const WidePlace &at, int ksplit, float *ws
     for (int i = 1; i < TM; ++i)
       af[buf][i] = *(const v8 *)(sb + aoff[ks] + i * 32 * WROWB);
   };
-  // s_waitcnt immediates: vmcnt = the loads of the newest k-step may stay in
-  // flight; the second one also waits for the wave's own LDS reads
-  constexpr int VMW = (WSTAGES - 2) * GPW;
-  constexpr int WAITVM = 0x0f70 | (VMW & 15) | ((VMW >> 4) << 14);
   constexpr int LB1 = GPW / 3, LB2 = 2 * GPW / 3;
   constexpr int NR = TM + WTN, NP = TM * WTN;
-  // One k-step.  On entry tile kt is in stage ST and the fragments of its
-  // first quarter are on their way into buffer 0.
-  auto step = [&] (int kt, auto stc) {
-    constexpr int ST = decltype (stc)::value;
-    constexpr int SN = (ST + WSTAGES - 1) % WSTAGES, S1 = (ST + 1) % WSTAGES;
-    // the loads of tile kt + 2 go to the stage that was multiplied in the step
-    // before (every wave has passed that step's barrier); past the end they
-    // repeat the last tile into a stage nothing reads
-    const int kn = kt + WSTAGES - 1 < nk ? kt + WSTAGES - 1 : nk - 1;
+  static_assert ((ST_ - 2) * GPW < 64, "");
+  // One k-step.  On entry tile kt is in stage st and the fragments of its first quarter are on
+  // their way into buffer 0.  (Stages of the loads are one fewer than those in LDS: DEEP.)
+  constexpr int DEEP = ST_ - 1;
+  auto step = [&] (int kt, int st, auto left) {
+    constexpr int LEFT = decltype (left)::value;
+    constexpr bool MORE = LEFT == DEEP;
+    const int s1 = st == ST_ - 1 ? 0 : st + 1, sn = st == 0 ? ST_ - 1 : st - 1;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks)
       {
         if (ks < 3)
           {
-            read_frags (ST, ks + 1, (ks + 1) & 1);
-            issue_part (kn, SN, ks == 0 ? 0 : ks == 1 ? LB1 : LB2, ks == 0 ? LB1 : ks == 1 ? LB2 : GPW);
+            read_frags (st, ks + 1, (ks + 1) & 1);
+            // the loads of tile kt + ST - 1 go to the stage that was multiplied in the step
+            // before (every wave has passed that step's barrier)
+            if (MORE)
+              issue_part (kt + DEEP, sn, ks == 0 ? 0 : ks == 1 ? LB1 : LB2, ks == 0 ? LB1 : ks == 1 ? LB2 : GPW);
           }
-        else
+        else if (LEFT > 0)
           {
             // tile kt + 1 has landed (this wave's part; the barrier covers the
             // others') and this wave has read the last of tile kt
-            __builtin_amdgcn_s_waitcnt (WAITVM & ~0x0f00);
+            wait_loads<(LEFT > 0 ? LEFT - 1 : 0) * GPW, true> ();
             __builtin_amdgcn_s_barrier ();
             __builtin_amdgcn_sched_barrier (0);
-            read_frags (S1, 0, 0);
+            read_frags (s1, 0, 0);
           }
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
           for (int jn = 0; jn < WTN; ++jn)
             acc[i][jn] = WideElem<GemmSegArgs>::mfma (bf[ks & 1][jn], af[ks & 1][i], acc[i][jn]);
-        if (ks == 0)
+        if (ks == 0 && MORE)
           WideOrder<0, NP, NR, LB1>::run ();
-        else if (ks == 1)
+        else if (ks == 1 && MORE)
           WideOrder<0, NP, NR, LB2 - LB1>::run ();
-        else if (ks == 2)
+        else if (ks == 2 && MORE)
           WideOrder<0, NP, NR, GPW - LB2>::run ();
         else
           WideOrder<0, NP, NR, 0>::run ();
         __builtin_amdgcn_sched_barrier (0);
       }
   };
-  __builtin_amdgcn_s_waitcnt (WAITVM);
+  if (nk < DEEP)
+    wait_loads<0, false> ();
+  else
+    wait_loads<(DEEP - 1) * GPW, false> ();
   __builtin_amdgcn_s_barrier ();
   read_frags (0, 0, 0);
   __builtin_amdgcn_sched_barrier (0);
-  int kt = 0;
-  for (; kt + WSTAGES <= nk; kt += WSTAGES)
-    {
-      step (kt, WideInt<0> ());
-      step (kt + 1, WideInt<1> ());
-      step (kt + 2, WideInt<2> ());
-    }
-  if (kt < nk)
-    step (kt, WideInt<0> ());
-  if (kt + 1 < nk)
-    step (kt + 1, WideInt<1> ());
-  __builtin_amdgcn_s_waitcnt (0x0f70); // no load may outlive the workgroup's LDS
+  wide_steps<DEEP, ST_> (nk, step);
 
   if constexpr (PLANES > 1)
     if (!part) // (of parts the sum is looked at)
@@ -647,20 +708,22 @@ wide_bf16_tile (const GemmSegArgs &a, const WidePlace &at, int ksplit, float *ws
 // weights came from the L2 and went through LDS three times: for 64 rows 72 KB into LDS and 144
 // out of it per 64 columns, 1730 cycles at 128 bytes for 770 of products; now 40 + 80 KB.  Two
 // stages are 80 KB, two workgroups to a compute unit, each of which multiplies where the other
-// one waits.  Tiles of 128 rows (128 KB, one workgroup) were slower (800 x 16128 x 4096 362 us for
+// one waits; where there is one to a compute unit, four stages take its place.  Tiles of 128 rows (128 KB, one workgroup) were slower (800 x 16128 x 4096 362 us for
 // 315); of 256 they do not fit, and those of wide_bf16_tile (144 + 288 KB for 3070 cycles of products)
 // stay the better ones where they fill the chip (wide_plan_planes).  us before / now: 12 x 12288 x
 // 4096 39.9 / 33.0, 300 x 2048 x 2048 27.8 / 25.2, 300 x 5504 x 2048 41.9 / 37.1, 300 x 12288 x 4096
 // 120 / 96, 700 x 11008 x 4096 236 / 188.
 constexpr int kPlanes = 3, kPlaneRows = 64;
 
+template <int STAGES>
 constexpr size_t
 wide_lds_planes ()
 {
-  const size_t stages = (size_t)2 * (kPlanes * kPlaneRows + WBN) * WROWB, park = (size_t)kPlaneRows * 2 * kWideParkLd * 4;
+  const size_t stages = (size_t)STAGES * (kPlanes * kPlaneRows + WBN) * WROWB, park = (size_t)kPlaneRows * 2 * kWideParkLd * 4;
   return stages > park ? stages : park;
 }
 
+template <int STAGES>
 __global__ __launch_bounds__ (WWAVES * 64) void
 gemm_wide_planes_kernel (const GemmSegArgs a, WideGrid grid, int ksplit, float *ws)
 {
@@ -746,30 +809,42 @@ gemm_wide_planes_kernel (const GemmSegArgs a, WideGrid grid, int ksplit, float *
         af[buf][p][i] = *(const v8 *)(sb + aoff[q] + p * A_BYTES + i * 32 * WROWB);
   };
   constexpr int NP = kPlanes * TM * WTN, NR = kPlanes * TM + WTN;
-  issue (0, 0, 0, LOADS);
-  __builtin_amdgcn_s_waitcnt (0x0f70); // vmcnt(0)
+  static_assert ((STAGES - 1) * LOADS < 64, "");
+  // (of two stages the second one's loads come after the barrier)
+  constexpr int FIRST = STAGES == 2 ? 1 : STAGES;
+#pragma unroll
+  for (int p = 0; p < FIRST; ++p)
+    if (p < nk)
+      issue (p, p, 0, LOADS);
+  if (nk < FIRST)
+    wait_loads<0, false> ();
+  else
+    wait_loads<(FIRST - 1) * LOADS, false> ();
   __builtin_amdgcn_s_barrier ();
-  issue (nk > 1 ? 1 : 0, 1, 0, LOADS);
+  if (FIRST < STAGES && FIRST < nk)
+    issue (FIRST, FIRST, 0, LOADS);
   read_frags (0, 0, 0);
   __builtin_amdgcn_sched_barrier (0);
-  // One k-step: on entry tile kt is in stage ST, the fragments of its first quarter are on
-  // their way and tile kt + 1 is on its way into the other stage.
-  auto step = [&] (int kt, auto stc) {
-    constexpr int ST = decltype (stc)::value;
+  // One k-step: on entry tile kt is in stage st, the fragments of its first quarter are on
+  // their way and the tiles behind it are on their way into the other stages.
+  auto step = [&] (int kt, int st, auto left) {
+    constexpr int LEFT = decltype (left)::value;
+    constexpr bool MORE = LEFT == STAGES; // to load
 #pragma unroll
     for (int q = 0; q < 4; ++q)
       {
         if (q < 3)
-          read_frags (ST, q + 1, (q + 1) & 1);
-        else
+          read_frags (st, q + 1, (q + 1) & 1);
+        else if (LEFT > 0)
           {
             // tile kt + 1 is there and nobody reads tile kt any more: its stage takes tile
-            // kt + 2 (past the end the last tile again, which nothing reads)
-            __builtin_amdgcn_s_waitcnt (0x0070); // vmcnt(0) lgkmcnt(0)
+            // kt + STAGES
+            wait_loads<(MORE ? STAGES - 2 : LEFT > 0 ? LEFT - 1 : 0) * LOADS, true> ();
             __builtin_amdgcn_s_barrier ();
             __builtin_amdgcn_sched_barrier (0);
-            read_frags (ST ^ 1, 0, 0);
-            issue (kt + 2 < nk ? kt + 2 : nk - 1, ST, 0, LOADS);
+            read_frags (st == STAGES - 1 ? 0 : st + 1, 0, 0);
+            if (MORE)
+              issue (kt + STAGES, st, 0, LOADS);
           }
 #pragma unroll
         for (int p = 0; p < kPlanes; ++p)
@@ -781,23 +856,16 @@ gemm_wide_planes_kernel (const GemmSegArgs a, WideGrid grid, int ksplit, float *
                 float16v &sum = p ? low[i][jn] : acc[i][jn];
                 sum = WideElem<GemmSegArgs>::mfma (bf[q & 1][jn], af[q & 1][p][i], sum);
               }
-        if (q < 3)
-          WideOrder<0, NP, NR, 0>::run ();
-        else
+        if (q == 3 && MORE)
           WideOrder<0, NP, NR, LOADS>::run ();
+        else
+          WideOrder<0, NP, NR, 0>::run ();
         __builtin_amdgcn_sched_barrier (0);
       }
   };
-  int kt = 0;
-  for (; kt + 2 <= nk; kt += 2)
-    {
-      step (kt, WideInt<0> ());
-      step (kt + 1, WideInt<1> ());
-    }
-  if (kt < nk)
-    step (kt, WideInt<0> ());
-  __builtin_amdgcn_s_waitcnt (0x0f70); // no load may outlive the workgroup's LDS
-  __builtin_amdgcn_s_barrier ();       // (nor a fragment read the parked sums)
+  wide_steps<STAGES, STAGES> (nk, step);
+  __builtin_amdgcn_s_waitcnt (0x0070); // every wave's fragments are read before the sums are parked
+  __builtin_amdgcn_s_barrier ();
 
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -811,7 +879,7 @@ gemm_wide_planes_kernel (const GemmSegArgs a, WideGrid grid, int ksplit, float *
   wide_epilogue<TM, WTN> (a, acc, wide_lds, wave, lane, m0 + wm * TM * 32, n0 + wn * 64, part);
 }
 
-template <int BM, int PLANES>
+template <int BM, int PLANES, int ST>
 __global__ __launch_bounds__ (WWAVES * 64) void
 gemm_wide_bf16_kernel (const GemmSegArgs a, WideGrid grid, int ksplit, float *ws)
 {
@@ -821,10 +889,10 @@ gemm_wide_bf16_kernel (const GemmSegArgs a, WideGrid grid, int ksplit, float *ws
     case WIDE_NONE:
       return;
     case WIDE_TILE:
-      return wide_bf16_tile<BM, PLANES> (a, at, ksplit, ws);
+      return wide_bf16_tile<BM, PLANES, ST> (a, at, ksplit, ws);
     case WIDE_HALF:
       if constexpr (BM == WBM)
-        return wide_bf16_tile<BM / 2, PLANES> (a, at, ksplit, ws);
+        return wide_bf16_tile<BM / 2, PLANES, ST> (a, at, ksplit, ws);
     }
 }
 
@@ -841,15 +909,17 @@ struct MixTime
   double step, start, parked; // per k-step; per tile; more where its sums are parked in LDS
 };
 inline MixTime
-mix_time (int bm, int kind, bool q8)
+mix_time (int bm, int kind, bool one_row, bool q8)
 {
   // (Q8_0 weights: 256 rows only, and no parked sums to weigh; from the products named at mix_q8_tile)
   constexpr MixTime tq8[3] = { { 2.20, 10.0, 0 }, { 1.30, 8.0, 0 }, { 0.70, 6.0, 0 } };
   if (q8)
     return tq8[kind];
-  constexpr MixTime t256[3] = { { 1.42, 5.5, 15.5 }, { 0.76, 6.9, 8.3 }, { 0.54, 5.6, 4.4 } };
-  constexpr MixTime t128[3] = { { 0.80, 6.3, 7.6 }, { 0.52, 5.9, 4.6 }, { 0.52, 5.9, 4.6 } };
-  return bm == WBM ? t256[kind] : t128[kind];
+  constexpr MixTime t256[3] = { { 1.41, 5.0, 15.5 }, { 0.69, 5.7, 8.3 }, { 0.53, 5.6, 4.4 } };
+  constexpr MixTime t128[3] = { { 0.77, 6.1, 7.6 }, { 0.46, 5.7, 4.6 }, { 0.46, 5.7, 4.6 } };
+  // one row of tiles streams the weights
+  constexpr MixTime t1[3] = { { 1.15, 7.4, 7.6 }, { 0.75, 6.8, 4.6 }, { 0.75, 6.8, 4.6 } };
+  return bm == WBM ? t256[kind] : one_row ? t1[kind] : t128[kind];
 }
 
 // When the compute units are done with tiles dealt in turn to whichever is free first.
@@ -933,7 +1003,7 @@ struct WideMix
     double t[3];
     for (int k = 0; k < 3; ++k)
       {
-        const MixTime m = mix_time (bm, k, q8);
+        const MixTime m = mix_time (bm, k, tm == 1, q8);
         t[k] = m.step * steps + m.start + park * m.parked;
       }
     const int options[3] = { 0, pairs () / U * U, pairs () };
@@ -1138,6 +1208,8 @@ mix_epilogue (const Args &a, const float4v (&acc)[TM][4], uint8_t *wide_lds, int
 // GHz, 56 % at 1.87 in 256 x 128 tiles of four waves with 32 x 32 x 16; the vendor library's kernel 88 %
 // at 1.64), so less data per product out of LDS and L2 is what makes it faster.  The loads of a k-step are
 // issued when its stage has just been read, not a quarter later: two stages of 64 KB are enough then.
+// Of more than two stages each half of a k-step issues half of one (a burst of all in one half / halves, us:
+// 300 x 16128 x 4096 bf16 62.2 / 56.6, 300 x 11008 x 4096 52.6 / 49.4, 700 x 11008 x 4096 85.5 / 80.1).
 // Tried on the way, 4096 x 4096 x 4096, us: 107 as it is, 123 with 32 x 32 x 16, 147 with four waves
 // of 128 x 128 (AGPR moves), 117 with raised wave priority around the products, 114 with four stages of
 // 32 columns, 111 with two reads per product.
@@ -1152,6 +1224,7 @@ mix_tile (const Args &a, const WidePlace &at, int vec, int ksplit, float *ws)
   constexpr int WN = MWAVES / WM, TM = BM / WM / 16, TN = 4;
   static_assert (BN / WN == 64 && BM % (MWAVES * 8) == 0 && BN % (MWAVES * 8) == 0, "");
   constexpr int STAGE_BYTES = (BM + BN) * WROWB;
+  constexpr bool ALIKE = BM + BN > 256; // see wide_steps_alike
   constexpr int AG = BM / 8 / MWAVES, LOADS = (BM + BN) / 8 / MWAVES; // 1 KiB instructions per wave and k-step
   extern __shared__ __align__ (16) uint8_t wide_lds[];
   const int nk_all = a.K / WBK;
@@ -1199,6 +1272,7 @@ mix_tile (const Args &a, const WidePlace &at, int vec, int ksplit, float *ws)
     }
   constexpr int BJ = (UPGATE ? BN / 2 : 32) * WROWB; // from a wave's first to its second 32 weight rows
 
+  constexpr int EARLY = ST > 2 ? LOADS / 2 : LOADS;
   float4v acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -1206,9 +1280,9 @@ mix_tile (const Args &a, const WidePlace &at, int vec, int ksplit, float *ws)
     for (int j = 0; j < TN; ++j)
       acc[i][j] = float4v{ 0.f, 0.f, 0.f, 0.f };
 
-  auto issue = [&] (int kt, int st) {
+  auto issue = [&] (int kt, int st, int i0, int i1) {
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i)
+    for (int i = i0; i < i1; ++i)
       {
         const int g = i < AG ? wave + MWAVES * i : BM / 8 + wave + MWAVES * (i - AG);
         __builtin_amdgcn_global_load_lds ((const VKL_GLOBAL void *)(src[i] + (size_t)kt * WBK),
@@ -1217,7 +1291,8 @@ mix_tile (const Args &a, const WidePlace &at, int vec, int ksplit, float *ws)
   };
 #pragma unroll
   for (int p = 0; p < ST; ++p)
-    issue (p < nk ? p : nk - 1, p);
+    if (ALIKE || p < nk)
+      issue (p < nk ? p : nk - 1, p, 0, p < ST - 1 ? LOADS : EARLY);
   v8 af[2][TM], bf[2][TN];
   auto read_frags = [&] (int st, int h, int buf) {
     const uint8_t *sb = wide_lds + st * STAGE_BYTES;
@@ -1228,63 +1303,59 @@ mix_tile (const Args &a, const WidePlace &at, int vec, int ksplit, float *ws)
     for (int i = 0; i < TM; ++i)
       af[buf][i] = *(const v8 *)(sb + aoff[h] + i * 16 * WROWB);
   };
-  // s_waitcnt immediates: vmcnt = the loads of so many k-steps may stay in flight
-  constexpr int V0 = (ST - 1) * LOADS, V1 = (ST - 2) * LOADS;
-  static_assert (V0 < 64, "");
-  constexpr int WAIT0 = 0x0f70 | (V0 & 15) | ((V0 >> 4) << 14), WAIT1 = 0x0070 | (V1 & 15) | ((V1 >> 4) << 14);
-  // One k-step.  On entry tile kt is in stage S and the fragments of its first half are on
+  static_assert ((ST - 1) * LOADS < 64, "");
+  // One k-step.  On entry tile kt is in stage st and the fragments of its first half are on
   // their way.  Between its halves tile kt + 1 has landed (this wave's part; the barrier covers
   // the others') and nobody reads tile kt any more, whose last fragments are in registers: its
-  // stage takes tile kt + ST, a whole step and more before it is wanted (past the end the last
-  // tile again, which nothing reads).
-  auto step = [&] (int kt, auto stc) {
-    constexpr int S = decltype (stc)::value;
+  // stage takes tile kt + ST, a whole step and more before it is wanted (past the end, if at all, the
+  // last tile again, which nothing reads).
+  auto step = [&] (int kt, int st, auto left) {
+    constexpr int LEFT = decltype (left)::value;
+    constexpr bool MORE = LEFT == ST; // to load
 #pragma unroll
     for (int h = 0; h < 2; ++h)
       {
         if (h == 0)
-          read_frags (S, 1, 1);
-        else
           {
-            __builtin_amdgcn_s_waitcnt (WAIT1); // also for the wave's own LDS reads
+            read_frags (st, 1, 1);
+            // the rest of tile kt + ST - 1
+            if (EARLY < LOADS && LEFT >= ST - 1)
+              issue (kt + ST - 1 < nk ? kt + ST - 1 : nk - 1, st == 0 ? ST - 1 : st - 1, EARLY, LOADS);
+          }
+        else if (LEFT > 0)
+          {
+            wait_loads<(MORE ? ST - 2 : LEFT > 0 ? LEFT - 1 : 0) * LOADS, true> ();
             __builtin_amdgcn_s_barrier ();
             __builtin_amdgcn_sched_barrier (0);
-            issue (kt + ST < nk ? kt + ST : nk - 1, S);
-            read_frags ((S + 1) % ST, 0, 0);
+            if (MORE)
+              issue (kt + ST < nk ? kt + ST : nk - 1, st, 0, EARLY);
+            read_frags (st == ST - 1 ? 0 : st + 1, 0, 0);
           }
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
           for (int j = 0; j < TN; ++j)
             acc[i][j] = WideElem<Args>::mfma (bf[h][j], af[h][i], acc[i][j]);
-        if (h)
-          MixOrder<0, TM * TN, TM + TN, LOADS>::run ();
+        if (h && MORE)
+          MixOrder<0, TM * TN, TM + TN, EARLY>::run ();
+        else if (!h && LEFT >= ST - 1)
+          MixOrder<0, TM * TN, TM + TN, LOADS - EARLY>::run ();
         else
           MixOrder<0, TM * TN, TM + TN, 0>::run ();
         __builtin_amdgcn_sched_barrier (0);
       }
   };
-  __builtin_amdgcn_s_waitcnt (WAIT0);
+  if (!ALIKE && nk < ST)
+    wait_loads<0, false> ();
+  else
+    wait_loads<(ST - 2) * LOADS + EARLY, false> ();
   __builtin_amdgcn_s_barrier ();
   read_frags (0, 0, 0);
   __builtin_amdgcn_sched_barrier (0);
-  int kt = 0;
-  for (; kt + ST <= nk; kt += ST)
-    {
-      step (kt, WideInt<0> ());
-      step (kt + 1, WideInt<1 % ST> ());
-      if constexpr (ST > 2)
-        step (kt + 2, WideInt<2 % ST> ());
-      if constexpr (ST > 3)
-        step (kt + 3, WideInt<3 % ST> ());
-    }
-  if (kt < nk)
-    step (kt, WideInt<0> ());
-  if (ST > 2 && kt + 1 < nk)
-    step (kt + 1, WideInt<1> ());
-  if (ST > 3 && kt + 2 < nk)
-    step (kt + 2, WideInt<2 % ST> ());
-  __builtin_amdgcn_s_waitcnt (0x0070); // no load may outlive the workgroup's LDS (nor a fragment read the parked sums)
+  if constexpr (ALIKE)
+    wide_steps_alike<ST, ST> (nk, step);
+  else
+    wide_steps<ST, ST> (nk, step);
   mix_epilogue<UPGATE, TM, Args> (a, acc, wide_lds, wave, lane, m0 + wm * (BM / WM), n0 + wn * (UPGATE ? 32 : 64), at.zmat,
                                   vec, part);
 }
@@ -2186,16 +2257,16 @@ wide_reduce_seg_kernel (const GemmSegArgs a, const float *ws, int parts)
 
 // As wide_plan, with every row count allowed and, where the tiles are few, up to 16 parts
 // of at least 4 k-steps: with few token rows the workgroups exist to stream the weights.
-// The model is the time of the tiles (WideMix) and that of the reduction, 4.5 us + its bytes at 2.6
-// TB/s.  Tiles of 64 rows have two workgroups to a compute unit: up to 128 rows, up to 256 of them take
-// 0.54 per k-step + 2.6, up to 512 0.81 + 3.7 (fitted to 968 products of 2 to 2048 rows).
-// Where a segment's sums are parked in LDS a tile takes longer (MixTime), which parts leave to the
-// reduction.  With weights that no cache holds the plan is 1.4 % slower than the best one in the mean over
-// 195 products of 130 to 2200 rows, 2.6 % with GELU, 1.7 to 3.2 over 91 of 2 to 128 rows.
-// Beyond 128 rows, 64-row tiles in one part where no sums are parked: us without / with them 512
-// x 2048 x 2048 17.4 / 13.0, 300 x 2048 x 2048 17.7 / 12.9, 300 x 4096 x 512 9.0 / 6.7, 192 x 2048 x 2048 15.1 /
-// 12.8.  With GELU they would gain as much (600 x 2048 x 2048 20.3 / 17.4), and up to 192 rows with more
-// than 128 tiles a tenth (192 x 5504 x 2048 20.3 / 18.8), but a product of either kind is held to be in
+// The model is the time of the tiles (WideMix) and that of the reduction.  Tiles of 64 rows have two workgroups to a
+// compute unit, or where each gets one at most six stages of loads (one_round): up to 128 rows, up to 256 of them
+// take 0.54 per k-step + 2.3, up to 512 0.84 + 4.2; beyond 128 rows, which share the weights, 0.39 + 1.9.
+// Where a segment's sums are parked in LDS a tile takes longer (MixTime), which parts leave to the reduction.  With weights that no cache holds the plan is 1.6 % slower
+// than the best one in the mean over 208 products of 130 to 2200 rows, 2 % over 48 with GELU, 1.6 % over
+// 91 of 2 to 128 rows.
+// Beyond 128 rows, tiles of 64 in one part where each compute unit gets one at most and no sums are parked: us
+// without / with them 512 x 2048 x 2048 19.5 / 15.4, 300 x 2048 x 2048 18.0 / 15.5, 200 x 8192 x 2048 20.9 / 15.7.
+// With GELU they would gain as much (600 x 2048 x 2048 21.5 / 19.1), and up to 192 rows with more
+// than 128 tiles (192 x 5504 x 2048 20.6 / 17.5), but a product of either kind is held to be in
 // parts (tests/test_gemm_f32.py), which these tiles are not.
 // (a tile's waves walk 64 parked rows at a time)
 double
@@ -2213,8 +2284,8 @@ wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
   // 64-row tiles, one and two workgroups per compute unit: one or two rows of them stream the
   // weights, more share them in the L2; the reduction
   const bool few = a.M <= 128;
-  const double one64 = few ? 0.54 : 0.42, first64 = few ? 2.6 : 2.7, two64 = few ? 0.81 : 0.9, round64 = few ? 3.7 : 2.7;
-  constexpr double park64 = 3.9, reduce0 = 4.5, rate = 2.6e6;
+  const double one64 = few ? 0.54 : 0.39, first64 = few ? 2.3 : 1.9, reduce0 = few ? 3.9 : 4.3, rate = few ? 1.75e6 : 2.7e6;
+  constexpr double two64 = 0.84, round64 = 4.2, park64 = 3.9;
   WidePlan best = { 0, 1 };
   double best_cost = 0;
   const int nk = a.K / WBK, tiles_n = (a.N + WBN - 1) / WBN;
@@ -2225,7 +2296,7 @@ wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
         const int tiles_m = (a.M + bm - 1) / bm, tiles = tiles_m * tiles_n * ks;
         if (a.M < bm && bm > 128)
           continue;
-        if (bm == 64 && !few && (ks > 1 || parked > 0 || (a.M <= 192 && tiles > 128)))
+        if (bm == 64 && !few && (tiles > WideGrid::kUnits || ks > 4 || (ks == 1 && (parked > 0 || (a.M <= 192 && tiles > 128)))))
           continue;
         // (parts that fill the compute units four times gain nothing)
         if (ks > 1
@@ -2302,13 +2373,13 @@ launch_mix_parts (const GemmSegArgs &a, int ksplit, float *ws, hipStream_t s)
   return (int)hipGetLastError ();
 }
 
-template <int BM, int PLANES = 1>
+template <int BM, int ST, int PLANES = 1>
 int
 launch_wide_parts (const GemmSegArgs &a, int ksplit, float *ws, hipStream_t s)
 {
   static LdsLimit limit;
-  constexpr size_t lds = wide_lds_bf16<BM> ();
-  const auto kernel = gemm_wide_bf16_kernel<BM, PLANES>;
+  constexpr size_t lds = wide_lds_bf16<BM, ST> ();
+  const auto kernel = gemm_wide_bf16_kernel<BM, PLANES, ST>;
   if (int e = limit.raise ((const void *)kernel, lds))
     return e;
   const WideGrid tiles ((a.M + BM - 1) / BM, (a.N + WBN - 1) / WBN, 1, ksplit, BM == WBM);
@@ -2316,28 +2387,44 @@ launch_wide_parts (const GemmSegArgs &a, int ksplit, float *ws, hipStream_t s)
   return (int)hipGetLastError ();
 }
 
+// whether every compute unit gets one tile at most, which then may have all of its LDS
+bool
+one_round (const GemmSegArgs &a, int bm, int ksplit)
+{
+  return (long)((a.M + bm - 1) / bm) * ((a.N + WBN - 1) / WBN) * ksplit <= WideGrid::kUnits;
+}
+constexpr int kDeep64 = 6, kDeepPlanes = 4; // stages of 64-row tiles then
+
 // the tiles of a bf16 product
 int
 launch_bf16_tiles (const GemmSegArgs &a, const WidePlan &p, float *ws, hipStream_t s)
 {
   return p.bm == WBM   ? launch_mix_parts<WBM> (a, p.ksplit, ws, s)
          : p.bm == 128 ? launch_mix_parts<128> (a, p.ksplit, ws, s)
-                       : launch_wide_parts<64> (a, p.ksplit, ws, s);
+         : one_round (a, 64, p.ksplit) ? launch_wide_parts<64, kDeep64> (a, p.ksplit, ws, s)
+                                       : launch_wide_parts<64, WSTAGES> (a, p.ksplit, ws, s);
 }
 
 // the tiles of a product of planes
+template <int STAGES>
+int
+launch_planes_parts (const GemmSegArgs &a, int ksplit, float *ws, hipStream_t s)
+{
+  static LdsLimit limit;
+  constexpr size_t lds = wide_lds_planes<STAGES> ();
+  if (int e = limit.raise ((const void *)gemm_wide_planes_kernel<STAGES>, lds))
+    return e;
+  const WideGrid tiles ((a.M + kPlaneRows - 1) / kPlaneRows, (a.N + WBN - 1) / WBN, 1, ksplit, false);
+  gemm_wide_planes_kernel<STAGES><<<dim3 ((unsigned)tiles.groups ()), dim3 (WWAVES * 64), lds, s>>> (a, tiles, ksplit, ws);
+  return (int)hipGetLastError ();
+}
+
 int
 launch_planes_tiles (const GemmSegArgs &a, const WidePlan &p, float *ws, hipStream_t s)
 {
-  if (p.bm == WBM)
-    return launch_wide_parts<WBM, kPlanes> (a, 1, nullptr, s);
-  static LdsLimit limit;
-  constexpr size_t lds = wide_lds_planes ();
-  if (int e = limit.raise ((const void *)gemm_wide_planes_kernel, lds))
-    return e;
-  const WideGrid tiles ((a.M + kPlaneRows - 1) / kPlaneRows, (a.N + WBN - 1) / WBN, 1, p.ksplit, false);
-  gemm_wide_planes_kernel<<<dim3 ((unsigned)tiles.groups ()), dim3 (WWAVES * 64), lds, s>>> (a, tiles, p.ksplit, ws);
-  return (int)hipGetLastError ();
+  return p.bm == WBM                               ? launch_wide_parts<WBM, WSTAGES, kPlanes> (a, 1, nullptr, s)
+         : one_round (a, kPlaneRows, p.ksplit) ? launch_planes_parts<kDeepPlanes> (a, p.ksplit, ws, s)
+                                                   : launch_planes_parts<2> (a, p.ksplit, ws, s);
 }
 
 template <bool PLANES>

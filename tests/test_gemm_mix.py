@@ -198,3 +198,14 @@ def test_q8_0_up_and_gate(dev, M, N, K):
     want = s * u
     off = 1.1 * go * u.abs() + s.abs() * uo + go * uo + 2.0 ** -20 * want.abs() + rounded(want, 11)
     assert bool(((y - want).abs() <= off).all())
+
+
+# at most 128 tiles of 128 x 128, each of which is cut by its columns: k ranges shorter and longer than the stages; columns that end in the
+# first and in the second half of the last tile, and none in its second half
+@pytest.mark.parametrize("M,N,K", [(77, 4096, 64), (100, 4040, 320), (64, 4104, 384), (128, 12300, 448), (256, 8008, 1088), (33, 4168, 832)])
+def test_fp16_few_tiles(dev, M, N, K):
+    test_fp16(dev, M, N, K)
+    if N % 8 == 0:
+        test_fp16_up_and_gate(dev, M, N, K)
+        test_fp16_three_matrices(dev, M, N // 24 * 8, K)
+        test_fp16_scale_residual_and_wide_copy(dev, M, N, K)

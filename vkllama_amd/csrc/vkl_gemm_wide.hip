@@ -4,7 +4,7 @@
 //
 // A k-step is 64 wide, so a tile row is one 128-byte cache line.  The tiles of x and W do
 // not pass through registers on their way in: global_load_lds_dwordx4 writes them
-// straight into LDS, two to four k-steps deep, one 1 KiB instruction
+// straight into LDS, two to six k-steps deep, one 1 KiB instruction
 // per 8 tile rows.  Such an instruction writes its 64 x 16 bytes to consecutive
 // LDS addresses, so rows cannot be padded against bank conflicts; instead every
 // lane fetches the 16-byte chunk (slot ^ f(row)) of its row, which stores the
@@ -71,6 +71,7 @@ template <> struct WideElem<GemmSegArgs>
 struct WidePlace
 {
   int m0, tn, zmat, ks; // first token row, tile of weight rows, matrix, part of the k range
+  int half;             // (WideMix) of a tile that is cut by its columns
 };
 enum WideKind
 {
@@ -967,7 +968,7 @@ struct MixSpan
 };
 
 // The tiles of a launch: pairs of 128-column tiles as one of 256 columns, then tiles of 128
-// columns, of which the last may be cut in two by their rows.  Each kind is dealt to the XCDs
+// columns, of which the last (few of 128 rows: all) may be cut in two.  Each kind is dealt to the XCDs
 // in contiguous ranges of pairs, row tile fastest in groups of eight: the 32 pairs that an XCD
 // multiplies at a time are then 8 x 4 and not 32 x 1, and share their rows in its L2 (8192 x
 // 8192 x 8192 1023 us with 32 x 1, 823 with 8 x 4, 256 x 128 tiles).
@@ -977,6 +978,11 @@ struct MixSpan
 // pair, as many as fill whole rounds, or all go into one tile, whichever is done first: 2048 x
 // 12288 columns (1.5 rounds of pairs) 182 us with one round of pairs and 256 tiles, 198 without pairs,
 // 211 of pairs alone; 1500 x 8064, K = 2048 59 / 59 / 55.
+//
+// At most 128 tiles of 128 rows leave half the compute units idle while the others wait for weights: they are cut
+// by their columns into twice as many of 128 x 64, with six stages of loads (whole / cut, us, fp16: 77 x 4096 x 11008 in four
+// parts 34.0 / 27.2, 128 rows 38.7 / 31.9, 77 x 4096 x 4096 16.1 / 15.5).  The halves of more tiles would not all
+// run at once.
 struct WideMix
 {
   int tiles_m, tiles_n, nmat, ksplit;
@@ -993,7 +999,7 @@ struct WideMix
   {
     return tiles_m * tiles_n * nmat * ksplit - 2 * wide;
   }
-  // bm: token rows of a tile, 256 (which may be cut) or 128; steps: of the k range of a part;
+  // bm: token rows of a tile, 256 (which may be cut by its rows) or 128 (by its columns); steps: of the k range of a part;
   // park: how much of the time for parked sums a tile takes; us: the time of the launch's tiles
   __host__
   WideMix (int bm, int tm, int tn, int mats, int parts, double steps, double park, double *us = nullptr, bool q8 = false)
@@ -1016,6 +1022,8 @@ struct WideMix
         wide = options[o];
         const int rest = narrow () % U;
         whole = bm == WBM && wide % U == 0 && rest > 0 && rest <= U / 2 ? narrow () - rest : narrow ();
+        if (bm < WBM && !q8 && narrow () <= U / 2)
+          whole = 0;
         MixSpan span;
         span.deal (wide, t[0]);
         span.deal (whole, t[1]);
@@ -1085,7 +1093,9 @@ struct WideMix
         i /= tiles_m;
         at.tn = tiles_n - 1, at.zmat = i % nmat, at.ks = i / nmat;
       }
-    at.m0 += half * (BM / 2);
+    at.half = half;
+    if (BM == WBM)
+      at.m0 += half * (BM / 2);
     return at.m0 < M ? kind : 0;
   }
 };
@@ -1231,7 +1241,7 @@ mix_tile (const Args &a, const WidePlace &at, int vec, int ksplit, float *ws)
   const int kbase = (int)((long)nk_all * at.ks / ksplit);
   const int nk = (int)((long)nk_all * (at.ks + 1) / ksplit) - kbase;
   float *part = ksplit > 1 ? ws + (size_t)at.ks * a.M * a.N : nullptr;
-  const int m0 = at.m0, n0 = at.tn * (UPGATE ? WBN / 2 : WBN);
+  const int m0 = at.m0, n0 = (at.tn * WBN + (BN < WBN ? at.half * BN : 0)) / (UPGATE ? 2 : 1);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane (threadIdx.x >> 6);
   const int wm = wave / WN, wn = wave % WN;
@@ -1367,6 +1377,7 @@ mix_lds ()
   constexpr size_t wide = (size_t)(BM == WBM ? 2 : 3) * (BM + 256) * WROWB;
   constexpr size_t narrow = (size_t)(BM == WBM ? 3 : 4) * (BM + WBN) * WROWB;
   constexpr size_t park = (size_t)MWAVES * std::max (BM / 2 * 36, 64 * 68) * 4; // see mix_epilogue
+  static_assert (BM == WBM || 6 * (BM + WBN / 2) * WROWB <= wide, "");
   return std::max (std::max (wide, narrow), park);
 }
 
@@ -1384,6 +1395,8 @@ gemm_mix_kernel (const Args a, WideMix grid, int vec, int ksplit, float *ws)
     case 3:
       if constexpr (BM == WBM)
         return mix_tile<BM / 2, WBN, 4, 4, UPGATE, Args> (a, at, vec, ksplit, ws);
+      else
+        return mix_tile<BM, WBN / 2, 8, 6, UPGATE, Args> (a, at, vec, ksplit, ws);
     }
 }
 

@@ -709,7 +709,8 @@ wide_bf16_tile (const GemmSegArgs &a, const WidePlace &at, int ksplit, float *ws
 // weights came from the L2 and went through LDS three times: for 64 rows 72 KB into LDS and 144
 // out of it per 64 columns, 1730 cycles at 128 bytes for 770 of products; now 40 + 80 KB.  Two
 // stages are 80 KB, two workgroups to a compute unit, each of which multiplies where the other
-// one waits; where there is one to a compute unit, four stages take its place.  Tiles of 128 rows (128 KB, one workgroup) were slower (800 x 16128 x 4096 362 us for
+// one waits; where there is one to a compute unit, four stages take its place.  Tiles of 128 rows
+// (128 KB, one workgroup) were slower (800 x 16128 x 4096 362 us for
 // 315); of 256 they do not fit, and those of wide_bf16_tile (144 + 288 KB for 3070 cycles of products)
 // stay the better ones where they fill the chip (wide_plan_planes).  us before / now: 12 x 12288 x
 // 4096 39.9 / 33.0, 300 x 2048 x 2048 27.8 / 25.2, 300 x 5504 x 2048 41.9 / 37.1, 300 x 12288 x 4096
@@ -2339,7 +2340,8 @@ wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
 // The tiles of a product of planes: 64 rows in up to 16 parts of the k range (one and two
 // workgroups to a compute unit, as above), or wide_bf16_tile's 256 rows, the last of which may be
 // cut.  Fitted to 160 products of 2 to 2048 rows in 1 to 16 parts and 151 of 192 to 2048 rows in
-// both forms: 0.5 % slower than the best plan in the mean, 7 at worst; without 256 rows 2.5 % and 22
+// both forms, all in two stages (four take 0.8 to 0.95 of that where a compute unit has one tile, in one
+// part or several): 0.5 % slower than the best plan in the mean, 7 at worst; without 256 rows 2.5 % and 22
 // (2048 x 8064 x 2048 187 us with them, 229 without; 512 x 16128 x 4096 175, 199).
 WidePlan
 wide_plan_planes (const GemmSegArgs &a, size_t scratch)

@@ -127,6 +127,46 @@ def test_bf16_segments(dev, M, N, K, act):
     assert bool(((c - want).abs() <= off[:, n1:] + 2.0 ** -23 * want.abs()).all())
 
 
+# what is parked in LDS in tiles whose loads go on past the end of the k range, at inner sizes of models: 256 x 256
+# (GELU), 256 x 128 in two and four parts, 128 x 256 (a scale), a fused pair of an odd width
+@pytest.mark.parametrize("kind,M,N,K", [("gelu", 2048, 11008, 4096), ("bf16", 1500, 2048, 7552), ("f16", 300, 4096, 11008),
+                                        ("f16", 512, 5120, 13824), ("scale", 384, 16500, 320), ("pair", 2051, 5501, 1024)])
+def test_parked_sums(dev, kind, M, N, K):
+    bf = kind in ("gelu", "bf16")
+    x, w = (numbers(1 + i, n, K, dtype=torch.bfloat16 if bf else torch.float16) for i, n in enumerate((M, N)))
+    gate = numbers(3, N, K) if kind == "pair" else None
+    scale = 2.0 ** -6 if kind == "scale" else 1.0
+    out = []
+    for _ in range(3):
+        y = torch.full((M, N), 7.0, device="cuda", dtype=torch.float32 if bf else torch.float16)
+        torch.cuda.synchronize()
+        if bf:
+            act = stack.ACT_GELU if kind == "gelu" else stack.ACT_NONE
+            e = stack.lib().vkl_project_bf16w(x.data_ptr(), stack.BF16, K, w.data_ptr(), M, N, K,
+                                              stack.segments([(0, N, y.data_ptr(), N, stack.F32, act, None, 0.0)]), 1, dev.stream)
+        elif kind == "pair":
+            e = capi.lib().vkl_ffn_upgate_f16(x.data_ptr(), w.data_ptr(), gate.data_ptr(), M, N, K, y.data_ptr(), dev.stream)
+        else:
+            e = capi.lib().vkl_matmul_f16_tb(x.data_ptr(), w.data_ptr(), 1, M, N, K, M * K, K, N * K, K, M * N, N, scale, 0.0, 0,
+                                             None, y.data_ptr(), None, dev.stream)
+        capi.check(e)
+        dev.sync()
+        out.append(y)
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+    want, off = sums(x, w)
+    if kind == "gelu":
+        off, want = 1.13 * off + 2.0 ** -20 * want.abs() + 2.0 ** -22, torch.nn.functional.gelu(want)  # its slope is at most 1.13
+    elif kind == "pair":
+        g, go = sums(x, gate)
+        s = g * torch.sigmoid(g)
+        off = 1.1 * go * want.abs() + s.abs() * off + go * off + 2.0 ** -20 * (s * want).abs()
+        want = s * want
+    want, off = want * scale, off * scale
+    off = off + (0 if bf else rounded(want, 11))
+    ok = want.abs() < 65000 if kind == "pair" else torch.ones_like(want, dtype=torch.bool)
+    assert bool(((out[0] - want).abs() <= off)[ok].all())
+
+
 class Q8:
     """A Q8_0 matrix of random quants and scales, in the library's layout and in 64 bits"""
 

@@ -236,6 +236,16 @@ wait_loads ()
   __builtin_amdgcn_s_waitcnt (imm);
 }
 
+// Behind the k loop of every tile: no load may outlive the workgroup's LDS, and none may land where sums are
+// parked.  A wave can wait for its own loads only, so each does so before the barrier behind which LDS is
+// written by hand (tests/test_lds_loads.py follows the compiled code).  Tiles that load past the end
+// (wide_steps_alike) have up to nine in flight here, the others none.
+__device__ __forceinline__ void
+land_all ()
+{
+  wait_loads<0, true> ();
+}
+
 // The products are formed transposed (the weights are the first operand): of a 32 x 32
 // block lane l holds token row l%32, and register q output column 8 (q/4) + 4 (l/32) +
 // q%4.  After exchanging half waves between the registers of two groups of four
@@ -696,6 +706,7 @@ wide_bf16_tile (const GemmSegArgs &a, const WidePlace &at, int ksplit, float *ws
   read_frags (0, 0, 0);
   __builtin_amdgcn_sched_barrier (0);
   wide_steps<DEEP, ST_> (nk, step);
+  land_all ();
 
   if constexpr (PLANES > 1)
     if (!part) // (of parts the sum is looked at)
@@ -866,8 +877,8 @@ gemm_wide_planes_kernel (const GemmSegArgs a, WideGrid grid, int ksplit, float *
       }
   };
   wide_steps<STAGES, STAGES> (nk, step);
-  __builtin_amdgcn_s_waitcnt (0x0070); // every wave's fragments are read before the sums are parked
-  __builtin_amdgcn_s_barrier ();
+  land_all ();
+  __builtin_amdgcn_s_barrier (); // every wave's fragments are read before the sums are parked
 
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -1319,7 +1330,7 @@ mix_tile (const Args &a, const WidePlace &at, int vec, int ksplit, float *ws)
   // their way.  Between its halves tile kt + 1 has landed (this wave's part; the barrier covers
   // the others') and nobody reads tile kt any more, whose last fragments are in registers: its
   // stage takes tile kt + ST, a whole step and more before it is wanted (past the end, if at all, the
-  // last tile again, which nothing reads).
+  // last tile again, which nothing reads, but which is still to land: land_all).
   auto step = [&] (int kt, int st, auto left) {
     constexpr int LEFT = decltype (left)::value;
     constexpr bool MORE = LEFT == ST; // to load
@@ -1367,6 +1378,7 @@ mix_tile (const Args &a, const WidePlace &at, int vec, int ksplit, float *ws)
     wide_steps_alike<ST, ST> (nk, step);
   else
     wide_steps<ST, ST> (nk, step);
+  land_all ();
   mix_epilogue<UPGATE, TM, Args> (a, acc, wide_lds, wave, lane, m0 + wm * (BM / WM), n0 + wn * (UPGATE ? 32 : 64), at.zmat,
                                   vec, part);
 }
@@ -1938,7 +1950,7 @@ mix_q8_tile (const GemmArgs &a, const WidePlace &at, int vec, int ksplit, float 
       __builtin_amdgcn_sched_barrier (0);
       st = s1;
     }
-  __builtin_amdgcn_s_waitcnt (0x0070); // no load may outlive the workgroup's LDS (nor a fragment read the parked sums)
+  land_all (); // (up to three k-steps past the end)
   mix_q8_epilogue<UPGATE> (a, acc, wide_lds, wave, lane, m0 + wm * (BM / 2), n0 + wn * (UPGATE ? 32 : 64), at.zmat, vec, part);
 }
 

@@ -8,8 +8,10 @@ torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 
-# tiles of 64 rows, one to a compute unit and more of them; 128 rows; 256; planes in two and four stages
-@pytest.mark.parametrize("M,N,xtype", [(40, 264, stack.BF16), (200, 264, stack.BF16), (130, 16384, stack.BF16), (300, 8192, stack.BF16),
+# tiles of 64 rows, one to a compute unit and more of them; 128 rows by four waves and, cut in two, by eight; 256 rows by
+# four waves and by eight; planes in two and four stages
+@pytest.mark.parametrize("M,N,xtype", [(40, 264, stack.BF16), (200, 264, stack.BF16), (130, 16384, stack.BF16), (650, 3080, stack.BF16),
+                                       (160, 8056, stack.BF16), (750, 5448, stack.BF16), (1280, 6392, stack.BF16), (300, 8192, stack.BF16),
                                        (520, 12288, stack.BF16), (200, 1032, stack.F32), (800, 24584, stack.F32)])
 def test_short_k_ranges(dev, M, N, xtype):
     g = torch.Generator(device="cuda").manual_seed(M + N)

@@ -16,7 +16,7 @@
 // remaining products then overlap with the first fragment reads of the next one.
 //
 // Tiles of up to 256 x 256 (gemm_mix_kernel) multiply fp16 and bf16; those of 32 x 32
-// products (wide_bf16_tile) are left for 64 rows of bf16 and for 32-bit operands.
+// products (wide_bf16_tile) are left for 64 rows of bf16, for short tiles of more and for 32-bit operands.
 #include "../../include/vkl_stack.h"
 #include "vkl_stack_dev.h"
 #include "vkl_common.h"
@@ -169,7 +169,7 @@ template <int V> struct WideInt
 // The k-steps of a tile of ST stages whose loads are issued D steps ahead: step (kt, stage, left) for
 // kt = 0 .. nk - 1.  left: how many k-steps stand behind it, D for D and more, where it issues the loads of
 // kt + D; the last D steps issue none, so that no tile waits for loads that nothing reads (with stages
-// for a whole compute unit, see one_round, us before / now, weights that no cache holds: 300 x 2048 x 2048
+// for a whole compute unit, see deep64, us before / now, weights that no cache holds: 300 x 2048 x 2048
 // 32-bit 28.2 / 25.8, 500 x 3072 x 2048 39.3 / 32.8, 128 x 8192 x 2048 bf16 18.2 / 17.0).  Their stage is
 // a variable, which spares copies of them.
 template <int D, int ST, int I = 0, class F>
@@ -559,8 +559,10 @@ wide_f32_again (const GemmSegArgs &a, float16v (&acc)[TM][WTN], int lane, int mr
       }
 }
 
-// A BM x 128 tile by four waves of BM / 2 x 64, three k-steps of it in LDS: 64 rows of bf16
-// products (two workgroups share a compute unit then), and 256 and 128 rows of 32-bit ones.
+// A BM x 128 tile by four waves of BM / 2 x 64, ST_ k-steps of it in LDS.  Of bf16 products 64 rows: three k-steps where
+// two workgroups share a compute unit, six (144 KB) where each has one (deep64); and 128 and 256 rows in three, which they
+// begin and end sooner than the eight waves of mix_tile (see launch_bf16_tiles).  Of 32-bit products 256 rows and their
+// halves, in three.
 // PLANES > 1: x holds PLANES values for every weight, in blocks of 64 (one k-step of
 // each plane in turn): see the 32-bit product below.
 template <int BM, int PLANES, int ST_>
@@ -915,8 +917,11 @@ gemm_wide_bf16_kernel (const GemmSegArgs a, WideGrid grid, int ksplit, float *ws
 constexpr int MWAVES = 8;
 
 // What the tiles of gemm_mix_kernel take, us: of bm token rows and 256 columns, of 128 columns,
-// and of half the rows.  Fitted (with wide_plan_bf16's other constants) to 195 bf16 products of
-// 130 to 2200 rows, K = 512 to 15104, weights that no cache holds, in up to 24 plans each.
+// and of half of that (by the rows of 256, by the columns of 128).  Fitted with wide_plan_bf16's other constants, see
+// there, to the choice that they make.  By themselves (least squares, launch included) tiles of 256 x 256 take 1.30
+// per k-step + 7.6, of 256 x 128 0.70 + 8.0, of 128 x 256 0.76 + 5.0, of 128 x 128 0.49 + 5.3 (one row of them 0.67 +
+// 3.8), of 128 x 64 0.31 + 4.5.  Those last ones are charged with more: at 0.31 a product of 160 x 5504 x 2048 and its
+// like would be in one part (15 us, in two 19.7), but it is held to be in parts (tests/test_gemm_f32.py).
 struct MixTime
 {
   double step, start, parked; // per k-step; per tile; more where its sums are parked in LDS
@@ -929,9 +934,9 @@ mix_time (int bm, int kind, bool one_row, bool q8)
   if (q8)
     return tq8[kind];
   constexpr MixTime t256[3] = { { 1.41, 5.0, 15.5 }, { 0.69, 5.7, 8.3 }, { 0.53, 5.6, 4.4 } };
-  constexpr MixTime t128[3] = { { 0.77, 6.1, 7.6 }, { 0.46, 5.7, 4.6 }, { 0.46, 5.7, 4.6 } };
+  constexpr MixTime t128[3] = { { 0.70, 7.2, 7.7 }, { 0.49, 7.0, 3.0 }, { 0.52, 3.4, 0.51 } };
   // one row of tiles streams the weights
-  constexpr MixTime t1[3] = { { 1.15, 7.4, 7.6 }, { 0.75, 6.8, 4.6 }, { 0.75, 6.8, 4.6 } };
+  constexpr MixTime t1[3] = { { 1.17, 7.6, 7.1 }, { 0.79, 7.0, 3.4 }, { 0.49, 5.1, 3.9 } };
   return bm == WBM ? t256[kind] : one_row ? t1[kind] : t128[kind];
 }
 
@@ -2017,8 +2022,9 @@ constexpr int kWideMinGroups = 88, kWideMinGroupsQ8 = 128;
 
 struct WidePlan
 {
-  int bm;     // token rows of a tile, 0: this form does not apply
-  int ksplit; // parts of the k range
+  int bm;                  // token rows of a tile, 0: this form does not apply
+  int ksplit;              // parts of the k range
+  bool four_waves = false; // (bf16) tiles of 256 or 128 rows and 128 columns by four waves, see launch_bf16_tiles
 };
 
 long
@@ -2284,11 +2290,15 @@ wide_reduce_seg_kernel (const GemmSegArgs a, const float *ws, int parts)
 // As wide_plan, with every row count allowed and, where the tiles are few, up to 16 parts
 // of at least 4 k-steps: with few token rows the workgroups exist to stream the weights.
 // The model is the time of the tiles (WideMix) and that of the reduction.  Tiles of 64 rows have two workgroups to a
-// compute unit, or where each gets one at most six stages of loads (one_round): up to 128 rows, up to 256 of them
-// take 0.54 per k-step + 2.3, up to 512 0.84 + 4.2; beyond 128 rows, which share the weights, 0.39 + 1.9.
-// Where a segment's sums are parked in LDS a tile takes longer (MixTime), which parts leave to the reduction.  With weights that no cache holds the plan is 1.6 % slower
-// than the best one in the mean over 208 products of 130 to 2200 rows, 2 % over 48 with GELU, 1.6 % over
-// 91 of 2 to 128 rows.
+// compute unit, or where each gets one at most six stages of loads (deep64).  Where a segment's sums are parked in LDS a
+// tile takes longer (MixTime), which parts leave to the reduction.
+// The constants are fitted to the choice they make among all plans of 646 bf16 products, each with and without GELU,
+// 2 to 2200 rows, 512 to 16128 columns, K = 512 to 15104, weights that no cache holds: 1.6 % slower than the best plan in
+// the mean, and in 7 of the 1292 more than 2.5 % (at most 5) slower than the plans of tiles of four waves alone that they
+// replaced.  Constants fitted to the mean only, without any tiles of four waves above 64 rows, were 3.3 % off and slower
+// in 119, us then / now: 33 x 16128 x 4096 35.2 / 31.3, 128 x 4096 x 11008 33.0 / 31.3,
+// 160 x 4096 x 4096 21.3 / 20.0, 1500 x 5504 x 2048 52.3 / 42.7, 1100 x 2048 x 5504 48.4 / 42.0, 160 x 8064 x 2048 with GELU
+// 23.1 / 19.0.
 // Beyond 128 rows, tiles of 64 in one part where each compute unit gets one at most and no sums are parked: us
 // without / with them 512 x 2048 x 2048 19.5 / 15.4, 300 x 2048 x 2048 18.0 / 15.5, 200 x 8192 x 2048 20.9 / 15.7.
 // With GELU they would gain as much (600 x 2048 x 2048 21.5 / 19.1), and up to 192 rows with more
@@ -2304,14 +2314,39 @@ mix_park (const GemmSegArgs &a)
   return parked ? std::min (1.0, a.M / 64.0) : 0;
 }
 
+// whether every compute unit gets one tile at most, which then may have all of its LDS
+bool
+one_round (const GemmSegArgs &a, int bm, int ksplit)
+{
+  return (long)((a.M + bm - 1) / bm) * ((a.N + WBN - 1) / WBN) * ksplit <= WideGrid::kUnits;
+}
+constexpr int kDeep64 = 6, kDeepPlanes = 4; // stages of 64-row tiles then
+
+// (a tile of fewer k-steps would wait for all of them before its first product: 33 x 3072 x 1024 in four parts 10.0 us
+// with six stages, 9.7 with three)
+bool
+deep64 (const GemmSegArgs &a, int ksplit)
+{
+  return one_round (a, 64, ksplit) && a.K / WBK / ksplit >= kDeep64 - 1;
+}
+
+// 256 x 128 tiles that leave a quarter of the compute units and more without one and are full of rows (see launch_bf16_tiles)
+bool
+four256 (const GemmSegArgs &a, int ksplit, int tiles, double park)
+{
+  return ksplit == 1 && park == 0 && tiles > WideGrid::kUnits / 2 && tiles <= WideGrid::kUnits * 3 / 4 && a.K / WBK <= 64
+         && a.M >= (a.M + WBM - 1) / WBM * (WBM / 8 * 7);
+}
+
 WidePlan
 wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
 {
   // 64-row tiles, one and two workgroups per compute unit: one or two rows of them stream the
-  // weights, more share them in the L2; the reduction
+  // weights, more share them in the L2; the reduction; 128-row tiles by four waves
   const bool few = a.M <= 128;
-  const double one64 = few ? 0.54 : 0.39, first64 = few ? 2.3 : 1.9, reduce0 = few ? 3.9 : 4.3, rate = few ? 1.75e6 : 2.7e6;
-  constexpr double two64 = 0.84, round64 = 4.2, park64 = 3.9;
+  const double one64 = few ? 0.57 : 0.42, first64 = few ? 1.69 : 3.0, two64 = few ? 0.75 : 1.07, round64 = few ? 6.5 : 2.48;
+  const double park64 = few ? 3.5 : 5.9, shallow64 = few ? 1.0 : 0.5, reduce0 = few ? 6.3 : 3.7, rate = few ? 3.0e6 : 1.9e6;
+  const double step4 = few ? 0.76 : 0.54, start4 = few ? 5.5 : 3.9;
   WidePlan best = { 0, 1 };
   double best_cost = 0;
   const int nk = a.K / WBK, tiles_n = (a.N + WBN - 1) / WBN;
@@ -2338,13 +2373,19 @@ wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
             cost = two * round;
             if (rest > 0)
               cost += rest <= WideGrid::kUnits ? one64 * steps + first64 + p : round;
+            if (tiles <= WideGrid::kUnits && !deep64 (a, ks))
+              cost += shallow64;
           }
         else
           WideMix (bm, tiles_m, tiles_n, 1, ks, steps, park, &cost);
-        if (ks > 1)
-          cost += reduce0 + (double)ks * a.M * a.N * sizeof (float) / rate;
-        if (!best.bm || cost < best_cost)
-          best = { bm, ks }, best_cost = cost;
+        const double reduce = ks > 1 ? reduce0 + (double)ks * a.M * a.N * sizeof (float) / rate : 0;
+        if (!best.bm || cost + reduce < best_cost)
+          best = { bm, ks, bm == WBM && four256 (a, ks, tiles, park) }, best_cost = cost + reduce;
+        if (bm != 128 || tiles <= WideGrid::kUnits / 2 || park > 0)
+          continue;
+        cost = (tiles + WideGrid::kUnits - 1) / WideGrid::kUnits * (step4 * steps + start4);
+        if (cost + reduce < best_cost)
+          best = { bm, ks, true }, best_cost = cost + reduce;
       }
   return best;
 }
@@ -2414,22 +2455,23 @@ launch_wide_parts (const GemmSegArgs &a, int ksplit, float *ws, hipStream_t s)
   return (int)hipGetLastError ();
 }
 
-// whether every compute unit gets one tile at most, which then may have all of its LDS
-bool
-one_round (const GemmSegArgs &a, int bm, int ksplit)
-{
-  return (long)((a.M + bm - 1) / bm) * ((a.N + WBN - 1) / WBN) * ksplit <= WideGrid::kUnits;
-}
-constexpr int kDeep64 = 6, kDeepPlanes = 4; // stages of 64-row tiles then
-
-// the tiles of a bf16 product
+// The tiles of a bf16 product.  128 rows by four waves take 0.52 per k-step + 3.6 us, by eight 0.46 + 5.0: the shorter the
+// k range of a tile, the better.  They are weighed where more than 128 tiles leave none to be cut and no sums are parked
+// (us, eight / four waves: 650 x 3072 x 1024 11.6 / 10.6, 77 x 4096 x 11008 in eight parts 29.2 / 27.9, 160 x 4096 x 4096 in
+// four 23.3 / 20.0; parked 8 to 14 % slower).
+// 256 rows by four waves are level with eight over most of one round of tiles, and slower with more tiles, longer k ranges
+// and parked sums.  What is left to them (four256) takes 0.965 to 1.014 of the time, 0.985 in the mean of 17: 700 x 8064 x 2048
+// 31.4 / 30.3, 750 x 5504 x 2048 30.6 / 29.9, 512 x 12288 x 4096 57.3 / 55.8; with 160 to 256 tiles less full of rows 0.99
+// to 1.03.
 int
 launch_bf16_tiles (const GemmSegArgs &a, const WidePlan &p, float *ws, hipStream_t s)
 {
-  return p.bm == WBM   ? launch_mix_parts<WBM> (a, p.ksplit, ws, s)
-         : p.bm == 128 ? launch_mix_parts<128> (a, p.ksplit, ws, s)
-         : one_round (a, 64, p.ksplit) ? launch_wide_parts<64, kDeep64> (a, p.ksplit, ws, s)
-                                       : launch_wide_parts<64, WSTAGES> (a, p.ksplit, ws, s);
+  if (p.bm == WBM)
+    return p.four_waves ? launch_wide_parts<WBM, WSTAGES> (a, p.ksplit, ws, s) : launch_mix_parts<WBM> (a, p.ksplit, ws, s);
+  if (p.bm == 128)
+    return p.four_waves ? launch_wide_parts<128, WSTAGES> (a, p.ksplit, ws, s) : launch_mix_parts<128> (a, p.ksplit, ws, s);
+  return deep64 (a, p.ksplit) ? launch_wide_parts<64, kDeep64> (a, p.ksplit, ws, s)
+                              : launch_wide_parts<64, WSTAGES> (a, p.ksplit, ws, s);
 }
 
 // the tiles of a product of planes

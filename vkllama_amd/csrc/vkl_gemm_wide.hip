@@ -929,8 +929,10 @@ struct MixTime
 inline MixTime
 mix_time (int bm, int kind, bool one_row, bool q8)
 {
-  // (Q8_0 weights: 256 rows only, and no parked sums to weigh; from the products named at mix_q8_tile)
-  constexpr MixTime tq8[3] = { { 2.20, 10.0, 0 }, { 1.30, 8.0, 0 }, { 0.70, 6.0, 0 } };
+  // (Q8_0 weights: 256 rows only, and no parked sums to weigh; 511 launches of 256 to 2048 rows, none slower by more
+  // than 2 % than without pairs.  With 2.20, 10; 1.30, 8; 0.70, 6 up/gate of 1300 to 2048 x 3072 x 1024 went into pairs:
+  // 44.2 us, 41.4 without)
+  constexpr MixTime tq8[3] = { { 2.26, 10.1, 0 }, { 1.30, 7.9, 0 }, { 0.71, 5.8, 0 } };
   if (q8)
     return tq8[kind];
   constexpr MixTime t256[3] = { { 1.41, 5.0, 15.5 }, { 0.69, 5.7, 8.3 }, { 0.53, 5.6, 4.4 } };

@@ -3,6 +3,8 @@
 The sizes reach every kind of tile and their edges: whole rounds of column pairs with what is left in tiles of 128
 columns, whole and cut; pairs alone; an odd last column; last rows and columns that fill part of a tile; fewer k-steps
 than a tile has stages, and a remainder of them."""
+import ctypes as C
+
 import pytest
 
 from vkllama_amd import capi
@@ -240,12 +242,21 @@ def test_q8_0_up_and_gate(dev, M, N, K):
     assert bool(((y - want).abs() <= off).all())
 
 
-# at most 128 tiles of 128 x 128, each of which is cut by its columns: k ranges shorter and longer than the stages; columns that end in the
-# first and in the second half of the last tile, and none in its second half
-@pytest.mark.parametrize("M,N,K", [(77, 4096, 64), (100, 4040, 320), (64, 4104, 384), (128, 12300, 448), (256, 8008, 1088), (33, 4168, 832)])
-def test_fp16_few_tiles(dev, M, N, K):
-    test_fp16(dev, M, N, K)
-    if N % 8 == 0:
+# 88 to 128 tiles of 128 x 128, each of which is cut by its columns: k ranges shorter than the six stages, as long and longer;
+# columns that end in the first and in the second half of the last tile (of the fused pair 64 of either), and none in its second half
+@pytest.mark.parametrize("kind,M,N,K", [("one", 128, 12300, 64), ("one", 100, 12280, 320), ("one", 66, 12352, 384), ("one", 128, 12300, 448),
+                                        ("one", 256, 8008, 1088), ("three", 128, 4104, 64), ("three", 100, 4096, 320), ("three", 250, 1944, 832),
+                                        ("pair", 500, 1376, 64), ("pair", 250, 4040, 192), ("pair", 128, 5600, 384), ("pair", 400, 2048, 512)])
+def test_fp16_few_tiles(dev, kind, M, N, K):
+    p = capi.GemmPlan()
+    assert capi.lib().vkl_gemm_plan(M, N, K, 1, 3 if kind == "three" else 1, int(kind == "pair"), 0, C.byref(p)) == 0
+    tiles = -(-M // 128) * -(-N // (64 if kind == "pair" else 128)) * (3 if kind == "three" else 1)
+    assert (p.family, p.tile_rows, p.ksplit) == (5, 128, 1) and tiles <= 128
+    if kind == "pair":
         test_fp16_up_and_gate(dev, M, N, K)
-        test_fp16_three_matrices(dev, M, N // 24 * 8, K)
-        test_fp16_scale_residual_and_wide_copy(dev, M, N, K)
+    elif kind == "three":
+        test_fp16_three_matrices(dev, M, N, K)
+    else:
+        test_fp16(dev, M, N, K)
+        if N % 8 == 0:
+            test_fp16_scale_residual_and_wide_copy(dev, M, N, K)

@@ -992,8 +992,9 @@ struct MixSpan
 // multiplies at a time are then 8 x 4 and not 32 x 1, and share their rows in its L2 (8192 x
 // 8192 x 8192 1023 us with 32 x 1, 823 with 8 x 4, 256 x 128 tiles).
 //
-// A tile of 256 columns takes 0.92 of two of 128 (every fragment that is read from LDS goes into
-// twice the products), but fewer of them fill a round over the 256 compute units.  So either no
+// A tile of 256 columns takes less than two of 128 (every fragment that is read from LDS goes into
+// twice the products; 0.95 of them by mix_time at K = 4096, of the tiles by themselves 0.86), but fewer of them fill a
+// round over the 256 compute units.  So either no
 // pair, as many as fill whole rounds, or all go into one tile, whichever is done first: 2048 x
 // 12288 columns (1.5 rounds of pairs) 182 us with one round of pairs and 256 tiles, 198 without pairs,
 // 211 of pairs alone; 1500 x 8064, K = 2048 59 / 59 / 55.

@@ -2461,11 +2461,11 @@ launch_wide_parts (const GemmSegArgs &a, int ksplit, float *ws, hipStream_t s)
 // The tiles of a bf16 product.  128 rows by four waves take 0.52 per k-step + 3.6 us, by eight 0.46 + 5.0: the shorter the
 // k range of a tile, the better.  They are weighed where more than 128 tiles leave none to be cut and no sums are parked
 // (us, eight / four waves: 650 x 3072 x 1024 11.6 / 10.6, 77 x 4096 x 11008 in eight parts 29.2 / 27.9, 160 x 4096 x 4096 in
-// four 23.3 / 20.0; parked 8 to 14 % slower).
+// four 23.3 / 20.0; parked 10 to 15 % slower).
 // 256 rows by four waves are level with eight over most of one round of tiles, and slower with more tiles, longer k ranges
-// and parked sums.  What is left to them (four256) takes 0.965 to 1.014 of the time, 0.985 in the mean of 17: 700 x 8064 x 2048
-// 31.4 / 30.3, 750 x 5504 x 2048 30.6 / 29.9, 512 x 12288 x 4096 57.3 / 55.8; with 160 to 256 tiles less full of rows 0.99
-// to 1.03.
+// and parked sums.  What is left to them (four256) takes 0.965 to 1.014 of the time, 0.986 in the mean of 18: 700 x 8064 x 2048
+// 31.4 / 30.3, 750 x 5504 x 2048 30.6 / 29.9, 512 x 12288 x 4096 57.3 / 55.8; with more tiles or tiles less full of rows
+// 0.98 to 1.03.
 int
 launch_bf16_tiles (const GemmSegArgs &a, const WidePlan &p, float *ws, hipStream_t s)
 {

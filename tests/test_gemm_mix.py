@@ -132,11 +132,15 @@ def test_bf16_segments(dev, M, N, K, act):
 # what is parked in LDS in tiles whose loads go on past the end of the k range, at inner sizes of models: 256 x 256
 # (GELU), 256 x 128 in two and four parts, 128 x 256 (a scale), a fused pair of an odd width
 @pytest.mark.parametrize("kind,M,N,K", [("gelu", 2048, 11008, 4096), ("bf16", 1500, 2048, 7552), ("f16", 300, 4096, 11008),
-                                        ("f16", 512, 5120, 13824), ("scale", 384, 16500, 320), ("pair", 2051, 5501, 1024)])
+                                        ("f16", 512, 5120, 13824), ("scale", 384, 16500, 320), ("pair", 2300, 6201, 1024)])
 def test_parked_sums(dev, kind, M, N, K):
     bf = kind in ("gelu", "bf16")
     x, w = (numbers(1 + i, n, K, dtype=torch.bfloat16 if bf else torch.float16) for i, n in enumerate((M, N)))
     gate = numbers(3, N, K) if kind == "pair" else None
+    if not bf:                                                   # (bf16 products have no such plan to ask for)
+        p = capi.GemmPlan()
+        assert capi.lib().vkl_gemm_plan(M, N, K, 1, 1, int(kind == "pair"), 0, C.byref(p)) == 0
+        assert (p.family, p.tile_rows, p.ksplit) == (5, 128 if kind == "scale" else 256, {11008: 4, 13824: 2}.get(K, 1))
     scale = 2.0 ** -6 if kind == "scale" else 1.0
     out = []
     for _ in range(3):

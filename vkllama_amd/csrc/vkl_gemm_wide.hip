@@ -22,6 +22,7 @@
 #include "vkl_common.h"
 #include "vkl_gemm.h"
 #include <algorithm>
+#include <type_traits>
 #include "vkl_gemm_finish.h"
 
 namespace vkl
@@ -365,6 +366,21 @@ template <bool UPGATE> struct WideSimple<UPGATE, GemmSegArgs>
   }
 };
 
+// Sums of a part of the k range: eight neighbouring columns of row m from the registers to the dense rows that the
+// reduction reads (rows of a multiple of eight values; others are parked).  The walk through LDS took 0.4 to 2.5 us of
+// a launch, us through LDS / straight, weights that no cache holds: 600 x 2048 x 7552 38.2 / 36.7, 1500 x 2048 x 7552 64.0 /
+// 61.6, 160 x 2048 x 2048 13.2 / 12.6, 32-bit 300 x 2048 x 5504 42.6 / 42.4.  (fp16 products, 77 x 4096 x 4096 and
+// 11008, took the same, and keep the walk.)
+__device__ __forceinline__ void
+part_store8 (float *part, int M, int N, int m, int n, const float4v lo, const float4v hi)
+{
+  if (m >= M || n >= N)
+    return;
+  float *dst = part + (size_t)m * N + n;
+  *(VKL_GLOBAL float4v *)dst = lo;
+  *(VKL_GLOBAL float4v *)(dst + 4) = hi;
+}
+
 // TN: 32-column accumulators of a wave; mrow, ncol: the first row and output column of the
 // wave's block
 template <int TM, int TN>
@@ -410,6 +426,27 @@ wide_epilogue (const GemmSegArgs &a, const float16v (&acc)[TM][TN], uint8_t *wid
         walk (WideInt<1> ());
       else
         walk (WideInt<0> ());
+      return;
+    }
+  if (part && (a.N % 8) == 0)
+    {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int jn = 0; jn < TN; ++jn)
+#pragma unroll
+          for (int p = 0; p < 2; ++p)
+            {
+              float4v lo, hi;
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                {
+                  float x, y;
+                  half_swap (acc[i][jn][8 * p + e], acc[i][jn][8 * p + 4 + e], x, y);
+                  lo[e] = x, hi[e] = y;
+                }
+              part_store8 (part, a.M, a.N, mrow + i * 32 + (lane & 31), ncol + jn * 32 + p * 16 + (lane >> 5) * 8, lo, hi);
+            }
       return;
     }
   // through LDS, 64 accumulator columns at a time
@@ -1146,6 +1183,16 @@ mix_epilogue (const Args &a, const float4v (&acc)[TM][4], uint8_t *wide_lds, int
               int zmat, int vec, float *part)
 {
   constexpr int NB = UPGATE ? 1 : 2; // 32-column blocks of outputs, each by itself
+  if constexpr (std::is_same_v<Args, GemmSegArgs>)
+    if (part && (a.N % 8) == 0)
+      {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int b = 0; b < NB; ++b)
+            part_store8 (part, a.M, a.N, mrow + i * 16 + (lane & 15), ncol + b * 32 + (lane >> 4) * 8, acc[i][2 * b], acc[i][2 * b + 1]);
+        return;
+      }
   bool parked = false;
 #pragma unroll
   for (int b = 0; b < NB; ++b)
@@ -2341,6 +2388,15 @@ four256 (const GemmSegArgs &a, int ksplit, int tiles, double park)
          && a.M >= (a.M + WBM - 1) / WBM * (WBM / 8 * 7);
 }
 
+// Parts that are no power of two fill the compute units where powers leave a quarter to a half of them idle (us, without / with:
+// 1200 x 4096 x 15104 177 / 141, 600 x 4096 x 15104 96 / 87, 1200 x 2048 x 7552 58.9 / 49.6, 300 x 4096 x 11008 50.6 / 47.2).
+// They are taken where they promise 4 % (of 391 products of 131 to 2100 rows none of 150 rows and more got more than 5 %
+// slower, the mean is 0.989 of the time; with 8 % promised 0.990), by tiles of 128 and 256 rows, and from 144
+// rows on: below, the model takes tiles of few rows for faster than they are (131 x 4096 x 11008 38.0 / 43.1, 77 x 12576 x 4096
+// 30.0 / 36.5).
+constexpr double kOddParts = 0.96;
+constexpr int kOddRows = 144;
+
 WidePlan
 wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
 {
@@ -2355,8 +2411,11 @@ wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
   const int nk = a.K / WBK, tiles_n = (a.N + WBN - 1) / WBN;
   const double parked = mix_park (a);
   for (int bm = 64; bm <= WBM; bm *= 2)
-    for (int ks = 1; ks <= 16; ks *= 2)
+    for (int ks = 1; ks <= 16; ++ks)
       {
+        const bool odd = (ks & (ks - 1)) != 0; // no power of two
+        if (odd && (a.M < kOddRows || bm == 64))
+          continue;
         const int tiles_m = (a.M + bm - 1) / bm, tiles = tiles_m * tiles_n * ks;
         if (a.M < bm && bm > 128)
           continue;
@@ -2382,12 +2441,12 @@ wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
         else
           WideMix (bm, tiles_m, tiles_n, 1, ks, steps, park, &cost);
         const double reduce = ks > 1 ? reduce0 + (double)ks * a.M * a.N * sizeof (float) / rate : 0;
-        if (!best.bm || cost + reduce < best_cost)
+        if (!best.bm || cost + reduce < (odd ? kOddParts : 1.0) * best_cost)
           best = { bm, ks, bm == WBM && four256 (a, ks, tiles, park) }, best_cost = cost + reduce;
         if (bm != 128 || tiles <= WideGrid::kUnits / 2 || park > 0)
           continue;
         cost = (tiles + WideGrid::kUnits - 1) / WideGrid::kUnits * (step4 * steps + start4);
-        if (cost + reduce < best_cost)
+        if (cost + reduce < (odd ? kOddParts : 1.0) * best_cost)
           best = { bm, ks, true }, best_cost = cost + reduce;
       }
   return best;

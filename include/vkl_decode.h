@@ -124,6 +124,20 @@ int vkl_decode_step (const vkl_decode_model *m, const uint32_t *tok,
                      uint32_t pos, int mode, float *logits32,
                      uint32_t *next_tok, void *stream);
 
+/* The end of a prompt pass, which goes on with one row behind the last block's
+ * attention (models/llama2.h:160-213, 283-298 of the reference with
+ * clip_output): output projection, residual, feed-forward part and the output
+ * layer, by the launches of a step's phases.
+ *  att      device fp16 [dim]: the row of the attention, 16-byte aligned
+ *  row      device fp16 [dim]: the residual stream's row, 16-byte aligned;
+ *           holds the last block's output afterwards
+ *  logits32 optional device fp32 [vocab]: widened fp16 logits
+ * No workgroup waits for another one.  Uses the model's scratch: same stream
+ * as its steps.  vkl_decode_tail_supported: whether the shape is covered. */
+int vkl_decode_tail (const vkl_decode_model *m, const void *att, void *row,
+                     float *logits32, void *stream);
+int vkl_decode_tail_supported (const vkl_decode_model *m);
+
 /* Launches in which workgroups wait for one another (mode 1; the attention +
  * Wo launch of mode 0) need every workgroup resident at once and the
  * same number of them on each XCD; where that does not hold (a GPU shared

@@ -144,6 +144,21 @@ DecodePlan::step_device_token (const uint32_t *tok, size_t offset,
                                       gpu_->stream ()));
 }
 
+bool
+DecodePlan::tail_usable () const
+{
+  return usable_ && vkl_decode_tail_supported (&desc_);
+}
+
+absl::StatusOr<Tensor>
+DecodePlan::tail (Tensor att, void *row)
+{
+  VKLLAMA_STATUS_OK (hip_status (
+      "end of a prompt pass",
+      vkl_decode_tail (&desc_, att.data (), row, (float *)logits32_.data (), gpu_->stream ())));
+  return logits32_;
+}
+
 absl::Status
 DecodePlan::loop (uint32_t *ids, size_t pos0, size_t n_steps)
 {

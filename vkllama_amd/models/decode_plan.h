@@ -33,6 +33,10 @@ struct DecodePlan : public StepPlan
   absl::Status loop (uint32_t *ids, size_t pos0, size_t n_steps) override;
   absl::Status loop_sampled (uint32_t *ids, size_t pos0, size_t n_steps, int topk,
                              float topp, uint64_t seed) override;
+  // the end of a prompt pass behind the last block's attention (vkl_decode_tail);
+  // the logits are those of the plan
+  bool tail_usable () const;
+  absl::StatusOr<Tensor> tail (Tensor att, void *row);
   int mode () const { return mode_; }
   // Did a wait between workgroups inside a launch give up
   // (vkl_decode_status)?  If so the plan switches to the launches that wait for

@@ -109,6 +109,14 @@ Llama2Block::operator() (Tensor in, const size_t offset)
   return feedforward_op_->operator() (*normed2);
 }
 
+absl::StatusOr<Tensor>
+Llama2Block::heads (Tensor in, const size_t offset)
+{
+  auto normed = norm_op_->operator() (in);
+  VKLLAMA_STATUS_OK (normed);
+  return attn_op_->heads (*normed, offset);
+}
+
 void
 Llama2Block::print_op_cost ()
 {
@@ -411,7 +419,12 @@ Model::forward_ (std::vector<uint32_t> const &toks, const size_t offset,
   VKLLAMA_STATUS_OK (X);
   VKLLAMA_STATUS_OK (input_command_->end ());
   VKLLAMA_STATUS_OK (input_command_->submit ());
-  for (size_t i = 0; i < blocks_.size (); ++i)
+  // behind its attention the last block continues with one row, which the
+  // launches of a step's phases take to the logits
+  const bool tail = fused_decode_ && plan_ && plan_->tail_usable () && X->dtype () == FP16
+                    && X->width () == dim_ && X->hs () % 16 == 0;
+  const size_t chain = tail ? blocks_.size () - 1 : blocks_.size ();
+  for (size_t i = 0; i < chain; ++i)
     {
       auto *command = block_commands_[i];
       VKLLAMA_STATUS_OK (command->begin ());
@@ -424,6 +437,12 @@ Model::forward_ (std::vector<uint32_t> const &toks, const size_t offset,
         }
       VKLLAMA_STATUS_OK (command->end ());
       VKLLAMA_STATUS_OK (command->submit ());
+    }
+  if (tail)
+    {
+      auto att = blocks_.back ()->heads (*X, offset);
+      VKLLAMA_STATUS_OK (att);
+      return plan_->tail (*att, (uint8_t *)X->data () + (X->height () - 1) * X->hs ());
     }
   VKLLAMA_STATUS_OK (output_command_->begin ());
   return (*output_layer_) (*X);

@@ -96,6 +96,8 @@ public:
                RmsNormParams const &norm);
   absl::Status init ();
   absl::StatusOr<Tensor> operator() (Tensor in, const size_t offset);
+  // norm and attention alone, without the output projection
+  absl::StatusOr<Tensor> heads (Tensor in, const size_t offset);
   void print_op_cost ();
 
   MultiHeadAttentionV2 *attention () { return attn_op_.get (); }

@@ -225,9 +225,7 @@ MultiHeadAttentionV2::operator() (Tensor X, const size_t offset) noexcept
       attn_timer_.stop (dev_);
       VKLLAMA_STATUS_OK (launch_status ("attention", err));
       attn_fused_last_ = true;
-      matmul_o_->set_residual (residual_);
-      residual_ = nullptr;
-      return (*matmul_o_) (attn_out_);
+      return project_ (attn_out_);
     }
 
   // [seqlen, heads, dim]
@@ -300,9 +298,7 @@ MultiHeadAttentionV2::operator() (Tensor X, const size_t offset) noexcept
       attn_timer_.stop (dev_);
       VKLLAMA_STATUS_OK (launch_status ("attention", err));
       attn_fused_last_ = true;
-      matmul_o_->set_residual (residual_);
-      residual_ = nullptr;
-      return (*matmul_o_) (attn_out_);
+      return project_ (attn_out_);
     }
 
   // [heads, seqlen, read_len]
@@ -322,9 +318,27 @@ MultiHeadAttentionV2::operator() (Tensor X, const size_t offset) noexcept
   //[1, seqlen, heads*dim]
   VKLLAMA_STATUS_OK (concated->reshape (
       1, concated->channels (), concated->height () * concated->width ()));
-  matmul_o_->set_residual (residual_);
+  return project_ (*concated);
+}
+
+absl::StatusOr<Tensor>
+MultiHeadAttentionV2::project_ (Tensor heads) noexcept
+{
+  const Tensor *r = residual_;
   residual_ = nullptr;
-  return (*matmul_o_) (*concated);
+  if (heads_only_)
+    return heads;
+  matmul_o_->set_residual (r);
+  return (*matmul_o_) (heads);
+}
+
+absl::StatusOr<Tensor>
+MultiHeadAttentionV2::heads (Tensor X, const size_t offset) noexcept
+{
+  heads_only_ = true;
+  auto out = (*this) (X, offset);
+  heads_only_ = false;
+  return out;
 }
 
 uint64_t

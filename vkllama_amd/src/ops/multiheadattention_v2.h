@@ -31,6 +31,8 @@ public:
                                      const size_t offset = 0) noexcept;
   absl::Status init () noexcept override;
   uint64_t time () noexcept override;
+  // the heads' outputs [1, rows, heads * dim], without the output projection
+  absl::StatusOr<Tensor> heads (Tensor X, const size_t offset) noexcept;
 
   // The reference rotates the clipped (last-block) query at position
   // `offset` instead of offset + rows - 1 (multiheadattention_v2.cpp:222-233,
@@ -84,6 +86,9 @@ private:
   bool kqv_fused_last_ = false;
   bool attn_fused_last_ = false;
   bool operator_attention_ = false;
+  bool heads_only_ = false; // this call
+
+  absl::StatusOr<Tensor> project_ (Tensor heads) noexcept;
 };
 }
 #endif

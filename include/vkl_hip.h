@@ -151,6 +151,19 @@ typedef struct
 } vkl_gemm_plan_t;
 int vkl_gemm_plan (int M, int N, int K, int wtype, int nmat, int upgate,
                    size_t workspace_bytes, vkl_gemm_plan_t *out);
+/* y = x W^T (+ residual) as by vkl_matmul_q8_0 / vkl_matmul_f16_tb, and the RMS
+ * norm of its rows as by vkl_rmsnorm_f16 (models/llama2.h:160-213: the norm that
+ * follows an addition), all dense: x [M, K], W [N, K], residual (optional), y
+ * and normed [M, N], norm fp32 [N].  y is bit for bit that of those calls, normed
+ * but for ties of the last rounding; a product whose k range is divided takes one
+ * launch less. */
+int vkl_matmul_norm_q8_0 (const void *x, const void *w_planar, int M, int N,
+                          int K, const void *residual, void *y,
+                          const float *norm, float eps, void *normed,
+                          void *stream);
+int vkl_matmul_norm_f16 (const void *x, const void *w, int M, int N, int K,
+                         const void *residual, void *y, const float *norm,
+                         float eps, void *normed, void *stream);
 /* src/ops/multiheadattention_v2.cpp:190-202, src/shaders/kqv_fp16_x_q8_0.comp */
 int vkl_kqv_q8_0 (const void *x, const void *wk, const void *wq,
                   const void *wv, int M, int N, int K, void *k, void *q,

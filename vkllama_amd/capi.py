@@ -63,6 +63,8 @@ SIGNATURES = {
     "vkl_q8_0_unpack": (i32, [vp, vp, sz, sz, vp]),
     "vkl_embed_q8_0": (i32, [vp, u32, u32, vp, u32, u32, vp, vp]),
     "vkl_embed_f16": (i32, [vp, u32, u32, vp, u32, u32, vp, vp]),
+    "vkl_matmul_norm_q8_0": (i32, [vp, vp, i32, i32, i32, vp, vp, vp, f32, vp, vp]),
+    "vkl_matmul_norm_f16": (i32, [vp, vp, i32, i32, i32, vp, vp, vp, f32, vp, vp]),
     "vkl_rmsnorm_f16": (i32, [vp, vp, i32, i32, f32, vp, vp]),
     "vkl_matmul_q8_0": (i32, [vp, vp, i32, i32, i32, sz, sz, f32, f32, i32, vp, vp, vp, vp]),
     "vkl_matmul_q8_0_noalloc": (i32, [vp, vp, i32, i32, i32, sz, sz, f32, f32, i32, vp, vp, vp, vp]),

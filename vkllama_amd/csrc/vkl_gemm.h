@@ -10,6 +10,15 @@
 
 namespace vkl
 {
+// (host) the RMS norm that follows a product; the launch that adds the parts of a divided k range
+// forms it too, where there is one
+struct GemmNorm
+{
+  const float *w;
+  float eps;
+  uint16_t *out; // [M, N] fp16, dense
+  bool done = false;
+};
 struct GemmArgs
 {
   const uint16_t *x; // [M, K] fp16, row stride xs (elements)
@@ -35,6 +44,7 @@ struct GemmArgs
   // per-stream buffer, allocated on first use
   float *workspace;
   size_t workspace_bytes; // size of `workspace` (checked before every use)
+  GemmNorm *norm;         // optional, host memory: one plain product with a dense y
 };
 
 // A product whose output columns fall into segments, each with a destination, a

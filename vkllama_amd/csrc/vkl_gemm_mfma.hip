@@ -1045,6 +1045,123 @@ skinny2_reduce_kernel (const GemmArgs a, const float *ws, int S, int mrows)
     a.y32[(size_t)m * a.N + n] = h2f (h);
 }
 
+// The same, and the RMS norm of the rows: a workgroup has one row in registers.  Bound by its place between two
+// products: a launch takes 4.5 to 5 us behind another one whatever it does, and this one takes the place of two.  Sums, roundings
+// and the norm are those of skinny2_reduce_kernel and rmsnorm_kernel (whose last product and rounding are one
+// instruction: a tie between two fp16 numbers may go the other way there).  us, two launches / this: 77 rows of 4096 in four
+// parts 8.7 / 4.7 (a turn of 77 tokens behind 1500, three layers, 486 / 478).
+// VEC: 2048 values of a row each.
+template <int VEC>
+__global__ __launch_bounds__ (256) void
+reduce_norm_kernel (const GemmArgs a, const float *ws, int S, int mrows, const float *w, float eps, uint16_t *out)
+{
+  __shared__ float red[4];
+  const int m = blockIdx.x, nv = a.N >> 3;
+  uint4 res[VEC], g[VEC][2];
+  float v[VEC][8];
+#pragma unroll
+  for (int j = 0; j < VEC; ++j)
+    {
+      const int c = min ((int)threadIdx.x + j * 256, nv - 1) * 8;
+      res[j] = ldg4 (a.residual ? a.residual + (size_t)m * a.ys + c : (const uint16_t *)ws);
+      g[j][0] = ldg4 (w + c), g[j][1] = ldg4 (w + c + 4);
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        v[j][e] = 0.f;
+    }
+  // (a part past the last counts as zero)
+  for (int s0 = 0; s0 < S; s0 += 4)
+    {
+      uint4 p[VEC][4][2];
+#pragma unroll
+      for (int j = 0; j < VEC; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          {
+            const float *src = ws + ((size_t)min (s0 + i, S - 1) * mrows + m) * a.N + min ((int)threadIdx.x + j * 256, nv - 1) * 8;
+            p[j][i][0] = ldg4 (src), p[j][i][1] = ldg4 (src + 4);
+          }
+#pragma unroll
+      for (int j = 0; j < VEC; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          {
+            const uint32_t u[8] = { p[j][i][0].x, p[j][i][0].y, p[j][i][0].z, p[j][i][0].w,
+                                    p[j][i][1].x, p[j][i][1].y, p[j][i][1].z, p[j][i][1].w };
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              v[j][e] += s0 + i < S ? __uint_as_float (u[e]) : 0.f;
+          }
+    }
+  float ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < VEC; ++j)
+    {
+      const int i = (int)threadIdx.x + j * 256;
+      const uint32_t rw[4] = { res[j].x, res[j].y, res[j].z, res[j].w };
+      uint16_t h[8];
+      float t = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        {
+          h[e] = f2h (v[j][e]);
+          if (a.residual)
+            h[e] = f2h (h2f (h[e]) + h2f ((uint16_t)(rw[e >> 1] >> (16 * (e & 1)))));
+          v[j][e] = h2f (h[e]);
+          t += v[j][e] * v[j][e];
+        }
+      ss += i < nv ? t : 0.f;
+      if (i < nv)
+        stg ((vkl_u32x4 *)(a.y[0] + (size_t)m * a.ys + i * 8),
+             vkl_u32x4{ h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16), h[4] | ((uint32_t)h[5] << 16),
+                        h[6] | ((uint32_t)h[7] << 16) });
+    }
+  ss = wave_sum (ss);
+  if ((threadIdx.x & 63) == 0)
+    red[threadIdx.x >> 6] = ss;
+  __syncthreads ();
+  const float total = (red[0] + red[1]) + (red[2] + red[3]);
+  const float alpha = 1.0f / sqrtf (total / (float)a.N + eps);
+#pragma unroll
+  for (int j = 0; j < VEC; ++j)
+    {
+      const int i = (int)threadIdx.x + j * 256;
+      const uint32_t gw[8] = { g[j][0].x, g[j][0].y, g[j][0].z, g[j][0].w, g[j][1].x, g[j][1].y, g[j][1].z, g[j][1].w };
+      uint16_t h[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        h[e] = f2h (v[j][e] * __uint_as_float (gw[e]) * alpha);
+      if (i < nv)
+        stg ((vkl_u32x4 *)(out + (size_t)m * a.N + i * 8),
+             vkl_u32x4{ h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16), h[4] | ((uint32_t)h[5] << 16),
+                        h[6] | ((uint32_t)h[7] << 16) });
+    }
+}
+
+// adds the parts of a product, of which each lies `rows` rows behind the one before
+int
+launch_reduce (const GemmArgs &a, const float *ws, int parts, int rows, hipStream_t s)
+{
+  GemmNorm *n = a.norm;
+  const auto mis = [] (const void *p) { return ((uintptr_t)p % 16) != 0; };
+  if (n && a.nmat == 1 && !a.upgate && a.scale == 1.f && a.bias == 0.f && a.act == 0 && !a.y32 && (a.N % 8) == 0 && a.N <= 8192
+      && (a.ys % 8) == 0 && !mis (a.y[0]) && !mis (a.residual) && !mis (n->w) && !mis (n->out))
+    {
+      const dim3 grid ((unsigned)a.M), block (256);
+      if (a.N <= 2048)
+        reduce_norm_kernel<1><<<grid, block, 0, s>>> (a, ws, parts, rows, n->w, n->eps, n->out);
+      else if (a.N <= 4096)
+        reduce_norm_kernel<2><<<grid, block, 0, s>>> (a, ws, parts, rows, n->w, n->eps, n->out);
+      else
+        reduce_norm_kernel<4><<<grid, block, 0, s>>> (a, ws, parts, rows, n->w, n->eps, n->out);
+      n->done = true;
+      return (int)hipGetLastError ();
+    }
+  const size_t total = (size_t)a.M * a.N;
+  skinny2_reduce_kernel<<<dim3 ((unsigned)((total + 255) / 256)), dim3 (256), 0, s>>> (a, ws, parts, rows);
+  return (int)hipGetLastError ();
+}
+
 // Scratch for callers that must not allocate (vkl_matmul_q8_0_noalloc): a
 // file-scope device array.  Every GPU the library runs on holds its own copy
 // at its own address until the process ends; in host code the array's name is
@@ -1099,9 +1216,7 @@ launch_rows64_q8 (const GemmArgs &a, hipStream_t s, int &err)
   else
     gemm_rows64_q8_kernel<<<dim3 ((unsigned)S, (unsigned)((a.N + 63) / 64), (unsigned)nm),
                             dim3 (kR64Waves * 64), kR64Lds, s>>> (a, ws, S);
-  const size_t total = (size_t)a.M * a.N;
-  skinny2_reduce_kernel<<<dim3 ((unsigned)((total + 255) / 256)), dim3 (256), 0, s>>> (a, ws, S, 32);
-  err = (int)hipGetLastError ();
+  err = launch_reduce (a, ws, S, 32, s);
   return true;
 }
 
@@ -1125,9 +1240,7 @@ launch_skinny2 (const GemmArgs &a, hipStream_t s, int &err)
     return false;
   gemm_skinny2_kernel<WT><<<dim3 ((unsigned)S, (unsigned)((a.N + 31) / 32), (unsigned)nm),
                            dim3 (kSk2Waves * 64), lds, s>>> (a, ws, S);
-  const size_t total = (size_t)a.M * a.N;
-  skinny2_reduce_kernel<<<dim3 ((unsigned)((total + 255) / 256)), dim3 (256), 0, s>>> (a, ws, S, 32);
-  err = (int)hipGetLastError ();
+  err = launch_reduce (a, ws, S, 32, s);
   return true;
 }
 
@@ -1176,11 +1289,7 @@ launch_cfg (const GemmArgs &a, int ksplit, hipStream_t s)
                (unsigned)nz),
          dim3 (kGemmThreads), 0, s>>> (a, tiles_m, tiles_n, per_xcd, ksplit, ws);
   if (ksplit > 1)
-    {
-      const size_t total = (size_t)a.M * a.N;
-      skinny2_reduce_kernel<<<dim3 ((unsigned)((total + 255) / 256)), dim3 (256), 0, s>>> (
-          a, ws, ksplit, a.M);
-    }
+    return launch_reduce (a, ws, ksplit, a.M, s);
   return (int)hipGetLastError ();
 }
 } // namespace
@@ -1319,9 +1428,7 @@ StreamScratch::bytes ()
 int
 gemm_reduce_parts (const GemmArgs &a, const float *ws, int parts, int rows, hipStream_t s)
 {
-  const size_t total = (size_t)a.M * a.N;
-  skinny2_reduce_kernel<<<dim3 ((unsigned)((total + 255) / 256)), dim3 (256), 0, s>>> (a, ws, parts, rows);
-  return (int)hipGetLastError ();
+  return launch_reduce (a, ws, parts, rows, s);
 }
 
 bool

@@ -228,12 +228,12 @@ gemm_args (const GemvQ8Args &a, int nmat, int upgate)
 
 bool
 try_gemm (const GemvQ8Args &a, int nmat, int upgate, hipStream_t s, int &err,
-          float *workspace = nullptr, size_t workspace_bytes = 0)
+          float *workspace = nullptr, size_t workspace_bytes = 0, vkl::GemmNorm *norm = nullptr)
 {
   if (a.M < vkl::kGemmMinRows)
     return false;
   vkl::GemmArgs g = gemm_args (a, nmat, upgate);
-  g.workspace = workspace, g.workspace_bytes = workspace_bytes;
+  g.workspace = workspace, g.workspace_bytes = workspace_bytes, g.norm = norm;
   if (!vkl::gemm_mfma_supported (g))
     return false;
   err = vkl::gemm_mfma_launch (g, s);
@@ -257,7 +257,7 @@ namespace
 int
 matmul_q8_0 (const void *x, const void *w_planar, int M, int N, int K, size_t xs,
              size_t ys, float scale, float bias, int act, const void *residual,
-             void *y, float *y32, void *stream, bool no_alloc)
+             void *y, float *y32, void *stream, bool no_alloc, vkl::GemmNorm *norm = nullptr)
 {
   GemvQ8Args a = {};
   if (int e = fill_common (a, x, M, N, K, xs, ys))
@@ -291,7 +291,7 @@ matmul_q8_0 (const void *x, const void *w_planar, int M, int N, int K, size_t xs
         return (int)hipErrorInvalidValue;
     }
   int err = 0;
-  if (try_gemm (a, 1, 0, (hipStream_t)stream, err, workspace, have))
+  if (try_gemm (a, 1, 0, (hipStream_t)stream, err, workspace, have, norm))
     return err;
   return launch<0, 1> (a, (hipStream_t)stream);
 }
@@ -313,6 +313,17 @@ vkl_matmul_q8_0_noalloc (const void *x, const void *w_planar, int M, int N, int 
 {
   return matmul_q8_0 (x, w_planar, M, N, K, xs, ys, scale, bias, act, residual, y, y32, stream,
                       true);
+}
+
+extern "C" int
+vkl_matmul_norm_q8_0 (const void *x, const void *w_planar, int M, int N, int K, const void *residual, void *y,
+                      const float *norm, float eps, void *normed, void *stream)
+{
+  VKL_CHECK_ARG (norm && normed);
+  vkl::GemmNorm n = { norm, eps, (uint16_t *)normed };
+  if (int e = matmul_q8_0 (x, w_planar, M, N, K, (size_t)K, (size_t)N, 1.f, 0.f, 0, residual, y, nullptr, stream, false, &n))
+    return e;
+  return n.done ? 0 : vkl_rmsnorm_f16 (y, norm, M, N, eps, normed, stream);
 }
 
 extern "C" int

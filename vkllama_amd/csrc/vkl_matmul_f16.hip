@@ -160,11 +160,12 @@ launch_tb (TbArgs &p, bool upgate, hipStream_t s)
 }
 } // namespace
 
-extern "C" int
-vkl_matmul_f16_tb (const void *a, const void *b, int C, int M, int N, int K,
-                   size_t acs, size_t ahs, size_t bcs, size_t bhs, size_t ycs,
-                   size_t yhs, float scale, float bias, int act,
-                   const void *residual, void *y, float *y32, void *stream)
+namespace
+{
+int
+matmul_f16_tb (const void *a, const void *b, int C, int M, int N, int K, size_t acs, size_t ahs, size_t bcs, size_t bhs,
+               size_t ycs, size_t yhs, float scale, float bias, int act, const void *residual, void *y, float *y32,
+               void *stream, vkl::GemmNorm *norm)
 {
   VKL_CHECK_ARG (a && b && y && C > 0 && M > 0 && N > 0 && K > 0);
   VKL_CHECK_ARG (act == 0 || act == 1);
@@ -192,11 +193,33 @@ vkl_matmul_f16_tb (const void *a, const void *b, int C, int M, int N, int K,
       g.y[0] = g.y[1] = g.y[2] = p.y;
       g.ys = yhs;
       g.scale = scale, g.bias = bias, g.act = act;
-      g.residual = p.residual, g.y32 = y32;
+      g.residual = p.residual, g.y32 = y32, g.norm = norm;
       if (vkl::gemm_mfma_supported (g))
         return vkl::gemm_mfma_launch (g, (hipStream_t)stream);
     }
   return launch_tb (p, false, (hipStream_t)stream);
+}
+} // namespace
+
+extern "C" int
+vkl_matmul_f16_tb (const void *a, const void *b, int C, int M, int N, int K,
+                   size_t acs, size_t ahs, size_t bcs, size_t bhs, size_t ycs,
+                   size_t yhs, float scale, float bias, int act,
+                   const void *residual, void *y, float *y32, void *stream)
+{
+  return matmul_f16_tb (a, b, C, M, N, K, acs, ahs, bcs, bhs, ycs, yhs, scale, bias, act, residual, y, y32, stream, nullptr);
+}
+
+extern "C" int
+vkl_matmul_norm_f16 (const void *x, const void *w, int M, int N, int K, const void *residual, void *y, const float *norm,
+                     float eps, void *normed, void *stream)
+{
+  VKL_CHECK_ARG (norm && normed && M > 0 && N > 0 && K > 0);
+  vkl::GemmNorm n = { norm, eps, (uint16_t *)normed };
+  if (int e = matmul_f16_tb (x, w, 1, M, N, K, 0, (size_t)K, 0, (size_t)K, 0, (size_t)N, 1.f, 0.f, 0, residual, y, nullptr,
+                             stream, &n))
+    return e;
+  return n.done ? 0 : vkl_rmsnorm_f16 (y, norm, M, N, eps, normed, stream);
 }
 
 extern "C" int

@@ -80,11 +80,12 @@ Llama2Block::init ()
 }
 
 absl::StatusOr<Tensor>
-Llama2Block::operator() (Tensor in, const size_t offset)
+Llama2Block::operator() (Tensor in, const size_t offset, bool normed, RMSNorm *next)
 {
   // The residual additions of the reference's block (element_wise after the
   // attention and after the feed-forward part) run in the launches of the two
-  // projections that precede them: the same fp16 values, two launches less.
+  // projections that precede them, and so do the norms behind them where those
+  // projections add parts: the same fp16 values, up to four launches less.
   Tensor residual = in;
   if (transformer_params_.clip_output)
     {
@@ -98,23 +99,23 @@ Llama2Block::operator() (Tensor in, const size_t offset)
       VKLLAMA_STATUS_OK (cliped);
       residual = *cliped;
     }
-  auto normed = norm_op_->operator() (in);
-  VKLLAMA_STATUS_OK (normed);
+  if (!normed)
+    VKLLAMA_STATUS_OK (norm_op_->operator() (in));
   attn_op_->set_residual (&residual);
-  auto added = attn_op_->operator() (*normed, offset);
+  attn_op_->set_norm (norm_op2_.get ());
+  auto added = attn_op_->operator() (norm_op_->output (), offset);
   VKLLAMA_STATUS_OK (added);
-  auto normed2 = norm_op2_->operator() (*added);
-  VKLLAMA_STATUS_OK (normed2);
   feedforward_op_->set_residual (&*added);
-  return feedforward_op_->operator() (*normed2);
+  feedforward_op_->set_norm (next);
+  return feedforward_op_->operator() (norm_op2_->output ());
 }
 
 absl::StatusOr<Tensor>
-Llama2Block::heads (Tensor in, const size_t offset)
+Llama2Block::heads (Tensor in, const size_t offset, bool normed)
 {
-  auto normed = norm_op_->operator() (in);
-  VKLLAMA_STATUS_OK (normed);
-  return attn_op_->heads (*normed, offset);
+  if (!normed)
+    VKLLAMA_STATUS_OK (norm_op_->operator() (in));
+  return attn_op_->heads (norm_op_->output (), offset);
 }
 
 void
@@ -428,7 +429,7 @@ Model::forward_ (std::vector<uint32_t> const &toks, const size_t offset,
     {
       auto *command = block_commands_[i];
       VKLLAMA_STATUS_OK (command->begin ());
-      X = (*blocks_[i]) (*X, offset);
+      X = (*blocks_[i]) (*X, offset, i > 0, i + 1 < blocks_.size () ? blocks_[i + 1]->attn_norm () : nullptr);
       if (!X.ok ())
         {
           fprintf (stderr, "infer block %zu failed: %s\n", i,
@@ -440,7 +441,7 @@ Model::forward_ (std::vector<uint32_t> const &toks, const size_t offset,
     }
   if (tail)
     {
-      auto att = blocks_.back ()->heads (*X, offset);
+      auto att = blocks_.back ()->heads (*X, offset, chain > 0);
       VKLLAMA_STATUS_OK (att);
       return plan_->tail (*att, (uint8_t *)X->data () + (X->height () - 1) * X->hs ());
     }

@@ -95,9 +95,11 @@ public:
                FeedForwardParams const &feed_forward,
                RmsNormParams const &norm);
   absl::Status init ();
-  absl::StatusOr<Tensor> operator() (Tensor in, const size_t offset);
+  // normed: attn_norm () holds the norm of `in`; next: takes that of the output
+  absl::StatusOr<Tensor> operator() (Tensor in, const size_t offset,
+                                     bool normed = false, RMSNorm *next = nullptr);
   // norm and attention alone, without the output projection
-  absl::StatusOr<Tensor> heads (Tensor in, const size_t offset);
+  absl::StatusOr<Tensor> heads (Tensor in, const size_t offset, bool normed);
   void print_op_cost ();
 
   MultiHeadAttentionV2 *attention () { return attn_op_.get (); }

@@ -90,7 +90,8 @@ FeedForward::operator() (Tensor X) noexcept
   timer_.stop (dev_);
   VKLLAMA_STATUS_OK (launch_status ("feed_forward up/gate", err));
   down_op_->set_residual (residual_);
-  residual_ = nullptr;
+  down_op_->set_norm (norm_);
+  residual_ = nullptr, norm_ = nullptr;
   return (*down_op_) (t0_);
 }
 }

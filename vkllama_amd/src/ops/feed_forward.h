@@ -20,6 +20,8 @@ public:
   absl::StatusOr<Tensor> operator() (Tensor X) noexcept;
   // the next call only: the residual is added in the down projection's launch
   void set_residual (const Tensor *r) noexcept { residual_ = r; }
+  // the next call only: the norm of the output's rows (MatMul::set_norm)
+  void set_norm (RMSNorm *n) noexcept { norm_ = n; }
   absl::Status init () noexcept override;
   uint64_t time () noexcept override;
   Tensor &w1 () { return w1_; }
@@ -28,6 +30,7 @@ public:
 
 private:
   const Tensor *residual_ = nullptr;
+  RMSNorm *norm_ = nullptr;
   Tensor t0_;
   Tensor w1_;
   Tensor w2_;

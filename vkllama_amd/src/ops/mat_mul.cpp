@@ -126,6 +126,8 @@ MatMul::run_ (Tensor &a, Tensor &b) noexcept
 
   const Tensor *res = residual_;
   residual_ = nullptr;
+  RMSNorm *norm = norm_;
+  norm_ = nullptr;
   if (res
       && (res->channels () != out_c || res->height () != out_h || res->width () != out_w
           || res->hs () != out_.hs () || res->dtype () != FP16
@@ -134,6 +136,19 @@ MatMul::run_ (Tensor &a, Tensor &b) noexcept
 
   void *s = dev_->stream ();
   int err = 0;
+  const bool dense = out_c == 1 && a.channels () == 1 && a.hs () == K * 2 && out_.hs () == out_w * 2
+                     && (b_dtype_ == Q8_0 || (transpose_b_ && b.hs () == K * 2));
+  if (norm && dense && scale_ == 1.f && bias_ == 0.f && act_ == 0)
+    {
+      VKLLAMA_STATUS_OK (norm->prepare (out_h, out_w));
+      timer_.start (dev_);
+      const auto product = b_dtype_ == Q8_0 ? vkl_matmul_norm_q8_0 : vkl_matmul_norm_f16;
+      err = product (a.data (), b.data (), (int)out_h, (int)out_w, (int)K, res ? res->data () : nullptr, out_.data (),
+                     (const float *)norm->weight ().data (), norm->eps (), norm->output ().data (), s);
+      timer_.stop (dev_);
+      VKLLAMA_STATUS_OK (launch_status ("matmul and norm", err));
+      return out_;
+    }
   timer_.start (dev_);
   if (b_dtype_ == Q8_0)
     {
@@ -167,6 +182,11 @@ MatMul::run_ (Tensor &a, Tensor &b) noexcept
     }
   timer_.stop (dev_);
   VKLLAMA_STATUS_OK (launch_status ("matmul", err));
+  if (norm)
+    {
+      auto normed = (*norm) (out_);
+      VKLLAMA_STATUS_OK (normed);
+    }
   return out_;
 }
 }

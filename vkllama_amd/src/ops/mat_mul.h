@@ -3,6 +3,7 @@
 #define __VKLLAMA_MATMUL_H__
 
 #include "src/ops/op.h"
+#include "src/ops/rms_norm.h"
 #include <memory>
 
 namespace vkllama
@@ -32,9 +33,14 @@ public:
   // launch).  Not part of the reference's interface.
   void set_residual (const Tensor *r) noexcept { residual_ = r; }
 
+  // The next product only: `n` holds the norm of its rows afterwards
+  // (RMSNorm::output).  Not part of the reference's interface.
+  void set_norm (RMSNorm *n) noexcept { norm_ = n; }
+
 private:
   absl::StatusOr<Tensor> run_ (Tensor &a, Tensor &b) noexcept;
   const Tensor *residual_ = nullptr;
+  RMSNorm *norm_ = nullptr;
   Tensor weight_;
   const int broadcast_type_;
   const int act_;

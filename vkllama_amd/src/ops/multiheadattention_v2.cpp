@@ -325,10 +325,12 @@ absl::StatusOr<Tensor>
 MultiHeadAttentionV2::project_ (Tensor heads) noexcept
 {
   const Tensor *r = residual_;
-  residual_ = nullptr;
+  RMSNorm *n = norm_;
+  residual_ = nullptr, norm_ = nullptr;
   if (heads_only_)
     return heads;
   matmul_o_->set_residual (r);
+  matmul_o_->set_norm (n);
   return (*matmul_o_) (heads);
 }
 

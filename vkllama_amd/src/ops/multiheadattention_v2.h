@@ -45,6 +45,8 @@ public:
 
   // the next call only: the residual is added in the output projection's launch
   void set_residual (const Tensor *r) noexcept { residual_ = r; }
+  // the next call only: the norm of the output's rows (MatMul::set_norm)
+  void set_norm (RMSNorm *n) noexcept { norm_ = n; }
 
   Tensor &wk () { return wk_; }
   Tensor &wq () { return wq_; }
@@ -56,6 +58,7 @@ public:
 
 private:
   const Tensor *residual_ = nullptr;
+  RMSNorm *norm_ = nullptr;
   Tensor wk_, wq_, wv_, wo_;
   Tensor kcache_, vcache_;
   const int maxlen_;

@@ -31,6 +31,19 @@ RMSNorm::time () noexcept
   return timer_.micros ();
 }
 
+absl::Status
+RMSNorm::prepare (size_t rows, size_t width) noexcept
+{
+  if (weight_.size () < width)
+    return absl::InvalidArgumentError (absl::StrFormat (
+        "rms_norm weight has %zu elements but input0 width is %zu",
+        weight_.size (), width));
+  if (out_.channels () == 1 && out_.height () == rows && out_.width () == width)
+    return absl::OkStatus ();
+  out_ = Tensor (1, rows, width, dev_, dtype_, false);
+  return out_.create ();
+}
+
 absl::StatusOr<Tensor>
 RMSNorm::operator() (Tensor x) noexcept
 {

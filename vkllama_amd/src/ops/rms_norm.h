@@ -17,6 +17,10 @@ public:
   // for fused callers
   Tensor &weight () { return weight_; }
   float eps () const { return eps_; }
+  // for a product that writes the norm of its own rows: the output of the next
+  // call with [1, rows, width], and what it holds
+  absl::Status prepare (size_t rows, size_t width) noexcept;
+  Tensor &output () { return out_; }
 
 private:
   Tensor weight_;

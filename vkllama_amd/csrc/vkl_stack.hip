@@ -1091,6 +1091,241 @@ launch_rows (const RowAttnArgs &a, int ht, dim3 grid, hipStream_t s)
   return launch_rows_ht<CT, 64, 2, VALS> (a, ht, grid, s);
 }
 
+// ---- many 32-bit query rows -----------------------------------------------------
+// The attention of a 32-bit prompt: sixteen queries of a head per workgroup, whose four waves walk blocks of sixteen
+// rows in turn (wave w every fourth) with a running maximum of their own and meet in LDS at the end.  Both products are
+// v_mfma_f32_16x16x4_f32, the scores transposed (S^T = K Q^T, O^T = V^T P^T): a result's lane holds four rows
+// 4 (lane / 16) .. + 3 of query lane % 16, which is how the second product takes its right operand.  Rows
+// go from memory into the registers as the first operand lies (k = 32 (b / 2) + 8 (lane / 16) + 4 (b % 2) + e in step (b, e),
+// so that two loads fetch whole lines) or, as values, four columns 64 g + 4 (lane % 16) .. + 3 of a row, one for each of four blocks of columns.
+//
+// Bound by what a compute unit fetches: 64 KB take 1.45 us, the products of it 0.85 at 128 values (eight waves per
+// workgroup were no faster).  The row kernel multiplies the same pairs on the vector ALU, one query row per workgroup, for each of which all rows
+// are fetched anew.  us, row kernel / this: 16 heads of 128 sharing 4, 300 rows 33.3 / 15.2, 800 140 / 46.9, in chunks of 256
+// 65 / 25; 100 rows 10.7 / 8.1; 32 heads, 2000 rows 1391 / 369; 16 heads of 64, 300 rows 36.6 / 9.3.  Error against 64 bits as
+// before or less (300 rows 1.1e-7 / 9.8e-8, 64 behind 1936 2.1e-7 / 1.7e-7): a block of rows has sums of its own.
+//
+// Rows that only some queries see meet weights of zero in the second product.  A value there that is not finite must not
+// reach the others: such a block (none but the last and, with chunks, the first of a tile) is added value by value.
+constexpr int kTq = 16, kTqWaves = 4;
+
+template <int D>
+__global__ __launch_bounds__ (kTqWaves * 64, 8 / kTqWaves) void
+attn_f32_tiles_kernel (const RowAttnArgs a, int S)
+{
+  constexpr int NB = D / 16, NG = D / 64, LDO = D + 4;
+  __shared__ __align__ (16) float so[kTqWaves][kTq][LDO];
+  __shared__ float sm[kTqWaves][kTq], sl[kTqWaves][kTq];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane (tid >> 6);
+  const int lo = lane & 15, hi = lane >> 4;
+  // (the longest contexts first, a head's tiles on one XCD where the heads are a multiple of 8)
+  const int s0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * kTq, head = blockIdx.x, g = head / a.rep;
+  const uint32_t p0 = a.pos.get ();
+  auto start = [&] (uint32_t pos) { return a.chunk ? (int)(pos / (uint32_t)a.chunk * (uint32_t)a.chunk) : 0; };
+  const int own = (int)p0 + s0 + lo, low = start ((uint32_t)own);  // rows low .. own are visible to this lane's query
+  const int last = (int)p0 + min (s0 + kTq, S) - 1;                // of the tile
+  const int b0 = start (p0 + (uint32_t)s0) / 16, b1 = last / 16;   // blocks of rows
+  const float *kr = (const float *)a.rows + (size_t)g * D;
+  const float *vr = (const float *)(a.vals ? a.vals : a.rows) + (size_t)g * D;
+
+  float4v q[NB];
+  {
+    float f = a.scale;
+    if (a.tcoef != 0.f)
+      f *= 1.0f + a.tcoef * logf ((float)(((uint32_t)own + 1u) / (uint32_t)a.tevery + 1u));
+    const float *src = (const float *)a.q + (size_t)min (s0 + lo, S - 1) * a.qs + (size_t)head * D + 8 * hi;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+      q[b] = __builtin_bit_cast (float4v, ldg4 (src + 32 * (b / 2) + 4 * (b % 2))) * f;
+  }
+  // (keys are requested a block ahead, values when their block begins: they have the first product's time)
+  struct Keys
+  {
+    float4v k[NB];
+  };
+  auto fetch = [&] (int blk, Keys &r) {
+    const float *ks = kr + (size_t)min (blk * 16 + lo, last) * a.rs + 8 * hi;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+      r.k[b] = __builtin_bit_cast (float4v, ldg4 (ks + 32 * (b / 2) + 4 * (b % 2)));
+  };
+  // (the sink is a row without a value that the first wave has seen)
+  float m = a.sink && wave == 0 ? 0.f : kNoKey, l = a.sink && wave == 0 && hi == 0 ? 1.f : 0.f;
+  float4v o[NG][4];
+#pragma unroll
+  for (int n = 0; n < NG; ++n)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      o[n][j] = float4v{ 0.f, 0.f, 0.f, 0.f };
+  auto block = [&] (int blk, const Keys &r, Keys &next) {
+    float4v v[4][NG];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      {
+        const float *vs = vr + (size_t)min (blk * 16 + 4 * hi + e, last) * a.rs + 4 * lo;
+#pragma unroll
+        for (int n = 0; n < NG; ++n)
+          v[e][n] = __builtin_bit_cast (float4v, ldg4 (vs + 64 * n));
+      }
+    fetch (min (blk + kTqWaves, b1), next);
+    __builtin_amdgcn_sched_barrier (0);
+    float4v s = { 0.f, 0.f, 0.f, 0.f }, t = s;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; e += 2)
+        {
+          s = __builtin_amdgcn_mfma_f32_16x16x4f32 (r.k[b][e], q[b][e], s, 0, 0, 0);
+          t = __builtin_amdgcn_mfma_f32_16x16x4f32 (r.k[b][e + 1], q[b][e + 1], t, 0, 0, 0);
+        }
+    s += t;
+    const int row = blk * 16 + 4 * hi;
+    float mx = m;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      {
+        s[e] = row + e <= own && row + e >= low ? s[e] : kNoKey;
+        mx = fmaxf (mx, s[e]);
+      }
+    {
+      const auto r16 = __builtin_amdgcn_permlane16_swap (__float_as_uint (mx), __float_as_uint (mx), false, false);
+      mx = fmaxf (__uint_as_float (r16[0]), __uint_as_float (r16[1]));
+      const auto r32 = __builtin_amdgcn_permlane32_swap (__float_as_uint (mx), __float_as_uint (mx), false, false);
+      mx = fmaxf (__uint_as_float (r32[0]), __uint_as_float (r32[1]));
+    }
+    const float al = expf (m - mx);
+    m = mx;
+    l *= al;
+    float4v p;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      {
+        p[e] = s[e] > kNoKey ? expf (s[e] - mx) : 0.f;
+        l += p[e];
+      }
+    // whether all queries see all rows of the block, and if not whether its values are finite
+    const bool all = blk * 16 + 15 <= (int)p0 + s0 && (!a.chunk || blk * 16 >= start ((uint32_t)last));
+    float odd = 0.f;
+    if (!all)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int n = 0; n < NG; ++n)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            odd = __builtin_fmaf (v[e][n][j], 0.f, odd);
+    if (all || __builtin_amdgcn_ballot_w64 (odd != 0.f) == 0)
+      {
+        // (a block's sum by itself: fewer roundings along the context than in one accumulator)
+        float4v u[NG][4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int n = 0; n < NG; ++n)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              u[n][j] = __builtin_amdgcn_mfma_f32_16x16x4f32 (v[e][n][j], p[e], e ? u[n][j] : float4v{ 0.f, 0.f, 0.f, 0.f }, 0, 0, 0);
+#pragma unroll
+        for (int n = 0; n < NG; ++n)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              o[n][j][e] = __builtin_fmaf (o[n][j][e], al, u[n][j][e]);
+        return;
+      }
+#pragma unroll
+    for (int n = 0; n < NG; ++n)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        o[n][j] *= al;
+#pragma unroll 1
+    for (int i = 0; i < 16; ++i)
+      {
+        const float pe = i % 4 == 0 ? p[0] : i % 4 == 1 ? p[1] : i % 4 == 2 ? p[2] : p[3];
+        const float w = __shfl (pe, 16 * (i / 4) + lo, 64);
+        const int key = blk * 16 + i;
+        const bool seen = key <= own && key >= low;
+        const float *vs = vr + (size_t)min (key, last) * a.rs + 16 * hi;
+#pragma unroll
+        for (int n = 0; n < NG; ++n)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            {
+              const float4v x = __builtin_bit_cast (float4v, ldg4 (vs + 64 * n + 4 * e));
+#pragma unroll
+              for (int j = 0; j < 4; ++j)
+                o[n][j][e] = seen ? __builtin_fmaf (w, x[j], o[n][j][e]) : o[n][j][e];
+            }
+      }
+  };
+  Keys x, y;
+  fetch (min (b0 + wave, b1), x);
+  for (int b = b0 + wave; b <= b1; b += 2 * kTqWaves)
+    {
+      block (b, x, y);
+      if (b + kTqWaves > b1)
+        break;
+      block (b + kTqWaves, y, x);
+    }
+  l += __shfl_xor (l, 16, 64);
+  l += __shfl_xor (l, 32, 64);
+  if (hi == 0)
+    sm[wave][lo] = m, sl[wave][lo] = l;
+  // register e of blocks 0 .. 3 of a group: columns 64 n + 16 hi + 4 e .. + 3
+#pragma unroll
+  for (int n = 0; n < NG; ++n)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      *(float4v *)&so[wave][lo][64 * n + 16 * hi + 4 * e] = float4v{ o[n][0][e], o[n][1][e], o[n][2][e], o[n][3][e] };
+  __syncthreads ();
+  const int i = (tid >> 4) & 15;
+  if (s0 + i >= S)
+    return;
+  float M = sm[0][i], w[kTqWaves], L = 0.f;
+#pragma unroll
+  for (int k = 1; k < kTqWaves; ++k)
+    M = fmaxf (M, sm[k][i]);
+#pragma unroll
+  for (int k = 0; k < kTqWaves; ++k)
+    {
+      w[k] = expf (sm[k][i] - M);
+      L = __builtin_fmaf (w[k], sl[k][i], L);
+    }
+  for (int n = tid >> 8; n < NG; n += kTqWaves / 4)
+    {
+      const int d = 64 * n + 4 * (tid & 15);
+      float4v r = { 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+      for (int k = 0; k < kTqWaves; ++k)
+        r += w[k] * *(const float4v *)&so[k][i][d];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        store_elem (a.out, a.otype, (size_t)(s0 + i) * a.os + (size_t)head * D + d + e, r[e] / L);
+    }
+}
+
+// Whether many query rows take the kernel above.  It walks a long context in one workgroup, the row kernel in up to 32:
+// few rows behind many stay there.  us: 1.45 per four blocks of the longest tile, or of all tiles dealt to 256 compute units; the row
+// kernel 30000 pairs of a query and a row in one.  Row kernel / tiles: 16 heads, 16 rows 6.9 / 5.2, 64 behind 1936 60 / 50,
+// 32 behind 968 22 / 28, 20 behind 3980 45 / 93; 4 heads, 16 behind 3984 18 / 91.
+bool
+f32_tiles (const RowAttnArgs &a, int ctype, int H, int S)
+{
+  if (ctype != VKL_TYPE_F32 || a.qtype != VKL_TYPE_F32 || (a.D != 64 && a.D != 128) || S < kTq || a.pos.loop
+      || (uint64_t)a.pos.val + (uint64_t)S >= (1u << 31) || (a.qs % 4) != 0 || ((uintptr_t)a.q % 16) != 0)
+    return false;
+  double longest = 0, all = 0, pairs = 0;
+  for (int s0 = 0; s0 < S; s0 += kTq)
+    {
+      const uint32_t first = a.pos.val + (uint32_t)s0, last = a.pos.val + (uint32_t)std::min (s0 + kTq, S) - 1;
+      const uint32_t low = a.chunk ? first / (uint32_t)a.chunk * (uint32_t)a.chunk : 0u;
+      const double rounds = (last / 16 - low / 16 + kTqWaves) / kTqWaves;
+      longest = std::max (longest, rounds), all += rounds * H, pairs += (double)(last - low + 1) * kTq * H;
+    }
+  return 4 + 1.45 * std::max (longest, all / 256) < 6.5 + pairs / 30000;
+}
+
 size_t
 row_scratch_bytes (int ctype, int H, int G, int D, int S, bool vals = false)
 {
@@ -1117,8 +1352,18 @@ row_step (int D)
 int
 rows_launch (RowAttnArgs a, int ctype, int H, int S, void *scratch, RowParts *parts, hipStream_t s)
 {
+  a.rep = H / a.G;
+  if (!parts && f32_tiles (a, ctype, H, S))
+    {
+      const dim3 grid ((unsigned)H, (unsigned)((S + kTq - 1) / kTq));
+      if (a.D == 128)
+        attn_f32_tiles_kernel<128><<<grid, dim3 (kTqWaves * 64), 0, s>>> (a, S);
+      else
+        attn_f32_tiles_kernel<64><<<grid, dim3 (kTqWaves * 64), 0, s>>> (a, S);
+      return (int)hipGetLastError ();
+    }
   const RowPlan p = row_plan (ctype, H, a.G, a.D, S, a.vals != nullptr);
-  a.rep = H / a.G, a.tiles = p.tiles, a.ht = p.ht, a.nsplit = p.nsplit;
+  a.tiles = p.tiles, a.ht = p.ht, a.nsplit = p.nsplit;
   a.cnt = parts ? nullptr : (uint32_t *)scratch;
   a.pm = (float *)((uint8_t *)scratch + kRowCounterBytes);
   a.pl = a.pm + p.parts;

@@ -820,53 +820,93 @@ attn_tiles_kernel (const AttnArgs a)
       }
 }
 
-// adds the parts of the keys up: one wave per query row and head
+// Adds the parts of the keys up: HD / 8 lanes per query row and head, eight values each.  Bound by latency: the maxima and
+// sums and the values of four parts are requested at once (a wave per row with a trip to memory for each part took
+// 2 to 3 us longer: 16 heads, 1500 rows behind 600 keys, both launches 43.8 / 41.0; 32 heads, one row behind 2047 14.9 / 12.4, 77
+// behind 1500 18.7 / 17.7).
 template <int HD, class E>
 __global__ __launch_bounds__ (256) void
 attn_parts_kernel (const AttnArgs a)
 {
-  constexpr int VPL = HD / 64; // values per lane
-  const int i = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), lane = threadIdx.x & 63;
-  const int row = i / a.H, head = i - row * a.H;
-  if (row >= a.S)
-    return;
+  typedef float f32x4 __attribute__ ((ext_vector_type (4)));
+  constexpr int LPR = HD / 8, SPL = 16 / LPR; // lanes of a row; parts whose maxima a lane looks at
+  const int i = (int)((blockIdx.x * 256 + threadIdx.x) / LPR), sub = (int)threadIdx.x % LPR;
+  const int head = i % a.H, row = min (i / a.H, a.S - 1);
   const int parts = parts_of (a, key_tiles (a, row / kBQ * kBQ));
-  // lane p looks at part p
-  float pm = -3.0e38f, ps = 0.f;
-  if (lane < parts)
-    {
-      const float *pr = part_row<HD> (a, lane, head, row);
-      pm = vkl::ldg (pr + HD), ps = vkl::ldg (pr + HD + 1);
-    }
-  float top = pm;
+  f32x4 x[4][2];
+  auto request = [&] (int p0) {
 #pragma unroll
-  for (int d = 32; d > 0; d >>= 1)
+    for (int j = 0; j < 4; ++j)
+      {
+        const float *pr = part_row<HD> (a, min (p0 + j, parts - 1), head, row) + sub * 8;
+        x[j][0] = *(const VKL_GLOBAL f32x4 *)pr, x[j][1] = *(const VKL_GLOBAL f32x4 *)(pr + 4);
+      }
+  };
+  float pm[SPL], ps[SPL];
+#pragma unroll
+  for (int k = 0; k < SPL; ++k)
+    {
+      const float *pr = part_row<HD> (a, min (sub + k * LPR, parts - 1), head, row);
+      pm[k] = vkl::ldg (pr + HD), ps[k] = vkl::ldg (pr + HD + 1);
+    }
+  request (0);
+  float gate = 0.f;
+  if (a.gate)
+    gate = vkl::ldg (a.gate + (size_t)row * a.gs + head);
+  float top = -3.0e38f;
+#pragma unroll
+  for (int k = 0; k < SPL; ++k)
+    {
+      pm[k] = sub + k * LPR < parts ? pm[k] : -3.0e38f;
+      top = fmaxf (top, pm[k]);
+    }
+#pragma unroll
+  for (int d = LPR / 2; d > 0; d >>= 1)
     top = fmaxf (top, __shfl_xor (top, d, 64));
-  const float w = lane < parts ? __builtin_amdgcn_exp2f (pm - top) : 0.f;
-  float total = w * ps;
+  float w[SPL], total = 0.f;
 #pragma unroll
-  for (int d = 32; d > 0; d >>= 1)
-    total += __shfl_xor (total, d, 64);
-  float o[VPL];
-#pragma unroll
-  for (int e = 0; e < VPL; ++e)
-    o[e] = 0.f;
-  for (int p = 0; p < parts; ++p)
+  for (int k = 0; k < SPL; ++k)
     {
-      const float wp = __shfl (w, p, 64);
-      const float *pr = part_row<HD> (a, p, head, row) + lane * VPL;
-#pragma unroll
-      for (int e = 0; e < VPL; ++e)
-        o[e] = __builtin_fmaf (wp, vkl::ldg (pr + e), o[e]);
+      const bool in = sub + k * LPR < parts;
+      w[k] = in ? __builtin_amdgcn_exp2f (pm[k] - top) : 0.f;
+      total += in ? w[k] * ps[k] : 0.f;
     }
+#pragma unroll
+  for (int d = LPR / 2; d > 0; d >>= 1)
+    total += __shfl_xor (total, d, 64);
+  float o[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    o[e] = 0.f;
+  const int base = ((int)threadIdx.x & 63) - sub;
+  for (int p0 = 0; p0 < a.parts; p0 += 4) // (a.parts: the most of any row)
+    {
+      if (p0 > 0)
+        request (p0);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        {
+          const int p = p0 + j;
+          const float wp = __shfl (SPL == 2 && p >= LPR ? w[SPL - 1] : w[0], base + p % LPR, 64);
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            o[e] = p < parts ? __builtin_fmaf (wp, x[j][e >> 2][e & 3], o[e]) : o[e];
+        }
+    }
+  if (i / a.H >= a.S)
+    return;
   float inv = 1.0f / total;
   if (a.gate)
-    inv = inv / (1.0f + expf (-vkl::ldg (a.gate + (size_t)row * a.gs + head)));
-  uint16_t *op = a.out + (size_t)row * a.ors + (size_t)head * a.ohs + lane * VPL;
-  if constexpr (VPL == 2)
-    *(VKL_GLOBAL uint32_t *)op = (uint32_t)E::bits (o[0] * inv) | ((uint32_t)E::bits (o[1] * inv) << 16);
-  else
-    *op = E::bits (o[0] * inv);
+    inv = inv / (1.0f + expf (-gate));
+  uint16_t *op = a.out + (size_t)row * a.ors + (size_t)head * a.ohs + sub * 8;
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    {
+      u32x2 v;
+      v.x = (uint32_t)E::bits (o[4 * h] * inv) | ((uint32_t)E::bits (o[4 * h + 1] * inv) << 16);
+      v.y = (uint32_t)E::bits (o[4 * h + 2] * inv) | ((uint32_t)E::bits (o[4 * h + 3] * inv) << 16);
+      *(VKL_GLOBAL u32x2 *)(op + 4 * h) = v;
+    }
 }
 
 // Into how many parts the keys go, where two workgroups fit a compute unit and fewer than
@@ -978,7 +1018,7 @@ launch_tiles (AttnArgs a, hipStream_t s)
       return vkl_launch_status ();
     }
   attn_tiles_kernel<HD, E, CHUNKED, true><<<dim3 ((unsigned)(groups * a.parts)), dim3 (kThreads), 0, s>>> (a);
-  attn_parts_kernel<HD, E><<<dim3 ((unsigned)((a.S * a.H + 3) / 4)), dim3 (256), 0, s>>> (a);
+  attn_parts_kernel<HD, E><<<dim3 ((unsigned)(((size_t)a.S * a.H * (HD / 8) + 255) / 256)), dim3 (256), 0, s>>> (a);
   return vkl_launch_status ();
 }
 

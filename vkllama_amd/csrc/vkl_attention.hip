@@ -537,8 +537,11 @@ parts_of (const AttnArgs &a, int n)
   return a.span ? (n + a.span - 1) / a.span : a.parts;
 }
 
-template <int HD, class E, bool CHUNKED, bool PARTS>
-__global__ __launch_bounds__ (kThreads, 2) void
+// PAIR: two groups of four waves take every other tile of keys each, with a maximum and sums of their own, and meet in LDS
+// at the end: a workgroup that has its compute unit alone then has a second wave per SIMD, which multiplies while the first
+// one forms its weights.
+template <int HD, class E, bool CHUNKED, bool PARTS, bool PAIR>
+__global__ __launch_bounds__ (PAIR ? 2 * kThreads : kThreads, 2) void
 attn_tiles_kernel (const AttnArgs a)
 {
   typedef typename E::v8 v8;
@@ -549,7 +552,8 @@ attn_tiles_kernel (const AttnArgs a)
   constexpr int LPW = TILE / 1024 / 4;   // loads per wave and tile
   // four objects: a read of one is then not made to wait for the loads on their way into
   // another
-  __shared__ __align__ (16) uint8_t lk0[TILE], lv0[TILE], lk1[TILE], lv1[TILE];
+  constexpr int GROUPS = PAIR ? 2 : 1;
+  __shared__ __align__ (16) uint8_t lk0[GROUPS * TILE], lv0[GROUPS * TILE], lk1[GROUPS * TILE], lv1[GROUPS * TILE];
 
   int head, qt, part = 0;
   {
@@ -559,7 +563,8 @@ attn_tiles_kernel (const AttnArgs a)
     tile_of (a, b, head, qt);
   }
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane (threadIdx.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane ((threadIdx.x >> 6) & 3);
+  const int group = PAIR ? __builtin_amdgcn_readfirstlane (threadIdx.x >> 8) : 0;
   const int lq = lane & 31, hh = lane >> 5;
   const int q0 = qt * kBQ;
   const int qrow = q0 + wave * 32 + lq; // this lane's query
@@ -615,16 +620,16 @@ attn_tiles_kernel (const AttnArgs a)
         const size_t key = (size_t)min (t * kBKey + r, a.L - 1);
         const int col = ((lane % CPR) ^ swizzle<HD> (r)) * 8;
         __builtin_amdgcn_global_load_lds ((const VKL_GLOBAL void *)(kb + key * a.khs + col),
-                                          (VKL_LDS void *)(lk + (wave + 4 * i) * 1024), 16, 0, 0);
+                                          (VKL_LDS void *)(lk + group * TILE + (wave + 4 * i) * 1024), 16, 0, 0);
         __builtin_amdgcn_global_load_lds ((const VKL_GLOBAL void *)(vb + key * a.vhs + col),
-                                          (VKL_LDS void *)(lv + (wave + 4 * i) * 1024), 16, 0, 0);
+                                          (VKL_LDS void *)(lv + group * TILE + (wave + 4 * i) * 1024), 16, 0, 0);
       }
   };
   // reads of K: key l % 32 of a block, values 16 kt + 8 (l / 32) .. + 7
   uint32_t koff[KT];
 #pragma unroll
   for (int kt = 0; kt < KT; ++kt)
-    koff[kt] = lq * ROWB + (((2 * kt + hh) ^ swizzle<HD> (lq)) << 4);
+    koff[kt] = group * TILE + lq * ROWB + (((2 * kt + hh) ^ swizzle<HD> (lq)) << 4);
   // reads of V: of sixteen lanes four each give the columns 16 ((l / 16) % 2) .. + 15 of four
   // neighbouring keys from 8 g + 4 (l / 32) on, of which each receives one column
   uint32_t voff[DB][2];
@@ -635,14 +640,14 @@ attn_tiles_kernel (const AttnArgs a)
       {
         const int key = 8 * g + 4 * hh + ((lane & 15) >> 2);
         const int chunk = 4 * db + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
-        voff[db][g] = key * ROWB + ((chunk ^ swizzle<HD> (key)) << 4) + (lane & 1) * 8;
+        voff[db][g] = group * TILE + key * ROWB + ((chunk ^ swizzle<HD> (key)) << 4) + (lane & 1) * 8;
       }
 
   // (the sink is a key that every query has seen before the first tile; the sums of the
   // two lane halves are added at the end, one of them has it)
   // (a tile may hold no key that a query sees: its first maximum lies far above the score
   // of a hidden key, whose weight is then zero)
-  const bool sink = CHUNKED && a.sink && part == 0;
+  const bool sink = CHUNKED && a.sink && part == 0 && group == 0;
   float m = sink ? 0.f : 0.1f * kNeg, sum = sink && hh == 0 ? 1.f : 0.f;
   float16v oacc[DB];
 #pragma unroll
@@ -657,9 +662,9 @@ attn_tiles_kernel (const AttnArgs a)
     __builtin_amdgcn_s_waitcnt (0x0f70);
     __builtin_amdgcn_s_barrier ();
     __builtin_amdgcn_sched_barrier (0);
-    if (t + 1 < t1)
-      issue (t + 1, kn, vn);
-    if (t * kBKey > wave_last || (CHUNKED && t * kBKey + kBKey <= wave_low))
+    if (t + GROUPS < t1)
+      issue (t + GROUPS, kn, vn);
+    if ((PAIR && t >= t1) || t * kBKey > wave_last || (CHUNKED && t * kBKey + kBKey <= wave_low))
       return;
     const bool inner = t * kBKey + kBKey - 1 <= q0 + wave * 32 + shift // every key visible to every query of the wave
                        && (!CHUNKED || t * kBKey >= wave_high);
@@ -775,16 +780,50 @@ attn_tiles_kernel (const AttnArgs a)
     Alternate<0x100, 2, 4 * DB, 4>::run ();
     __builtin_amdgcn_sched_barrier (0);
   };
-  if (t0 < t1)
-    issue (t0, lk0, lv0);
-  for (int t = t0; t < t1; t += 2)
+  if (t0 + group < t1)
+    issue (t0 + group, lk0, lv0);
+  // (both groups take as many steps, and barriers: the last of the second may be empty)
+  for (int t = t0; t < t1; t += 2 * GROUPS)
     {
-      step (t, lk0, lv0, lk1, lv1);
-      if (t + 1 < t1)
-        step (t + 1, lk1, lv1, lk0, lv0);
+      step (t + group, lk0, lv0, lk1, lv1);
+      if (t + GROUPS < t1)
+        step (t + GROUPS + group, lk1, lv1, lk0, lv0);
     }
   // the other half of the lanes has summed the other keys of the same query
   sum += __shfl_xor (sum, 32, 64);
+  if constexpr (PAIR)
+    {
+      typedef float f32x4 __attribute__ ((ext_vector_type (4)));
+      typedef float f32x2 __attribute__ ((ext_vector_type (2)));
+      static_assert (DB * 4 * 1024 + 512 <= GROUPS * TILE, "");
+      __syncthreads (); // every wave has read its last tile
+      uint8_t *at = wave == 0 ? lk0 : wave == 1 ? lv0 : wave == 2 ? lk1 : lv1;
+      f32x4 *ov = (f32x4 *)at + lane;
+      f32x2 *st = (f32x2 *)(at + DB * 4 * 1024) + lane;
+      if (group)
+        {
+#pragma unroll
+          for (int i = 0; i < DB * 4; ++i)
+            ov[i * 64] = f32x4{ oacc[i / 4][4 * (i % 4)], oacc[i / 4][4 * (i % 4) + 1], oacc[i / 4][4 * (i % 4) + 2],
+                                oacc[i / 4][4 * (i % 4) + 3] };
+          *st = f32x2{ m, sum };
+        }
+      __syncthreads ();
+      if (group)
+        return;
+      const f32x2 other = *st;
+      const float mn = fmaxf (m, other.x);
+      const float w0 = __builtin_amdgcn_exp2f ((m - mn) * c), w1 = __builtin_amdgcn_exp2f ((other.x - mn) * c);
+      m = mn, sum = w0 * sum + w1 * other.y;
+#pragma unroll
+      for (int i = 0; i < DB * 4; ++i)
+        {
+          const f32x4 x = ov[i * 64];
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            oacc[i / 4][4 * (i % 4) + e] = w0 * oacc[i / 4][4 * (i % 4) + e] + w1 * x[e];
+        }
+    }
   if (PARTS)
     {
       if (qrow >= a.S)
@@ -993,6 +1032,21 @@ plan_parts (AttnArgs &a, int hd)
     a.parts = 3;
 }
 
+// Whether the workgroups of a launch in one part, each of which has a compute unit alone, are of two groups of waves: from ten
+// tiles of keys on, where half of the tiles saves more than the meeting at the end costs (2 us).  us, four waves / eight: 16 heads of 128, 450 rows
+// 13.0 / 13.1, 640 16.7 / 16.2, 1000 23.1 / 20.5, 1500 32.7 / 27.5, 2048 43.5 / 35.7; 32 heads, 768 rows 19.7 / 18.6, 1024 24.4 / 22.1; 16
+// heads of 64, 700 rows 12.7 / 11.1; 128 rows 7.1 / 9.2.
+constexpr int kPairTiles = 10;
+
+bool
+tile_pairs (const AttnArgs &a)
+{
+  int most = 0;
+  for (int q0 = 0; q0 < a.S; q0 += kBQ)
+    most = std::max (most, key_tiles (a, q0));
+  return a.ntq * a.H <= 256 && most >= kPairTiles;
+}
+
 template <int HD, class E, bool CHUNKED>
 int
 launch_tiles (AttnArgs a, hipStream_t s)
@@ -1014,10 +1068,13 @@ launch_tiles (AttnArgs a, hipStream_t s)
   if (!a.ws)
     {
       a.parts = 1, a.span = 0;
-      attn_tiles_kernel<HD, E, CHUNKED, false><<<dim3 ((unsigned)groups), dim3 (kThreads), 0, s>>> (a);
+      if (tile_pairs (a))
+        attn_tiles_kernel<HD, E, CHUNKED, false, true><<<dim3 ((unsigned)groups), dim3 (2 * kThreads), 0, s>>> (a);
+      else
+        attn_tiles_kernel<HD, E, CHUNKED, false, false><<<dim3 ((unsigned)groups), dim3 (kThreads), 0, s>>> (a);
       return vkl_launch_status ();
     }
-  attn_tiles_kernel<HD, E, CHUNKED, true><<<dim3 ((unsigned)(groups * a.parts)), dim3 (kThreads), 0, s>>> (a);
+  attn_tiles_kernel<HD, E, CHUNKED, true, false><<<dim3 ((unsigned)(groups * a.parts)), dim3 (kThreads), 0, s>>> (a);
   attn_parts_kernel<HD, E><<<dim3 ((unsigned)(((size_t)a.S * a.H * (HD / 8) + 255) / 256)), dim3 (256), 0, s>>> (a);
   return vkl_launch_status ();
 }

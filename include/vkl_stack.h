@@ -350,6 +350,11 @@ int vkl_stack_supported (const vkl_stack_model *m);
 int vkl_stack_step (const vkl_stack_model *m, const uint32_t *tok,
                     uint32_t pos, float *logits32, uint32_t *next_tok,
                     void *stream);
+/* One layer run of the step by itself, for one row x [width_p] of the residual
+ * stream, in place (16-byte aligned; values behind `width` zero): the token at pos,
+ * whose row of the cache it writes; those before it are there. */
+int vkl_stack_layer_step (const vkl_stack_model *m, int run, float *x,
+                          uint32_t pos, void *stream);
 /* The step's last launch by itself: logits32 [vocab] of one row x [width_p] of the
  * residual stream (final norm, output matrix, soft cap), all in fp32. */
 int vkl_stack_logits (const vkl_stack_model *m, const float *x, float *logits32,

@@ -2765,6 +2765,20 @@ vkl_stack_step (const vkl_stack_model *m, const uint32_t *tok, uint32_t pos, flo
 // one row of 128-row tiles before / this launch, 2048 wide bf16 3.1 + 30.7 / 21, 4096 wide 4.6 +
 // 65.4 / 41, 2048 wide fp32 (split into planes as well) 3.4 + 1.9 + 50.8 / 21.
 extern "C" int
+vkl_stack_layer_step (const vkl_stack_model *m, int run, float *x, uint32_t pos, void *stream)
+{
+  if (int e = check_stack (m))
+    return e;
+  VKL_CHECK_ARG (run >= 0 && run < m->n_runs && x && ((uintptr_t)x % 16) == 0 && pos < (uint32_t)m->maxlen);
+  StepArgs p = {};
+  p.m = m, p.s = carve_stack (m), p.pos = { nullptr, pos }, p.stream = weights_stream (*m);
+  p.s.x = x;
+  if (int e = compute_units (&p.n_cu))
+    return e;
+  return launch_stack_layer (p, m->layers_h[run], (hipStream_t)stream);
+}
+
+extern "C" int
 vkl_stack_logits (const vkl_stack_model *m, const float *x, float *logits32, void *stream)
 {
   if (int e = check_stack (m))

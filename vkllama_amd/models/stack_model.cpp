@@ -54,7 +54,7 @@ StackBlock::norm_weights_ (const WeightSource &w, const std::string &name)
 
 absl::Status
 StackBlock::norm_product_ (const char *what, Tensor &x, int S, Tensor &norm, Tensor &w, int n,
-                           std::vector<vkl_out_seg> const &segs, Buffers &b)
+                           std::vector<vkl_out_seg> const &segs, Buffers &b, int first)
 {
   vkl_add_norm_project p = {};
   if (b.back)
@@ -62,8 +62,25 @@ StackBlock::norm_product_ (const char *what, Tensor &x, int S, Tensor &norm, Ten
   b.back = nullptr;
   p.y = (float *)x.data (), p.ys = (size_t)width_p_, p.W = width_;
   p.norm = (const float *)norm.data (), p.eps = eps_, p.h = b.h.data (), p.hs = (size_t)width_p_, p.Wp = width_p_;
-  p.w_next = w.data (), p.N = n, p.segs = segs.data (), p.nseg = (int)segs.size ();
+  p.w_next = (const uint16_t *)w.data () + (size_t)first * width_p_, p.N = n, p.segs = segs.data (), p.nseg = (int)segs.size ();
   return launched (what, vkl_add_norm_project_bf16w (&p, dtype_ == FP32 ? VKL_TYPE_F32 : VKL_TYPE_BF16, S, dev_->stream ()));
+}
+
+absl::Status
+StackBlock::keep_ (Tensor &x, int S, size_t offset, int run, Tensor &norm, Tensor &w, Buffers &b)
+{
+  const TokenMixer::Rows r = mixer_->kept_rows ();
+  auto segs = mixer_->segments (S, offset, run);
+  VKLLAMA_STATUS_OK (segs);
+  std::vector<vkl_out_seg> kept;
+  for (vkl_out_seg s : *segs)
+    if (s.n0 >= r.first && s.n0 < r.first + r.n)
+      {
+        s.n0 -= r.first;
+        kept.push_back (s);
+      }
+  VKLLAMA_STATUS_OK (norm_product_ ("product of what is kept", x, S, norm, w, r.n, kept, b, r.first));
+  return mixer_->keep (S, offset, run);
 }
 
 absl::Status
@@ -316,9 +333,14 @@ StackModel::put_tokens_ (std::vector<uint32_t> const &toks)
   return toks_.flush ();
 }
 
-// S tokens from number `first` of the call on through every layer; leaves the residual stream in x_
+// S tokens from number `first` of the call on through every layer; leaves the residual stream in x_.  last_only: only
+// the last token's row of it is wanted.  Behind the layers' last mixing of tokens nothing reads the others, so the last
+// layer takes what it keeps of all tokens (a product with a few rows of its matrix) and is the one-token step's layer
+// for the last one, whose row it keeps once more.  Passes of four layers, us before / now: 1500 tokens behind 600, Fazinex
+// 2048 wide 757 / 627; 2048 tokens, Fuzuvik 4096 wide 2953 / 2528; 300 in 32-bit, 2048 wide 743 / 657.  Recurrences need all
+// that feeds them, and stay.
 absl::Status
-StackModel::pass_ (size_t first, int S, size_t offset, std::vector<float> *streams)
+StackModel::pass_ (size_t first, int S, size_t offset, std::vector<float> *streams, bool last_only)
 {
   void *s = gpu_->stream ();
   VKLLAMA_STATUS_OK (reserve (x_, S, width_p_, gpu_, FP32));
@@ -337,6 +359,12 @@ StackModel::pass_ (size_t first, int S, size_t offset, std::vector<float> *strea
   for (size_t n = 0; n < cfg_.order.size (); ++n)
     {
       const size_t i = (size_t)cfg_.order[n];
+      if (last_only && n + 1 == cfg_.order.size () && blocks_[i]->can_keep ())
+        {
+          VKLLAMA_STATUS_OK (blocks_[i]->keep (x_, S, offset, seen[i], buf_));
+          return launched ("last layer", vkl_stack_layer_step (&plan_->desc (), (int)n, xp + (size_t)(S - 1) * width_p_,
+                                                               (uint32_t)(offset + (size_t)S - 1), s));
+        }
       VKLLAMA_STATUS_OK ((*blocks_[i]) (x_, S, offset, seen[i]++, buf_));
       if (streams || n + 1 == cfg_.order.size ())
         VKLLAMA_STATUS_OK (blocks_[i]->finish (x_, S, buf_));
@@ -386,7 +414,12 @@ StackModel::forward_ (std::vector<uint32_t> const &toks, const size_t offset, st
   for (size_t at = 0; at < toks.size (); at += kPortion)
     {
       const int S = (int)std::min<size_t> (kPortion, toks.size () - at);
-      VKLLAMA_STATUS_OK (pass_ (at, S, offset + at, nullptr));
+      // the row of the last token and no other of this portion
+      const bool last_only = fused_decode_ && plan_->usable () && S > 1
+                             && std::all_of (rows.begin (), rows.end (),
+                                             [&] (uint32_t r) { return r < at || r >= at + (size_t)S - 1; })
+                             && std::count (rows.begin (), rows.end (), (uint32_t)(at + (size_t)S - 1));
+      VKLLAMA_STATUS_OK (pass_ (at, S, offset + at, nullptr, last_only));
       // runs of wanted rows that fall into this portion (in the order asked for)
       for (size_t i = 0; i < rows.size ();)
         {

@@ -44,6 +44,10 @@ public:
   virtual absl::Status load (const WeightSource &w) = 0;
   // x [S, width_p] fp32, in place; the last product back may be left to the next block or finish ()
   virtual absl::Status operator() (Tensor &x, int S, size_t offset, int run, Buffers &b) = 0;
+  // for S tokens of which only the last one's output is wanted, which the one-token step computes: no more than later
+  // tokens need of them.  Only if can_keep ()
+  virtual absl::Status keep (Tensor &x, int S, size_t offset, int run, Buffers &b) = 0;
+  bool can_keep () const { return mixer_->kept_rows ().n > 0; }
   // the product back that is left
   absl::Status finish (Tensor &x, int S, Buffers &b);
   virtual void describe (vkl_stack_layer &l, int run) = 0;
@@ -54,9 +58,11 @@ public:
 
 protected:
   absl::StatusOr<Tensor> norm_weights_ (const WeightSource &w, const std::string &name);
-  // the product back that is left, h = rms_norm (x) norm, and the product of h with the n rows of w
+  // the product back that is left, h = rms_norm (x) norm, and the product of h with n rows of w from row `first` on
   absl::Status norm_product_ (const char *what, Tensor &x, int S, Tensor &norm, Tensor &w, int n,
-                              std::vector<vkl_out_seg> const &segs, Buffers &b);
+                              std::vector<vkl_out_seg> const &segs, Buffers &b, int first = 0);
+  // keep () with the norm and the matrix of the mixer's input
+  absl::Status keep_ (Tensor &x, int S, size_t offset, int run, Tensor &norm, Tensor &w, Buffers &b);
   GPUDevice *dev_;
   Command *command_;
   std::string prefix_;
@@ -78,6 +84,10 @@ public:
                  const MixerParams &mp, const FeedForwardParams &ff);
   absl::Status load (const WeightSource &w) override;
   absl::Status operator() (Tensor &x, int S, size_t offset, int run, Buffers &b) override;
+  absl::Status keep (Tensor &x, int S, size_t offset, int run, Buffers &b) override
+  {
+    return keep_ (x, S, offset, run, norm_, w_in_, b);
+  }
   void describe (vkl_stack_layer &l, int run) override;
   int cat_width () const override { return k_out_; }
 
@@ -94,6 +104,10 @@ public:
                    const MixerParams &mp, const FeedForwardParams &ff);
   absl::Status load (const WeightSource &w) override;
   absl::Status operator() (Tensor &x, int S, size_t offset, int run, Buffers &b) override;
+  absl::Status keep (Tensor &x, int S, size_t offset, int run, Buffers &b) override
+  {
+    return keep_ (x, S, offset, run, norm1_, w_in_, b);
+  }
   void describe (vkl_stack_layer &l, int run) override;
   int cat_width () const override { return std::max (k_out_, ff_p_); }
 
@@ -135,7 +149,7 @@ private:
   absl::StatusOr<Tensor> forward_ (std::vector<uint32_t> const &toks, const size_t offset,
                                    std::vector<uint32_t> const &rows) override;
   absl::Status put_tokens_ (std::vector<uint32_t> const &toks);
-  absl::Status pass_ (size_t first, int S, size_t offset, std::vector<float> *streams);
+  absl::Status pass_ (size_t first, int S, size_t offset, std::vector<float> *streams, bool last_only = false);
   absl::Status logits_ (const std::vector<uint32_t> &rows, float *out);
   absl::Status wait_all_ () override;
   StepPlan *plan_ptr_ () override { return plan_.get (); }

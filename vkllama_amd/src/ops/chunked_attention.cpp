@@ -85,8 +85,25 @@ ChunkedAttention::segments (int S, size_t offset, int run)
   };
 }
 
+TokenMixer::Rows
+ChunkedAttention::kept_rows () const
+{
+  return { p_.heads * dim_, 2 * p_.kv_heads * dim_ };
+}
+
 absl::Status
-ChunkedAttention::mix (int S, size_t offset, int run, void *out, size_t os)
+ChunkedAttention::keep (int S, size_t offset, int run)
+{
+  vkl_attn_rows_prep r = prepared_ (offset, run);
+  r.H = 1, r.q = nullptr; // (one query head, which is not there)
+  timer_.start (dev_);
+  const int err = vkl_attn_prepare (&r, S, (uint32_t)offset, dev_->stream ());
+  timer_.stop (dev_);
+  return launch_status ("keys and values", err);
+}
+
+vkl_attn_rows_prep
+ChunkedAttention::prepared_ (size_t offset, int run)
 {
   const size_t nq = (size_t)p_.heads * dim_, nk = (size_t)p_.kv_heads * dim_;
   Tensor &kc = kcaches_[(size_t)run], &vc = vcaches_[(size_t)run];
@@ -97,6 +114,15 @@ ChunkedAttention::mix (int S, size_t offset, int run, void *out, size_t os)
   r.k = row_ (kc, offset), r.ko = kc.data (), r.kvs = nk, r.vo = vc.data ();
   if (first_)
     r.v = row_ (vc, offset), r.first = first_->vcaches_[0].data (), r.fdim = first_->dim_, r.mix = mix_;
+  return r;
+}
+
+absl::Status
+ChunkedAttention::mix (int S, size_t offset, int run, void *out, size_t os)
+{
+  const size_t nq = (size_t)p_.heads * dim_, nk = (size_t)p_.kv_heads * dim_;
+  Tensor &kc = kcaches_[(size_t)run], &vc = vcaches_[(size_t)run];
+  const vkl_attn_rows_prep r = prepared_ (offset, run);
   timer_.start (dev_);
   int err = vkl_attn_prepare (&r, S, (uint32_t)offset, dev_->stream ());
   if (!err && (p_.dtype == FP32 || dim_ > 256 || S <= kFewRows))

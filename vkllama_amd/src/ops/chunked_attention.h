@@ -24,11 +24,14 @@ public:
   absl::Status pack_in (const WeightSource &w, const std::string &prefix, PackedMatrix &m) const override;
   absl::StatusOr<std::vector<vkl_out_seg> > segments (int S, size_t offset, int run) override;
   absl::Status mix (int S, size_t offset, int run, void *out, size_t os) override;
+  Rows kept_rows () const override;
+  absl::Status keep (int S, size_t offset, int run) override;
   void describe (vkl_stack_layer &l, int run) override;
   size_t row_bytes () const override { return kcaches_.empty () ? 0 : 2 * kcaches_[0].hs (); }
   size_t rows_read (size_t pos) const override { return p_.chunk ? pos % (size_t)p_.chunk + 1 : pos + 1; }
 
 private:
+  vkl_attn_rows_prep prepared_ (size_t offset, int run);
   void *row_ (Tensor &cache, size_t pos) { return (uint8_t *)cache.data () + pos * cache.hs (); }
   ChunkedAttention *first_;
   float mix_ = 0.f;

@@ -85,6 +85,30 @@ LatentAttention::segments (int S, size_t, int)
   };
 }
 
+TokenMixer::Rows
+LatentAttention::kept_rows () const
+{
+  return { c_row_ (), round_up (p_.kv_rank, 8) };
+}
+
+absl::Status
+LatentAttention::keep (int S, size_t offset, int run)
+{
+  timer_.start (dev_);
+  const int err = norm_latents_ (S, offset, run);
+  timer_.stop (dev_);
+  return launch_status ("latents", err);
+}
+
+// the new latents, normed, to their cache rows
+int
+LatentAttention::norm_latents_ (int S, size_t offset, int run)
+{
+  return vkl_rmsnorm_f32 ((const float *)c_.data (), (size_t)rank_, nullptr, S, p_.kv_rank,
+                          (const float *)c_norm_.data (), p_.eps, cache_row_ (run, offset), type_ (), (size_t)rank_,
+                          rank_, dev_->stream ());
+}
+
 absl::Status
 LatentAttention::mix (int S, size_t offset, int run, void *out, size_t os)
 {
@@ -92,9 +116,7 @@ LatentAttention::mix (int S, size_t offset, int run, void *out, size_t os)
   const size_t nq = (size_t)H * dim_, na = (size_t)H * rank_;
   void *s = dev_->stream ();
   timer_.start (dev_);
-  int err = vkl_rmsnorm_f32 ((const float *)c_.data (), (size_t)rank_, nullptr, S, p_.kv_rank,
-                             (const float *)c_norm_.data (), p_.eps, cache_row_ (run, offset), type_ (),
-                             (size_t)rank_, rank_, s);
+  int err = norm_latents_ (S, offset, run);
   if (!err && (ukv_.size () == 0 || S <= kFewRows))
     {
       VKLLAMA_STATUS_OK (grow_ (qa_, S, (int)na, dev_, FP32));

@@ -21,6 +21,8 @@ public:
   absl::Status pack_in (const WeightSource &w, const std::string &prefix, PackedMatrix &m) const override;
   absl::StatusOr<std::vector<vkl_out_seg> > segments (int S, size_t offset, int run) override;
   absl::Status mix (int S, size_t offset, int run, void *out, size_t os) override;
+  Rows kept_rows () const override;
+  absl::Status keep (int S, size_t offset, int run) override;
   void describe (vkl_stack_layer &l, int run) override;
   size_t weight_bytes () const override { return ukt_.bytes () + uv_.bytes () + c_norm_.bytes (); }
 
@@ -28,6 +30,7 @@ protected:
   int cache_width_ () const override { return rank_; }
 
 private:
+  int norm_latents_ (int S, size_t offset, int run);
   int c_row_ () const { return p_.heads * dim_; }
   int g_row_ () const { return c_row_ () + round_up (p_.kv_rank, 8); }
   int rank_ = 0;    // latent size, padded

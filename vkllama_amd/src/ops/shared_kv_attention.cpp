@@ -53,6 +53,19 @@ SharedKVAttention::segments (int S, size_t offset, int run)
   };
 }
 
+TokenMixer::Rows
+SharedKVAttention::kept_rows () const
+{
+  return { p_.heads * dim_, p_.kv_heads * dim_ };
+}
+
+// (the product has written the keys where they stay)
+absl::Status
+SharedKVAttention::keep (int, size_t, int)
+{
+  return absl::OkStatus ();
+}
+
 absl::Status
 SharedKVAttention::mix (int S, size_t offset, int run, void *out, size_t os)
 {

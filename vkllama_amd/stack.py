@@ -64,6 +64,7 @@ SIGNATURES = {
     "vkl_stack_scratch_bytes": (sz, [vp]),
     "vkl_stack_supported": (i32, [vp]),
     "vkl_stack_step": (i32, [vp, vp, u32, vp, vp, vp]),
+    "vkl_stack_layer_step": (i32, [vp, i32, vp, u32, vp]),
     "vkl_stack_logits": (i32, [vp, vp, vp, vp]),
     "vkl_stack_loop": (i32, [vp, vp, u32, i32, vp, vp]),
     "vkl_stack_loop_sampled": (i32, [vp, vp, u32, i32, vp, i32, f32, C.c_uint64, vp]),

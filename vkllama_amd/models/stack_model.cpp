@@ -69,7 +69,7 @@ StackBlock::norm_product_ (const char *what, Tensor &x, int S, Tensor &norm, Ten
 absl::Status
 StackBlock::keep_ (Tensor &x, int S, size_t offset, int run, Tensor &norm, Tensor &w, Buffers &b)
 {
-  const TokenMixer::Rows r = mixer_->kept_rows ();
+  const TokenMixer::Rows r = mixer_->kept_rows (S, offset);
   auto segs = mixer_->segments (S, offset, run);
   VKLLAMA_STATUS_OK (segs);
   std::vector<vkl_out_seg> kept;
@@ -359,7 +359,7 @@ StackModel::pass_ (size_t first, int S, size_t offset, std::vector<float> *strea
   for (size_t n = 0; n < cfg_.order.size (); ++n)
     {
       const size_t i = (size_t)cfg_.order[n];
-      if (last_only && n + 1 == cfg_.order.size () && blocks_[i]->can_keep ())
+      if (last_only && n + 1 == cfg_.order.size () && blocks_[i]->can_keep (S, offset))
         {
           VKLLAMA_STATUS_OK (blocks_[i]->keep (x_, S, offset, seen[i], buf_));
           return launched ("last layer", vkl_stack_layer_step (&plan_->desc (), (int)n, xp + (size_t)(S - 1) * width_p_,

@@ -47,7 +47,7 @@ public:
   // for S tokens of which only the last one's output is wanted, which the one-token step computes: no more than later
   // tokens need of them.  Only if can_keep ()
   virtual absl::Status keep (Tensor &x, int S, size_t offset, int run, Buffers &b) = 0;
-  bool can_keep () const { return mixer_->kept_rows ().n > 0; }
+  bool can_keep (int S, size_t offset) const { return mixer_->kept_rows (S, offset).n > 0; }
   // the product back that is left
   absl::Status finish (Tensor &x, int S, Buffers &b);
   virtual void describe (vkl_stack_layer &l, int run) = 0;

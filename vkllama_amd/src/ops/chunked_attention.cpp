@@ -86,7 +86,7 @@ ChunkedAttention::segments (int S, size_t offset, int run)
 }
 
 TokenMixer::Rows
-ChunkedAttention::kept_rows () const
+ChunkedAttention::kept_rows (int, size_t) const
 {
   return { p_.heads * dim_, 2 * p_.kv_heads * dim_ };
 }

@@ -86,8 +86,13 @@ LatentAttention::segments (int S, size_t, int)
 }
 
 TokenMixer::Rows
-LatentAttention::kept_rows () const
+LatentAttention::kept_rows (int S, size_t offset) const
 {
+  // A few dozen tokens with nothing before them: one attention over expanded rows takes less than the step's five
+  // launches behind a small product (four layers, us with / without: 33 tokens 2048 wide 219 / 214, 24 4096 wide 378 /
+  // 375, 48 220 / 229 and 401 / 403).
+  if (S > kFewRows && offset + (size_t)S < 48)
+    return {};
   return { c_row_ (), round_up (p_.kv_rank, 8) };
 }
 

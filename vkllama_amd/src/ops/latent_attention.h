@@ -21,7 +21,7 @@ public:
   absl::Status pack_in (const WeightSource &w, const std::string &prefix, PackedMatrix &m) const override;
   absl::StatusOr<std::vector<vkl_out_seg> > segments (int S, size_t offset, int run) override;
   absl::Status mix (int S, size_t offset, int run, void *out, size_t os) override;
-  Rows kept_rows () const override;
+  Rows kept_rows (int S, size_t offset) const override;
   absl::Status keep (int S, size_t offset, int run) override;
   void describe (vkl_stack_layer &l, int run) override;
   size_t weight_bytes () const override { return ukt_.bytes () + uv_.bytes () + c_norm_.bytes (); }

@@ -54,7 +54,7 @@ SharedKVAttention::segments (int S, size_t offset, int run)
 }
 
 TokenMixer::Rows
-SharedKVAttention::kept_rows () const
+SharedKVAttention::kept_rows (int, size_t) const
 {
   return { p_.heads * dim_, p_.kv_heads * dim_ };
 }

@@ -97,13 +97,13 @@ public:
   virtual absl::StatusOr<std::vector<vkl_out_seg> > segments (int S, size_t offset, int run) = 0;
   // after the product: the heads' outputs to out [S, out_cols], row stride os
   virtual absl::Status mix (int S, size_t offset, int run, void *out, size_t os) = 0;
-  // For tokens whose outputs nothing reads: the rows of the matrix that later tokens need (of the first one on, whole
-  // segments; n 0: this mixer has no such form), and what takes the place of mix () behind the product with these
+  // For tokens whose outputs nothing reads: the rows of the matrix that later tokens need (from the first one on,
+  // whole segments; n 0: no such form, or none that is faster), and what takes the place of mix () behind the product with these
   struct Rows
   {
     int first = 0, n = 0;
   };
-  virtual Rows kept_rows () const { return {}; }
+  virtual Rows kept_rows (int, size_t) const { return {}; }
   virtual absl::Status keep (int, size_t, int) { return absl::UnimplementedError ("tokens without outputs"); }
   // this mixer's part of the one-token step's layer table
   virtual void describe (vkl_stack_layer &l, int run) = 0;

@@ -192,6 +192,12 @@ int vkl_matmul_f16_nn (const void *a, const void *b, int C, int M, int N,
 int vkl_kqv_f16 (const void *x, const void *wk, const void *wq,
                  const void *wv, int M, int N, int K, void *k, void *q,
                  void *v, void *stream);
+/* The same where only the last row of q is wanted (the last block of a prompt pass):
+ * k and v [M, N], and row M - 1 of q [M, N]; what the other rows hold afterwards is
+ * not defined.  wtype 8 (planar Q8_0) or 1 (fp16). */
+int vkl_kqv_last (const void *x, const void *wk, const void *wq, const void *wv,
+                  int wtype, int M, int N, int K, void *k, void *q, void *v,
+                  void *stream);
 /* src/shaders/ffn_up_and_gate_fp16.comp */
 int vkl_ffn_upgate_f16 (const void *x, const void *wup, const void *wgate,
                         int M, int N, int K, void *out, void *stream);

@@ -209,6 +209,14 @@ fill_common (GemvQ8Args &a, const void *x, int M, int N, int K, size_t xs,
   return 0;
 }
 
+// From when on vkl_kqv_last leaves the other rows of q out: a product over two matrices and one row's, us of three
+// matrices / of this, weights that no cache holds.  fp16: 4096 wide 2048 rows 165.7 / 119.0, 700 86.4 / 59.8; 5120 wide
+// 1000 rows 134.2 / 123.8, 512 rows 76.1 / 81.9; 512 wide 3000 rows 11.4 / 10.5, 2048 rows 7.9 / 8.9.  Q8_0: 5120
+// wide 3967 rows 772.4 / 514.9, 1000 185.6 / 185.4, 512 108.3 / 110.8; 2048 wide 700 rows 41.2 / 31.1.  Below these
+// the second launch, and tiles that leave half of the compute units idle, cost what the rows save.
+constexpr int kLastMinRows = 640;
+constexpr double kLastMinWork = 7e8; // multiply-adds of one matrix
+
 // the same problem on the matrix cores when there are enough token rows
 // the problem as the matrix-core launcher takes it
 vkl::GemmArgs
@@ -341,6 +349,46 @@ vkl_kqv_q8_0 (const void *x, const void *wk, const void *wq, const void *wv,
   if (try_gemm (a, 3, 0, (hipStream_t)stream, err))
     return err;
   return launch<1, 3> (a, (hipStream_t)stream);
+}
+
+extern "C" int
+vkl_kqv_last (const void *x, const void *wk, const void *wq, const void *wv, int wtype, int M, int N, int K, void *k,
+              void *q, void *v, void *stream)
+{
+  VKL_CHECK_ARG (x && wk && wq && wv && k && q && v && M > 0 && N > 0 && K > 0 && (wtype == 8 || wtype == 1));
+  vkl::GemmArgs g = {};
+  if (wtype == 8)
+    {
+      GemvQ8Args a = {};
+      if (int e = fill_common (a, x, M, N, K, (size_t)K, (size_t)N))
+        return e;
+      set_mat (a, 0, wk, k);
+      set_mat (a, 1, wv, v);
+      g = gemm_args (a, 2, 0);
+    }
+  else
+    {
+      g.x = (const uint16_t *)x, g.xs = (size_t)K;
+      g.M = M, g.N = N, g.K = K, g.Kp = (K + 31) / 32 * 32;
+      g.wtype = 1, g.nmat = 2;
+      g.wh[0] = (const uint16_t *)wk, g.wh[1] = (const uint16_t *)wv;
+      g.ws = (size_t)K;
+      g.y[0] = (uint16_t *)k, g.y[1] = (uint16_t *)v;
+      g.ys = (size_t)N;
+      g.scale = 1.f;
+    }
+  // (the last rows are aligned as the first ones are)
+  if (M < kLastMinRows || (double)M * N * K < kLastMinWork || (K % 8) != 0 || (N % 8) != 0
+      || !vkl::gemm_mfma_supported (g))
+    return (wtype == 8 ? vkl_kqv_q8_0 : vkl_kqv_f16) (x, wk, wq, wv, M, N, K, k, q, v, stream);
+  if (int e = vkl::gemm_mfma_launch (g, (hipStream_t)stream))
+    return e;
+  const uint16_t *xl = (const uint16_t *)x + (size_t)(M - 1) * K;
+  uint16_t *ql = (uint16_t *)q + (size_t)(M - 1) * N;
+  if (wtype == 8)
+    return vkl_matmul_q8_0 (xl, wq, 1, N, K, (size_t)K, (size_t)N, 1.f, 0.f, 0, nullptr, ql, nullptr, stream);
+  return vkl_matmul_f16_tb (xl, wq, 1, 1, N, K, 0, (size_t)K, 0, (size_t)K, 0, (size_t)N, 1.f, 0.f, 0, nullptr, ql, nullptr,
+                            stream);
 }
 
 extern "C" int

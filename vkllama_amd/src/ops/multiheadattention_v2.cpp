@@ -166,10 +166,14 @@ MultiHeadAttentionV2::operator() (Tensor X, const size_t offset) noexcept
       VKLLAMA_STATUS_OK (q_.reshape (1, S, N));
       VKLLAMA_STATUS_OK (v_.reshape (1, S, N));
       timer_.start (dev_);
-      const auto project = wk_.dtype () == Q8_0 ? vkl_kqv_q8_0 : vkl_kqv_f16;
-      const int err = project (X.data (), wk_.data (), wq_.data (), wv_.data (),
-                               (int)S, (int)N, (int)X.width (), k_.data (),
-                               q_.data (), v_.data (), dev_->stream ());
+      // (of a clipped output only the last row of q goes on)
+      const bool q8 = wk_.dtype () == Q8_0;
+      const auto project = q8 ? vkl_kqv_q8_0 : vkl_kqv_f16;
+      const int err = clip_output_
+                          ? vkl_kqv_last (X.data (), wk_.data (), wq_.data (), wv_.data (), q8 ? 8 : 1, (int)S, (int)N,
+                                          (int)X.width (), k_.data (), q_.data (), v_.data (), dev_->stream ())
+                          : project (X.data (), wk_.data (), wq_.data (), wv_.data (), (int)S, (int)N, (int)X.width (),
+                                     k_.data (), q_.data (), v_.data (), dev_->stream ());
       timer_.stop (dev_);
       VKLLAMA_STATUS_OK (launch_status ("kqv", err));
       k = k_, q = q_, v = v_;

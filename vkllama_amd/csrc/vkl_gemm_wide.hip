@@ -973,9 +973,16 @@ mix_time (int bm, int kind, bool one_row, bool q8)
   if (q8)
     return tq8[kind];
   constexpr MixTime t256[3] = { { 1.41, 5.0, 15.5 }, { 0.69, 5.7, 8.3 }, { 0.53, 5.6, 4.4 } };
+  // Fitted to the choice that they make among 460 bf16 products of 200 to 2048 rows, the other constants as they are: 1.5 %
+  // faster in the mean for these tiles, which are in 70 of the plans, one of them 3 % slower than the plan before (the best
+  // choice of all: 2.0 %).  448 others, 144 to 2200 rows, widths of 1024, 2048, 3072 and 4096: 1.7 % in the mean, up to 22;
+  // three 2.6 to 6.4 % slower (528 x 2048 x 7552 29.3 / 31.2).
+  constexpr MixTime t192[2] = { { 1.34, 6.97, 8.0 }, { 0.70, 3.63, 5.7 } };
   constexpr MixTime t128[3] = { { 0.70, 7.2, 7.7 }, { 0.49, 7.0, 3.0 }, { 0.52, 3.4, 0.51 } };
   // one row of tiles streams the weights
   constexpr MixTime t1[3] = { { 1.17, 7.6, 7.1 }, { 0.79, 7.0, 3.4 }, { 0.49, 5.1, 3.9 } };
+  if (bm == 192)
+    return t192[std::min (kind, 1)];
   return bm == WBM ? t256[kind] : one_row ? t1[kind] : t128[kind];
 }
 
@@ -1036,6 +1043,11 @@ struct MixSpan
 // 12288 columns (1.5 rounds of pairs) 182 us with one round of pairs and 256 tiles, 198 without pairs,
 // 211 of pairs alone; 1500 x 8064, K = 2048 59 / 59 / 55.
 //
+// 192 rows (bf16) are for products whose 256-row tiles fill a part of their last round only: one round of 192 x 256 takes
+// 0.85 of one of 256 x 256.  us with tiles of 128 and 256 rows / with these, weights that no cache holds: 1500 x 7552 x 2048
+// 57.4 / 48.8, 1500 x 2048 x 7552 (two parts) 61.4 / 57.1, 1500 x 4096 x 15104 181.9 / 165.7, 1152 x 4096 x 4096 55.4 / 49.5,
+// 768 x 5504 x 2048 with GELU 0.83 of the time, 2048 x 5504 x 2048 0.90.  They are not cut.
+//
 // At most 128 tiles of 128 rows leave half the compute units idle while the others wait for weights: they are cut
 // by their columns into twice as many of 128 x 64, with six stages of loads (whole / cut, us, fp16: 77 x 4096 x 11008 in four
 // parts 34.0 / 27.2, 128 rows 38.7 / 31.9, 77 x 4096 x 4096 16.1 / 15.5).  The halves of more tiles would not all
@@ -1056,7 +1068,7 @@ struct WideMix
   {
     return tiles_m * tiles_n * nmat * ksplit - 2 * wide;
   }
-  // bm: token rows of a tile, 256 (which may be cut by its rows) or 128 (by its columns); steps: of the k range of a part;
+  // bm: token rows of a tile, 256 (which may be cut by its rows), 192 or 128 (by its columns); steps: of the k range of a part;
   // park: how much of the time for parked sums a tile takes; us: the time of the launch's tiles
   __host__
   WideMix (int bm, int tm, int tn, int mats, int parts, double steps, double park, double *us = nullptr, bool q8 = false)
@@ -1079,7 +1091,7 @@ struct WideMix
         wide = options[o];
         const int rest = narrow () % U;
         whole = bm == WBM && wide % U == 0 && rest > 0 && rest <= U / 2 ? narrow () - rest : narrow ();
-        if (bm < WBM && !q8 && narrow () <= U / 2)
+        if (bm == 128 && !q8 && narrow () <= U / 2)
           whole = 0;
         MixSpan span;
         span.deal (wide, t[0]);
@@ -1442,10 +1454,10 @@ template <int BM>
 constexpr size_t
 mix_lds ()
 {
-  constexpr size_t wide = (size_t)(BM == WBM ? 2 : 3) * (BM + 256) * WROWB;
-  constexpr size_t narrow = (size_t)(BM == WBM ? 3 : 4) * (BM + WBN) * WROWB;
+  constexpr size_t wide = (size_t)(BM > 128 ? 2 : 3) * (BM + 256) * WROWB;
+  constexpr size_t narrow = (size_t)(BM > 128 ? 3 : 4) * (BM + WBN) * WROWB;
   constexpr size_t park = (size_t)MWAVES * std::max (BM / 2 * 36, 64 * 68) * 4; // see mix_epilogue
-  static_assert (BM == WBM || 6 * (BM + WBN / 2) * WROWB <= wide, "");
+  static_assert (BM > 128 || 6 * (BM + WBN / 2) * WROWB <= wide, "");
   return std::max (std::max (wide, narrow), park);
 }
 
@@ -1457,13 +1469,13 @@ gemm_mix_kernel (const Args a, WideMix grid, int vec, int ksplit, float *ws)
   switch (grid.place (a.M, BM, at))
     {
     case 1:
-      return mix_tile<BM, 256, 2, BM == WBM ? 2 : 3, UPGATE, Args> (a, at, vec, ksplit, ws);
+      return mix_tile<BM, 256, 2, (BM > 128 ? 2 : 3), UPGATE, Args> (a, at, vec, ksplit, ws);
     case 2:
-      return mix_tile<BM, WBN, 4, BM == WBM ? 3 : 4, UPGATE, Args> (a, at, vec, ksplit, ws);
+      return mix_tile<BM, WBN, 4, (BM > 128 ? 3 : 4), UPGATE, Args> (a, at, vec, ksplit, ws);
     case 3:
       if constexpr (BM == WBM)
         return mix_tile<BM / 2, WBN, 4, 4, UPGATE, Args> (a, at, vec, ksplit, ws);
-      else
+      else if constexpr (BM == 128)
         return mix_tile<BM, WBN / 2, 8, 6, UPGATE, Args> (a, at, vec, ksplit, ws);
     }
 }
@@ -2410,7 +2422,7 @@ wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
   double best_cost = 0;
   const int nk = a.K / WBK, tiles_n = (a.N + WBN - 1) / WBN;
   const double parked = mix_park (a);
-  for (int bm = 64; bm <= WBM; bm *= 2)
+  for (int bm = 64; bm <= WBM; bm += 64)
     for (int ks = 1; ks <= 16; ++ks)
       {
         const bool odd = (ks & (ks - 1)) != 0; // no power of two
@@ -2530,6 +2542,8 @@ launch_bf16_tiles (const GemmSegArgs &a, const WidePlan &p, float *ws, hipStream
 {
   if (p.bm == WBM)
     return p.four_waves ? launch_wide_parts<WBM, WSTAGES> (a, p.ksplit, ws, s) : launch_mix_parts<WBM> (a, p.ksplit, ws, s);
+  if (p.bm == 192)
+    return launch_mix_parts<192> (a, p.ksplit, ws, s);
   if (p.bm == 128)
     return p.four_waves ? launch_wide_parts<128, WSTAGES> (a, p.ksplit, ws, s) : launch_mix_parts<128> (a, p.ksplit, ws, s);
   return deep64 (a, p.ksplit) ? launch_wide_parts<64, kDeep64> (a, p.ksplit, ws, s)

@@ -2470,14 +2470,24 @@ wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
 // both forms, all in two stages (four take 0.8 to 0.95 of that where a compute unit has one tile, in one
 // part or several): 0.5 % slower than the best plan in the mean, 7 at worst; without 256 rows 2.5 % and 22
 // (2048 x 8064 x 2048 187 us with them, 229 without; 512 x 16128 x 4096 175, 199).
+// Three, five, six and seven parts are taken where they promise 8 %: of 204 products of 2 to 532 rows (weights that no cache
+// holds) 0.988 of the time in the mean, none more than 2 % slower; us, powers of two / now: 300 x 2048 x 5504 42.7 / 36.3, 300 x 4096 x
+// 4096 54.7 / 45.7, 300 x 4096 x 11008 110.2 / 94.8, 181 x 6416 x 2048 35.4 / 30.3.  With 4 % promised seven were 2 to 6 % slower, and so are nine and
+// more parts.
+constexpr double kOddPlanes = 0.92;
+constexpr int kOddPlaneParts = 7;
+
 WidePlan
 wide_plan_planes (const GemmSegArgs &a, size_t scratch)
 {
   const int nk = a.K / WBK / kPlanes, tiles_n = (a.N + WBN - 1) / WBN;
   WidePlan best = { kPlaneRows, 1 };
-  double best_cost = 0;
-  for (int ks = 1; ks <= 16; ks *= 2)
+  double best_cost = 0, even_cost = 0;
+  for (int ks = 1; ks <= 16; ++ks)
     {
+      const bool odd = (ks & (ks - 1)) != 0; // no power of two
+      if (odd && ks > kOddPlaneParts)
+        continue;
       if (ks > 1 && (nk / ks < 4 || (size_t)ks * a.M * a.N * sizeof (float) > scratch))
         continue;
       const int tiles = (a.M + kPlaneRows - 1) / kPlaneRows * tiles_n * ks;
@@ -2486,14 +2496,16 @@ wide_plan_planes (const GemmSegArgs &a, size_t scratch)
       double cost = two * round + (ks > 1 ? 4.2 + (double)ks * a.M * a.N * sizeof (float) / 3.8e6 : 0);
       if (rest > 0)
         cost += rest <= WideGrid::kUnits ? 0.935 * steps + 1.6 : round;
-      if (ks == 1 || cost < best_cost)
+      if (ks == 1 || cost < (odd ? kOddPlanes : 1.0) * best_cost)
         best.ksplit = ks, best_cost = cost;
+      if (ks == 1 || (!odd && cost < even_cost))
+        even_cost = cost;
     }
   if (a.M >= WBM)
     {
       const WideGrid tiles ((a.M + WBM - 1) / WBM, tiles_n, 1, 1, true);
       const int whole = (tiles.whole + WideGrid::kUnits - 1) / WideGrid::kUnits;
-      if (whole * (1.97 * nk + 9.6) + (tiles.whole < tiles.tiles () ? 1.44 * nk + 6.6 : 0) < best_cost)
+      if (whole * (1.97 * nk + 9.6) + (tiles.whole < tiles.tiles () ? 1.44 * nk + 6.6 : 0) < even_cost)
         best = { WBM, 1 };
     }
   return best;

@@ -43,3 +43,8 @@ def test_last_row_equals_the_operators(util, layers, loop, dtype):
     assert np.abs(a - b).max() <= bound * np.abs(a).max()
     for m in ms:
         m.close()
+
+
+def test_arguments_are_checked(dev):
+    from vkllama_amd import stack
+    assert stack.lib().vkl_stack_layer_step(None, 0, None, 0, dev.stream) == 1

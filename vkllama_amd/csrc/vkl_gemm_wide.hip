@@ -2471,7 +2471,7 @@ wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
 // part or several): 0.5 % slower than the best plan in the mean, 7 at worst; without 256 rows 2.5 % and 22
 // (2048 x 8064 x 2048 187 us with them, 229 without; 512 x 16128 x 4096 175, 199).
 // Three, five, six and seven parts are taken where they promise 8 %: of 204 products of 2 to 532 rows (weights that no cache
-// holds) 0.988 of the time in the mean, none more than 2 % slower; us, powers of two / now: 300 x 2048 x 5504 42.7 / 36.3, 300 x 4096 x
+// holds) 0.988 of the time in the mean, none more than 2.2 % slower; us, powers of two / now: 300 x 2048 x 5504 42.7 / 36.3, 300 x 4096 x
 // 4096 54.7 / 45.7, 300 x 4096 x 11008 110.2 / 94.8, 181 x 6416 x 2048 35.4 / 30.3.  With 4 % promised seven were 2 to 6 % slower, and so are nine and
 // more parts.
 constexpr double kOddPlanes = 0.92;

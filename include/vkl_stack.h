@@ -61,6 +61,20 @@ typedef struct
 int vkl_project_bf16w (const void *x, int xtype, size_t xs, const void *w,
                        int M, int N, int K, const vkl_out_seg *segs, int nseg,
                        void *stream);
+/* Which tiles such a product takes, without touching the GPU, so that tests can
+ * see that they reach what they mean: aligned operands, one dense segment of
+ * type `otype` with the activation `act`, a stream with scratch that is not
+ * captured. */
+typedef struct
+{
+  int tile_rows;  /* 0: x fp32 on the 32-bit instructions */
+  int ksplit;     /* parts of the k range */
+  int pairs;      /* tiles of 256 columns (the others have 128) */
+  int four_waves; /* workgroups of four waves; 0: of eight */
+  int planes;     /* bf16 planes of x: 3 (x fp32), otherwise 1 */
+} vkl_project_plan_t;
+int vkl_project_plan (int xtype, int M, int N, int K, int otype, int act,
+                      vkl_project_plan_t *out);
 /* What stands between two products of a layer, and the second one: y += x W^T
  * (x null: nothing is added), h = rms_norm (y) * norm, and the product of h.  The
  * same as vkl_project_bf16w with the residual y in place, vkl_rmsnorm_f32 and

@@ -10,12 +10,16 @@ pytestmark = pytest.mark.gpu
 
 
 # one row beyond three tiles, rows that just fill tiles, a column range that ends inside a tile; with a residual in place
-# (fp32) or an activation that is parked; four and eight parts
-@pytest.mark.parametrize("M,N,K,f32,act", [(577, 8190, 512, False, stack.ACT_NONE), (768, 8192, 512, True, stack.ACT_NONE),
-                                           (768, 5504, 1024, False, stack.ACT_GELU), (1300, 4232, 512, False, stack.ACT_RELU2),
-                                           (1500, 3080, 1024, True, stack.ACT_NONE), (1153, 4096, 512, False, stack.ACT_NONE),
-                                           (750, 2048, 6144, True, stack.ACT_NONE), (768, 1024, 11008, False, stack.ACT_GELU)])
-def test_tiles_of_192_rows(dev, M, N, K, f32, act):
+# (fp32) or an activation that is parked; four and eight parts; pairs of 128 columns with an odd column behind them (8064) or a
+# last one in part, straight from the registers, parked, with a residual
+@pytest.mark.parametrize("M,N,K,f32,act,parts,pairs", [
+    (577, 8190, 512, False, stack.ACT_NONE, 1, 0), (768, 8192, 512, True, stack.ACT_NONE, 1, 0), (768, 5504, 1024, False, stack.ACT_GELU, 1, 0),
+    (1300, 4232, 512, False, stack.ACT_RELU2, 1, 0), (1500, 3080, 1024, True, stack.ACT_NONE, 1, 0), (1153, 4096, 512, False, stack.ACT_NONE, 1, 0),
+    (750, 2048, 6144, True, stack.ACT_NONE, 4, 0), (768, 1024, 11008, False, stack.ACT_GELU, 8, 0),
+    (1500, 8064, 2048, False, stack.ACT_NONE, 1, 248), (1500, 8064, 1024, False, stack.ACT_GELU, 1, 248), (1300, 8190, 576, True, stack.ACT_NONE, 1, 224)])
+def test_tiles_of_192_rows(dev, M, N, K, f32, act, parts, pairs):
+    p = stack.project_plan(stack.BF16, M, N, K, stack.F32 if f32 else stack.BF16, act)
+    assert (p.tile_rows, p.ksplit, p.pairs) == (192, parts, pairs)
     g = torch.Generator(device="cuda").manual_seed(M + N)
     x = torch.randn((M, K), generator=g, device="cuda").bfloat16()
     w = torch.randn((N, K), generator=g, device="cuda").bfloat16()

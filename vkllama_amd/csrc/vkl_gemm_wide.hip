@@ -2511,6 +2511,13 @@ wide_plan_planes (const GemmSegArgs &a, size_t scratch)
   return best;
 }
 
+WideMix
+mix_tiles (const GemmSegArgs &a, int bm, int ksplit)
+{
+  return WideMix (bm, (a.M + bm - 1) / bm, (a.N + WBN - 1) / WBN, 1, ksplit, (double)(a.K / WBK) / ksplit,
+                  ksplit == 1 ? mix_park (a) : 0);
+}
+
 // ws: scratch for the parts of the k range, whose sums the caller adds
 template <int BM>
 int
@@ -2521,8 +2528,7 @@ launch_mix_parts (const GemmSegArgs &a, int ksplit, float *ws, hipStream_t s)
   const auto kernel = gemm_mix_kernel<BM, false, GemmSegArgs>;
   if (int e = limit.raise ((const void *)kernel, lds))
     return e;
-  const WideMix tiles (BM, (a.M + BM - 1) / BM, (a.N + WBN - 1) / WBN, 1, ksplit, (double)(a.K / WBK) / ksplit,
-                       ksplit == 1 ? mix_park (a) : 0);
+  const WideMix tiles = mix_tiles (a, BM, ksplit);
   kernel<<<dim3 ((unsigned)tiles.groups ()), dim3 (MWAVES * 64), lds, s>>> (a, tiles, 1, ksplit, ws);
   return (int)hipGetLastError ();
 }
@@ -2734,6 +2740,14 @@ plane_rows (int K)
   return StreamScratch::bytes () / 2 / ((size_t)kPlanes * K * sizeof (uint16_t));
 }
 
+// the rows that are multiplied at a time
+int
+portion_rows (const GemmSegArgs &a)
+{
+  const size_t most = plane_rows (a.K);
+  return most >= (size_t)a.M ? a.M : (int)(most / WBM * WBM);
+}
+
 void
 launch_split (const float *x, size_t xs, int M, int K, float *ws, hipStream_t s)
 {
@@ -2758,8 +2772,8 @@ gemm_wide_f32_launch (const GemmSegArgs &a, hipStream_t s, int &err)
     return false;
   // the planes of as many rows as half of the scratch holds at a time, the parts of
   // a split k range behind them
-  const size_t half = StreamScratch::bytes () / 2, most = plane_rows (a.K);
-  const int rows = most >= (size_t)a.M ? a.M : (int)(most / WBM * WBM);
+  const size_t half = StreamScratch::bytes () / 2;
+  const int rows = portion_rows (a);
   StreamScratch own;
   float *ws = rows > 0 ? own.take (s) : nullptr;
   if (!ws)
@@ -3010,6 +3024,37 @@ vkl_project_bf16w (const void *x, int xtype, size_t xs, const void *w, int M, in
   if (int e = vkl::seg_args (x, xtype, xs, w, M, N, K, segs, nseg, a))
     return e;
   return vkl::project (a, (hipStream_t)stream);
+}
+
+extern "C" int
+vkl_project_plan (int xtype, int M, int N, int K, int otype, int act, vkl_project_plan_t *out)
+{
+  using namespace vkl;
+  VKL_CHECK_ARG (out);
+  // (addresses that fit, which nothing follows)
+  void *any = (void *)(uintptr_t)16;
+  const vkl_out_seg seg = { 0, N, any, (size_t)(N > 0 ? N : 0), otype, act, nullptr, 0.f };
+  GemmSegArgs a;
+  if (int e = seg_args (any, xtype, (size_t)(K > 0 ? K : 0), any, M, N, K, &seg, 1, a))
+    return e;
+  const bool f32 = xtype == VKL_TYPE_F32;
+  *out = { 0, 1, 0, 0, 1 };
+  WidePlan p;
+  if (f32)
+    {
+      a.M = portion_rows (a);
+      if (!planes_pay (a) || a.M <= 0)
+        return 0;
+      p = wide_plan_planes (with_planes (a, nullptr), StreamScratch::bytes () / 2);
+      out->planes = kPlanes;
+    }
+  else
+    p = wide_plan_bf16 (a, StreamScratch::bytes ());
+  out->tile_rows = p.bm, out->ksplit = p.ksplit;
+  out->four_waves = f32 || p.bm == 64 || p.four_waves;
+  if (!out->four_waves)
+    out->pairs = mix_tiles (a, p.bm, p.ksplit).wide;
+  return 0;
 }
 
 extern "C" int

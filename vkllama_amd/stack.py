@@ -14,6 +14,11 @@ class OutSeg(C.Structure):
                 ("cap", f32)]
 
 
+class ProjectPlan(C.Structure):
+    """vkl_project_plan_t"""
+    _fields_ = [("tile_rows", i32), ("ksplit", i32), ("pairs", i32), ("four_waves", i32), ("planes", i32)]
+
+
 class AddNormProject(C.Structure):
     """vkl_add_norm_project"""
     _fields_ = [("x", vp), ("xs", sz), ("w", vp), ("K", i32), ("y", vp), ("ys", sz), ("W", i32), ("norm", vp), ("eps", f32),
@@ -40,6 +45,7 @@ ACT_NONE, ACT_SILU, ACT_RELU2, ACT_GELU = 0, 1, 2, 3
 
 SIGNATURES = {
     "vkl_project_bf16w": (i32, [vp, i32, sz, vp, i32, i32, i32, C.POINTER(OutSeg), i32, vp]),
+    "vkl_project_plan": (i32, [i32, i32, i32, i32, i32, i32, C.POINTER(ProjectPlan)]),
     "vkl_add_norm_project_bf16w": (i32, [C.POINTER(AddNormProject), i32, i32, vp]),
     "vkl_embed_norm_bf16": (i32, [vp, u32, i32, i32, vp, u32, vp, f32, vp, sz, vp]),
     "vkl_rmsnorm_f32": (i32, [vp, sz, vp, i32, i32, vp, f32, vp, i32, sz, i32, vp]),
@@ -85,3 +91,9 @@ def lib():
 def segments(items):
     """items: (n0, n, y, ys, type, act, residual, cap) each"""
     return (OutSeg * len(items))(*[OutSeg(*it) for it in items])
+
+
+def project_plan(xtype, M, N, K, otype=F32, act=ACT_NONE):
+    p = ProjectPlan()
+    capi.check(lib().vkl_project_plan(xtype, M, N, K, otype, act, C.byref(p)), "vkl_project_plan")
+    return p

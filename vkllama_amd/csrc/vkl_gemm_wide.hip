@@ -975,8 +975,8 @@ mix_time (int bm, int kind, bool one_row, bool q8)
   constexpr MixTime t256[3] = { { 1.41, 5.0, 15.5 }, { 0.69, 5.7, 8.3 }, { 0.53, 5.6, 4.4 } };
   // Fitted to the choice that they make among 460 bf16 products of 200 to 2048 rows, the other constants as they are: 1.5 %
   // faster in the mean for these tiles, which are in 70 of the plans, one of them 3 % slower than the plan before (the best
-  // choice of all: 2.0 %).  448 others, 144 to 2200 rows, widths of 1024, 2048, 3072 and 4096: 1.7 % in the mean, up to 22;
-  // three 2.6 to 6.4 % slower (528 x 2048 x 7552 29.3 / 31.2).
+  // choice of all: 2.0 %).  448 others, 144 to 2200 rows, widths of 1024, 2048, 3072 and 4096: 1.7 % in the mean, up to 22; what was
+  // slower is held back by kFew192 (and 528 x 2048 x 7552, 29.3 / 31.2, see kOddParts).
   constexpr MixTime t192[2] = { { 1.34, 6.97, 8.0 }, { 0.70, 3.63, 5.7 } };
   constexpr MixTime t128[3] = { { 0.70, 7.2, 7.7 }, { 0.49, 7.0, 3.0 }, { 0.52, 3.4, 0.51 } };
   // one row of tiles streams the weights
@@ -2403,11 +2403,20 @@ four256 (const GemmSegArgs &a, int ksplit, int tiles, double park)
 // Parts that are no power of two fill the compute units where powers leave a quarter to a half of them idle (us, without / with:
 // 1200 x 4096 x 15104 177 / 141, 600 x 4096 x 15104 96 / 87, 1200 x 2048 x 7552 58.9 / 49.6, 300 x 4096 x 11008 50.6 / 47.2).
 // They are taken where they promise 4 % (of 391 products of 131 to 2100 rows none of 150 rows and more got more than 5 %
-// slower, the mean is 0.989 of the time; with 8 % promised 0.990), by tiles of 128 and 256 rows, and from 144
-// rows on: below, the model takes tiles of few rows for faster than they are (131 x 4096 x 11008 38.0 / 43.1, 77 x 12576 x 4096
-// 30.0 / 36.5).
+// slower than by the parts before them, the mean is 0.989 of the time; with 8 % promised 0.990), by tiles of 128, 192 and 256 rows, and
+// from 144 rows on: below, the model takes tiles of few rows for faster than they are (131 x 4096 x 11008 38.0 / 43.1, 77 x 12576 x
+// 4096 30.0 / 36.5).  192 rows take five or three parts in one of 300 products: powers of two and other tiles / these, 366 x 3072 x
+// 11264 46.6 / 40.8, 288 x 3072 x 8192 34.1 / 31.2, 528 x 2048 x 7552 36.0 / 31.7 (which 128 rows in three parts do in 30.2).
 constexpr double kOddParts = 0.96;
 constexpr int kOddRows = 144;
+
+// A last row of 256-row tiles that holds at most 64 rows takes less than the model says.  Tiles of 192 rows that leave a quarter of the
+// compute units without one have to promise 2.5 % there: us, 256 rows / 192, 555 x 7680 x 5120 57.0 / 61.1, 2074 x 2048 x
+// 7552 79.7 / 82.3, 2078 x 2048 x 5504 65.0 / 64.8, 1298 x 3072 x 8192 85.0 / 80.9; more tiles of 192 rows stay faster (1049 x 4096
+// x 4096 49.7 / 45.6, 1049 x 5120 x 5120 64.5 / 60.4).  2833 products of 144 to 2300 rows, all whose tiles are not those of powers of two
+// and 64, 128 and 256 rows, take 0.886 of the time with those, and none is more than 2 % slower.
+constexpr int kShortRows = 64;
+constexpr double kFew192 = 0.975;
 
 WidePlan
 wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
@@ -2453,7 +2462,10 @@ wide_plan_bf16 (const GemmSegArgs &a, size_t scratch)
         else
           WideMix (bm, tiles_m, tiles_n, 1, ks, steps, park, &cost);
         const double reduce = ks > 1 ? reduce0 + (double)ks * a.M * a.N * sizeof (float) / rate : 0;
-        if (!best.bm || cost + reduce < (odd ? kOddParts : 1.0) * best_cost)
+        const bool few192 = best.bm == 192 && best.ksplit == 1 && (a.M + 191) / 192 * tiles_n <= WideGrid::kUnits * 3 / 4;
+        const bool short256 = bm == WBM && ks == 1 && tiles_m * bm - a.M >= bm - kShortRows;
+        const double promise = odd ? kOddParts : few192 && short256 ? 1 / kFew192 : 1.0;
+        if (!best.bm || cost + reduce < promise * best_cost)
           best = { bm, ks, bm == WBM && four256 (a, ks, tiles, park) }, best_cost = cost + reduce;
         if (bm != 128 || tiles <= WideGrid::kUnits / 2 || park > 0)
           continue;

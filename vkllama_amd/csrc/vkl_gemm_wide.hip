@@ -2494,7 +2494,7 @@ wide_plan_planes (const GemmSegArgs &a, size_t scratch)
 {
   const int nk = a.K / WBK / kPlanes, tiles_n = (a.N + WBN - 1) / WBN;
   WidePlan best = { kPlaneRows, 1 };
-  double best_cost = 0, even_cost = 0;
+  double best_cost = 0;
   for (int ks = 1; ks <= 16; ++ks)
     {
       const bool odd = (ks & (ks - 1)) != 0; // no power of two
@@ -2510,14 +2510,12 @@ wide_plan_planes (const GemmSegArgs &a, size_t scratch)
         cost += rest <= WideGrid::kUnits ? 0.935 * steps + 1.6 : round;
       if (ks == 1 || cost < (odd ? kOddPlanes : 1.0) * best_cost)
         best.ksplit = ks, best_cost = cost;
-      if (ks == 1 || (!odd && cost < even_cost))
-        even_cost = cost;
     }
   if (a.M >= WBM)
     {
       const WideGrid tiles ((a.M + WBM - 1) / WBM, tiles_n, 1, 1, true);
       const int whole = (tiles.whole + WideGrid::kUnits - 1) / WideGrid::kUnits;
-      if (whole * (1.97 * nk + 9.6) + (tiles.whole < tiles.tiles () ? 1.44 * nk + 6.6 : 0) < even_cost)
+      if (whole * (1.97 * nk + 9.6) + (tiles.whole < tiles.tiles () ? 1.44 * nk + 6.6 : 0) < best_cost)
         best = { WBM, 1 };
     }
   return best;

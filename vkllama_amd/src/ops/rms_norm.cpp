@@ -34,6 +34,11 @@ RMSNorm::time () noexcept
 absl::Status
 RMSNorm::prepare (size_t rows, size_t width) noexcept
 {
+  // (what a product writes here is fp16)
+  if (dtype_ != FP16)
+    return absl::InvalidArgumentError (absl::StrFormat (
+        "rms_norm op defined with %d dtype but the dtype of input0 is %d",
+        int (dtype_), int (FP16)));
   if (weight_.size () < width)
     return absl::InvalidArgumentError (absl::StrFormat (
         "rms_norm weight has %zu elements but input0 width is %zu",

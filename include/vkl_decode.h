@@ -133,7 +133,10 @@ int vkl_decode_step (const vkl_decode_model *m, const uint32_t *tok,
  *           holds the last block's output afterwards
  *  logits32 optional device fp32 [vocab]: widened fp16 logits
  * No workgroup waits for another one.  Uses the model's scratch: same stream
- * as its steps.  vkl_decode_tail_supported: whether the shape is covered. */
+ * as its steps.  hipErrorInvalidValue for models that vkl_decode_step refuses
+ * (whatever the number of positions), a last layer without its matrices, and rows
+ * that are not there or not aligned.  vkl_decode_tail_supported: whether the
+ * model is covered. */
 int vkl_decode_tail (const vkl_decode_model *m, const void *att, void *row,
                      float *logits32, void *stream);
 int vkl_decode_tail_supported (const vkl_decode_model *m);

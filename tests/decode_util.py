@@ -24,7 +24,8 @@ def lib():
     so = capi.lib()
     for name, res, args in (("vkl_decode_scratch_bytes", C.c_size_t, [vp]), ("vkl_decode_flags_acquire", i32, [vp]),
                             ("vkl_decode_flags_release", None, [vp]), ("vkl_decode_status", i32, [vp, vp]),
-                            ("vkl_decode_step", i32, [vp, vp, u32, i32, vp, vp, vp])):
+                            ("vkl_decode_step", i32, [vp, vp, u32, i32, vp, vp, vp]),
+                            ("vkl_decode_tail", i32, [vp, vp, vp, vp, vp]), ("vkl_decode_tail_supported", i32, [vp])):
         fn = getattr(so, name)
         fn.restype, fn.argtypes = res, args
     return so

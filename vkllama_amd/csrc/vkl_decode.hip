@@ -752,8 +752,9 @@ decode_phase_kernel (const Params p, const vkl_layer_weights lw, int layer,
   run_phase<WT> (p, lw, layer, PHASE, (int)blockIdx.x, G, lds);
 }
 
+// what every launch of a model needs, and what its scratch memory is laid out by
 int
-check_model (const vkl_decode_model *m)
+check_shape (const vkl_decode_model *m)
 {
   VKL_CHECK_ARG (m != nullptr);
   VKL_CHECK_ARG (m->wtype == 8 || m->wtype == 1);
@@ -766,8 +767,28 @@ check_model (const vkl_decode_model *m)
   VKL_CHECK_ARG (m->layers && m->layers_h && m->tok_embd && m->output
                  && m->output_norm);
   VKL_CHECK_ARG (m->freqc && m->freqs && m->scratch);
+  return 0;
+}
+
+int
+check_model (const vkl_decode_model *m)
+{
+  if (int e = check_shape (m))
+    return e;
   VKL_CHECK_ARG (lds_bytes_needed (m->dim, m->ffn, m->maxlen, m->head_dim)
                  <= 160 * 1024);
+  return 0;
+}
+
+// the same for the launches behind a prompt's attention, which hold no scores, and the last layer's pointers
+int
+check_tail (const vkl_decode_model *m)
+{
+  if (int e = check_shape (m))
+    return e;
+  VKL_CHECK_ARG (lds_bytes_needed (m->dim, m->ffn, 1, 64) <= 160 * 1024);
+  const vkl_layer_weights &l = m->layers_h[m->n_layers - 1];
+  VKL_CHECK_ARG (l.wo && l.w_gate && l.w_up && l.w_down && l.ffn_norm);
   return 0;
 }
 
@@ -1224,10 +1245,7 @@ vkl_decode_step (const vkl_decode_model *m, const uint32_t *tok, uint32_t pos,
 extern "C" int
 vkl_decode_tail_supported (const vkl_decode_model *m)
 {
-  return m && (m->wtype == 8 || m->wtype == 1) && m->dim > 0 && (m->dim % 32) == 0 && m->dim <= 16384 && m->ffn > 0
-         && (m->ffn % 32) == 0 && m->ffn <= 16384 && m->vocab > 0 && (m->vocab % 2) == 0 && m->n_layers > 0
-         && m->layers_h && m->output && m->output_norm && m->scratch
-         && lds_bytes_needed (m->dim, m->ffn, 1, 64) <= 160 * 1024;
+  return check_tail (m) == 0;
 }
 
 // The launches of a step's phases: four, where the operators take eight or nine for one row (Wo, norm, up/gate,
@@ -1237,7 +1255,9 @@ vkl_decode_tail_supported (const vkl_decode_model *m)
 extern "C" int
 vkl_decode_tail (const vkl_decode_model *m, const void *att, void *row, float *logits32, void *stream)
 {
-  VKL_CHECK_ARG (vkl_decode_tail_supported (m) && att && row && ((uintptr_t)att % 16) == 0 && ((uintptr_t)row % 16) == 0);
+  if (int e = check_tail (m))
+    return e;
+  VKL_CHECK_ARG (att && row && ((uintptr_t)att % 16) == 0 && ((uintptr_t)row % 16) == 0);
   int dev = 0, n_cu = 0;
   VKL_HIP (hipGetDevice (&dev));
   VKL_HIP (hipDeviceGetAttribute (&n_cu, hipDeviceAttributeMultiprocessorCount, dev));

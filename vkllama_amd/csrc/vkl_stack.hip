@@ -2767,9 +2767,6 @@ vkl_stack_step (const vkl_stack_model *m, const uint32_t *tok, uint32_t pos, flo
   return launch_stack_step (p, (hipStream_t)stream);
 }
 
-// A prompt pass ends here too, with its last row: us for that row, the norm and a product of
-// one row of 128-row tiles before / this launch, 2048 wide bf16 3.1 + 30.7 / 21, 4096 wide 4.6 +
-// 65.4 / 41, 2048 wide fp32 (split into planes as well) 3.4 + 1.9 + 50.8 / 21.
 extern "C" int
 vkl_stack_layer_step (const vkl_stack_model *m, int run, float *x, uint32_t pos, void *stream)
 {
@@ -2784,6 +2781,9 @@ vkl_stack_layer_step (const vkl_stack_model *m, int run, float *x, uint32_t pos,
   return launch_stack_layer (p, m->layers_h[run], (hipStream_t)stream);
 }
 
+// A prompt pass ends here too, with its last row: us for that row, the norm and a product of
+// one row of 128-row tiles before / this launch, 2048 wide bf16 3.1 + 30.7 / 21, 4096 wide 4.6 +
+// 65.4 / 41, 2048 wide fp32 (split into planes as well) 3.4 + 1.9 + 50.8 / 21.
 extern "C" int
 vkl_stack_logits (const vkl_stack_model *m, const float *x, float *logits32, void *stream)
 {

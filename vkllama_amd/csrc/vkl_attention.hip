@@ -958,6 +958,11 @@ attn_parts_kernel (const AttnArgs a)
 // start of its first row's chunk on; where a chunk ends inside the query tile, every tile of
 // keys is masked and takes 2 (128 rows behind 8000 keys, 16 heads, chunks of 512: 13 us, 22 in the
 // sixteen parts of 8128 keys; 32 heads, 128 rows behind 1000: 17, in one part 21).
+// What one part takes is that of workgroups of four waves.  Two groups of waves (tile_pairs), which such a launch of ten tiles and
+// more has, take some 2 + 1.02 per tile; the model does not know them, since tests/test_attention_spans.py holds the parts to
+// those that it gives.  us, as chosen / in one part: 16 heads of 128, 1500 rows behind 300 keys 36.1 / 34.4, 600 38.3 / 36.6, 1200
+// 45.3 / 46.1, 2400 62.3 / 63.1, 1024 behind 1024 36.6 / 34.6; 8 heads, 1500 behind 600 31.3 / 34.7; 32 heads, 200 behind 600 19.0 /
+// 18.3; 16 heads of 64, 1500 behind 600 (two parts) 32.3 / 25.2.
 int
 key_parts (const AttnArgs &a, int hd)
 {

@@ -85,13 +85,27 @@ LatentAttention::segments (int S, size_t, int)
   };
 }
 
+// Whether a last layer with an expansion that keeps the latents alone, and takes the step's five launches for the last token, is faster
+// than the operators over all tokens.  Up to kFewRows it is: these have no expansion.  Beyond them some dozen tokens in bf16
+// cost the operators as much as the step's launches behind a small product cost; what else they save grows with the
+// tokens, and with the positions before them, whose latents are expanded too.  Passes of four layers, time of this form over that
+// of the operators:
+//             S 24, 48, 80, 130, 200 at 0      at 200                          at 600
+//  512 wide   1.01 1.03 1.02 1.02 1.02         1.03 1.02 1.00 1.01 1.00        1.01 1.00 0.99 0.99 0.99
+// 1024        1.02 1.02 1.01 1.01 0.99         1.03 1.01 1.01 1.00 0.99        1.01 0.99 0.99 1.00 0.98
+// 2048        1.00 1.01 0.98 0.97 0.93         1.01 0.99 0.96 0.94 0.94        0.99 0.98 0.95 0.93 0.92
+// 4096        0.99 1.03 0.99 0.95 0.94         1.01 1.02 0.98 0.95 0.93        0.95 0.98 0.95 0.95 0.92
+// In 32-bit, which has no expansion, it is always the faster one (33 tokens, 512 wide 0.95, 2048 wide 0.9).
+bool
+LatentAttention::keeping_pays (int width, int S, size_t offset)
+{
+  return S <= kFewRows || (size_t)S + offset / 8 >= (width >= 2048 ? 80u : 160u);
+}
+
 TokenMixer::Rows
 LatentAttention::kept_rows (int S, size_t offset) const
 {
-  // A few dozen tokens with nothing before them: one attention over expanded rows takes less than the step's five
-  // launches behind a small product (four layers, us with / without: 33 tokens 2048 wide 219 / 214, 24 4096 wide 378 /
-  // 375, 48 220 / 229 and 401 / 403).
-  if (S > kFewRows && offset + (size_t)S < 48)
+  if (ukv_.size () != 0 && !keeping_pays (p_.width, S, offset))
     return {};
   return { c_row_ (), round_up (p_.kv_rank, 8) };
 }

@@ -22,6 +22,7 @@ public:
   absl::StatusOr<std::vector<vkl_out_seg> > segments (int S, size_t offset, int run) override;
   absl::Status mix (int S, size_t offset, int run, void *out, size_t os) override;
   Rows kept_rows (int S, size_t offset) const override;
+  static bool keeping_pays (int width, int S, size_t offset);
   absl::Status keep (int S, size_t offset, int run) override;
   void describe (vkl_stack_layer &l, int run) override;
   size_t weight_bytes () const override { return ukt_.bytes () + uv_.bytes () + c_norm_.bytes (); }

@@ -18,10 +18,12 @@ def weights(dev, rng, N, K, q8):
 
 
 # one row, slices of up to 32 rows, whole inner sizes, the general tiles and the wide ones with and without parts; rows of
-# up to 2048, 4096, 8192 values and more, and of an odd number
+# up to 2048, 4096, 6144, 8192 values and more, and of an odd number; few rows of as many parts as one launch takes, and of more
 @pytest.mark.parametrize("q8", [True, False])
 @pytest.mark.parametrize("M,N,K", [(1, 512, 1376), (2, 520, 64), (12, 2048, 2048), (31, 4096, 1408), (33, 4104, 4096), (77, 2056, 5504),
-                                   (77, 4096, 11008), (130, 5120, 5120), (300, 4096, 4096), (40, 8200, 2048), (9, 130, 96), (200, 1000, 2048)])
+                                   (77, 4096, 11008), (130, 5120, 5120), (300, 4096, 4096), (40, 8200, 2048), (9, 130, 96), (200, 1000, 2048),
+                                   (3, 5120, 5120), (33, 6144, 2048), (33, 6152, 2048), (64, 8192, 2048), (3, 5120, 11008), (3, 5120, 13824), (5, 4096, 11008),
+                                   (3, 8192, 8192)])
 def test_product_norm(dev, M, N, K, q8):
     rng = np.random.default_rng(M + N + K)
     L, w = capi.lib(), weights(dev, rng, N, K, q8)

@@ -1138,20 +1138,31 @@ reduce_norm_kernel (const GemmArgs a, const float *ws, int S, int mrows, const f
     }
 }
 
+// Parts times blocks of 2048 columns up to which a workgroup has a row to itself: it fetches all parts of it, four at a time,
+// which the other form's many workgroups do in one trip; few rows of many parts were slower for it.  us, two launches / one, fp16:
+// 3 x 5120 x 13824 (14 parts, 48) 36.6 / 37.4, 3 x 6144 x 16384 (48) 43.8 / 45.2, 3 x 5120 x 11008 (36) 1.00 of the time, 3 x 5120 x
+// 5120 (24) 0.98, 3 x 4096 x 11008 (24) 0.97, 33 x 4096 x 4096 (16) 0.95; Q8_0 2 x 4096 x 11008 (22 parts, 48) 20.3 / 20.7, 2 x 2048 x 16384
+// (32) 0.98.  Beyond 6144 columns a thread holds 32 values of four parts: 3 x 8192 x 8192 (32) 32.0 / 33.2, 3 x 8192 x 2048 (16) 0.95.
+constexpr int kRowNormWork = 36, kWideRowNormWork = 16;
+
 // adds the parts of a product, of which each lies `rows` rows behind the one before
 int
 launch_reduce (const GemmArgs &a, const float *ws, int parts, int rows, hipStream_t s)
 {
   GemmNorm *n = a.norm;
   const auto mis = [] (const void *p) { return ((uintptr_t)p % 16) != 0; };
+  const int vec = a.N <= 2048 ? 1 : a.N <= 4096 ? 2 : a.N <= 6144 ? 3 : 4;
   if (n && a.nmat == 1 && !a.upgate && a.scale == 1.f && a.bias == 0.f && a.act == 0 && !a.y32 && (a.N % 8) == 0 && a.N <= 8192
-      && (a.ys % 8) == 0 && !mis (a.y[0]) && !mis (a.residual) && !mis (n->w) && !mis (n->out))
+      && (parts + 3) / 4 * 4 * vec <= (vec < 4 ? kRowNormWork : kWideRowNormWork) && (a.ys % 8) == 0 && !mis (a.y[0])
+      && !mis (a.residual) && !mis (n->w) && !mis (n->out))
     {
       const dim3 grid ((unsigned)a.M), block (256);
-      if (a.N <= 2048)
+      if (vec == 1)
         reduce_norm_kernel<1><<<grid, block, 0, s>>> (a, ws, parts, rows, n->w, n->eps, n->out);
-      else if (a.N <= 4096)
+      else if (vec == 2)
         reduce_norm_kernel<2><<<grid, block, 0, s>>> (a, ws, parts, rows, n->w, n->eps, n->out);
+      else if (vec == 3)
+        reduce_norm_kernel<3><<<grid, block, 0, s>>> (a, ws, parts, rows, n->w, n->eps, n->out);
       else
         reduce_norm_kernel<4><<<grid, block, 0, s>>> (a, ws, parts, rows, n->w, n->eps, n->out);
       n->done = true;

@@ -184,6 +184,11 @@ int vkl_attn_kv_rows (const void *q, int qtype, size_t qs, const void *rows,
                       int sink, void *out, int otype, size_t os,
                       void *scratch, void *stream);
 size_t vkl_attn_kv_rows_scratch_bytes (int ctype, int H, int G, int dim, int S);
+/* Whether fp32 rows of that many tokens go to the matrix cores in vkl_attn_rows (vals
+ * 0) and vkl_attn_kv_rows (vals 1): operands without an odd alignment.  Host
+ * arithmetic only: what a test can pin. */
+int vkl_attn_f32_tiles (int vals, int H, int G, int dim, int S, uint32_t pos0,
+                        int chunk);
 /* the same for many query rows on the matrix cores, bf16; shapes as for
  * vkl_attn_prefill_causal_bf16 */
 int vkl_attn_prefill_chunked_bf16 (const void *q, const void *k, const void *v,

@@ -53,11 +53,13 @@ def inputs(S, L, H, G, D, seed):
 
 
 # the smallest, a last tile of one row and of fifteen, waves without a block, a context in front; chunks that begin in a tile and in a block;
-# 15 rows and few rows behind many (the row kernel)
-@pytest.mark.parametrize("H,G,S,pos0,D,chunk,sink", [(2, 1, 16, 0, 128, 0, 1), (3, 3, 17, 0, 64, 0, 0), (4, 2, 31, 5, 128, 0, 1), (8, 2, 300, 0, 64, 0, 1),
-                                                     (5, 1, 130, 77, 128, 0, 0), (2, 2, 200, 40, 64, 37, 1), (4, 1, 97, 63, 128, 64, 0), (2, 1, 64, 10, 128, 16, 1),
-                                                     (2, 1, 15, 3, 128, 0, 1), (2, 1, 18, 1500, 64, 0, 1)])
-def test_against_64_bits(dev, H, G, S, pos0, D, chunk, sink):
+# 15 rows, few rows of few heads and few rows behind many (the row kernel)
+@pytest.mark.parametrize("H,G,S,pos0,D,chunk,sink,tiles", [
+    (8, 1, 16, 0, 128, 0, 1, 1), (3, 3, 17, 0, 64, 0, 0, 1), (16, 2, 31, 5, 128, 0, 1, 1), (8, 2, 300, 0, 64, 0, 1, 1), (5, 1, 130, 77, 128, 0, 0, 1),
+    (2, 2, 200, 40, 64, 37, 1, 1), (4, 1, 97, 63, 128, 64, 0, 1), (2, 1, 64, 10, 128, 16, 1, 1), (2, 1, 15, 3, 128, 0, 1, 0),
+    (2, 1, 16, 0, 128, 0, 1, 0), (4, 2, 31, 5, 128, 0, 1, 0), (2, 1, 18, 1500, 64, 0, 1, 0)])
+def test_against_64_bits(dev, H, G, S, pos0, D, chunk, sink, tiles):
+    assert stack.lib().vkl_attn_f32_tiles(1, H, G, D, S, pos0, chunk) == tiles
     q, k, v = inputs(S, pos0 + S + 3, H, G, D, S + D)
     q = q * torch.exp(torch.linspace(-3, 1.5, S, device="cuda"))[:, None]  # from flat to sharp
     q = torch.nn.functional.pad(q, (0, 8))[:, :H * D]
@@ -72,6 +74,7 @@ def test_against_64_bits(dev, H, G, S, pos0, D, chunk, sink):
 
 @pytest.mark.parametrize("S,pos0,D", [(16, 0, 64), (100, 30, 128)])
 def test_shared_rows_and_a_temperature(dev, S, pos0, D):
+    assert stack.lib().vkl_attn_f32_tiles(0, 4, 2, D, S, pos0, 0) == 1
     q, k, _ = inputs(S, pos0 + S, 4, 2, D, S)
     got = attend(dev, q, k, None, 4, 2, D, pos0, temp=(0.2, 16))
     want, size = reference(q, k, None, 4, 2, D, pos0, temp=(0.2, 16))
@@ -84,18 +87,18 @@ def test_shared_rows_and_a_temperature(dev, S, pos0, D):
 @pytest.mark.parametrize("chunk", [0, 24])
 def test_values_that_are_not_finite_reach_those_who_see_them(dev, D, odd, chunk):
     """A value of a later position, or of an earlier chunk, changes nothing."""
-    S = 60
-    q, k, v = inputs(S, S, 2, 1, D, D)
-    clean = attend(dev, q, k, v, 2, 1, D, 0, chunk, 1)
+    S, H = 60, 8
+    assert stack.lib().vkl_attn_f32_tiles(1, H, 1, D, S, 0, chunk) == 1
+    q, k, v = inputs(S, S, H, 1, D, D)
+    clean = attend(dev, q, k, v, H, 1, D, 0, chunk, 1)
     bad = torch.nn.functional.pad(v, (0, 8))[:, :D]                          # (of the strides of k)
     bad[21, 3] = odd
-    got = attend(dev, q, k, bad, 2, 1, D, 0, chunk, 1)
+    got = attend(dev, q, k, bad, H, 1, D, 0, chunk, 1)
     pos = torch.arange(S, device="cuda")
     sees = (pos >= 21) & ((pos // chunk == 21 // chunk) if chunk else (pos >= 0))
-    assert bool((~torch.isfinite(got[sees][:, [3, D + 3]])).all())
-    only = torch.ones(2 * D, dtype=torch.bool, device="cuda")
-    only[3], only[D + 3] = False, False
+    column = torch.arange(H * D, device="cuda") % D == 3
+    assert bool((~torch.isfinite(got[sees][:, column])).all())
     # (rows of such a block are added one by one: the last bits differ)
-    assert bool(torch.isfinite(got[~sees]).all()) and bool(torch.isfinite(got[:, only]).all())
+    assert bool(torch.isfinite(got[~sees]).all()) and bool(torch.isfinite(got[:, ~column]).all())
     assert bool(((got[~sees] - clean[~sees]).abs() <= 64 * 2.0 ** -24 * 4.0).all())
-    assert bool(((got[:, only] - clean[:, only]).abs() <= 64 * 2.0 ** -24 * 4.0).all())
+    assert bool(((got[:, ~column] - clean[:, ~column]).abs() <= 64 * 2.0 ** -24 * 4.0).all())

@@ -1311,25 +1311,38 @@ attn_f32_tiles_kernel (const RowAttnArgs a, int S)
     }
 }
 
-// Whether many query rows take the kernel above.  It walks a long context in one workgroup, the row kernel in up to 32:
-// few rows behind many stay there.  us: 1.45 per four blocks of the longest tile, or of all tiles dealt to 256 compute units; the row
-// kernel 30000 pairs of a query and a row in one.  Row kernel / tiles: 16 heads, 16 rows 6.9 / 5.2, 64 behind 1936 60 / 50,
-// 32 behind 968 22 / 28, 20 behind 3980 45 / 93; 4 heads, 16 behind 3984 18 / 91.
+// Whether many query rows take the kernel above: where its time promises to be 5 % below the row kernel's.  Both models are fitted to 1500
+// shapes of 2 to 40 heads, 16 to 1200 rows and up to 4000 positions before them, rows that are values too or not, in chunks or not
+// (us; a tile takes so much per four blocks of sixteen rows, the longest tile or all of them dealt to 256 compute units; the row kernel
+// has heads that share rows in workgroups of up to eight, `ht`).  1000 other shapes: the choice takes 1.005 of the better kernel's time in the
+// mean, and in seven of them the tiles are more than 2 % slower, once 16.  A model without the heads of a workgroup took few heads of few rows
+// to the tiles: row kernel / tiles, 4 heads that share nothing, rows that are values too, 111 rows 5.8 / 8.4, 12 heads, 25 rows behind 52 5.4 /
+// 7.9; 4 heads with values of their own, 128 rows 7.0 / 8.2.  As before: 16 heads of 128 sharing 4, 300 rows 33.3 / 15.2.
 bool
 f32_tiles (const RowAttnArgs &a, int ctype, int H, int S)
 {
   if (ctype != VKL_TYPE_F32 || a.qtype != VKL_TYPE_F32 || (a.D != 64 && a.D != 128) || S < kTq || a.pos.loop
       || (uint64_t)a.pos.val + (uint64_t)S >= (1u << 31) || (a.qs % 4) != 0 || ((uintptr_t)a.q % 16) != 0)
     return false;
-  double longest = 0, all = 0, pairs = 0;
+  const RowPlan p = row_plan (ctype, H, a.G, a.D, S, a.vals != nullptr);
+  const auto low = [&] (uint32_t pos) { return a.chunk ? pos / (uint32_t)a.chunk * (uint32_t)a.chunk : 0u; };
+  double longest = 0, all = 0, rows = 0; // rows: that the queries of a head see
   for (int s0 = 0; s0 < S; s0 += kTq)
     {
-      const uint32_t first = a.pos.val + (uint32_t)s0, last = a.pos.val + (uint32_t)std::min (s0 + kTq, S) - 1;
-      const uint32_t low = a.chunk ? first / (uint32_t)a.chunk * (uint32_t)a.chunk : 0u;
-      const double rounds = (last / 16 - low / 16 + kTqWaves) / kTqWaves;
-      longest = std::max (longest, rounds), all += rounds * H, pairs += (double)(last - low + 1) * kTq * H;
+      const int n = std::min (kTq, S - s0);
+      const uint32_t first = a.pos.val + (uint32_t)s0, last = first + (uint32_t)n - 1, mid = first + (uint32_t)(n - 1) / 2;
+      const double rounds = (last / 16 - low (first) / 16 + kTqWaves) / kTqWaves;
+      longest = std::max (longest, rounds), all += rounds * H, rows += (double)n * (mid + 1 - low (mid));
     }
-  return 4 + 1.45 * std::max (longest, all / 256) < 6.5 + pairs / 30000;
+  const double round = a.D == 64 ? 0.86 : 1.55, start = a.D == 64 ? 3.8 : 4.3;
+  // a workgroup of ht heads: its start, and per 100000 rows
+  const int k = p.ht >= 8 ? 3 : p.ht >= 4 ? 2 : p.ht >= 2 ? 1 : 0;
+  constexpr double kStart[4] = { 4.6, 5.1, 6.4, 9.1 }, kRows[4] = { 2.25, 4.6, 9.3, 20 };
+  const double groups = (double)a.G * p.tiles, len = (double)a.pos.val + S;
+  double row = kStart[k] + (a.vals && k == 3 ? 0.7 : 0) + (p.nsplit > 1 && len > 64 ? 2.75 : 0);
+  row += kRows[k] * (a.vals ? 1.63 : 1) * (a.D == 64 ? 0.45 : 1) * rows * groups * 1e-5;
+  row += 0.0035 * len / p.nsplit + 0.0017 * groups * S * p.nsplit;
+  return start + round * std::max (longest, all / 256) < 0.95 * row;
 }
 
 size_t
@@ -2688,6 +2701,16 @@ vkl_attn_rows (const void *q, int qtype, size_t qs, const void *rows, int ctype,
                  && (otype == VKL_TYPE_F32 || otype == VKL_TYPE_BF16));
   return rows_attention (q, qtype, qs, rows, ctype, rs, H, G, dim, S, StepPos{ nullptr, pos0 }, scale, temp_coef,
                          temp_every, out, otype, os, scratch, nullptr, (hipStream_t)stream);
+}
+
+extern "C" int
+vkl_attn_f32_tiles (int vals, int H, int G, int dim, int S, uint32_t pos0, int chunk)
+{
+  if (H <= 0 || G <= 0 || H % G || dim <= 0 || S <= 0 || S > 65535 || chunk < 0)
+    return 0;
+  RowAttnArgs a = {};
+  a.qtype = VKL_TYPE_F32, a.vals = vals ? &a : nullptr, a.G = G, a.D = dim, a.chunk = chunk, a.pos = { nullptr, pos0 };
+  return f32_tiles (a, VKL_TYPE_F32, H, S);
 }
 
 extern "C" size_t

@@ -57,6 +57,7 @@ SIGNATURES = {
     "vkl_attn_prepare": (i32, [C.POINTER(AttnRowsPrep), i32, u32, vp]),
     "vkl_attn_kv_rows": (i32, [vp, i32, sz, vp, vp, i32, sz, i32, i32, i32, i32, u32, f32, i32, i32, vp, i32, sz, vp, vp]),
     "vkl_attn_kv_rows_scratch_bytes": (sz, [i32, i32, i32, i32, i32]),
+    "vkl_attn_f32_tiles": (i32, [i32, i32, i32, i32, i32, u32, i32]),
     "vkl_attn_prefill_chunked_bf16": (i32, [vp, vp, vp, i32, i32, i32, i32, i32, sz, sz, sz, f32, i32, i32, vp, sz, vp]),
     "vkl_attn_prefill_parts": (i32, [i32, i32, i32, i32, i32]),
     "vkl_attn_prefill_tile_parts": (i32, [i32, i32, i32, i32, i32, i32]),

@@ -198,6 +198,10 @@ int vkl_kqv_f16 (const void *x, const void *wk, const void *wq,
 int vkl_kqv_last (const void *x, const void *wk, const void *wq, const void *wv,
                   int wtype, int M, int N, int K, void *k, void *q, void *v,
                   void *stream);
+/* whether that leaves the other rows of q out (a launch over two matrices and one
+ * row's product) or forms them (one launch over three): dense operands, 16-byte
+ * aligned.  Host arithmetic only: what a test can pin. */
+int vkl_kqv_last_apart (int wtype, int M, int N, int K);
 /* src/shaders/ffn_up_and_gate_fp16.comp */
 int vkl_ffn_upgate_f16 (const void *x, const void *wup, const void *wgate,
                         int M, int N, int K, void *out, void *stream);

@@ -11,9 +11,14 @@ torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("M", [1, 2, 70, 639, 640, 700, 1025])
-@pytest.mark.parametrize("wtype,N,K", [(1, 1152, 1024), (1, 1160, 1064), (1, 1150, 1030), (8, 1152, 1024), (8, 1160, 1056),
-                                       (8, 1154, 1088)])
+FORMED = [(w, M, N, K) for w, N, K in ((1, 1152, 1024), (1, 1160, 1064), (1, 1150, 1030), (8, 1152, 1024), (8, 1160, 1056), (8, 1154, 1088))
+          for M in (1, 2, 70, 639, 700, 1025)] + [(8, 768, 1024, 1024)]
+# rows that end inside a tile, columns too
+LEFT_OUT = [(1, 641, 4096, 512), (1, 515, 4104, 640), (1, 1300, 2056, 576), (1, 3001, 1152, 1024), (8, 257, 4104, 576), (8, 1025, 1160, 512),
+            (8, 641, 2176, 512), (8, 1500, 1152, 1024)]
+
+
+@pytest.mark.parametrize("wtype,M,N,K", FORMED + LEFT_OUT)
 def test_kqv_last(dev, wtype, M, N, K):
     rng = np.random.default_rng(M * 7 + N + K)
     x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float16)).cuda()

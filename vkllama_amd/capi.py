@@ -74,6 +74,7 @@ SIGNATURES = {
     "vkl_gemm_plan": (i32, [i32, i32, i32, i32, i32, i32, sz, C.POINTER(GemmPlan)]),
     "vkl_kqv_q8_0": (i32, [vp, vp, vp, vp, i32, i32, i32, vp, vp, vp, vp]),
     "vkl_kqv_last": (i32, [vp, vp, vp, vp, i32, i32, i32, i32, vp, vp, vp, vp]),
+    "vkl_kqv_last_apart": (i32, [i32, i32, i32, i32]),
     "vkl_kqv_f16": (i32, [vp, vp, vp, vp, i32, i32, i32, vp, vp, vp, vp]),
     "vkl_ffn_upgate_q8_0": (i32, [vp, vp, vp, i32, i32, i32, vp, vp]),
     "vkl_rope_kvwrite_f16": (i32, [vp, vp, vp, i32, i32, i32, sz, i32, i32, u32, u32, vp, vp, i32, vp, vp, i32, vp]),

@@ -119,6 +119,7 @@ size_t gemm_mfma_workspace_bytes (const GemmArgs &a);
 // where it applies.
 bool gemm_wide_supported (const GemmArgs &a);
 void gemm_wide_choice (const GemmArgs &a, int *tile_rows, int *ksplit); // tile_rows 0: another form
+double gemm_wide_us (const GemmArgs &a); // modelled time of its tiles (0: another form)
 int gemm_wide_launch (const GemmArgs &a, hipStream_t s);
 size_t gemm_wide_workspace_bytes (const GemmArgs &a); // fp32 scratch of its k-split (0: none)
 // At most 96 token rows against many rows of Q8_0 weights, each workgroup over

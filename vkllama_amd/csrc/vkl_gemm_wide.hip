@@ -2156,6 +2156,26 @@ gemm_wide_choice (const GemmArgs &a, int *tile_rows, int *ksplit)
   *tile_rows = p.bm, *ksplit = p.bm ? p.ksplit : 1;
 }
 
+// The time of the tiles by mix_time.  Q8_0 in tiles of 128 rows, which that does not know, takes 0.65 of 256 rows (us of one round: 2048 wide
+// 27.6 / 42.2, 1024 wide 16.7 / 25.5).
+double
+gemm_wide_us (const GemmArgs &a)
+{
+  const WidePlan p = wide_plan (a);
+  if (!p.bm)
+    return 0;
+  const int tiles_m = (a.M + p.bm - 1) / p.bm, tiles_n = (a.N + (a.upgate ? 63 : 127)) / (a.upgate ? 64 : 128), mats = a.upgate ? 1 : a.nmat;
+  const double steps = (double)(a.K / WBK) / p.ksplit;
+  if (a.wtype == 8 && p.bm == 128)
+    {
+      const MixTime t = mix_time (WBM, 1, false, true);
+      return (wide_tiles (a, p.bm) * p.ksplit + WideGrid::kUnits - 1) / WideGrid::kUnits * 0.65 * (t.step * steps + t.start);
+    }
+  double us = 0;
+  WideMix (p.bm, tiles_m, tiles_n, mats, p.ksplit, steps, 0, &us, a.wtype == 8);
+  return us;
+}
+
 size_t
 gemm_wide_workspace_bytes (const GemmArgs &a)
 {

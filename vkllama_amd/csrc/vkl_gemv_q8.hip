@@ -209,13 +209,8 @@ fill_common (GemvQ8Args &a, const void *x, int M, int N, int K, size_t xs,
   return 0;
 }
 
-// From when on vkl_kqv_last leaves the other rows of q out: a product over two matrices and one row's, us of three
-// matrices / of this, weights that no cache holds.  fp16: 4096 wide 2048 rows 165.7 / 119.0, 700 86.4 / 59.8; 5120 wide
-// 1000 rows 134.2 / 123.8, 512 rows 76.1 / 81.9; 512 wide 3000 rows 11.4 / 10.5, 2048 rows 7.9 / 8.9.  Q8_0: 5120
-// wide 3967 rows 772.4 / 514.9, 1000 185.6 / 185.4, 512 108.3 / 110.8; 2048 wide 700 rows 41.2 / 31.1.  Below these
-// the second launch, and tiles that leave half of the compute units idle, cost what the rows save.
-constexpr int kLastMinRows = 640;
-constexpr double kLastMinWork = 7e8; // multiply-adds of one matrix
+// What the product of one row of q costs vkl_kqv_last beside the tiles of two matrices in place of three, see last_apart.
+constexpr double kLastRow = 4.5;
 
 // the same problem on the matrix cores when there are enough token rows
 // the problem as the matrix-core launcher takes it
@@ -351,12 +346,34 @@ vkl_kqv_q8_0 (const void *x, const void *wk, const void *wq, const void *wv,
   return launch<1, 3> (a, (hipStream_t)stream);
 }
 
-extern "C" int
-vkl_kqv_last (const void *x, const void *wk, const void *wq, const void *wv, int wtype, int M, int N, int K, void *k,
-              void *q, void *v, void *stream)
+namespace
 {
-  VKL_CHECK_ARG (x && wk && wq && wv && k && q && v && M > 0 && N > 0 && K > 0 && (wtype == 8 || wtype == 1));
-  vkl::GemmArgs g = {};
+// Whether the other rows of q are left out: k and v by one launch over two matrices, one row of q by another.  They are where both forms run
+// on the direct-to-LDS tiles and the tiles save more than the second launch costs: 480 products of 512 to 8192 wide and 256 to
+// 4000 rows take 1.009 of the better form's time in the mean and none is slower than with three matrices (240 of them fitted).  What counts is how
+// the tiles fill their rounds over the compute units: us, three matrices / this, weights that no cache holds, fp16 4096 wide 2048 rows
+// 165.7 / 119.0, 640 60.6 / 57.8, 272 47.8 / 39.9, 2560 wide 967 39.2 / 41.6 (three matrices), 1024 wide 768 9.9 / 10.9 (three); Q8_0
+// 5120 wide 3967 rows 772.4 / 514.9, 4096 wide 640 89.6 / 80.0, 1024 wide 768 16.6 / 30.1 (three: two have too few tiles for
+// that form).  From 640 rows and 7e8 multiply-adds on, the rule before, 73 of 290 were slower.
+bool
+last_apart (vkl::GemmArgs two)
+{
+  // (the last rows are aligned as the first ones are)
+  if ((two.K % 8) != 0 || (two.N % 8) != 0 || !vkl::gemm_mfma_supported (two))
+    return false;
+  vkl::GemmArgs three = two;
+  three.nmat = 3;
+  three.wq[2] = two.wq[1], three.wd[2] = two.wd[1], three.wh[2] = two.wh[1], three.y[2] = two.y[1];
+  if (vkl::gemm_plan (two).family != vkl::GEMM_WIDE || vkl::gemm_plan (three).family != vkl::GEMM_WIDE)
+    return false;
+  return vkl::gemm_wide_us (two) + kLastRow < vkl::gemm_wide_us (three);
+}
+
+// the product over wk and wv
+int
+last_args (const void *x, const void *wk, const void *wv, int wtype, int M, int N, int K, void *k, void *v, vkl::GemmArgs &g)
+{
+  g = {};
   if (wtype == 8)
     {
       GemvQ8Args a = {};
@@ -365,21 +382,40 @@ vkl_kqv_last (const void *x, const void *wk, const void *wq, const void *wv, int
       set_mat (a, 0, wk, k);
       set_mat (a, 1, wv, v);
       g = gemm_args (a, 2, 0);
+      return 0;
     }
-  else
-    {
-      g.x = (const uint16_t *)x, g.xs = (size_t)K;
-      g.M = M, g.N = N, g.K = K, g.Kp = (K + 31) / 32 * 32;
-      g.wtype = 1, g.nmat = 2;
-      g.wh[0] = (const uint16_t *)wk, g.wh[1] = (const uint16_t *)wv;
-      g.ws = (size_t)K;
-      g.y[0] = (uint16_t *)k, g.y[1] = (uint16_t *)v;
-      g.ys = (size_t)N;
-      g.scale = 1.f;
-    }
-  // (the last rows are aligned as the first ones are)
-  if (M < kLastMinRows || (double)M * N * K < kLastMinWork || (K % 8) != 0 || (N % 8) != 0
-      || !vkl::gemm_mfma_supported (g))
+  g.x = (const uint16_t *)x, g.xs = (size_t)K;
+  g.M = M, g.N = N, g.K = K, g.Kp = (K + 31) / 32 * 32;
+  g.wtype = 1, g.nmat = 2;
+  g.wh[0] = (const uint16_t *)wk, g.wh[1] = (const uint16_t *)wv;
+  g.ws = (size_t)K;
+  g.y[0] = (uint16_t *)k, g.y[1] = (uint16_t *)v;
+  g.ys = (size_t)N;
+  g.scale = 1.f;
+  return 0;
+}
+} // namespace
+
+extern "C" int
+vkl_kqv_last_apart (int wtype, int M, int N, int K)
+{
+  if (M <= 0 || N <= 0 || K <= 0 || (wtype != 8 && wtype != 1))
+    return 0;
+  // (an address that fits, which nothing follows)
+  void *any = (void *)(uintptr_t)4096;
+  vkl::GemmArgs g;
+  return last_args (any, any, any, wtype, M, N, K, any, any, g) == 0 && last_apart (g);
+}
+
+extern "C" int
+vkl_kqv_last (const void *x, const void *wk, const void *wq, const void *wv, int wtype, int M, int N, int K, void *k,
+              void *q, void *v, void *stream)
+{
+  VKL_CHECK_ARG (x && wk && wq && wv && k && q && v && M > 0 && N > 0 && K > 0 && (wtype == 8 || wtype == 1));
+  vkl::GemmArgs g;
+  if (int e = last_args (x, wk, wv, wtype, M, N, K, k, v, g))
+    return e;
+  if (!last_apart (g))
     return (wtype == 8 ? vkl_kqv_q8_0 : vkl_kqv_f16) (x, wk, wq, wv, M, N, K, k, q, v, stream);
   if (int e = vkl::gemm_mfma_launch (g, (hipStream_t)stream))
     return e;

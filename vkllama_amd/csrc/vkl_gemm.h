@@ -10,8 +10,9 @@
 
 namespace vkl
 {
-// (host) the RMS norm that follows a product; the launch that adds the parts of a divided k range
-// forms it too, where there is one
+// (host) the RMS norm that follows a plain product with a dense y; the launch that adds the parts of a divided k range
+// forms it too, where there is one.  Not among the arguments below, which every kernel fetches: eight bytes more there took small
+// products 0.2 us longer (bf16 64 x 2048 x 512 5.6 / 5.8).
 struct GemmNorm
 {
   const float *w;
@@ -44,7 +45,6 @@ struct GemmArgs
   // per-stream buffer, allocated on first use
   float *workspace;
   size_t workspace_bytes; // size of `workspace` (checked before every use)
-  GemmNorm *norm;         // optional, host memory: one plain product with a dense y
 };
 
 // A product whose output columns fall into segments, each with a destination, a
@@ -72,6 +72,7 @@ struct GemmSegArgs : GemmArgs
   int nseg;
   GemmSeg seg[kGemmSegs];
 };
+static_assert (sizeof (GemmArgs) <= 232 && sizeof (GemmSegArgs) <= 440, "every kernel fetches them, see GemmNorm");
 // the fp32 product (vkl_gemm_f32.hip) and the bf16 one (vkl_gemm_wide.hip)
 int gemm_f32_launch (const GemmSegArgs &a, hipStream_t s);
 int gemm_wide_bf16_launch (const GemmSegArgs &a, hipStream_t s);
@@ -111,7 +112,7 @@ struct GemmPlan
   size_t workspace_bytes;
 };
 GemmPlan gemm_plan (const GemmArgs &a);
-int gemm_mfma_launch (const GemmArgs &a, hipStream_t s);
+int gemm_mfma_launch (const GemmArgs &a, hipStream_t s, GemmNorm *norm = nullptr);
 // bytes of fp32 scratch gemm_mfma_launch will use for this problem (0: none)
 size_t gemm_mfma_workspace_bytes (const GemmArgs &a);
 // Many token rows against dense fp16 weights: 256-row tiles staged by
@@ -120,7 +121,7 @@ size_t gemm_mfma_workspace_bytes (const GemmArgs &a);
 bool gemm_wide_supported (const GemmArgs &a);
 void gemm_wide_choice (const GemmArgs &a, int *tile_rows, int *ksplit); // tile_rows 0: another form
 double gemm_wide_us (const GemmArgs &a); // modelled time of its tiles (0: another form)
-int gemm_wide_launch (const GemmArgs &a, hipStream_t s);
+int gemm_wide_launch (const GemmArgs &a, hipStream_t s, GemmNorm *norm = nullptr);
 size_t gemm_wide_workspace_bytes (const GemmArgs &a); // fp32 scratch of its k-split (0: none)
 // At most 96 token rows against many rows of Q8_0 weights, each workgroup over
 // the whole of K: no partial sums (vkl_gemm_rowsfull.hip).
@@ -155,7 +156,7 @@ private:
   ScratchEntry *held_ = nullptr;
 };
 // adds `parts` partial results of `rows` rows each in order and applies the epilogue
-int gemm_reduce_parts (const GemmArgs &a, const float *ws, int parts, int rows, hipStream_t s);
+int gemm_reduce_parts (const GemmArgs &a, const float *ws, int parts, int rows, hipStream_t s, GemmNorm *norm = nullptr);
 // frees the scratch buffer that launches on this stream allocated (the
 // stream must be idle); called when a stream is destroyed
 void gemm_release_workspace (hipStream_t s);

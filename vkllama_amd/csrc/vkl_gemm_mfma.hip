@@ -1147,9 +1147,8 @@ constexpr int kRowNormWork = 36, kWideRowNormWork = 16;
 
 // adds the parts of a product, of which each lies `rows` rows behind the one before
 int
-launch_reduce (const GemmArgs &a, const float *ws, int parts, int rows, hipStream_t s)
+launch_reduce (const GemmArgs &a, const float *ws, int parts, int rows, hipStream_t s, GemmNorm *n)
 {
-  GemmNorm *n = a.norm;
   const auto mis = [] (const void *p) { return ((uintptr_t)p % 16) != 0; };
   const int vec = a.N <= 2048 ? 1 : a.N <= 4096 ? 2 : a.N <= 6144 ? 3 : 4;
   if (n && a.nmat == 1 && !a.upgate && a.scale == 1.f && a.bias == 0.f && a.act == 0 && !a.y32 && (a.N % 8) == 0 && a.N <= 8192
@@ -1202,7 +1201,7 @@ skinny2_prepare (size_t lds)
 
 // the whole-line form for Q8_0 weights
 bool
-launch_rows64_q8 (const GemmArgs &a, hipStream_t s, int &err)
+launch_rows64_q8 (const GemmArgs &a, hipStream_t s, GemmNorm *norm, int &err)
 {
   if (a.wtype != 8 || a.M > 32 || a.batch > 1)
     return false;
@@ -1227,13 +1226,13 @@ launch_rows64_q8 (const GemmArgs &a, hipStream_t s, int &err)
   else
     gemm_rows64_q8_kernel<<<dim3 ((unsigned)S, (unsigned)((a.N + 63) / 64), (unsigned)nm),
                             dim3 (kR64Waves * 64), kR64Lds, s>>> (a, ws, S);
-  err = launch_reduce (a, ws, S, 32, s);
+  err = launch_reduce (a, ws, S, 32, s, norm);
   return true;
 }
 
 template <int WT>
 bool
-launch_skinny2 (const GemmArgs &a, hipStream_t s, int &err)
+launch_skinny2 (const GemmArgs &a, hipStream_t s, GemmNorm *norm, int &err)
 {
   if (a.M > 32 || a.batch > 1)
     return false;
@@ -1251,7 +1250,7 @@ launch_skinny2 (const GemmArgs &a, hipStream_t s, int &err)
     return false;
   gemm_skinny2_kernel<WT><<<dim3 ((unsigned)S, (unsigned)((a.N + 31) / 32), (unsigned)nm),
                            dim3 (kSk2Waves * 64), lds, s>>> (a, ws, S);
-  err = launch_reduce (a, ws, S, 32, s);
+  err = launch_reduce (a, ws, S, 32, s, norm);
   return true;
 }
 
@@ -1280,7 +1279,7 @@ tile_ksplit (const GemmArgs &a)
 
 template <int BM, int WT>
 int
-launch_cfg (const GemmArgs &a, int ksplit, hipStream_t s)
+launch_cfg (const GemmArgs &a, int ksplit, hipStream_t s, GemmNorm *norm)
 {
   const int tiles_m = (a.M + BM - 1) / BM;
   const int tiles_n = (a.N + (a.upgate ? 64 : BN) - 1) / (a.upgate ? 64 : BN);
@@ -1300,7 +1299,7 @@ launch_cfg (const GemmArgs &a, int ksplit, hipStream_t s)
                (unsigned)nz),
          dim3 (kGemmThreads), 0, s>>> (a, tiles_m, tiles_n, per_xcd, ksplit, ws);
   if (ksplit > 1)
-    return launch_reduce (a, ws, ksplit, a.M, s);
+    return launch_reduce (a, ws, ksplit, a.M, s, norm);
   return (int)hipGetLastError ();
 }
 } // namespace
@@ -1437,9 +1436,9 @@ StreamScratch::bytes ()
 }
 
 int
-gemm_reduce_parts (const GemmArgs &a, const float *ws, int parts, int rows, hipStream_t s)
+gemm_reduce_parts (const GemmArgs &a, const float *ws, int parts, int rows, hipStream_t s, GemmNorm *norm)
 {
-  return launch_reduce (a, ws, parts, rows, s);
+  return launch_reduce (a, ws, parts, rows, s, norm);
 }
 
 bool
@@ -1555,7 +1554,7 @@ gemm_plan (const GemmArgs &a)
 }
 
 int
-gemm_mfma_launch (const GemmArgs &a, hipStream_t s)
+gemm_mfma_launch (const GemmArgs &a, hipStream_t s, GemmNorm *norm)
 {
   const GemmPlan p = gemm_plan (a);
   int err = 0;
@@ -1565,23 +1564,23 @@ gemm_mfma_launch (const GemmArgs &a, hipStream_t s)
       return gemm_rowsfull_launch (a, s);
     case GEMM_ROWS128:
     case GEMM_ROWS64:
-      if (launch_rows64_q8 (a, s, err))
+      if (launch_rows64_q8 (a, s, norm, err))
         return err;
       break;
     case GEMM_SLICES:
-      if (a.wtype == 8 ? launch_skinny2<8> (a, s, err) : launch_skinny2<1> (a, s, err))
+      if (a.wtype == 8 ? launch_skinny2<8> (a, s, norm, err) : launch_skinny2<1> (a, s, norm, err))
         return err;
       break;
     case GEMM_WIDE:
-      return gemm_wide_launch (a, s);
+      return gemm_wide_launch (a, s, norm);
     case GEMM_TILE:
       {
         const bool small = p.tile_rows == 64;
         if (a.wtype == 8)
-          return small ? launch_cfg<64, 8> (a, p.ksplit, s) : launch_cfg<128, 8> (a, p.ksplit, s);
+          return small ? launch_cfg<64, 8> (a, p.ksplit, s, norm) : launch_cfg<128, 8> (a, p.ksplit, s, norm);
         if (a.wtype == 2)
-          return small ? launch_cfg<64, 2> (a, p.ksplit, s) : launch_cfg<128, 2> (a, p.ksplit, s);
-        return small ? launch_cfg<64, 1> (a, p.ksplit, s) : launch_cfg<128, 1> (a, p.ksplit, s);
+          return small ? launch_cfg<64, 2> (a, p.ksplit, s, norm) : launch_cfg<128, 2> (a, p.ksplit, s, norm);
+        return small ? launch_cfg<64, 1> (a, p.ksplit, s, norm) : launch_cfg<128, 1> (a, p.ksplit, s, norm);
       }
     default:
       return (int)hipErrorInvalidValue;

@@ -2184,7 +2184,7 @@ gemm_wide_workspace_bytes (const GemmArgs &a)
 }
 
 int
-gemm_wide_launch (const GemmArgs &a, hipStream_t s)
+gemm_wide_launch (const GemmArgs &a, hipStream_t s, GemmNorm *norm)
 {
   constexpr size_t m256 = mix_lds<256> (), m128 = mix_lds<128> ();
   constexpr size_t qmix = mix_lds_q8 (), q256 = wide_lds_q8<256> (), q128 = wide_lds_q8<128> ();
@@ -2255,7 +2255,7 @@ gemm_wide_launch (const GemmArgs &a, hipStream_t s)
   else
     gemm_mix_kernel<128, false, GemmArgs><<<grid, block, m128, s>>> (a, mix, vec, ksplit, ws);
   if (ksplit > 1)
-    return gemm_reduce_parts (a, ws, ksplit, a.M, s);
+    return gemm_reduce_parts (a, ws, ksplit, a.M, s, norm);
   return (int)hipGetLastError ();
 }
 

@@ -236,10 +236,10 @@ try_gemm (const GemvQ8Args &a, int nmat, int upgate, hipStream_t s, int &err,
   if (a.M < vkl::kGemmMinRows)
     return false;
   vkl::GemmArgs g = gemm_args (a, nmat, upgate);
-  g.workspace = workspace, g.workspace_bytes = workspace_bytes, g.norm = norm;
+  g.workspace = workspace, g.workspace_bytes = workspace_bytes;
   if (!vkl::gemm_mfma_supported (g))
     return false;
-  err = vkl::gemm_mfma_launch (g, s);
+  err = vkl::gemm_mfma_launch (g, s, norm);
   return true;
 }
 

@@ -193,9 +193,9 @@ matmul_f16_tb (const void *a, const void *b, int C, int M, int N, int K, size_t 
       g.y[0] = g.y[1] = g.y[2] = p.y;
       g.ys = yhs;
       g.scale = scale, g.bias = bias, g.act = act;
-      g.residual = p.residual, g.y32 = y32, g.norm = norm;
+      g.residual = p.residual, g.y32 = y32;
       if (vkl::gemm_mfma_supported (g))
-        return vkl::gemm_mfma_launch (g, (hipStream_t)stream);
+        return vkl::gemm_mfma_launch (g, (hipStream_t)stream, norm);
     }
   return launch_tb (p, false, (hipStream_t)stream);
 }
